@@ -7,7 +7,7 @@ import torch
 import torch.nn.functional as F
 
 from wtconv_amd import _lib
-from wtconv_amd.wavelet import _Haar, _prep
+from wtconv_amd.wavelet import _haar, _prep
 
 MAX_KERNEL_SIZE = 7             # wtconv_max_kernel_size() of the built library (haar_cuda.py:62: the default ceiling)
 HARD_MAX_KERNEL_SIZE = 7        # the kernels are instantiated for K = 1, 3, 5, 7; nothing larger can be built in
@@ -28,12 +28,12 @@ def haar2d(x: torch.Tensor) -> torch.Tensor:
     x = _prep(x, 4, "haar2d")
     if x.shape[2] % 2 or x.shape[3] % 2:
         x = F.pad(x, (0, x.shape[3] % 2, 0, x.shape[2] % 2))
-    return _Haar.apply(x, 2, False)
+    return _haar(x, 2, False)
 
 
 def ihaar2d(x: torch.Tensor, output_size=None) -> torch.Tensor:
     """(B, C, 4, h, w) -> (B, C, 2h, 2w), cropped to `output_size` (H, W) if given (haar_cuda.py:536-537)."""
-    out = _Haar.apply(_prep(x, 5, "ihaar2d"), 2, True)
+    out = _haar(_prep(x, 5, "ihaar2d"), 2, True)
     if output_size is not None:
         out = out[:, :, :output_size[0], :output_size[1]]
     return out

@@ -211,6 +211,15 @@ int wtconv_block_residual_backward(const void* dout, const void* y, const void* 
 int wtconv_haar2d(const void* x, void* out, long long planes, int H, int W, int dtype, int inverse, void* stream);
 int wtconv_haar1d(const void* x, void* out, long long rows, int N, int dtype, int inverse, void* stream);
 
+/* The same with the filter bank that the caller was given: the launch compares the taps of its first channel (device
+ * memory, `bank_dtype`; 4 x 2 x 2 or 2 x 2 values) with db1's and stores 1 (they are) or 2 (they are not) in *verdict,
+ * a word of pinned, coherent host memory that the caller has cleared.  It is written early in the kernel, before the
+ * transform is complete; whatever the verdict, the transform computed is db1's. */
+int wtconv_haar2d_checked(const void* x, void* out, long long planes, int H, int W, int dtype, int inverse,
+                          const void* bank, int bank_dtype, unsigned* verdict, void* stream);
+int wtconv_haar1d_checked(const void* x, void* out, long long rows, int N, int dtype, int inverse,
+                          const void* bank, int bank_dtype, unsigned* verdict, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

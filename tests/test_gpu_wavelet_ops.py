@@ -95,3 +95,33 @@ def test_fast_twin_haar_utilities(hip_device):
         H.check_kernel_size(9)
     with pytest.raises(ValueError):
         H.check_kernel_size(4)
+
+
+@pytest.mark.parametrize("dims", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_bank_in_gpu_memory_is_checked_by_the_launch(hip_device, dims, dtype):
+    """db1 banks pass in every dtype; one wrong tap, a NaN or a swapped filter is refused (float64 and strided banks
+    take the check on the host)."""
+    from wtconv.util import wavelet as Wv
+    create = Wv.create_2d_wavelet_filter if dims == 2 else Wv.create_1d_wavelet_filter
+    fwd = Wv.wavelet_2d_transform if dims == 2 else Wv.wavelet_1d_transform
+    inv = Wv.inverse_2d_wavelet_transform if dims == 2 else Wv.inverse_1d_wavelet_transform
+    x = torch.randn((2, 3, 6, 8) if dims == 2 else (2, 3, 8), device=hip_device)
+    dec = create("db1", 3, 3)[0].to(device=hip_device, dtype=dtype)
+    want = fwd(x, create("db1", 3, 3)[0])
+    assert torch.equal(fwd(x, dec), want)
+    strided = torch.stack([dec, dec], dim=-1)[..., 0]
+    assert not strided.is_contiguous() and torch.equal(fwd(x, strided), want)
+    torch.testing.assert_close(inv(want, dec), x, rtol=1e-5, atol=1e-5)
+    taps = 2 ** dims
+    for i in range(taps * taps):
+        bad = dec.clone()
+        bad.view(-1)[i] *= -1
+        with pytest.raises(NotImplementedError):
+            fwd(x, bad)
+    bad = dec.clone()
+    bad.view(-1)[1] = float("nan")
+    with pytest.raises(NotImplementedError):
+        inv(want, bad)
+    with pytest.raises(ValueError):
+        fwd(x, dec[1:])

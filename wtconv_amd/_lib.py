@@ -53,6 +53,8 @@ EXPORTS["wtconv_block_residual_backward"] = (_i, [_p, _p, _p, _p, _p, _i, _i, _i
 _ll = ctypes.c_longlong
 EXPORTS["wtconv_haar2d"] = (_i, [_p, _p, _ll, _i, _i, _i, _i, _p])
 EXPORTS["wtconv_haar1d"] = (_i, [_p, _p, _ll, _i, _i, _i, _p])
+EXPORTS["wtconv_haar2d_checked"] = (_i, [_p, _p, _ll, _i, _i, _i, _i, _p, _i, _p, _p])
+EXPORTS["wtconv_haar1d_checked"] = (_i, [_p, _p, _ll, _i, _i, _i, _p, _i, _p, _p])
 
 _lib = None
 _lock = threading.Lock()

@@ -35,11 +35,8 @@ dim3 unit_grid(unsigned gx, long long units) {
     else { using T_ = f16_t; CALL; }                                           \
   } while (0)
 
-}  // namespace
-
-extern "C" int wtconv_haar2d(const void* x, void* out, long long planes, int H, int W, int dtype, int inverse,
-                             void* stream_) {
-  const char* fn = "wtconv_haar2d";
+int haar2d(const char* fn, const void* x, void* out, long long planes, int H, int W, int dtype, int inverse,
+           const BankCheck& bank, void* stream_) {
   if (int e = check_haar(fn, x, out, planes, dtype)) return e;
   if (H <= 0 || W <= 0 || H % 2 || W % 2)
     return fail(WTCONV_E_ARG, "%s: the plane must have even, positive extents (got %dx%d)", fn, H, W);
@@ -50,21 +47,53 @@ extern "C" int wtconv_haar2d(const void* x, void* out, long long planes, int H, 
   const dim3 grid = unit_grid(gx, planes);
   if (inverse)
     WT_HAAR_BY_DTYPE(dtype, WT_LAUNCH(haar2d_synthesis_kernel<T_>, grid, dim3(kHaarThreads), 0, stream,
-                                      static_cast<const T_*>(x), static_cast<T_*>(out), h, w, planes));
+                                      static_cast<const T_*>(x), static_cast<T_*>(out), h, w, planes, bank));
   else
     WT_HAAR_BY_DTYPE(dtype, WT_LAUNCH(haar2d_analysis_kernel<T_>, grid, dim3(kHaarThreads), 0, stream,
-                                      static_cast<const T_*>(x), static_cast<T_*>(out), h, w, planes));
+                                      static_cast<const T_*>(x), static_cast<T_*>(out), h, w, planes, bank));
   return check_launch(fn);
 }
 
-extern "C" int wtconv_haar1d(const void* x, void* out, long long rows, int N, int dtype, int inverse, void* stream_) {
-  const char* fn = "wtconv_haar1d";
+int haar1d(const char* fn, const void* x, void* out, long long rows, int N, int dtype, int inverse,
+           const BankCheck& bank, void* stream_) {
   if (int e = check_haar(fn, x, out, rows, dtype)) return e;
   if (N <= 0 || N % 2) return fail(WTCONV_E_ARG, "%s: the row length must be even and positive (got %d)", fn, N);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int n = N / 2;
   const dim3 grid = unit_grid(static_cast<unsigned>((n + kHaarThreads - 1) / kHaarThreads), rows);
   WT_HAAR_BY_DTYPE(dtype, WT_LAUNCH(haar1d_kernel<T_>, grid, dim3(kHaarThreads), 0, stream, static_cast<const T_*>(x),
-                                    static_cast<T_*>(out), n, rows, inverse));
+                                    static_cast<T_*>(out), n, rows, inverse, bank));
   return check_launch(fn);
+}
+
+int check_bank_args(const char* fn, const void* bank, int bank_dtype, const unsigned* verdict) {
+  if (bank == nullptr || verdict == nullptr) return fail(WTCONV_E_ARG, "%s: null bank or verdict pointer", fn);
+  if (bank_dtype != WTCONV_F32 && bank_dtype != WTCONV_BF16 && bank_dtype != WTCONV_F16)
+    return fail(WTCONV_E_ARG, "%s: unknown bank dtype %d", fn, bank_dtype);
+  return 0;
+}
+
+}  // namespace
+
+extern "C" int wtconv_haar2d(const void* x, void* out, long long planes, int H, int W, int dtype, int inverse,
+                             void* stream) {
+  return haar2d("wtconv_haar2d", x, out, planes, H, W, dtype, inverse, BankCheck{}, stream);
+}
+
+extern "C" int wtconv_haar1d(const void* x, void* out, long long rows, int N, int dtype, int inverse, void* stream) {
+  return haar1d("wtconv_haar1d", x, out, rows, N, dtype, inverse, BankCheck{}, stream);
+}
+
+extern "C" int wtconv_haar2d_checked(const void* x, void* out, long long planes, int H, int W, int dtype, int inverse,
+                                     const void* bank, int bank_dtype, unsigned* verdict, void* stream) {
+  const char* fn = "wtconv_haar2d_checked";
+  if (int e = check_bank_args(fn, bank, bank_dtype, verdict)) return e;
+  return haar2d(fn, x, out, planes, H, W, dtype, inverse, BankCheck{bank, bank_dtype, 2, verdict}, stream);
+}
+
+extern "C" int wtconv_haar1d_checked(const void* x, void* out, long long rows, int N, int dtype, int inverse,
+                                     const void* bank, int bank_dtype, unsigned* verdict, void* stream) {
+  const char* fn = "wtconv_haar1d_checked";
+  if (int e = check_bank_args(fn, bank, bank_dtype, verdict)) return e;
+  return haar1d(fn, x, out, rows, N, dtype, inverse, BankCheck{bank, bank_dtype, 1, verdict}, stream);
 }

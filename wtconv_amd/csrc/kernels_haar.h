@@ -13,10 +13,41 @@ namespace wt {
 
 constexpr int kHaarThreads = 256;
 
+// The filter bank that came with a call, checked by the launch that computes the transform: its first thread compares
+// the taps of the first channel with db1's and leaves the verdict (kBankOk / kBankOther) in a word of host memory that
+// the caller waits for.  The word is written while the transform runs, so the caller learns it at the start of the
+// kernel: nothing is copied and the stream is not drained.  verdict == nullptr: no check.
+constexpr unsigned kBankOk = 1, kBankOther = 2;
+struct BankCheck {
+  const void* bank;      // 4 filters of 2 x 2 taps (dims == 2), or 2 filters of 2 taps
+  int dtype;
+  int dims;
+  unsigned* verdict;
+};
+
+__device__ __forceinline__ void check_bank(const BankCheck& b) {
+  if (b.verdict == nullptr || (blockIdx.x | blockIdx.y | blockIdx.z | threadIdx.x) != 0) return;
+  const int n = b.dims == 2 ? 16 : 4;
+  const float tap = b.dims == 2 ? 0.5f : 0.70710678118654752440f;
+  bool ok = true;
+  for (int i = 0; i < n; ++i) {
+    // filter s = i / taps; its sign flips along rows for bit 0 of s, along columns for bit 1 (1-D: along the row)
+    const int neg = b.dims == 2 ? (((i >> 2) & (i >> 1)) ^ ((i >> 3) & i)) & 1 : (i >> 1) & i & 1;
+    const float v = load_param(b.bank, b.dtype, i);
+    ok = ok && fabsf(v - (neg ? -tap : tap)) <= 4e-3f;      // (bf16 banks pass, NaN does not)
+  }
+#ifdef WT_EMULATE
+  *b.verdict = ok ? kBankOk : kBankOther;
+#else
+  __hip_atomic_store(b.verdict, ok ? kBankOk : kBankOther, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#endif
+}
+
 // x (planes, H, W) -> out (planes, 4, H/2, W/2).  Grid (ceil(h * ceil(w / 2) / 256), planes folded into y and z).
 template <typename T>
 __global__ void __launch_bounds__(kHaarThreads)
-haar2d_analysis_kernel(const T* __restrict__ x, T* __restrict__ out, int h, int w, long long planes) {
+haar2d_analysis_kernel(const T* __restrict__ x, T* __restrict__ out, int h, int w, long long planes, BankCheck bank) {
+  check_bank(bank);
   const long long plane = static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y;
   if (plane >= planes) return;
   const int wp = (w + 1) >> 1;                       // pairs of coefficient columns per row
@@ -42,7 +73,8 @@ haar2d_analysis_kernel(const T* __restrict__ x, T* __restrict__ out, int h, int 
 // coef (planes, 4, h, w) -> out (planes, 2h, 2w)
 template <typename T>
 __global__ void __launch_bounds__(kHaarThreads)
-haar2d_synthesis_kernel(const T* __restrict__ coef, T* __restrict__ out, int h, int w, long long planes) {
+haar2d_synthesis_kernel(const T* __restrict__ coef, T* __restrict__ out, int h, int w, long long planes, BankCheck bank) {
+  check_bank(bank);
   const long long plane = static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y;
   if (plane >= planes) return;
   const int wp = (w + 1) >> 1;
@@ -69,7 +101,8 @@ haar2d_synthesis_kernel(const T* __restrict__ coef, T* __restrict__ out, int h, 
 // folded into y and z).
 template <typename T>
 __global__ void __launch_bounds__(kHaarThreads)
-haar1d_kernel(const T* __restrict__ x, T* __restrict__ out, int n, long long rows, int inverse) {
+haar1d_kernel(const T* __restrict__ x, T* __restrict__ out, int n, long long rows, int inverse, BankCheck bank) {
+  check_bank(bank);
   const long long row = static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y;
   if (row >= rows) return;
   const int q = blockIdx.x * kHaarThreads + threadIdx.x;

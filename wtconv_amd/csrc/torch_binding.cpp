@@ -14,9 +14,12 @@
 
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 
+#include <chrono>
+#include <mutex>
 #include <optional>
 #include <vector>
 
@@ -45,6 +48,10 @@ struct Abi {
                  int, void*, size_t, void*);
   size_t (*ws1)(int, int, int, int, int, int);
   const char* (*last_error)();
+  int (*haar2)(const void*, void*, long long, int, int, int, int, void*);
+  int (*haar1)(const void*, void*, long long, int, int, int, void*);
+  int (*haar2c)(const void*, void*, long long, int, int, int, int, const void*, int, unsigned*, void*);
+  int (*haar1c)(const void*, void*, long long, int, int, int, const void*, int, unsigned*, void*);
   bool bound = false;
 } abi;
 
@@ -53,10 +60,11 @@ void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 11, "bind: expected 11 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 15, "bind: expected 15 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
+  take(abi.haar2, a[11]); take(abi.haar1, a[12]); take(abi.haar2c, a[13]); take(abi.haar1c, a[14]);
   abi.bound = true;
 }
 
@@ -264,9 +272,137 @@ py::object layer(const Tensor& x, const Tensor& base_w, const std::optional<Tens
   return py::cast(out);
 }
 
+// ---- the single-level Haar transforms (wtconv_amd/wavelet.py), with the check of the filter bank they are handed.
+
+// Words of pinned host memory that a kernel writes its verdict into while the caller waits: one page, taken when the
+// first bank is checked, its words lent for one call each.
+class VerdictPool {
+ public:
+  unsigned* lend() {
+    const std::lock_guard<std::mutex> lock(m_);
+    if (page_ == nullptr) {
+      if (hipHostMalloc(reinterpret_cast<void**>(&page_), kWords * kStride * sizeof(unsigned),
+                        hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        page_ = nullptr;
+        return nullptr;
+      }
+      for (int i = 0; i < kWords; ++i) free_.push_back(page_ + i * kStride);
+    }
+    if (free_.empty()) return nullptr;
+    unsigned* w = free_.back();
+    free_.pop_back();
+    *static_cast<volatile unsigned*>(w) = 0u;
+    return w;
+  }
+  void give_back(unsigned* w) {
+    const std::lock_guard<std::mutex> lock(m_);
+    free_.push_back(w);
+  }
+
+ private:
+  static constexpr int kWords = 64, kStride = 16;      // a cache line each
+  std::mutex m_;
+  unsigned* page_ = nullptr;
+  std::vector<unsigned*> free_;
+};
+VerdictPool verdicts;
+
+// Waits for the kernel that writes *w.  It writes early, so this is a short spin; should nothing arrive in two seconds
+// (a long queue ahead of it on the stream), the stream is waited for instead.
+unsigned await_verdict(const unsigned* w, hipStream_t stream) {
+  const volatile unsigned* v = w;
+  const auto begin = std::chrono::steady_clock::now();
+  for (unsigned spins = 0;; ++spins) {
+    if (const unsigned got = *v) return got;
+    __builtin_ia32_pause();
+    if ((spins & 0xfffu) == 0xfffu && std::chrono::steady_clock::now() - begin > std::chrono::seconds(2)) break;
+  }
+  TORCH_CHECK(hipStreamSynchronize(stream) == hipSuccess, "the stream failed while a filter bank was being checked");
+  return *v;
+}
+
+class HaarNode : public torch::autograd::Function<HaarNode> {
+ public:
+  // bank / verdict: addresses (0 = no check)
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, int64_t dims, bool inverse, int64_t bank,
+                        int64_t bank_dtype, int64_t verdict) {
+    ctx->saved_data["dims"] = dims;
+    ctx->saved_data["inverse"] = inverse;
+    const c10::DeviceGuard guard(x.device());
+    const int64_t b = x.size(0), c = x.size(1);
+    const int64_t h = dims == 2 ? (inverse ? 2 * x.size(3) : x.size(2)) : 1;
+    const int64_t w = inverse ? 2 * x.size(dims == 2 ? 4 : 3) : x.size(dims == 2 ? 3 : 2);
+    Tensor out = dims == 2 ? (inverse ? at::empty({b, c, h, w}, x.options()) : at::empty({b, c, 4, h / 2, w / 2}, x.options()))
+                           : (inverse ? at::empty({b, c, w}, x.options()) : at::empty({b, c, 2, w / 2}, x.options()));
+    void* stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+    const int dt = dtype_code(x.scalar_type());
+    int rc;
+    if (verdict == 0)
+      rc = dims == 2 ? abi.haar2(x.data_ptr(), out.data_ptr(), b * c, h, w, dt, inverse, stream)
+                     : abi.haar1(x.data_ptr(), out.data_ptr(), b * c, w, dt, inverse, stream);
+    else
+      rc = dims == 2 ? abi.haar2c(x.data_ptr(), out.data_ptr(), b * c, h, w, dt, inverse, reinterpret_cast<const void*>(bank),
+                                  bank_dtype, reinterpret_cast<unsigned*>(verdict), stream)
+                     : abi.haar1c(x.data_ptr(), out.data_ptr(), b * c, w, dt, inverse, reinterpret_cast<const void*>(bank),
+                                  bank_dtype, reinterpret_cast<unsigned*>(verdict), stream);
+    if (rc) fail(rc, "wtconv haar");
+    return out;
+  }
+
+  // The transforms are orthogonal: each one's backward is the other.
+  static variable_list backward(AutogradContext* ctx, variable_list grad_outputs) {
+    variable_list res(6);
+    if (grad_outputs[0].defined())
+      res[0] = HaarNode::apply(grad_outputs[0].contiguous(), ctx->saved_data["dims"].toInt(),
+                               !ctx->saved_data["inverse"].toBool(), int64_t{0}, int64_t{0}, int64_t{0});
+    return res;
+  }
+};
+
+// The transform of a contiguous GPU tensor.  With a bank: the result if it is db1's, False if it is another one, None
+// if it is not one that a kernel can look at (host memory, another dtype, strided) and nothing was done.
+py::object haar(const Tensor& x, const std::optional<Tensor>& bank, int64_t dims, bool inverse) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (!bank.has_value()) {
+    Tensor out;
+    {
+      py::gil_scoped_release nogil;
+      out = HaarNode::apply(x, dims, inverse, int64_t{0}, int64_t{0}, int64_t{0});
+    }
+    return py::cast(out);
+  }
+  const int bdt = dtype_code(bank->scalar_type());
+  if (bdt < 0 || bank->device() != x.device() || !bank->is_contiguous() || x.numel() == 0) return py::none();
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  TORCH_CHECK(hipStreamIsCapturing(stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone,
+              "a filter bank in GPU memory cannot be checked while the stream is being captured");
+  unsigned* w = verdicts.lend();
+  if (w == nullptr) return py::none();
+  Tensor out;
+  unsigned got;
+  {
+    py::gil_scoped_release nogil;
+    // (an exception of the launch itself leaves nothing that would write the word)
+    try {
+      out = HaarNode::apply(x, dims, inverse, reinterpret_cast<int64_t>(bank->data_ptr()), int64_t{bdt},
+                            reinterpret_cast<int64_t>(w));
+    } catch (...) {
+      verdicts.give_back(w);
+      throw;
+    }
+    got = await_verdict(w, stream);
+    verdicts.give_back(w);
+  }
+  if (got != 1u) return py::bool_(false);
+  return py::cast(out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind, "hand over the addresses of the C-ABI entry points");
   m.def("layer", &layer, "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical");
+  m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }

@@ -10,7 +10,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _ext, _lib
 
 _R = 0.7071067811865476
 _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
@@ -44,16 +44,40 @@ def create_2d_wavelet_filter(wave, in_size, out_size, type=torch.float):
     return bank(dlo, dhi, in_size), bank(rlo, rhi, out_size)
 
 
-def _check_bank(filters, channels, dims):
+def _refuse_bank():
+    raise NotImplementedError("only the Haar (db1) filter bank is supported by the HIP transforms")
+
+
+def _check_bank(filters, dims):
     """The kernels compute the db1 transform whatever `filters` holds, so anything else must be refused."""
     S = 4 if dims == 2 else 2
-    shape = (S * channels, 1, 2, 2) if dims == 2 else (S * channels, 1, 2)
-    if tuple(filters.shape) != shape:
-        raise ValueError(f"filters of shape {tuple(filters.shape)}: expected the db1 bank {shape}")
     ref = (create_2d_wavelet_filter if dims == 2 else create_1d_wavelet_filter)("db1", 1, 1, torch.float32)[0]
     got = filters[:S].detach().to(device="cpu", dtype=torch.float32)      # (a few values: the first channel's bank)
     if not torch.allclose(got, ref, rtol=0, atol=4e-3):                   # bf16 banks included
-        raise NotImplementedError("only the Haar (db1) filter bank is supported by the HIP transforms")
+        _refuse_bank()
+
+
+def _transform(x, filters, dims, inverse):
+    """The transform of x with the bank it came with.  A bank in GPU memory is checked by the launch itself (the first
+    thread of the transform's kernel compares the taps): reading it back would drain the stream on every call."""
+    S = 4 if dims == 2 else 2
+    shape = (S * x.shape[1], 1, 2, 2) if dims == 2 else (S * x.shape[1], 1, 2)
+    if tuple(filters.shape) != shape:
+        raise ValueError(f"filters of shape {tuple(filters.shape)}: expected the db1 bank {shape}")
+    ext = None if torch.compiler.is_compiling() else _ext.get()
+    if ext is not None:
+        out = ext.haar(x, filters, dims, inverse)
+        if out is False:
+            _refuse_bank()
+        if out is not None:
+            return out
+    _check_bank(filters, dims)
+    return _haar(x, dims, inverse)
+
+
+def _haar(x, dims, inverse):
+    ext = None if torch.compiler.is_compiling() else _ext.get()
+    return _Haar.apply(x, dims, inverse) if ext is None else ext.haar(x, None, dims, inverse)
 
 
 def _launch(x, out, dims, inverse):
@@ -115,8 +139,7 @@ def wavelet_2d_transform(x, filters):
     x = _prep(x, 4, "wavelet_2d_transform")
     if x.shape[2] % 2 or x.shape[3] % 2:
         raise ValueError(f"wavelet_2d_transform: extents must be even, got {tuple(x.shape[2:])} (pad first, as wtconv2d.py:49-51 does)")
-    _check_bank(filters, x.shape[1], 2)
-    return _Haar.apply(x, 2, False)
+    return _transform(x, filters, 2, False)
 
 
 def inverse_2d_wavelet_transform(x, filters):
@@ -124,8 +147,7 @@ def inverse_2d_wavelet_transform(x, filters):
     x = _prep(x, 5, "inverse_2d_wavelet_transform")
     if x.shape[2] != 4:
         raise ValueError(f"inverse_2d_wavelet_transform: expected 4 sub-bands, got shape {tuple(x.shape)}")
-    _check_bank(filters, x.shape[1], 2)
-    return _Haar.apply(x, 2, True)
+    return _transform(x, filters, 2, True)
 
 
 def wavelet_1d_transform(x, filters):
@@ -133,8 +155,7 @@ def wavelet_1d_transform(x, filters):
     x = _prep(x, 3, "wavelet_1d_transform")
     if x.shape[2] % 2:
         raise ValueError(f"wavelet_1d_transform: the length must be even, got {x.shape[2]} (pad first, as wtconv1d.py:49-51 does)")
-    _check_bank(filters, x.shape[1], 1)
-    return _Haar.apply(x, 1, False)
+    return _transform(x, filters, 1, False)
 
 
 def inverse_1d_wavelet_transform(x, filters):
@@ -142,5 +163,4 @@ def inverse_1d_wavelet_transform(x, filters):
     x = _prep(x, 4, "inverse_1d_wavelet_transform")
     if x.shape[2] != 2:
         raise ValueError(f"inverse_1d_wavelet_transform: expected 2 sub-bands, got shape {tuple(x.shape)}")
-    _check_bank(filters, x.shape[1], 1)
-    return _Haar.apply(x, 1, True)
+    return _transform(x, filters, 1, True)
