@@ -201,6 +201,25 @@ int wtconv_block_residual_backward(const void* dout, const void* y, const void* 
                                    int B, int C, int HW, int dtype, int param_dtype, void* workspace,
                                    size_t workspace_bytes, void* stream);
 
+/* ---- the whole of a WTConvNeXt block behind its WTConv layer, for inference (wtconvnext/wtconvnext.py:125-140 without
+ * drop_path): out = shortcut + gamma * (fc2 gelu(fc1 LayerNorm_c(x))), with x, shortcut and out (B, C, HW), exact (erf)
+ * GELU, fc1_weight (hidden, C) and fc2_weight (C, hidden) as nn.Linear keeps them.  bfloat16 tensors and parameters, the
+ * latter 16-byte aligned; gamma may be NULL.  out may be the shortcut, but not x.  Products, sums, LayerNorm and GELU in
+ * float; the normalised values and the hidden activations are rounded to bfloat16 once.
+ * wtconv_block_mlp_supported says whether a size has a kernel; the workspace takes partial sums of small batches. */
+typedef struct {
+  const void *norm_weight, *norm_bias;      /* (C) */
+  const void *fc1_weight, *fc1_bias;        /* (hidden, C), (hidden) */
+  const void *fc2_weight, *fc2_bias;        /* (C, hidden), (C) */
+  const void *gamma;                        /* (C) or NULL */
+} wtconv_mlp_params;
+
+int wtconv_block_mlp_supported(int B, int C, int HW, int hidden);
+size_t wtconv_block_mlp_workspace_bytes(int B, int C, int HW, int hidden);
+int wtconv_block_mlp(const void* x, const void* shortcut, void* out, const wtconv_mlp_params* params, int B, int C,
+                     int HW, int hidden, float eps, int dtype, int param_dtype, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* ---- single-level Haar (db1) transforms as operators of their own: wavelet_2d_transform /
  * inverse_2d_wavelet_transform and their 1-D twins with the db1 bank (wtconv/util/wavelet.py:46-75; the fast
  * twin's haar2d / ihaar2d utilities, fast_wtconv/cuda_haar/__init__.py:52-55).  Even extents only (the reference

@@ -318,3 +318,75 @@ def test_autocast_keeps_the_plain_passes(hip_device):
         finally:
             block_ops.usable = real
     assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape,hidden", [
+    ((2, 96, 8, 8), 384),        # one tile exactly, rows of whole 8-pixel vectors
+    ((5, 96, 7, 9), 384),        # odd pixel count: pixel by pixel, tile over several images, remainder
+    ((3, 128, 6, 6), 512),       # 4-pixel vectors
+    ((1, 192, 11, 3), 768),      # one pixel more than the smallest taken
+    ((70, 192, 28, 28), 64),     # a single slice of hidden units, many tiles
+    ((2, 256, 14, 14), 1024),    # hidden units dealt to several workgroups
+    ((2, 384, 14, 14), 1536),
+    ((168, 384, 14, 14), 1536),  # enough tiles to go unsplit
+    ((1, 384, 13, 11), 192),
+])
+@pytest.mark.parametrize("layer_scale", [True, False])
+def test_fused_block_against_fp64(hip_device, shape, hidden, layer_scale):
+    """LayerNorm, MLP, layer scale and shortcut in one kernel against float64 on the same bfloat16 values."""
+    import torch.nn.functional as F
+    from wtconv_amd import _ext
+    B, C, H, W = shape
+    gen = torch.Generator(device=hip_device).manual_seed(C + H)
+    r = lambda *s, k=1.0: (torch.randn(*s, generator=gen, device=hip_device) * k).bfloat16()
+    x, sc = r(B, C, H, W), r(B, C, H, W)
+    x[0, :, 0, 0] *= 30                                  # large activations: GELU's far ends
+    nw, nb, w1, b1 = 1 + r(C, k=.2), r(C, k=.2), r(hidden, C, k=C ** -.5), r(hidden, k=3.0)
+    w2, b2, gm = r(C, hidden, k=hidden ** -.5), r(C, k=.3), r(C) if layer_scale else None
+    with torch.no_grad():
+        got = _ext.get().block_mlp(x, sc, nw, nb, 1e-6, w1, b1, w2, b2, gm)
+    assert got is not None and got.shape == x.shape and got.dtype == torch.bfloat16
+    d = lambda t: t.double()
+    y = F.layer_norm(d(x).permute(0, 2, 3, 1), (C,), d(nw), d(nb), 1e-6)
+    y = F.linear(F.gelu(F.linear(y, d(w1), d(b1))), d(w2), d(b2))
+    want = d(sc) + (y if gm is None else y * d(gm)).permute(0, 3, 1, 2)
+    rel = ((d(got) - want).norm() / want.norm()).item()
+    assert rel < 4e-3, rel
+    rms = want.pow(2).mean().sqrt()
+    assert ((d(got) - want).abs() / torch.maximum(want.abs(), rms)).max().item() < 6e-2
+
+
+def test_fused_block_keeps_infinities_and_nans_to_their_pixels(hip_device):
+    from wtconv_amd import _ext
+    C = 96
+    g = torch.Generator(device=hip_device).manual_seed(0)
+    r = lambda *s: torch.randn(*s, generator=g, device=hip_device).bfloat16()
+    x, sc = r(2, C, 8, 8), r(2, C, 8, 8)
+    args = (1 + r(C), r(C), 1e-6, r(4 * C, C), r(4 * C), r(C, 4 * C), r(C), r(C))
+    with torch.no_grad():
+        clean = _ext.get().block_mlp(x, sc, *args)
+        x[1, 5, 3, 2] = float("nan")
+        got = _ext.get().block_mlp(x, sc, *args)
+        assert torch.isnan(got[1, :, 3, 2]).all()
+        got[1, :, 3, 2] = clean[1, :, 3, 2]
+        assert torch.equal(got, clean)
+        big = torch.full((4 * C,), float("inf"), device=hip_device, dtype=torch.bfloat16)      # gelu(inf) is inf, not nan
+        w2 = torch.ones(C, 4 * C, device=hip_device, dtype=torch.bfloat16)
+        assert torch.isinf(_ext.get().block_mlp(clean, sc, *args[:4], big, w2, args[6], None)).all()
+
+
+def test_fused_block_is_left_alone_where_modules_are_watched(hip_device):
+    """Recording, hooks and other activations take the separate passes; the results agree."""
+    from wtconvnext.wtconvnext import WTConvNeXtBlock
+    torch.manual_seed(0)
+    blk = WTConvNeXtBlock(96, wt_levels=2, ls_init_value=0.5).to(hip_device).bfloat16().eval()
+    x = torch.randn(2, 96, 14, 14, device=hip_device).bfloat16()
+    with torch.no_grad():
+        fused = blk(x)
+        seen = []
+        handle = blk.mlp.fc1.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        apart = blk(x)
+        handle.remove()
+    assert seen and (fused.float() - apart.float()).norm() < 1e-2 * apart.float().norm()
+    blk(x).float().sum().backward()
+    assert blk.mlp.fc1.weight.grad is not None

@@ -7,16 +7,18 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libwtconv_hip.so")
 SOURCES = [os.path.join(CSRC, "api.hip"), os.path.join(CSRC, "mfma2d.hip"), os.path.join(CSRC, "block.hip"),
-           os.path.join(CSRC, "haar.hip")]
-HEADERS = [os.path.join(CSRC, f) for f in ("common.h", "host_util.h", "kernels1d.h", "kernels1d_row.h", "kernels2d.h", "kernels2d_mfma.h", "kernels2d_mfma_wgrad.h", "kernels_block.h", "kernels_haar.h", "wgrad_finish.h",
+           os.path.join(CSRC, "haar.hip"), os.path.join(CSRC, "mlp.hip")]
+HEADERS = [os.path.join(CSRC, f) for f in ("common.h", "host_util.h", "kernels1d.h", "kernels1d_row.h", "kernels2d.h", "kernels2d_mfma.h", "kernels2d_mfma_wgrad.h", "kernels_block.h", "kernels_haar.h", "kernels_mlp.h", "wgrad_finish.h",
                                          "kernels2d_stream.h", "mfma2d.h", "plan.h")] + [
     os.path.join(os.path.dirname(PKG_DIR), "include", "wtconv_hip.h")]
 
 # packed-FP32 code generation is switched off on purpose: every float op is a scalar VALU op
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-               "-mllvm", "-amdgpu-mfma-vgpr-form=1",     # MFMA accumulators in ordinary VGPRs: no copies to and from AGPRs
                "-Wno-unused-command-line-argument"]
+# MFMA accumulators in ordinary VGPRs: no copies to and from AGPRs.  Not for mlp.hip, whose kernels keep more than 256
+# registers a lane and need the AGPR half of the file for the accumulators.
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 OBJ_DIR = os.path.join(PKG_DIR, "build")
 
 
@@ -33,7 +35,7 @@ def build_library(verbose=False):
     objs, procs = [], []
     for src in SOURCES:
         obj = os.path.join(OBJ_DIR, os.path.splitext(os.path.basename(src))[0] + ".o")
-        cmd = [hipcc_path()] + HIPCC_FLAGS + ["-c", src, "-o", obj]
+        cmd = [hipcc_path()] + HIPCC_FLAGS + ([] if src.endswith("mlp.hip") else VGPR_FORM) + ["-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
         objs.append(obj)

@@ -21,6 +21,11 @@ class ParamGrads(ctypes.Structure):
     _fields_ = Params._fields_
 
 
+class MlpParams(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("norm_weight", "norm_bias", "fc1_weight", "fc1_bias", "fc2_weight",
+                                               "fc2_bias", "gamma")]
+
+
 EXPORTS = {
     "wtconv_abi_version": (ctypes.c_int, []),
     "wtconv_last_error": (ctypes.c_char_p, []),
@@ -49,6 +54,9 @@ EXPORTS["wtconv_block_residual"] = (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p]
 EXPORTS["wtconv_block_workspace_bytes"] = (_z, [_i, _i, _i, _i])
 EXPORTS["wtconv_channel_norm_backward"] = (_i, [_p, _p, _p, _p, _p, _p, _i, _i, _i, _f, _i, _i, _i, _p, _z, _p])
 EXPORTS["wtconv_block_residual_backward"] = (_i, [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _p, _z, _p])
+EXPORTS["wtconv_block_mlp_supported"] = (_i, [_i] * 4)
+EXPORTS["wtconv_block_mlp_workspace_bytes"] = (_z, [_i] * 4)
+EXPORTS["wtconv_block_mlp"] = (_i, [_p, _p, _p, ctypes.POINTER(MlpParams), _i, _i, _i, _i, _f, _i, _i, _p, _z, _p])
 
 _ll = ctypes.c_longlong
 EXPORTS["wtconv_haar2d"] = (_i, [_p, _p, _ll, _i, _i, _i, _i, _p])

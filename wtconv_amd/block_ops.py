@@ -9,7 +9,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _ext, _lib
 
 _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}
 
@@ -45,6 +45,24 @@ def usable(x, *params, training=False):
 def usable_nhwc(y, shortcut):
     """Whether the residual kernels take the MLP output `y` (B, H, W, C) for this shortcut: same dtype and device."""
     return y.dtype == shortcut.dtype and y.device == shortcut.device and y.dim() == 4
+
+
+def _hooked(*modules):
+    return any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
+def block_mlp(x, shortcut, norm, mlp, gamma):
+    """shortcut + gamma * fc2(gelu(fc1(norm(x)))) of a WTConvNeXt block, with x and shortcut (B, C, H, W), in one kernel;
+    None where it does not apply: autograd records, another dtype than bfloat16, a channel count without a kernel, an
+    activation other than the exact GELU, or hooks that expect to see the modules called."""
+    ext = _ext.get()
+    if ext is None or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+        return None
+    fc1, act, fc2 = mlp.fc1, mlp.act, mlp.fc2
+    if (type(fc1) is not torch.nn.Linear or type(fc2) is not torch.nn.Linear or type(act) is not torch.nn.GELU
+            or act.approximate != "none" or norm.weight is None or norm.bias is None or _hooked(norm, mlp, fc1, act, fc2)):
+        return None
+    return ext.block_mlp(x, shortcut, norm.weight, norm.bias, norm.eps, fc1.weight, fc1.bias, fc2.weight, fc2.bias, gamma)
 
 
 def _stream():

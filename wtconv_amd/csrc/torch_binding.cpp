@@ -52,6 +52,10 @@ struct Abi {
   int (*haar1)(const void*, void*, long long, int, int, int, void*);
   int (*haar2c)(const void*, void*, long long, int, int, int, int, const void*, int, unsigned*, void*);
   int (*haar1c)(const void*, void*, long long, int, int, int, const void*, int, unsigned*, void*);
+  int (*mlp_ok)(int, int, int, int);
+  size_t (*mlp_ws)(int, int, int, int);
+  int (*mlp)(const void*, const void*, void*, const wtconv_mlp_params*, int, int, int, int, float, int, int, void*, size_t,
+             void*);
   bool bound = false;
 } abi;
 
@@ -60,11 +64,12 @@ void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 15, "bind: expected 15 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 18, "bind: expected 18 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
   take(abi.haar2, a[11]); take(abi.haar1, a[12]); take(abi.haar2c, a[13]); take(abi.haar1c, a[14]);
+  take(abi.mlp_ok, a[15]); take(abi.mlp_ws, a[16]); take(abi.mlp, a[17]);
   abi.bound = true;
 }
 
@@ -399,10 +404,48 @@ py::object haar(const Tensor& x, const std::optional<Tensor>& bank, int64_t dims
   return py::cast(out);
 }
 
+// The block behind its WTConv layer in one kernel (inference): None if the kernel does not take these arguments or
+// autograd would record the call.
+py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm_w, const Tensor& norm_b, double eps,
+                     const Tensor& w1, const std::optional<Tensor>& b1, const Tensor& w2, const std::optional<Tensor>& b2,
+                     const std::optional<Tensor>& gamma) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (x.dim() != 4 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous()) return py::none();
+  if (shortcut.sizes() != x.sizes() || !b1.has_value() || !b2.has_value()) return py::none();
+  const int64_t B = x.size(0), C = x.size(1), HW = x.size(2) * x.size(3);
+  if (w1.dim() != 2 || w2.dim() != 2 || w1.size(1) != C || w2.size(0) != C || w1.size(0) != w2.size(1)) return py::none();
+  const int64_t hidden = w1.size(0);
+  if (norm_w.numel() != C || norm_b.numel() != C || b1->numel() != hidden || b2->numel() != C) return py::none();
+  if (gamma.has_value() && gamma->numel() != C) return py::none();
+  const bool grad = at::GradMode::is_enabled();
+  if (grad && x.requires_grad()) return py::none();
+  const Tensor* all[] = {&shortcut, &norm_w, &norm_b, &w1, &*b1, &w2, &*b2, gamma.has_value() ? &*gamma : nullptr};
+  uintptr_t bits = 0;
+  for (const Tensor* t : all) {
+    if (t == nullptr) continue;
+    if (!canonical(*t, x.device(), at::kBFloat16) || (grad && t->requires_grad())) return py::none();
+    if (t != &shortcut) bits |= reinterpret_cast<uintptr_t>(t->data_ptr());
+  }
+  if (bits % 16 || x.numel() == 0 || B * HW > (1LL << 30) || !abi.mlp_ok(B, C, HW, hidden)) return py::none();
+  const c10::DeviceGuard guard(x.device());
+  Tensor out = at::empty_like(x, at::MemoryFormat::Contiguous);
+  const size_t wsz = abi.mlp_ws(B, C, HW, hidden);
+  Tensor ws;
+  if (wsz) ws = at::empty({static_cast<int64_t>(wsz)}, x.options().dtype(at::kByte));
+  const wtconv_mlp_params p = {norm_w.data_ptr(), norm_b.data_ptr(), w1.data_ptr(), b1->data_ptr(), w2.data_ptr(),
+                               b2->data_ptr(), gamma.has_value() ? gamma->data_ptr() : nullptr};
+  const int rc = abi.mlp(x.data_ptr(), shortcut.data_ptr(), out.data_ptr(), &p, B, C, HW, hidden, static_cast<float>(eps),
+                         WTCONV_BF16, WTCONV_BF16, wsz ? ws.data_ptr() : nullptr, wsz,
+                         c10::hip::getCurrentHIPStream(x.device().index()).stream());
+  if (rc) fail(rc, "wtconv block mlp");
+  return py::cast(out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind, "hand over the addresses of the C-ABI entry points");
   m.def("layer", &layer, "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical");
+  m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
   m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }

@@ -93,6 +93,10 @@ class WTConvNeXtBlock(nn.Module):
         x = self.conv_dw(x)
         ops = _block_ops()
         drops = self.training and not isinstance(self.drop_path, nn.Identity)
+        if ops is not None and not drops and type(self.mlp) is Mlp:
+            out = ops.block_mlp(x, shortcut, self.norm, self.mlp, self.gamma)      # inference on the GPU: one kernel
+            if out is not None:
+                return out
         if (ops is not None and not drops and x.is_contiguous() and shortcut.is_contiguous()
                 and ops.usable(x, self.norm.weight, self.norm.bias, self.gamma, training=True)
                 and ops.usable(shortcut, training=True)):
