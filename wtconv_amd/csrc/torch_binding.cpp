@@ -17,6 +17,10 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/Exceptions.h>
 
 #include <chrono>
 #include <mutex>
@@ -84,7 +88,7 @@ int dtype_code(at::ScalarType t) {
 
 void fail(int rc, const char* what) {
   const char* msg = abi.last_error ? abi.last_error() : "";
-  if (rc == WTCONV_E_ARG) throw py::value_error(std::string(msg && *msg ? msg : what));
+  TORCH_CHECK_VALUE(rc != WTCONV_E_ARG, msg && *msg ? msg : what);
   TORCH_CHECK(false, (msg && *msg) ? msg : what, " (code ", rc, ")");
 }
 
@@ -107,144 +111,147 @@ void fill(Table& t, const Tensor& base_w, const Tensor& base_b, const Tensor& ba
   }
 }
 
-class WTConvNode : public torch::autograd::Function<WTConvNode> {
- public:
-  // wt = the L level weights followed by the L level scales.
-  static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& base_w,
-                        const std::optional<Tensor>& base_b_opt, const Tensor& base_s, at::TensorList wt,
-                        int64_t dims, int64_t K, int64_t L) {
-    const Tensor x = x_in.contiguous();
-    const Tensor base_b = base_b_opt.has_value() ? *base_b_opt : Tensor();
-    const c10::DeviceGuard guard(x.device());      // (PyTorch on ROCm names the device type "cuda")
-    const Shape s = dims == 2 ? Shape{(int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3)}
-                              : Shape{(int)x.size(0), (int)x.size(1), 1, (int)x.size(2)};
-    Tensor out = at::empty_like(x, at::MemoryFormat::Contiguous);
-    const size_t wsz = workspace_bytes(dims, s, K, L, 0);
-    Tensor ws = at::empty({static_cast<int64_t>(wsz)}, x.options().dtype(at::kByte));
-    wtconv_params p;
-    fill(p, base_w, base_b, base_s, wt, L);
-    void* stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-    const int dt = dtype_code(x.scalar_type()), pdt = dtype_code(base_w.scalar_type());
-    const int rc = dims == 2 ? abi.fwd2(x.data_ptr(), out.data_ptr(), &p, s.B, s.C, s.H, s.W, K, L, dt, pdt,
-                                        ws.data_ptr(), wsz, stream)
-                             : abi.fwd1(x.data_ptr(), out.data_ptr(), &p, s.B, s.C, s.W, K, L, dt, pdt, ws.data_ptr(),
-                                        wsz, stream);
-    if (rc) fail(rc, "wtconv forward");
-    variable_list saved = {x, base_w, base_b, base_s};
-    saved.insert(saved.end(), wt.begin(), wt.end());
-    ctx->save_for_backward(saved);
-    ctx->saved_data["dims"] = dims;
-    ctx->saved_data["K"] = K;
-    ctx->saved_data["L"] = L;
-    return out;
+// Device memory of one call, given back to PyTorch's stream-ordered allocator when the launches are queued.
+c10::DataPtr scratch(const Tensor& like, size_t bytes) { return c10::GetAllocator(like.device().type())->allocate(bytes); }
+
+// A tensor over part of `flat`'s storage (what narrow().view() gives, without two trips through the dispatcher).
+Tensor part_of(const Tensor& flat, int64_t at, at::IntArrayRef sizes) {
+  Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(flat.storage()), flat.key_set(), flat.dtype());
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+  t.unsafeGetTensorImpl()->set_storage_offset(flat.storage_offset() + at);
+  return t;
+}
+
+constexpr int kMaxTensors = 3 + 2 * WTCONV_MAX_LEVELS;
+
+// The parameters of a layer: base weight, base bias (may be undefined), base scale, L level weights, L level scales.
+struct LayerParams {
+  Tensor t[kMaxTensors];
+  int L = 0;
+  int count() const { return 3 + 2 * L; }
+  at::TensorList levels() const { return at::TensorList(t + 3, 2 * L); }
+};
+
+Shape shape_of(const Tensor& x, int dims) {
+  return dims == 2 ? Shape{(int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3)}
+                   : Shape{(int)x.size(0), (int)x.size(1), 1, (int)x.size(2)};
+}
+
+Tensor layer_forward(const Tensor& x, const LayerParams& lp, int dims, int K) {
+  const c10::DeviceGuard guard(x.device());      // (PyTorch on ROCm names the device type "cuda")
+  const Shape s = shape_of(x, dims);
+  Tensor out = at::empty(x.sizes(), x.options().requires_grad(false));
+  const size_t wsz = workspace_bytes(dims, s, K, lp.L, 0);
+  const c10::DataPtr ws = scratch(x, wsz);
+  wtconv_params p;
+  fill(p, lp.t[0], lp.t[1], lp.t[2], lp.levels(), lp.L);
+  void* stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+  const int dt = dtype_code(x.scalar_type()), pdt = dtype_code(lp.t[0].scalar_type());
+  const int rc = dims == 2 ? abi.fwd2(x.const_data_ptr(), out.mutable_data_ptr(), &p, s.B, s.C, s.H, s.W, K, lp.L, dt, pdt,
+                                      ws.get(), wsz, stream)
+                           : abi.fwd1(x.const_data_ptr(), out.mutable_data_ptr(), &p, s.B, s.C, s.W, K, lp.L, dt, pdt,
+                                      ws.get(), wsz, stream);
+  if (rc) fail(rc, "wtconv forward");
+  return out;
+}
+
+// Gradients of x and of the parameters: edges 0 and 1..count() of the node.
+struct WTConvNode : public torch::autograd::Node {
+  torch::autograd::SavedVariable x_, p_[kMaxTensors];
+  int dims_ = 0, K_ = 0, L_ = 0;
+
+  std::string name() const override { return "WTConvLayerBackward"; }
+
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    x_.reset_data();
+    for (int i = 0; i < 3 + 2 * L_; ++i) p_[i].reset_data();
   }
 
-  static variable_list backward(AutogradContext* ctx, variable_list grad_outputs) {
-    const variable_list saved = ctx->get_saved_variables();
-    const int dims = ctx->saved_data["dims"].toInt(), K = ctx->saved_data["K"].toInt(), L = ctx->saved_data["L"].toInt();
-    const Tensor &x = saved[0], &base_w = saved[1], &base_b = saved[2], &base_s = saved[3];
-    const at::TensorList wt(saved.data() + 4, 2 * L);
-    const bool has_bias = base_b.defined();
-    // one result per argument of forward: x, base_w, base_b, base_s, 2L level tensors, dims, K, L
-    variable_list res(4 + 2 * L + 3);
-    Tensor g = grad_outputs[0];
-    if (!g.defined()) return res;
-    // needs_input_grad counts the tensor arguments only (a missing bias is not one of them)
-    const int nt = 3 + (has_bias ? 1 : 0) + 2 * L;
-    const bool need_x = ctx->needs_input_grad(0);
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const int dims = dims_, K = K_, L = L_;
+    const Tensor x = x_.unpack();
+    LayerParams lp;
+    lp.L = L;
+    const int n = lp.count();
+    for (int i = 0; i < n; ++i) lp.t[i] = p_[i].unpack();
+    variable_list res(1 + n);
+    if (!grads[0].defined()) return res;
+    const bool need_x = task_should_compute_output(0);
     bool need_params = false;
-    for (int i = 1; i < nt; ++i) need_params = need_params || ctx->needs_input_grad(i);
+    for (int i = 1; i <= n; ++i) need_params = need_params || task_should_compute_output(i);
     if (!need_x && !need_params) return res;
-    if (g.scalar_type() != x.scalar_type()) g = g.to(x.scalar_type());
-    g = g.contiguous();
-    const c10::DeviceGuard guard(x.device());      // (PyTorch on ROCm names the device type "cuda")
-    const Shape s = dims == 2 ? Shape{(int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3)}
-                              : Shape{(int)x.size(0), (int)x.size(1), 1, (int)x.size(2)};
-    const int pass = need_x && need_params ? 3 : (need_x ? 1 : 2);
-    const size_t wsz = workspace_bytes(dims, s, K, L, pass);
-    Tensor ws = at::empty({static_cast<int64_t>(wsz)}, x.options().dtype(at::kByte));
-    wtconv_params p;
-    fill(p, base_w, base_b, base_s, wt, L);
-    void* stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-    const int dt = dtype_code(x.scalar_type()), pdt = dtype_code(base_w.scalar_type());
-    Tensor grad_x;
-    if (need_x) grad_x = at::empty_like(x, at::MemoryFormat::Contiguous);
-    // parameter gradients are written as fp32 into one flat buffer (one allocation for the 5 + 2 L tensors): fp32
-    // parameters get views of it in their own shapes, others views of one cast of it
-    const bool f32 = base_w.scalar_type() == at::kFloat;
-    std::vector<Tensor> views(3 + 2 * L);      // base_w, base_b, base_s, levels
-    Tensor flat;
-    wtconv_param_grads gt;
-    if (need_params) {
-      std::vector<const Tensor*> plist = {&base_w, &base_b, &base_s};
-      for (int i = 0; i < 2 * L; ++i) plist.push_back(&wt[i]);
-      int64_t total = 0;
-      for (const Tensor* t : plist) total += t->defined() ? t->numel() : 0;
-      flat = at::empty({total}, x.options().dtype(at::kFloat));
-      int64_t pos = 0;
-      for (size_t i = 0; i < plist.size(); ++i)
-        if (plist[i]->defined()) {
-          views[i] = flat.narrow(0, pos, plist[i]->numel());
-          if (f32) views[i] = views[i].view(plist[i]->sizes());
-          pos += plist[i]->numel();
-        }
-      const at::TensorList lv(views.data() + 3, 2 * L);
-      fill(gt, views[0], views[1], views[2], lv, L);
-    }
-    int rc;
-    if (dims == 2) {
-      if (pass == 3)
-        rc = abi.bwd2(x.data_ptr(), g.data_ptr(), grad_x.data_ptr(), &p, &gt, s.B, s.C, s.H, s.W, K, L, dt, pdt,
-                      ws.data_ptr(), wsz, stream);
-      else if (pass == 1)
-        rc = abi.bwdin2(g.data_ptr(), grad_x.data_ptr(), &p, s.B, s.C, s.H, s.W, K, L, dt, pdt, ws.data_ptr(), wsz, stream);
-      else
-        rc = abi.bwdpar2(x.data_ptr(), g.data_ptr(), &p, &gt, s.B, s.C, s.H, s.W, K, L, dt, pdt, ws.data_ptr(), wsz, stream);
-    } else {
-      if (pass == 3)
-        rc = abi.bwd1(x.data_ptr(), g.data_ptr(), grad_x.data_ptr(), &p, &gt, s.B, s.C, s.W, K, L, dt, pdt, ws.data_ptr(),
-                      wsz, stream);
-      else if (pass == 1)
-        rc = abi.bwdin1(g.data_ptr(), grad_x.data_ptr(), &p, s.B, s.C, s.W, K, L, dt, pdt, ws.data_ptr(), wsz, stream);
-      else
-        rc = abi.bwdpar1(x.data_ptr(), g.data_ptr(), &p, &gt, s.B, s.C, s.W, K, L, dt, pdt, ws.data_ptr(), wsz, stream);
-    }
-    if (rc) fail(rc, "wtconv backward");
-    // The gradients come from raw pointers and carry no graph.  Under create_graph=True every result that something
-    // differentiable went into gets a node that raises when it is differentiated (what once_differentiable does for
-    // the Python function): a second-order term is refused instead of being treated as a constant.
+    // Under create_graph=True every result that something differentiable went into is refused a second derivative
+    // (the gradients come from raw pointers and carry no graph) instead of being treated as a constant.
     bool twice = false;
     if (at::GradMode::is_enabled()) {
-      twice = grad_outputs[0].requires_grad();
-      for (const Tensor& t : saved) twice = twice || (t.defined() && t.requires_grad());
+      twice = grads[0].requires_grad() || x.requires_grad();
+      for (int i = 0; i < n; ++i) twice = twice || (lp.t[i].defined() && lp.t[i].requires_grad());
     }
-    auto refuse = [&](Tensor& t) {
-      if (!twice || !t.defined()) return;
-      auto err = std::make_shared<torch::autograd::Error>(
-          "the backward pass of the WTConv layer is not differentiable (double backward / create_graph=True through "
-          "this layer is not supported)", torch::autograd::edge_list());
-      torch::autograd::create_gradient_edge(t, err);
-    };
-    res[0] = grad_x;
-    refuse(res[0]);
+    const at::NoGradGuard no_grad;
+    Tensor g = grads[0];
+    if (g.scalar_type() != x.scalar_type()) g = g.to(x.scalar_type());
+    if (!g.is_contiguous()) g = g.contiguous();
+    const c10::DeviceGuard guard(x.device());
+    const Shape s = shape_of(x, dims);
+    const int pass = need_x && need_params ? 3 : (need_x ? 1 : 2);
+    const size_t wsz = workspace_bytes(dims, s, K, L, pass);
+    const c10::DataPtr ws = scratch(x, wsz);
+    wtconv_params p;
+    fill(p, lp.t[0], lp.t[1], lp.t[2], lp.levels(), L);
+    void* stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+    const int dt = dtype_code(x.scalar_type()), pdt = dtype_code(lp.t[0].scalar_type());
+    Tensor grad_x;
+    if (need_x) grad_x = at::empty(x.sizes(), x.options().requires_grad(false));
+    // parameter gradients are written as fp32 into one flat buffer (one allocation for the 3 + 2 L tensors): fp32
+    // parameters get parts of it in their own shapes, others parts of one cast of it
+    const bool f32 = lp.t[0].scalar_type() == at::kFloat;
+    int64_t pos[kMaxTensors], total = 0;
+    Tensor flat;
+    wtconv_param_grads gt = {};
     if (need_params) {
-      if (!f32) {
-        const Tensor cast = flat.to(base_w.scalar_type());
-        int64_t pos = 0;
-        std::vector<const Tensor*> plist = {&base_w, &base_b, &base_s};
-        for (int i = 0; i < 2 * L; ++i) plist.push_back(&wt[i]);
-        for (size_t i = 0; i < plist.size(); ++i)
-          if (plist[i]->defined()) {
-            views[i] = cast.narrow(0, pos, plist[i]->numel()).view(plist[i]->sizes());
-            pos += plist[i]->numel();
-          }
+      for (int i = 0; i < n; ++i) {
+        pos[i] = total;
+        if (lp.t[i].defined()) total += lp.t[i].numel();
       }
-      res[1] = views[0];
-      res[2] = views[1];
-      res[3] = views[2];
-      for (int i = 0; i < 2 * L; ++i) res[4 + i] = views[3 + i];
-      for (int i = 1; i < 4 + 2 * L; ++i) refuse(res[i]);
+      flat = at::empty({total}, x.options().dtype(at::kFloat).requires_grad(false));
+      float* f = flat.mutable_data_ptr<float>();
+      gt.base_weight = f + pos[0];
+      gt.base_bias = lp.t[1].defined() ? f + pos[1] : nullptr;
+      gt.base_scale = f + pos[2];
+      for (int l = 0; l < L; ++l) {
+        gt.wt_weight[l] = f + pos[3 + l];
+        gt.wt_scale[l] = f + pos[3 + L + l];
+      }
     }
+    const void *xp = x.const_data_ptr(), *gp = g.const_data_ptr();
+    void* gxp = need_x ? grad_x.mutable_data_ptr() : nullptr;
+    int rc;
+    if (dims == 2) {
+      rc = pass == 3   ? abi.bwd2(xp, gp, gxp, &p, &gt, s.B, s.C, s.H, s.W, K, L, dt, pdt, ws.get(), wsz, stream)
+           : pass == 1 ? abi.bwdin2(gp, gxp, &p, s.B, s.C, s.H, s.W, K, L, dt, pdt, ws.get(), wsz, stream)
+                       : abi.bwdpar2(xp, gp, &p, &gt, s.B, s.C, s.H, s.W, K, L, dt, pdt, ws.get(), wsz, stream);
+    } else {
+      rc = pass == 3   ? abi.bwd1(xp, gp, gxp, &p, &gt, s.B, s.C, s.W, K, L, dt, pdt, ws.get(), wsz, stream)
+           : pass == 1 ? abi.bwdin1(gp, gxp, &p, s.B, s.C, s.W, K, L, dt, pdt, ws.get(), wsz, stream)
+                       : abi.bwdpar1(xp, gp, &p, &gt, s.B, s.C, s.W, K, L, dt, pdt, ws.get(), wsz, stream);
+    }
+    if (rc) fail(rc, "wtconv backward");
+    res[0] = std::move(grad_x);
+    if (need_params) {
+      const Tensor src = f32 ? flat : flat.to(lp.t[0].scalar_type());
+      for (int i = 0; i < n; ++i)
+        if (lp.t[i].defined() && task_should_compute_output(1 + i)) res[1 + i] = part_of(src, pos[i], lp.t[i].sizes());
+    }
+    if (twice)
+      for (Tensor& t : res)
+        if (t.defined()) {
+          auto err = std::make_shared<torch::autograd::Error>(
+              "the backward pass of the WTConv layer is not differentiable (double backward / create_graph=True through "
+              "this layer is not supported)", torch::autograd::edge_list());
+          torch::autograd::create_gradient_edge(t, err);
+        }
     return res;
   }
 };
@@ -253,28 +260,84 @@ bool canonical(const Tensor& t, const at::Device& dev, at::ScalarType pd) {
   return t.device() == dev && t.scalar_type() == pd && t.is_contiguous();
 }
 
-// The layer with its C++ autograd node, or None when the arguments need the conversions of the Python path.
-py::object layer(const Tensor& x, const Tensor& base_w, const std::optional<Tensor>& base_b, const Tensor& base_s,
-                 const std::vector<Tensor>& wt_ws, const std::vector<Tensor>& wt_ss, int64_t dims, int64_t K, int64_t L) {
+// The tensors of a list or tuple, as levels lp.t[at...]; false if it is neither or holds anything else.
+bool take_levels(PyObject* seq, LayerParams& lp, int L, int at) {
+  const bool list = PyList_CheckExact(seq);
+  if (!list && !PyTuple_CheckExact(seq)) return false;
+  if ((list ? PyList_GET_SIZE(seq) : PyTuple_GET_SIZE(seq)) != L) return false;
+  for (int i = 0; i < L; ++i) {
+    PyObject* o = list ? PyList_GET_ITEM(seq, i) : PyTuple_GET_ITEM(seq, i);
+    if (!THPVariable_Check(o)) return false;
+    lp.t[at + i] = THPVariable_Unpack(o);
+  }
+  return true;
+}
+
+// layer(x, base_weight, base_bias or None, base_scale, level weights, level scales, dims, K, L): the layer with its C++
+// autograd node, or None when the arguments are not the canonical ones (the caller then takes the Python path, which
+// converts what can be converted and says what is wrong with the rest).  A plain CPython function: the argument
+// conversions of pybind11 cost more than the checks below.
+PyObject* layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 9, "layer: expected 9 arguments, got ", nargs);
   TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
-  if (!x.is_cuda() || dtype_code(x.scalar_type()) < 0) return py::none();
-  const at::ScalarType pd = base_w.scalar_type();
-  if (dtype_code(pd) < 0) return py::none();
-  if (static_cast<int64_t>(wt_ws.size()) != L || static_cast<int64_t>(wt_ss.size()) != L) return py::none();
-  const at::Device dev = x.device();
-  if (!canonical(base_w, dev, pd) || !canonical(base_s, dev, pd)) return py::none();
-  if (base_b.has_value() && base_b->defined() && !canonical(*base_b, dev, pd)) return py::none();
-  std::vector<Tensor> wt;
-  wt.reserve(2 * L);
-  for (const Tensor& t : wt_ws) { if (!canonical(t, dev, pd)) return py::none(); wt.push_back(t); }
-  for (const Tensor& t : wt_ss) { if (!canonical(t, dev, pd)) return py::none(); wt.push_back(t); }
-  const std::optional<Tensor> bias = (base_b.has_value() && base_b->defined()) ? base_b : std::nullopt;
+  const int dims = static_cast<int>(PyLong_AsLong(args[6]));
+  const long K = PyLong_AsLong(args[7]), L = PyLong_AsLong(args[8]);
+  if (PyErr_Occurred()) return nullptr;
+  if ((dims != 1 && dims != 2) || L < 1 || L > WTCONV_MAX_LEVELS || K < 1 || K % 2 == 0) Py_RETURN_NONE;
+  for (int i = 0; i < 4; ++i)
+    if (!THPVariable_Check(args[i]) && !(i == 2 && args[i] == Py_None)) Py_RETURN_NONE;
+  const Tensor& x_in = THPVariable_Unpack(args[0]);
+  if (!x_in.is_cuda() || x_in.dim() != dims + 2 || dtype_code(x_in.scalar_type()) < 0 || x_in.numel() == 0) Py_RETURN_NONE;
+  LayerParams lp;
+  lp.L = static_cast<int>(L);
+  lp.t[0] = THPVariable_Unpack(args[1]);
+  if (args[2] != Py_None) lp.t[1] = THPVariable_Unpack(args[2]);
+  lp.t[2] = THPVariable_Unpack(args[3]);
+  if (!take_levels(args[4], lp, lp.L, 3) || !take_levels(args[5], lp, lp.L, 3 + lp.L)) Py_RETURN_NONE;
+  const at::ScalarType pd = lp.t[0].scalar_type();
+  const at::Device dev = x_in.device();
+  if (dtype_code(pd) < 0) Py_RETURN_NONE;
+  const int64_t C = x_in.size(1), taps = dims == 2 ? K * K : K, S = dims == 2 ? 4 : 2;
+  bool record = at::GradMode::is_enabled(), any = x_in.requires_grad();
+  for (int i = 0; i < lp.count(); ++i) {
+    const Tensor& t = lp.t[i];
+    if (!t.defined()) continue;
+    const int64_t want = i == 0 ? C * taps : i < 3 ? C : i < 3 + L ? S * C * taps : S * C;
+    if (!canonical(t, dev, pd) || t.numel() != want || t._fw_grad(0).defined()) Py_RETURN_NONE;
+    any = any || t.requires_grad();
+  }
+  if (x_in._fw_grad(0).defined()) Py_RETURN_NONE;      // forward-mode differentiation: refused by the Python function
+  record = record && any;
   Tensor out;
   {
-    py::gil_scoped_release nogil;
-    out = WTConvNode::apply(x, base_w, bias, base_s, at::TensorList(wt), dims, K, L);
+    const pybind11::gil_scoped_release nogil;
+    Tensor x = x_in;
+    if (!x.is_contiguous()) {
+      const at::NoGradGuard no_grad;
+      x = x.contiguous();
+    }
+    out = layer_forward(x, lp, dims, static_cast<int>(K));
+    if (record) {
+      const std::shared_ptr<WTConvNode> node(new WTConvNode(), torch::autograd::deleteNode);
+      torch::autograd::edge_list next;
+      next.reserve(1 + lp.count());
+      auto edge = [&](const Tensor& t) {
+        next.push_back(t.defined() ? torch::autograd::impl::gradient_edge(t) : torch::autograd::Edge());
+      };
+      edge(x_in);
+      for (int i = 0; i < lp.count(); ++i) edge(lp.t[i]);
+      node->set_next_edges(std::move(next));
+      node->x_ = torch::autograd::SavedVariable(x, false);
+      for (int i = 0; i < lp.count(); ++i) node->p_[i] = torch::autograd::SavedVariable(lp.t[i], false);
+      node->dims_ = dims;
+      node->K_ = static_cast<int>(K);
+      node->L_ = lp.L;
+      torch::autograd::set_history(out, node);
+    }
   }
-  return py::cast(out);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
 }
 
 // ---- the single-level Haar transforms (wtconv_amd/wavelet.py), with the check of the filter bank they are handed.
@@ -445,7 +508,11 @@ py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind, "hand over the addresses of the C-ABI entry points");
-  m.def("layer", &layer, "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical");
+  static PyMethodDef functions[] = {
+      {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&layer)), METH_FASTCALL,
+       "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical"},
+      {nullptr, nullptr, 0, nullptr}};
+  if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
   m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
   m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }

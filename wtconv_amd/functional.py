@@ -5,6 +5,7 @@ wavelet level, the inverse cascade); PyTorch only supplies device memory and the
 Semantics follow the reference layer (wtconv/wtconv2d.py:38-87, wtconv/wtconv1d.py:38-87).
 """
 import ctypes
+import functools
 from typing import List, Optional
 
 import torch
@@ -14,6 +15,11 @@ from . import _ext, _lib
 _DT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 
 
+@functools.lru_cache(maxsize=None)
+def _max_kernel_size():
+    return _lib.load().wtconv_max_kernel_size()
+
+
 def check_kernel_size(kernel_size):
     """Raise early if no built kernel covers this size (cf. the reference's
     fast_wtconv/cuda_haar/haar_cuda.py:86-105)."""
@@ -21,7 +27,7 @@ def check_kernel_size(kernel_size):
         raise ValueError(f"kernel_size must be odd and positive, got {kernel_size}")
     if torch.compiler.is_compiling():     # no ctypes under tracing; modules check at construction
         return
-    kmax = _lib.load().wtconv_max_kernel_size()
+    kmax = _max_kernel_size()
     if kernel_size > kmax:
         raise ValueError(f"kernel_size {kernel_size} exceeds the largest built kernel ({kmax})")
 
@@ -328,16 +334,19 @@ def _op_autograd_backward(ctx, grad_out):
 _op_forward.register_autograd(_op_autograd_backward, setup_context=_op_setup_context)
 
 
+def _node(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, dims, K, L):
+    """The layer through the C++ autograd node (no interpreter between PyTorch's engine and the library), which checks
+    the arguments itself; None for anything it does not take as it comes: parameters that need a conversion first (mixed
+    dtypes, another device, not contiguous), and whatever has to be refused with a message."""
+    if torch.compiler.is_compiling() or K > _max_kernel_size():
+        return None
+    ext = _ext.get()
+    return None if ext is None else ext.layer(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, dims, K, L)
+
+
 def _apply(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, dims, K, L):
     if torch.compiler.is_compiling():
         return _op_forward(x, base_weight, base_bias, base_scale, list(wt_weights), list(wt_scales), dims)
-    ext = _ext.get()
-    if ext is not None:
-        # the same launches from a C++ autograd node (no interpreter between PyTorch's engine and the library);
-        # None: parameters that need a conversion first (mixed dtypes, another device, not contiguous)
-        out = ext.layer(x, base_weight, base_bias, base_scale, list(wt_weights), list(wt_scales), dims, K, L)
-        if out is not None:
-            return out
     return _WTConvFn.apply(x, base_weight, base_bias, base_scale, dims, K, L, *wt_weights, *wt_scales)
 
 
@@ -361,13 +370,15 @@ def wtconv2d(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, strid
     base_weight (C,1,K,K); base_bias (C,) or None; base_scale (1,C,1,1);
     wt_weights[l] (4C,1,K,K); wt_scales[l] (1,4C,1,1).  Stride sub-samples the stride-1
     result, as the reference does (wtconv2d.py:33-36,84-85)."""
-    _check_input(x, 4, "wtconv2d")
-    C, K, L = x.shape[1], base_weight.shape[-1], len(wt_weights)
-    if not 1 <= L <= _lib.MAX_LEVELS:
-        raise ValueError(f"wt_levels must be 1-{_lib.MAX_LEVELS}, got {L}")
-    check_kernel_size(int(K))
-    _check_params(C, K, L, 4, 2, base_weight, base_bias, base_scale, wt_weights, wt_scales)
-    out = _apply(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 2, int(K), L)
+    K, L = int(base_weight.size(-1)), len(wt_weights)
+    out = _node(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 2, K, L)
+    if out is None:
+        _check_input(x, 4, "wtconv2d")
+        if not 1 <= L <= _lib.MAX_LEVELS:
+            raise ValueError(f"wt_levels must be 1-{_lib.MAX_LEVELS}, got {L}")
+        check_kernel_size(K)
+        _check_params(x.shape[1], K, L, 4, 2, base_weight, base_bias, base_scale, wt_weights, wt_scales)
+        out = _apply(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 2, K, L)
     if stride > 1:
         out = out[:, :, ::stride, ::stride]
     return out
@@ -377,13 +388,15 @@ def wtconv1d(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, strid
     """WTConv1d forward (differentiable).  x (B,C,N); base_weight (C,1,K);
     wt_weights[l] (2C,1,K); scales (1,C,1) / (1,2C,1).  Stride is a true average pool
     (wtconv1d.py:33-36)."""
-    _check_input(x, 3, "wtconv1d")
-    C, K, L = x.shape[1], base_weight.shape[-1], len(wt_weights)
-    if not 1 <= L <= _lib.MAX_LEVELS:
-        raise ValueError(f"wt_levels must be 1-{_lib.MAX_LEVELS}, got {L}")
-    check_kernel_size(int(K))
-    _check_params(C, K, L, 2, 1, base_weight, base_bias, base_scale, wt_weights, wt_scales)
-    out = _apply(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 1, int(K), L)
+    K, L = int(base_weight.size(-1)), len(wt_weights)
+    out = _node(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 1, K, L)
+    if out is None:
+        _check_input(x, 3, "wtconv1d")
+        if not 1 <= L <= _lib.MAX_LEVELS:
+            raise ValueError(f"wt_levels must be 1-{_lib.MAX_LEVELS}, got {L}")
+        check_kernel_size(K)
+        _check_params(x.shape[1], K, L, 2, 1, base_weight, base_bias, base_scale, wt_weights, wt_scales)
+        out = _apply(x, base_weight, base_bias, base_scale, wt_weights, wt_scales, 1, K, L)
     if stride > 1:
         out = torch.nn.functional.avg_pool1d(out, kernel_size=stride, stride=stride)
     return out

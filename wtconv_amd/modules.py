@@ -57,6 +57,22 @@ class _ScaleModule(nn.Module):
         return torch.mul(self.weight, x)
 
 
+def _weight(module):
+    """module.weight, without nn.Module's attribute lookup where it is an ordinary parameter."""
+    w = module._parameters.get("weight")
+    return module.weight if w is None else w
+
+
+def _layer_params(module):
+    """base weight, bias, scale, level weights, level scales of a WTConv2d / WTConv1d (a call reads 3 + 2 L of them, and
+    through `module.base_conv.weight` and the like that alone takes 4 us)."""
+    sub = module._modules
+    base = sub["base_conv"]
+    return (_weight(base), base.bias if "bias" not in base._parameters else base._parameters["bias"],
+            _weight(sub["base_scale"]), [_weight(m) for m in sub["wavelet_convs"]._modules.values()],
+            [_weight(m) for m in sub["wavelet_scale"]._modules.values()])
+
+
 class WTConv2d(nn.Module):
     def __init__(self, in_channels, out_channels, kernel_size=5, stride=1, bias=True, wt_levels=1,
                  wt_type='db1'):
@@ -87,9 +103,7 @@ class WTConv2d(nn.Module):
         self.do_stride = nn.AvgPool2d(kernel_size=1, stride=stride) if stride > 1 else None
 
     def forward(self, x):
-        return Fn.wtconv2d(x, self.base_conv.weight, self.base_conv.bias, self.base_scale.weight,
-                           [m.weight for m in self.wavelet_convs],
-                           [m.weight for m in self.wavelet_scale], stride=self.stride)
+        return Fn.wtconv2d(x, *_layer_params(self), stride=self.stride)
 
     def extra_repr(self):
         return (f"{self.in_channels}, kernel_size={self.kernel_size}, wt_levels={self.wt_levels}, "
@@ -126,9 +140,7 @@ class WTConv1d(nn.Module):
         self.do_stride = nn.AvgPool1d(kernel_size=stride, stride=stride) if stride > 1 else None
 
     def forward(self, x):
-        return Fn.wtconv1d(x, self.base_conv.weight, self.base_conv.bias, self.base_scale.weight,
-                           [m.weight for m in self.wavelet_convs],
-                           [m.weight for m in self.wavelet_scale], stride=self.stride)
+        return Fn.wtconv1d(x, *_layer_params(self), stride=self.stride)
 
     def extra_repr(self):
         return (f"{self.in_channels}, kernel_size={self.kernel_size}, wt_levels={self.wt_levels}, "
@@ -176,5 +188,9 @@ class FastWTConv2d(nn.Module):
             nn.init.kaiming_uniform_(w, a=math.sqrt(5))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return Fn.wtconv2d(x, self.base_weight, self.base_bias, self.base_scale,
+        p = self._parameters
+        if len(p) == 3:
+            return Fn.wtconv2d(x, p["base_weight"], p["base_bias"], p["base_scale"], list(self.wt_weights._parameters.values()),
+                               list(self.wt_scales._parameters.values()), stride=self.stride)
+        return Fn.wtconv2d(x, self.base_weight, self.base_bias, self.base_scale,      # (a parametrized attribute)
                            list(self.wt_weights), list(self.wt_scales), stride=self.stride)
