@@ -7,20 +7,21 @@
 
 #include "common.h"
 #include "host_util.h"
+#include "launch.h"
 #include "mfma2d.h"
 #include "kernels1d.h"
 #include "kernels1d_row.h"
 #include "kernels2d.h"
 #include "kernels2d_stream.h"
 #include "plan.h"
+#ifdef WT_EMULATE      // one translation unit for the host build
+#include "conv1d.hip"
+#include "plane2d.hip"
+#include "stream2d.hip"
+#include "wgrad2d.hip"
+#endif
 
 namespace wt {
-
-// The element type of the activations as the template argument `T_` of a launcher call.
-#define WT_BY_DTYPE(dtype, CALL)                                              \
-  ((dtype) == WTCONV_F32 ? [&] { using T_ = float; return CALL; }()          \
-   : (dtype) == WTCONV_BF16 ? [&] { using T_ = bf16_t; return CALL; }()      \
-                            : [&] { using T_ = f16_t; return CALL; }())
 
 // Threads of wgrad_finish_kernel: one per entry of a channel's record (taps of every filter + sumG) where that fits.
 static inline int finish_threads(int nrec) { return nrec >= 1024 ? 1024 : (nrec + kWave - 1) / kWave * kWave; }
@@ -62,128 +63,6 @@ static int launch_fold(const wtconv_params* params, int pdtype, float* fw, float
   return check_launch("fold_params_kernel");
 }
 
-// ---- 2-D dispatch over (dtype, K, level-1 strip width) -------------------------------
-template <typename T, int K, int TJ1, int MODE, typename Geo = PlaneGeoRuntime>
-static int run_plane2d_mode(const void* x, void* out, const float* fw, const float* fb, const Plan2D& pl,
-                            hipStream_t stream) {
-  auto kern = wt2d_plane_kernel<T, K, TJ1, kTJC, MODE, Geo>;
-  const size_t lds = static_cast<size_t>(pl.lds_floats) * sizeof(float);
-  if (int e = allow_lds(kern, lds)) return e;
-  const int sg = 1 << pl.sg_shift;
-  const int slots = pl.block / sg;
-  const int nunits = sg < kWave ? (pl.C * pl.groups_per_channel + 3) / 4 : (pl.nplanes + slots - 1) / slots;
-  int nwg = compute_units() * resident_per_cu(kern, pl.block, lds);
-  if (nwg > nunits) nwg = nunits;
-  WT_LAUNCH(kern, dim3(nwg), dim3(pl.block), lds, stream, static_cast<const T*>(x), static_cast<T*>(out), fw, fb, pl);
-  return check_launch("wt2d_plane_kernel");
-}
-
-// Plane shapes of the WTConvNeXt stages with K = 5: geometry as a compile-time constant.  Returns 1 if the shape
-// is not one of them (or the run-time plan differs, e.g. unaligned pointers), else the launch's result.
-template <typename T>
-static int run_plane2d_static(int K, int tj1, const void* x, void* out, const float* fw, const float* fb,
-                              const Plan2D& pl, hipStream_t stream) {
-  if (K != 5 || pl.H != pl.W) return 1;
-#define WT_TRY(H_, L_)                                                                                  \
-  if (pl.H == H_ && pl.L == L_) {                                                                       \
-    using G = PlaneGeoStatic<H_, H_, 5, L_>;                                                            \
-    constexpr Plan2D g = G::plan();                                                                     \
-    if (tj1 == G::tj1() && same_plane_geometry(g, pl))                                                  \
-      return run_plane2d_mode<T, 5, G::tj1(), G::mode(), G>(x, out, fw, fb, pl, stream);                \
-    return 1;                                                                                           \
-  }
-  WT_TRY(56, 3) WT_TRY(28, 3) WT_TRY(14, 2) WT_TRY(7, 2)
-#undef WT_TRY
-  return 1;
-}
-
-template <typename T, int K, int TJ1>
-static int run_plane2d(const void* x, void* out, const float* fw, const float* fb, const Plan2D& pl,
-                       hipStream_t stream) {
-  if (pl.prefetch && pl.fuse >= 2) return run_plane2d_mode<T, K, TJ1, 3>(x, out, fw, fb, pl, stream);
-  if (pl.prefetch) return run_plane2d_mode<T, K, TJ1, 0>(x, out, fw, fb, pl, stream);
-  if (pl.vec_ok) return run_plane2d_mode<T, K, TJ1, 1>(x, out, fw, fb, pl, stream);
-  return run_plane2d_mode<T, K, TJ1, 2>(x, out, fw, fb, pl, stream);
-}
-
-template <typename T, int K>
-static int run_plane2d_tj(int tj1, const void* x, void* out, const float* fw, const float* fb, const Plan2D& pl,
-                          hipStream_t stream) {
-  switch (tj1) {
-    case 1: return run_plane2d<T, K, 1>(x, out, fw, fb, pl, stream);
-    case 2: return run_plane2d<T, K, 2>(x, out, fw, fb, pl, stream);
-    default: return run_plane2d<T, K, 4>(x, out, fw, fb, pl, stream);
-  }
-}
-
-template <typename T>
-static int run_plane2d_k(int K, int tj1, const void* x, void* out, const float* fw, const float* fb,
-                         const Plan2D& pl, hipStream_t stream) {
-  switch (K) {
-    case 1: return run_plane2d_tj<T, 1>(tj1, x, out, fw, fb, pl, stream);
-    case 3: return run_plane2d_tj<T, 3>(tj1, x, out, fw, fb, pl, stream);
-    case 5: return run_plane2d_tj<T, 5>(tj1, x, out, fw, fb, pl, stream);
-    case 7: return run_plane2d_tj<T, 7>(tj1, x, out, fw, fb, pl, stream);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
-}
-
-template <typename T, int K, int L, typename Geo = PlaneGeoRuntime>
-static int run_wgrad2d(const void* x, const void* g, float* partial, const Plan2D& pl, int B, int bchunk,
-                       int nchunk, const FinishArgs& fin, hipStream_t stream) {
-  auto kern = wt2d_wgrad_kernel<T, K, L, kTJW, Geo>;
-  const size_t lds = static_cast<size_t>(pl.lds_floats) * sizeof(float);
-  if (int e = allow_lds(kern, lds)) return e;
-  WT_LAUNCH(kern, dim3(pl.C, nchunk), dim3(512), lds, stream, static_cast<const T*>(x), static_cast<const T*>(g),
-            partial, pl, B, bchunk, fin);
-  return check_launch("wt2d_wgrad_kernel");
-}
-
-// Plane shapes of the WTConvNeXt stages with K = 5 at their usual planes per iteration: geometry as a compile-time
-// constant.  Returns 1 if the launch is not one of them, else the launch's result.
-template <typename T>
-static int run_wgrad2d_static(int K, int L, const void* x, const void* g, float* partial, const Plan2D& pl, int B,
-                              int bchunk, int nchunk, const FinishArgs& fin, hipStream_t stream) {
-  if (K != 5 || pl.H != pl.W) return 1;
-#define WT_TRY(H_, L_)                                                                                   \
-  if (pl.H == H_ && L == L_) {                                                                           \
-    constexpr int PB = wgrad_planes_per_iter(128, H_, H_, 5, L_);                                        \
-    using G = WgradGeoStatic<H_, H_, 5, L_, PB>;                                                         \
-    constexpr Plan2D gp = G::plan();                                                                     \
-    if (same_wgrad_geometry(gp, pl))                                                                     \
-      return run_wgrad2d<T, 5, L_, G>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);                     \
-    return 1;                                                                                            \
-  }
-  WT_TRY(56, 3) WT_TRY(28, 3) WT_TRY(14, 2) WT_TRY(7, 2)
-#undef WT_TRY
-  return 1;
-}
-
-template <typename T, int K>
-static int run_wgrad2d_l(int L, const void* x, const void* g, float* partial, const Plan2D& pl, int B,
-                         int bchunk, int nchunk, const FinishArgs& fin, hipStream_t stream) {
-  switch (L) {
-    case 1: return run_wgrad2d<T, K, 1>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 2: return run_wgrad2d<T, K, 2>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 3: return run_wgrad2d<T, K, 3>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 4: return run_wgrad2d<T, K, 4>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 5: return run_wgrad2d<T, K, 5>(x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-  }
-  return fail(WTCONV_E_ARG, "wt_levels %d", L);
-}
-
-template <typename T>
-static int run_wgrad2d_k(int K, int L, const void* x, const void* g, float* partial, const Plan2D& pl, int B,
-                         int bchunk, int nchunk, const FinishArgs& fin, hipStream_t stream) {
-  switch (K) {
-    case 1: return run_wgrad2d_l<T, 1>(L, x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 3: return run_wgrad2d_l<T, 3>(L, x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 5: return run_wgrad2d_l<T, 5>(L, x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-    case 7: return run_wgrad2d_l<T, 7>(L, x, g, partial, pl, B, bchunk, nchunk, fin, stream);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
-}
-
 // ---- planes that do not fit LDS: level-by-level kernels through an HBM pyramid ----------
 static size_t lds_fit_limit() {
 #ifdef WT_EMULATE   // host emulation only: send small planes through the level-by-level kernels
@@ -202,7 +81,6 @@ static bool wgrad_fits_lds(int B, int C, int H, int W, int K, int L) {
   return static_cast<size_t>(pl.plane_lds_floats) * 4 <= lds_fit_limit();
 }
 
-static size_t round_up64(size_t v) { return (v + 63) / 64 * 64; }
 constexpr long long kMaxPlaneElems = 1LL << 28;
 
 static Stream2D make_stream2d(int B, int C, int H, int W, int L) {
@@ -239,122 +117,6 @@ static int stream_chunks(int B, int C, int H, int W) {
   return static_cast<int>(want);
 }
 
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
-// `ll_only`: the level-1 detail bands are not stored (forward / input-gradient pass: its last
-// synthesis level rebuilds them from the pixels; the weight-gradient pass needs them).
-template <typename T>
-static int stream_analysis_chain(const T* src, float* pyr, const Stream2D& sp, hipStream_t stream, bool ll_only) {
-  const unsigned gy = sp.nplanes < 65535 ? sp.nplanes : 65535;
-  for (int l = 1; l <= sp.L; ++l) {
-    const int n = sp.h[l] * sp.w[l];
-    const unsigned gx = static_cast<unsigned>((n + 255) / 256);
-    if (l == 1 && ll_only) {
-      WT_LAUNCH((stream_analysis_kernel<T, true>), dim3(gx, gy), dim3(256), 0, stream, src,
-                static_cast<size_t>(sp.H) * sp.W, sp.H, sp.W, pyr + sp.aoff[1], sp.h[1], sp.w[1], sp.nplanes);
-    } else if (l == 1) {
-      WT_LAUNCH((stream_analysis_kernel<T, false>), dim3(gx, gy), dim3(256), 0, stream, src,
-                static_cast<size_t>(sp.H) * sp.W, sp.H, sp.W, pyr + sp.aoff[1], sp.h[1], sp.w[1], sp.nplanes);
-    } else {
-      WT_LAUNCH((stream_analysis_kernel<float, false>), dim3(gx, gy), dim3(256), 0, stream,
-                static_cast<const float*>(pyr + sp.aoff[l - 1]), static_cast<size_t>(4) * sp.h[l - 1] * sp.w[l - 1],
-                sp.h[l - 1], sp.w[l - 1], pyr + sp.aoff[l], sp.h[l], sp.w[l], sp.nplanes);
-    }
-    if (int e = check_launch("stream_analysis_kernel")) return e;
-  }
-  return 0;
-}
-
-// `have_pyramid`: the pyramid of x is in `pyr` already (the whole backward pass shares the one of grad_out).
-template <typename T, int K>
-static int run_stream2d(const void* x_, void* out_, const float* fw, const float* fb, float* pyr, const Stream2D& sp,
-                        hipStream_t stream, bool have_pyramid = false) {
-  const T* x = static_cast<const T*>(x_);
-  T* out = static_cast<T*>(out_);
-  if (sp.L > 1 && !have_pyramid) {      // a single level is synthesised from the pixels alone
-    if (int e = stream_analysis_chain<T>(x, pyr, sp, stream, true)) return e;
-  }
-  const unsigned gy = sp.nplanes < 65535 ? sp.nplanes : 65535;
-  const unsigned gz = (sp.nplanes + gy - 1) / gy;
-  const int NF = 1 + 4 * sp.L;
-  for (int l = sp.L; l >= 1; --l) {
-    const unsigned tiles = static_cast<unsigned>(((sp.h[l] + kStreamTile - 1) / kStreamTile) *
-                                                 ((sp.w[l] + kStreamTileW - 1) / kStreamTileW));
-    const float* zin = l < sp.L ? pyr + sp.zoff[l + 1] : nullptr;
-    const bool io_ok = l > 1 || (aligned16(x) && aligned16(out));
-    const int vec = (sp.w[l] % 4 == 0 && aligned16(pyr) ? 1 : 0) | (sp.w[l - 1] % 4 == 0 && io_ok ? 2 : 0);
-    if (l > 1) {
-      WT_LAUNCH((stream_synth_kernel<T, K, false>), dim3(tiles, gy, gz), dim3(256), 0, stream,
-                static_cast<const float*>(pyr + sp.aoff[l]), sp.h[l], sp.w[l], zin, pyr + sp.zoff[l], sp.h[l - 1],
-                sp.w[l - 1], static_cast<const T*>(nullptr), static_cast<T*>(nullptr), fw, fb, sp.C, NF,
-                1 + 4 * (l - 1), sp.nplanes, vec);
-    } else {
-      WT_LAUNCH((stream_synth_kernel<T, K, true>), dim3(tiles, gy, gz), dim3(256), 0, stream,
-                static_cast<const float*>(pyr + sp.aoff[1]), sp.h[1], sp.w[1], zin, static_cast<float*>(nullptr), sp.H,
-                sp.W, x, out, fw, fb, sp.C, NF, 1, sp.nplanes, vec);
-    }
-    if (int e = check_launch("stream_synth_kernel")) return e;
-  }
-  return 0;
-}
-
-template <typename T>
-static int run_stream2d_k(int K, const void* x, void* out, const float* fw, const float* fb, float* pyr,
-                          const Stream2D& sp, hipStream_t stream, bool have_pyramid = false) {
-  switch (K) {
-    case 1: return run_stream2d<T, 1>(x, out, fw, fb, pyr, sp, stream, have_pyramid);
-    case 3: return run_stream2d<T, 3>(x, out, fw, fb, pyr, sp, stream, have_pyramid);
-    case 5: return run_stream2d<T, 5>(x, out, fw, fb, pyr, sp, stream, have_pyramid);
-    case 7: return run_stream2d<T, 7>(x, out, fw, fb, pyr, sp, stream, have_pyramid);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
-}
-
-// `have_g_pyramid`: the pyramid of grad_out is in `pyr_g` already (left there by the input-gradient pass of the same call).
-template <typename T, int K>
-static int run_stream2d_wgrad(const void* x_, const void* g_, float* partial, float* pyr_x, float* pyr_g,
-                              const Stream2D& sp, int B, int nchunk, hipStream_t stream, bool have_g_pyramid = false) {
-  const T* x = static_cast<const T*>(x_);
-  const T* g = static_cast<const T*>(g_);
-  if (int e = stream_analysis_chain<T>(x, pyr_x, sp, stream, false)) return e;
-  if (!have_g_pyramid)
-    if (int e = stream_analysis_chain<T>(g, pyr_g, sp, stream, false)) return e;
-  const int rec = (1 + 4 * sp.L) * K * K + 1;
-  const bool pyr_ok = aligned16(pyr_x) && aligned16(pyr_g);
-  // chunks of a launch: at least four (batch item, tile) units per workgroup where the level has them
-  auto level_chunks = [&](int h, int w) {
-    const long units = static_cast<long>(B) * ((h + kStreamTile - 1) / kStreamTile) *
-                       ((w + kStreamTileW - 1) / kStreamTileW);
-    const long nc = units / 4;
-    return static_cast<unsigned>(nc < 1 ? 1 : (nc > nchunk ? nchunk : nc));
-  };
-  WT_LAUNCH((stream_corr_kernel<T, K>), dim3(sp.C, level_chunks(sp.H, sp.W)), dim3(256), 0, stream, x, g,
-            static_cast<size_t>(sp.H) * sp.W, static_cast<size_t>(0), sp.H, sp.W, partial, rec, 0, 1, 1, B, sp.C,
-            (sp.W % 4 == 0 && aligned16(x) && aligned16(g)) ? 1 : 0, nchunk);
-  if (int e = check_launch("stream_corr_kernel")) return e;
-  for (int l = 1; l <= sp.L; ++l) {
-    const size_t n = static_cast<size_t>(sp.h[l]) * sp.w[l];
-    WT_LAUNCH((stream_corr_kernel<float, K>), dim3(sp.C * 4, level_chunks(sp.h[l], sp.w[l])), dim3(256), 0, stream,
-              static_cast<const float*>(pyr_x + sp.aoff[l]), static_cast<const float*>(pyr_g + sp.aoff[l]), 4 * n, n,
-              sp.h[l], sp.w[l], partial, rec, 1 + 4 * (l - 1), 4, 0, B, sp.C,
-              (sp.w[l] % 4 == 0 && pyr_ok) ? 1 : 0, nchunk);
-    if (int e = check_launch("stream_corr_kernel")) return e;
-  }
-  return 0;
-}
-
-template <typename T>
-static int run_stream2d_wgrad_k(int K, const void* x, const void* g, float* partial, float* pyr_x, float* pyr_g,
-                                const Stream2D& sp, int B, int nchunk, hipStream_t stream, bool have_g_pyramid = false) {
-  switch (K) {
-    case 1: return run_stream2d_wgrad<T, 1>(x, g, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
-    case 3: return run_stream2d_wgrad<T, 3>(x, g, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
-    case 5: return run_stream2d_wgrad<T, 5>(x, g, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
-    case 7: return run_stream2d_wgrad<T, 7>(x, g, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
-}
-
 // `shared_pyr` (level-by-level path only): where to build the whole pyramid of x -- detail bands of level 1 included --
 // for a later pass of the same call to reuse; the folded parameters then go to `shared_fw` instead of the workspace start.
 // `tickets` (plane-resident paths only): C words this pass clears on its way, for the parameter-gradient pass that
@@ -386,9 +148,9 @@ static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_p
     float* pyr = shared_pyr != nullptr ? shared_pyr : fw + round_up64(fold_floats(C, 4, L, K * K));
     if (int e = launch_fold(params, pdtype, fw, fb, C, 4, L, K * K, flip, flip ? 0 : 1, stream)) return e;
     if (shared_pyr != nullptr) {
-      if (int e = WT_BY_DTYPE(dtype, stream_analysis_chain<T_>(static_cast<const T_*>(x), pyr, sp, stream, false))) return e;
+      if (int e = launch_stream_analysis(dtype, x, pyr, sp, stream, false)) return e;
     }
-    return WT_BY_DTYPE(dtype, run_stream2d_k<T_>(K, x, out, fw, fb, pyr, sp, stream, shared_pyr != nullptr));
+    return launch_stream2d(dtype, K, x, out, fw, fb, pyr, sp, stream, shared_pyr != nullptr);
   }
   Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256, esz, x, out, nullptr);
   int tj1 = 4, sg_shift = 8;
@@ -403,77 +165,7 @@ static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_p
   float* fw = static_cast<float*>(ws);
   float* fb = fw + static_cast<size_t>(C) * (1 + 4 * L) * K * K;
   if (int e = launch_fold(params, pdtype, fw, fb, C, 4, L, K * K, flip, flip ? 0 : 1, stream, tickets, C)) return e;
-  if (dtype != WTCONV_BF16) {     // (bf16 tensors of these shapes are on the matrix-core kernels)
-    const int e = dtype == WTCONV_F32 ? run_plane2d_static<float>(K, tj1, x, out, fw, fb, pl, stream)
-                                      : run_plane2d_static<f16_t>(K, tj1, x, out, fw, fb, pl, stream);
-    if (e != 1) return e;
-  }
-  return WT_BY_DTYPE(dtype, run_plane2d_k<T_>(K, tj1, x, out, fw, fb, pl, stream));
-}
-
-// ---- 1-D dispatch -------------------------------------------------------------------
-template <typename T, int K>
-static int run_tile1d(const void* x, void* out, const float* fw, const float* fb, const Plan1D& pl, int B,
-                      hipStream_t stream) {
-  auto kern = wt1d_tile_kernel<T, K, kTJ1D>;
-  const size_t lds = static_cast<size_t>(pl.lds_floats) * sizeof(float);
-  if (int e = allow_lds(kern, lds)) return e;
-  const long long nrows = static_cast<long long>(B) * pl.C;
-  if (nrows > 0x7fffffffLL) return fail(WTCONV_E_UNSUPPORTED, "batch*channels = %lld is too large", nrows);
-  const unsigned gy = nrows < 65535 ? static_cast<unsigned>(nrows) : 65535u;
-  const unsigned gz = static_cast<unsigned>((nrows + gy - 1) / gy);
-  if (gz > 65535u) return fail(WTCONV_E_UNSUPPORTED, "batch*channels = %lld is too large", nrows);
-  WT_LAUNCH(kern, dim3(pl.ntiles, gy, gz), dim3(kBlock1D), lds, stream, static_cast<const T*>(x),
-            static_cast<T*>(out), fw, fb, pl, static_cast<int>(nrows));
-  return check_launch("wt1d_tile_kernel");
-}
-
-template <typename T>
-static int run_tile1d_k(int K, const void* x, void* out, const float* fw, const float* fb, const Plan1D& pl,
-                        int B, hipStream_t stream) {
-  switch (K) {
-    case 1: return run_tile1d<T, 1>(x, out, fw, fb, pl, B, stream);
-    case 3: return run_tile1d<T, 3>(x, out, fw, fb, pl, B, stream);
-    case 5: return run_tile1d<T, 5>(x, out, fw, fb, pl, B, stream);
-    case 7: return run_tile1d<T, 7>(x, out, fw, fb, pl, B, stream);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
-}
-
-template <typename T, int K, int L>
-static int run_wgrad1d(const void* x, const void* g, float* partial, const Plan1D& pl, int B, int per_chunk,
-                       int nchunk, hipStream_t stream) {
-  auto kern = wt1d_wgrad_kernel<T, K, L, kTJ1D>;
-  const size_t lds = static_cast<size_t>(pl.lds_floats) * sizeof(float);
-  if (int e = allow_lds(kern, lds)) return e;
-  WT_LAUNCH(kern, dim3(pl.C, nchunk), dim3(kBlock1D), lds, stream, static_cast<const T*>(x),
-            static_cast<const T*>(g), partial, pl, B, per_chunk);
-  return check_launch("wt1d_wgrad_kernel");
-}
-
-template <typename T, int K>
-static int run_wgrad1d_l(int L, const void* x, const void* g, float* partial, const Plan1D& pl, int B,
-                         int per_chunk, int nchunk, hipStream_t stream) {
-  switch (L) {
-    case 1: return run_wgrad1d<T, K, 1>(x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 2: return run_wgrad1d<T, K, 2>(x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 3: return run_wgrad1d<T, K, 3>(x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 4: return run_wgrad1d<T, K, 4>(x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 5: return run_wgrad1d<T, K, 5>(x, g, partial, pl, B, per_chunk, nchunk, stream);
-  }
-  return fail(WTCONV_E_ARG, "wt_levels %d", L);
-}
-
-template <typename T>
-static int run_wgrad1d_k(int K, int L, const void* x, const void* g, float* partial, const Plan1D& pl, int B,
-                         int per_chunk, int nchunk, hipStream_t stream) {
-  switch (K) {
-    case 1: return run_wgrad1d_l<T, 1>(L, x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 3: return run_wgrad1d_l<T, 3>(L, x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 5: return run_wgrad1d_l<T, 5>(L, x, g, partial, pl, B, per_chunk, nchunk, stream);
-    case 7: return run_wgrad1d_l<T, 7>(L, x, g, partial, pl, B, per_chunk, nchunk, stream);
-  }
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d is not built", K);
+  return launch_plane2d(dtype, K, tj1, x, out, fw, fb, pl, stream);
 }
 
 // ---- row-resident 1-D kernels ----------------------------------------------------------
@@ -501,19 +193,6 @@ static Row1D make_row1d(int C, int N, int nl, size_t esz, const void* p0, const 
   return r;
 }
 
-// Batch chunks of a row-resident kernel: C * nchunk workgroups that all run at once (one round: a second, partly
-// filled round costs as much as a full one), `per_cu` of them per CU on 256 CUs -- constants, so that workspace
-// sizes do not depend on the device queried.
-static void row1d_chunks(int B, int C, int per_cu, int* per_chunk, int* nchunk) {
-  if (per_cu < 1) per_cu = 1;
-  int want = 256 * per_cu / C;
-  if (want < 1) want = 1;
-  if (want > B) want = B;
-  const int pc = (B + want - 1) / want;
-  *per_chunk = pc;
-  *nchunk = (B + pc - 1) / pc;
-}
-
 // Workgroups per CU the kernels with two slot regions (parameter gradients, fused backward) are planned for: what
 // LDS allows, at most two waves per SIMD (they need up to 256 registers).
 static int row1d_two_region_per_cu(int K, int L, const Row1DShape& sh) {
@@ -521,109 +200,6 @@ static int row1d_two_region_per_cu(int K, int L, const Row1DShape& sh) {
   int per_cu = static_cast<int>(kLdsLimitBytes / lds);
   if (per_cu > 512 / sh.block) per_cu = 512 / sh.block;
   return per_cu < 1 ? 1 : per_cu;
-}
-
-template <typename T, int K, int L, int S>
-static int run_row1d(const void* x, void* out, const wtconv_params* params, int pdtype, int flip, const Row1D& pl,
-                     int B, int block, hipStream_t stream) {
-  if constexpr (row1d_built(K, L, S)) {
-    auto kern = wt1d_row_kernel<T, K, L, S>;
-    const size_t lds = row1d_region(K, L, S, block) * sizeof(float);
-    if (int e = allow_lds(kern, lds)) return e;
-    int per_chunk, nchunk;
-    row1d_chunks(B, pl.C, resident_per_cu(kern, block, lds), &per_chunk, &nchunk);   // (no workspace depends on this)
-    if (nchunk > 65535) return fail(WTCONV_E_UNSUPPORTED, "too many batch chunks (%d)", nchunk);
-    WT_LAUNCH(kern, dim3(pl.C, nchunk), dim3(block), lds, stream, static_cast<const T*>(x), static_cast<T*>(out),
-              to_table(params, L), pdtype, flip, pl, B, per_chunk);
-    return check_launch("wt1d_row_kernel");
-  } else {
-    return fail(WTCONV_E_UNSUPPORTED, "row-resident 1-D kernel not built for kernel_size %d, %d levels", K, L);
-  }
-}
-
-// The fused backward kernel: grad_x, the chunks' partial sums and (by the last workgroup of each channel) the
-// parameter gradients.  `tickets`: C words, cleared by a launch of their own right before.
-template <typename T, int K, int L, int S>
-static int run_row1d_bwd(const void* x, const void* g, void* gx, float* partial, unsigned* tickets,
-                         const wtconv_params* params, int pdtype, const GradTable& gt, const Row1D& pl, int B,
-                         int block, int per_chunk, int nchunk, hipStream_t stream) {
-  if constexpr (row1d_bwd_built(K, L, S)) {
-    auto kern = wt1d_row_bwd_kernel<T, K, L, S>;
-    const size_t lds = 2 * row1d_region(K, L, S, block) * sizeof(float);
-    if (int e = allow_lds(kern, lds)) return e;
-    WT_LAUNCH(zero_tickets_kernel, dim3((pl.C + 255) / 256), dim3(256), 0, stream, tickets, pl.C);
-    if (int e = check_launch("zero_tickets_kernel")) return e;
-    WT_LAUNCH(kern, dim3(pl.C, nchunk), dim3(block), lds, stream, static_cast<const T*>(x),
-              static_cast<const T*>(g), static_cast<T*>(gx), partial, tickets, to_table(params, L), pdtype, gt, pl, B,
-              per_chunk, nchunk);
-    return check_launch("wt1d_row_bwd_kernel");
-  } else {
-    return fail(WTCONV_E_UNSUPPORTED, "row-resident 1-D kernel not built for kernel_size %d, %d levels", K, L);
-  }
-}
-
-template <typename T, int K, int L, int S>
-static int run_row1d_wgrad(const void* x, const void* g, float* partial, const Row1D& pl, int B, int block,
-                           int per_chunk, int nchunk, hipStream_t stream) {
-  if constexpr (row1d_built(K, L, S)) {
-    auto kern = wt1d_row_wgrad_kernel<T, K, L, S>;
-    const size_t lds = 2 * row1d_region(K, L, S, block) * sizeof(float);
-    if (int e = allow_lds(kern, lds)) return e;
-    WT_LAUNCH(kern, dim3(pl.C, nchunk), dim3(block), lds, stream, static_cast<const T*>(x),
-              static_cast<const T*>(g), partial, pl, B, per_chunk);
-    return check_launch("wt1d_row_wgrad_kernel");
-  } else {
-    return fail(WTCONV_E_UNSUPPORTED, "row-resident 1-D kernel not built for kernel_size %d, %d levels", K, L);
-  }
-}
-
-#define WT_ROW1D_SWITCH_S(T, K, L, CALL)                              \
-  return S == 16 ? CALL(T, K, L, 16) : CALL(T, K, L, 32);
-#define WT_ROW1D_SWITCH_L(T, K, CALL)                                 \
-  switch (L) {                                                        \
-    case 1: WT_ROW1D_SWITCH_S(T, K, 1, CALL)                          \
-    case 2: WT_ROW1D_SWITCH_S(T, K, 2, CALL)                          \
-    case 3: WT_ROW1D_SWITCH_S(T, K, 3, CALL)                          \
-    case 4: WT_ROW1D_SWITCH_S(T, K, 4, CALL)                          \
-    case 5: WT_ROW1D_SWITCH_S(T, K, 5, CALL)                          \
-  }                                                                   \
-  break;
-#define WT_ROW1D_SWITCH(T, CALL)                                      \
-  switch (K) {                                                        \
-    case 3: WT_ROW1D_SWITCH_L(T, 3, CALL)                             \
-    case 5: WT_ROW1D_SWITCH_L(T, 5, CALL)                             \
-    case 7: WT_ROW1D_SWITCH_L(T, 7, CALL)                             \
-  }
-
-template <typename T>
-static int run_row1d_kl(int K, int L, int S, const void* x, void* out, const wtconv_params* params, int pdtype,
-                        int flip, const Row1D& pl, int B, int block, hipStream_t stream) {
-#define WT_CALL(T_, K_, L_, S_) run_row1d<T_, K_, L_, S_>(x, out, params, pdtype, flip, pl, B, block, stream)
-  WT_ROW1D_SWITCH(T, WT_CALL)
-#undef WT_CALL
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d / %d levels not built", K, L);
-}
-
-template <typename T>
-static int run_row1d_bwd_kl(int K, int L, int S, const void* x, const void* g, void* gx, float* partial,
-                            unsigned* tickets, const wtconv_params* params, int pdtype, const GradTable& gt,
-                            const Row1D& pl, int B, int block, int per_chunk, int nchunk, hipStream_t stream) {
-#define WT_CALL(T_, K_, L_, S_)                                                                                 \
-  run_row1d_bwd<T_, K_, L_, S_>(x, g, gx, partial, tickets, params, pdtype, gt, pl, B, block, per_chunk, nchunk, \
-                                stream)
-  WT_ROW1D_SWITCH(T, WT_CALL)
-#undef WT_CALL
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d / %d levels not built", K, L);
-}
-
-template <typename T>
-static int run_row1d_wgrad_kl(int K, int L, int S, const void* x, const void* g, float* partial, const Row1D& pl,
-                              int B, int block, int per_chunk, int nchunk, hipStream_t stream) {
-#define WT_CALL(T_, K_, L_, S_) \
-  run_row1d_wgrad<T_, K_, L_, S_>(x, g, partial, pl, B, block, per_chunk, nchunk, stream)
-  WT_ROW1D_SWITCH(T, WT_CALL)
-#undef WT_CALL
-  return fail(WTCONV_E_UNSUPPORTED, "kernel_size %d / %d levels not built", K, L);
 }
 
 static int tile1d_pass(const char* fn, const void* x, void* out, const wtconv_params* params, int B, int C,
@@ -644,12 +220,12 @@ static int tile1d_pass(const char* fn, const void* x, void* out, const wtconv_pa
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   if (row_resident) {      // (these kernels fold their channel's parameters themselves: no fold launch, no table)
     const Row1D rp = make_row1d(C, N, sh.nl, esz, x, out);
-    return WT_BY_DTYPE(dtype, run_row1d_kl<T_>(K, L, sh.S, x, out, params, pdtype, flip, rp, B, sh.block, stream));
+    return launch_row1d(dtype, K, L, sh.S, x, out, params, pdtype, flip, rp, B, sh.block, stream);
   }
   float* fw = static_cast<float*>(ws);
   float* fb = fw + static_cast<size_t>(C) * (1 + 2 * L) * K;
   if (int e = launch_fold(params, pdtype, fw, fb, C, 2, L, K, flip, flip ? 0 : 1, stream)) return e;
-  return WT_BY_DTYPE(dtype, run_tile1d_k<T_>(K, x, out, fw, fb, pl, B, stream));
+  return launch_tile1d(dtype, K, x, out, fw, fb, pl, B, stream);
 }
 
 // ---- static scratch for callers that may not allocate ------------------------------------
@@ -843,19 +419,14 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
     Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, esz, x, grad_out, nullptr, pb);
     finish_wgrad_plan(&pl, K);
     wgrad_chunks(B, C, pb, kWgradResident, &bchunk, &nchunk);
-    e = dtype == WTCONV_F32   ? run_wgrad2d_static<float>(K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream)
-        : dtype == WTCONV_F16 ? run_wgrad2d_static<f16_t>(K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream)
-                              : 1;
-    if (e == 1)
-      e = WT_BY_DTYPE(dtype, run_wgrad2d_k<T_>(K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream));
+    e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream);
   } else {
     const Stream2D sp = make_stream2d(B, C, H, W, L);
     nchunk = stream_chunks(B, C, H, W);
     if (nchunk > 65535 || C > 0x7fffffff / 4) return fail(WTCONV_E_UNSUPPORTED, "%s: too many chunks (%d)", fn, nchunk);
     float* pyr_x = partial + round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * L) * K * K + 1));
     float* pyr_g = pyr_x + sp.floats;
-    e = WT_BY_DTYPE(dtype, run_stream2d_wgrad_k<T_>(K, x, grad_out, partial, pyr_x, pyr_g, sp, B, nchunk, stream,
-                                                    have_g_pyramid));
+    e = launch_stream2d_wgrad(dtype, K, x, grad_out, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
   }
   if (e || resident) return e;
   const GradTable gt = to_grad_table(grads, L);
@@ -996,10 +567,9 @@ int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_p
   int e;
   if (row_resident) {
     const Row1D rp = make_row1d(C, N, sh.nl, esz, x, grad_out);
-    e = WT_BY_DTYPE(dtype, run_row1d_wgrad_kl<T_>(K, L, sh.S, x, grad_out, partial, rp, B, sh.block, per_chunk, nchunk,
-                                                  stream));
+    e = launch_row1d_wgrad(dtype, K, L, sh.S, x, grad_out, partial, rp, B, sh.block, per_chunk, nchunk, stream);
   } else {
-    e = WT_BY_DTYPE(dtype, run_wgrad1d_k<T_>(K, L, x, grad_out, partial, pl, B, per_chunk, nchunk, stream));
+    e = launch_wgrad1d(dtype, K, L, x, grad_out, partial, pl, B, per_chunk, nchunk, stream);
   }
   if (e) return e;
   GradTable gt = {};
@@ -1043,9 +613,8 @@ int wtconv1d_backward(const void* x, const void* grad_out, void* grad_x, const w
     Row1D rp = make_row1d(C, N, sh.nl, esz, x, grad_out);
     rp.vec_ok = rp.vec_ok && (reinterpret_cast<uintptr_t>(grad_x) & 15u) == 0;
     const GradTable gt = to_grad_table(grads, L);
-    return WT_BY_DTYPE(dtype, run_row1d_bwd_kl<T_>(K, L, sh.S, x, grad_out, grad_x, partial, tickets, params, param_dtype,
-                                                    gt, rp, B, sh.block, per_chunk, nchunk,
-                                                    static_cast<hipStream_t>(stream)));
+    return launch_row1d_bwd(dtype, K, L, sh.S, x, grad_out, grad_x, partial, tickets, params, param_dtype, gt, rp, B, sh.block,
+                            per_chunk, nchunk, static_cast<hipStream_t>(stream));
   }
   if (int e = wtconv1d_backward_input(grad_out, grad_x, params, B, C, N, K, levels, dtype, param_dtype, workspace,
                                       workspace_bytes, stream))

@@ -56,7 +56,7 @@ struct Plan2D {
 // fw[c][f][t]: f = 0 base conv, f = 1 + S*l + s level l sub-band s; value gamma * w, taps
 // reversed when flip != 0.  fb[c] = gamma_b * bias (0 without bias).  Also clears the `nzero` words at `zero_words`
 // (the channel tickets of a parameter-gradient pass that follows on the stream).
-__global__ void fold_params_kernel(ParamTable p, int pdtype, float* __restrict__ fw,
+static __global__ void fold_params_kernel(ParamTable p, int pdtype, float* __restrict__ fw,
                                    float* __restrict__ fb, int C, int S, int L, int KK,
                                    int flip, int use_bias, unsigned* __restrict__ zero_words, int nzero) {
   const int NF = 1 + S * L;
@@ -1080,7 +1080,7 @@ __global__ __launch_bounds__(512, 4) void wt2d_wgrad_kernel(const T* __restrict_
 
 // The second stage as a launch of its own (one workgroup per channel, dynamic LDS NF*KK + 1 floats): after a first
 // stage that does not finish its channels itself.
-__global__ void wgrad_finish_kernel(const float* __restrict__ partial, int nchunk, ParamTable p,
+static __global__ void wgrad_finish_kernel(const float* __restrict__ partial, int nchunk, ParamTable p,
                                     int pdtype, GradTable gt, int C, int S, int L, int KK) {
   WT_SHARED_FLOATS(prod);
   wgrad_finish_channel<false>(partial, nchunk, p, pdtype, gt, C, static_cast<int>(blockIdx.x), S, L, KK, prod);
@@ -1088,7 +1088,7 @@ __global__ void wgrad_finish_kernel(const float* __restrict__ partial, int nchun
 
 // Clears the ticket words of a first stage that finishes its channels itself (a kernel rather than a memset, so
 // that a caller may record the call into a HIP graph).
-__global__ void zero_tickets_kernel(unsigned* __restrict__ t, int n) {
+static __global__ void zero_tickets_kernel(unsigned* __restrict__ t, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) t[i] = 0u;
 }
 
