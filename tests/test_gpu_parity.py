@@ -186,13 +186,39 @@ def test_config4_1d_small_batch(hip_device):
     ((1, 1, 1), 3, 1, True, 1),
     ((3, 2, 517), 5, 3, True, 1),      # row-resident, 16 samples per lane, rows not 16-byte sized
     ((2, 3, 700), 7, 3, False, 1),     # row-resident, K = 7
-    ((1, 2, 8192), 3, 2, True, 1),     # row-resident at the 512-lane limit
-    ((1, 2, 20000), 5, 4, True, 1),    # beyond it: tiled kernels, 20 tiles
+    ((1, 2, 8192), 3, 2, True, 1),     # three segments
+    ((1, 2, 20000), 5, 4, True, 1),    # five segments
+    ((2, 2, 4096), 7, 4, True, 1),     # a row of exactly a workgroup
+    ((2, 2, 4097), 7, 4, True, 1),     # one sample more: two segments
+    ((1, 2, 8193), 7, 5, True, 1),     # 32 samples per lane, two segments, halos of three lanes
+    ((2, 2, 60), 1, 2, True, 1),       # kernel size 1: tiled kernels
     ((5, 4, 4096), 5, 4, True, 1),     # several rows per chunk in the parameter-gradient kernel
-    ((35000, 2, 8), 3, 2, True, 1),    # 70 000 short rows: the tiled kernels beyond one 65 535-row grid slice
+    ((35000, 2, 8), 3, 2, True, 1),    # 70 000 rows of less than a lane
 ])
 def test_edge_shapes_1d(hip_device, shape, K, L, bias, stride):
     _run_fp32("1d", shape[1], K, L, shape, hip_device, bias=bias, stride=stride, seed=5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,K,L", [(3, 3, 1), (8, 5, 2), (517, 5, 3), (4104, 5, 4), (9001, 7, 5)])
+def test_1d_rows_at_any_address(hip_device, dtype, N, K, L):
+    """Rows that start at any element's address give, bit for bit, what rows at a 16-byte boundary give."""
+    _, W1 = _mods()
+    torch.manual_seed(0)
+    mod = W1(3, 3, K, wt_levels=L).to(hip_device)
+    got = []
+    for off in (0, 1, 3):
+        x = torch.empty(2 * 3 * N + off, device=hip_device, dtype=dtype)[off:].view(2, 3, N)
+        g = torch.empty(2 * 3 * N + off, device=hip_device, dtype=dtype)[off:].view(2, 3, N)
+        gen = torch.Generator(device=hip_device).manual_seed(5)
+        x.normal_(generator=gen)
+        g.normal_(generator=gen)
+        x.requires_grad_(True)
+        out = mod(x)
+        got.append([out.detach()] + list(torch.autograd.grad(out, [x] + [p for p in mod.parameters() if p.requires_grad], g)))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert torch.equal(a, b)
 
 
 def test_1d_bf16(hip_device):
@@ -238,7 +264,7 @@ def test_under_autocast_and_channels_last(hip_device):
     ("2d", (3, 4, 56, 56), 5, 3),        # rows of whole vectors (the stage-1 plane)
     ("2d", (2, 3, 17, 31), 7, 3),        # odd sizes, K = 7
     ("2d", (1, 2, 230, 250), 3, 2),      # beyond LDS: the level-by-level kernels
-    ("1d", (2, 4, 300), 5, 3),           # short rows: tiled kernels
+    ("1d", (2, 4, 300), 5, 3),           # rows of less than a wave
     ("1d", (2, 3, 4096), 5, 4),          # row-resident kernels, vector rows
     ("1d", (1, 2, 1001), 3, 5),          # row-resident, scalar rows
 ])

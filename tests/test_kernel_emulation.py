@@ -265,7 +265,9 @@ def _case1d(B, C, N, K, L, bias, seed=0):
     (1, 1, 700, 7, 3, False),      # row-resident, K = 7: level 3 holds 2 < R entries per lane
     (1, 1, 600, 3, 5, True),       # row-resident, five levels
     (1, 1, 800, 5, 5, True),       # row-resident, one level-5 entry per lane: edges from two lanes away
-])                                 # (rows beyond 512 lanes, on the tiled kernels: test_emulated_1d_fused_backward)
+    (1, 1, 4101, 7, 4, True),      # two segments of a row, edges from up to three lanes away, odd length
+    (1, 1, 8193, 5, 5, False),     # 32 samples per lane, two segments, a single sample in the last lane
+])                                 # (segments on the fused backward kernel: test_emulated_1d_fused_backward)
 def test_emulated_1d_fp32(B, C, N, K, L, bias):
     x, g, bw, bb, bs, ws, ss = _case1d(B, C, N, K, L, bias)
     got = emu_util.run(1, x, g, bw, bb, bs, ws, ss, K)
@@ -295,7 +297,9 @@ def test_emulated_1d_row_resident_bf16():
     (1, 1, 700, 7, 3, True, 0, 0),       # K = 7
     (1, 2, 800, 3, 5, True, 0, 0),       # five levels
     (2, 1, 1000, 5, 4, True, 1, 1),      # bf16 rows and parameters
-    (1, 1, 17000, 5, 4, True, 0, 0),     # longer than 512 lanes: every pass on the tiled kernels (17 tiles)
+    (1, 1, 12291, 5, 4, True, 0, 0),     # longer than a workgroup: four segments, odd length
+    (2, 1, 4099, 7, 3, False, 1, 0),     # two segments, bf16 rows that start at odd elements
+    (2, 1, 13, 3, 3, True, 1, 0),        # a single lane
 ])
 def test_emulated_1d_fused_backward(B, C, N, K, L, bias, dtype, pdtype):
     """wtconv1d_backward as one call: grad_x and every parameter gradient from the fused row kernel (the last

@@ -169,28 +169,26 @@ static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_p
 }
 
 // ---- row-resident 1-D kernels ----------------------------------------------------------
-// Rows of 16 to `max_lanes` lanes' worth of samples run on the register-resident kernels, with 16 samples per lane
-// where the row fits the workgroup that way and 32 otherwise; shorter or longer rows and K = 1 use the tiled ones.
-struct Row1DShape { int S, nl, block; };
+// Rows of any length run on the register-resident kernels, those longer than a workgroup in segments of about equal
+// length; K = 1, whose convolutions have no neighbours to fetch, uses the tiled ones.  (Measured down to rows of four
+// lanes, 64 samples: 16.9 us against 35.4 on tiles for [256,64,64] float32, K = 5, three levels.)
+struct Row1DShape { int S, block; Row1D pl; };
 
-static bool row1d_shape(int N, int K, int L, int max_lanes, Row1DShape* sh) {
+static bool row1d_shape(int C, int N, int K, int L, Row1DShape* sh) {
   if (K < 3 || K > 7 || L < 1 || L > kMaxLevels || N <= 0) return false;
-  for (int S : {16, 32}) {
-    if (!row1d_built(K, L, S)) continue;
-    const int n = (N + S - 1) / S;
-    if (n < 16 || n > max_lanes) continue;
-    sh->S = S; sh->nl = n; sh->block = (n + 63) / 64 * 64;
-    return true;
-  }
-  return false;
-}
-
-static Row1D make_row1d(int C, int N, int nl, size_t esz, const void* p0, const void* p1) {
-  Row1D r = {};
-  r.C = C; r.N = N; r.nl = nl;
-  auto aligned = [](const void* p) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-  r.vec_ok = (static_cast<size_t>(N) * esz % 16 == 0) && aligned(p0) && aligned(p1);
-  return r;
+  const int S = row1d_samples(L);
+  const int n = N / S + (N % S != 0 ? 1 : 0);
+  const bool one = n <= kRow1dMaxLanes;
+  const int hal = one ? 0 : row1d_guard(K, L, S);
+  const int most = kRow1dMaxLanes - 2 * hal;
+  Row1D& r = sh->pl;
+  r.C = C; r.N = N; r.hal = hal;
+  r.nseg = one ? 1 : (n + most - 1) / most;
+  r.use = (n + r.nseg - 1) / r.nseg;
+  r.nl = r.use + 2 * hal;
+  sh->S = S;
+  sh->block = (r.nl + 63) / 64 * 64;
+  return true;
 }
 
 // Workgroups per CU the kernels with two slot regions (parameter gradients, fused backward) are planned for: what
@@ -212,20 +210,19 @@ static int tile1d_pass(const char* fn, const void* x, void* out, const wtconv_pa
   if ((reinterpret_cast<uintptr_t>(x) % esz) || (reinterpret_cast<uintptr_t>(out) % esz))
     return fail(WTCONV_E_ARG, "%s: tensor pointer not aligned to its element size", fn);
   Row1DShape sh = {};
-  const bool row_resident = row1d_shape(N, K, L, kRow1dMaxLanes, &sh);
+  const bool row_resident = row1d_shape(C, N, K, L, &sh);
   const Plan1D pl = make_plan1d(C, N, K, L, false, esz, x, out, nullptr);
   const size_t need = wtconv1d_workspace_bytes(B, C, N, K, L, flip ? WTCONV_PASS_BACKWARD_INPUT : WTCONV_PASS_FORWARD);
   if (ws == nullptr || ws_bytes < need)
     return fail(WTCONV_E_WORKSPACE, "%s: workspace of %zu B needed, %zu given", fn, need, ws_bytes);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   if (row_resident) {      // (these kernels fold their channel's parameters themselves: no fold launch, no table)
-    const Row1D rp = make_row1d(C, N, sh.nl, esz, x, out);
-    return launch_row1d(dtype, K, L, sh.S, x, out, params, pdtype, flip, rp, B, sh.block, stream);
+    return launch_row1d(dtype, K, L, x, out, params, pdtype, flip, sh.pl, B, sh.block, stream);
   }
   float* fw = static_cast<float*>(ws);
   float* fb = fw + static_cast<size_t>(C) * (1 + 2 * L) * K;
   if (int e = launch_fold(params, pdtype, fw, fb, C, 2, L, K, flip, flip ? 0 : 1, stream)) return e;
-  return launch_tile1d(dtype, K, x, out, fw, fb, pl, B, stream);
+  return launch_tile1d(dtype, x, out, fw, fb, pl, B, stream);
 }
 
 // ---- static scratch for callers that may not allocate ------------------------------------
@@ -506,8 +503,8 @@ size_t wtconv1d_workspace_bytes(int B, int C, int N, int K, int levels, int pass
     const Plan1D pl = make_plan1d(C, N, K, levels, true, 4, nullptr, nullptr, nullptr);
     int per_chunk, nchunk;
     Row1DShape sh = {};
-    if (row1d_shape(N, K, levels, kRow1dMaxLanes, &sh))
-      row1d_chunks(B, C, row1d_two_region_per_cu(K, levels, sh), &per_chunk, &nchunk);
+    if (row1d_shape(C, N, K, levels, &sh))
+      row1d_chunks(B * sh.pl.nseg, C, row1d_two_region_per_cu(K, levels, sh), &per_chunk, &nchunk);
     else
       wgrad_chunks1d(B, C, pl.ntiles, &per_chunk, &nchunk);
     // partial sums, then one ticket word per channel (fused backward kernel)
@@ -557,19 +554,18 @@ int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_p
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   int per_chunk, nchunk;
   Row1DShape sh = {};
-  const bool row_resident = row1d_shape(N, K, L, kRow1dMaxLanes, &sh);
+  const bool row_resident = row1d_shape(C, N, K, L, &sh);
   if (row_resident)
-    row1d_chunks(B, C, row1d_two_region_per_cu(K, L, sh), &per_chunk, &nchunk);
+    row1d_chunks(B * sh.pl.nseg, C, row1d_two_region_per_cu(K, L, sh), &per_chunk, &nchunk);
   else
     wgrad_chunks1d(B, C, pl.ntiles, &per_chunk, &nchunk);
   if (nchunk > 65535) return fail(WTCONV_E_UNSUPPORTED, "%s: too many chunks (%d)", fn, nchunk);
   float* partial = static_cast<float*>(workspace);
   int e;
   if (row_resident) {
-    const Row1D rp = make_row1d(C, N, sh.nl, esz, x, grad_out);
-    e = launch_row1d_wgrad(dtype, K, L, sh.S, x, grad_out, partial, rp, B, sh.block, per_chunk, nchunk, stream);
+    e = launch_row1d_wgrad(dtype, K, L, x, grad_out, partial, sh.pl, B, sh.block, per_chunk, nchunk, stream);
   } else {
-    e = launch_wgrad1d(dtype, K, L, x, grad_out, partial, pl, B, per_chunk, nchunk, stream);
+    e = launch_wgrad1d(dtype, L, x, grad_out, partial, pl, B, per_chunk, nchunk, stream);
   }
   if (e) return e;
   GradTable gt = {};
@@ -590,8 +586,7 @@ int wtconv1d_backward(const void* x, const void* grad_out, void* grad_x, const w
   // rows that the register-resident kernels take run the whole backward pass as one kernel -- with the lanes, chunks
   // and workspace layout of the separate parameter-gradient pass, so the two share wtconv1d_workspace_bytes
   Row1DShape sh = {};
-  if (K >= 1 && levels >= 1 && levels <= kMaxLevels && row1d_shape(N, K, levels, kRow1dMaxLanes, &sh) &&
-      sh.block <= kRow1dBwdMaxLanes && row1d_bwd_built(K, levels, sh.S)) {
+  if (row1d_shape(C, N, K, levels, &sh) && row1d_bwd_built(K, levels, sh.S)) {
     const int L = levels;
     if (int e = check_common(fn, params, B, C, K, L, dtype, param_dtype)) return e;
     if (x == nullptr || grad_out == nullptr || grad_x == nullptr) return fail(WTCONV_E_ARG, "%s: null tensor pointer", fn);
@@ -606,14 +601,12 @@ int wtconv1d_backward(const void* x, const void* grad_out, void* grad_x, const w
     if (reinterpret_cast<uintptr_t>(workspace) % 4)
       return fail(WTCONV_E_ARG, "%s: workspace not aligned", fn);
     int per_chunk, nchunk;
-    row1d_chunks(B, C, row1d_two_region_per_cu(K, L, sh), &per_chunk, &nchunk);
+    row1d_chunks(B * sh.pl.nseg, C, row1d_two_region_per_cu(K, L, sh), &per_chunk, &nchunk);
     if (nchunk > 65535) return fail(WTCONV_E_UNSUPPORTED, "%s: too many chunks (%d)", fn, nchunk);
     float* partial = static_cast<float*>(workspace);
     unsigned* tickets = reinterpret_cast<unsigned*>(partial + round_up64(static_cast<size_t>(nchunk) * C * ((1 + 2 * L) * K + 1)));
-    Row1D rp = make_row1d(C, N, sh.nl, esz, x, grad_out);
-    rp.vec_ok = rp.vec_ok && (reinterpret_cast<uintptr_t>(grad_x) & 15u) == 0;
     const GradTable gt = to_grad_table(grads, L);
-    return launch_row1d_bwd(dtype, K, L, sh.S, x, grad_out, grad_x, partial, tickets, params, param_dtype, gt, rp, B, sh.block,
+    return launch_row1d_bwd(dtype, K, L, x, grad_out, grad_x, partial, tickets, params, param_dtype, gt, sh.pl, B, sh.block,
                             per_chunk, nchunk, static_cast<hipStream_t>(stream));
   }
   if (int e = wtconv1d_backward_input(grad_out, grad_x, params, B, C, N, K, levels, dtype, param_dtype, workspace,

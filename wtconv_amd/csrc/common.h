@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 #endif
 #include <stdint.h>
+#include <string.h>
 #include <type_traits>
 
 #include "../../include/wtconv_hip.h"
@@ -303,27 +304,45 @@ __device__ __forceinline__ void pin_values(float (&v)[N]) {
 
 // 16-byte global accesses of data that is touched once (activations streaming through a kernel): marked
 // non-temporal, so that they do not displace what the caches should keep.
-__device__ __forceinline__ uint4 load_stream_u4(const void* p) {
+// load_u4: an ordinary one.  ALIGN: what the address is a multiple of, the element's size where rows start anywhere
+// (the hardware takes 16-byte accesses at any such address).
 #ifdef WT_EMULATE
-  return *reinterpret_cast<const uint4*>(p);
+template <int ALIGN = 16>
+__device__ __forceinline__ uint4 load_u4(const void* p) {
+  uint4 r;
+  memcpy(&r, p, sizeof(r));
+  return r;
+}
+template <int ALIGN = 16>
+__device__ __forceinline__ uint4 load_stream_u4(const void* p) { return load_u4<ALIGN>(p); }
+template <int ALIGN = 16>
+__device__ __forceinline__ void store_stream_u4(void* p, const uint4& q) { memcpy(p, &q, sizeof(q)); }
 #else
-  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+template <int ALIGN> struct U4At { typedef u32x4_t type; };
+template <> struct U4At<4> { typedef u32x4_t type __attribute__((aligned(4))); };
+template <> struct U4At<2> { typedef u32x4_t type __attribute__((aligned(2))); };
+template <int ALIGN = 16>
+__device__ __forceinline__ uint4 load_u4(const void* p) {
+  const u32x4_t v = *reinterpret_cast<const typename U4At<ALIGN>::type*>(p);
   uint4 r;
   r.x = v.x; r.y = v.y; r.z = v.z; r.w = v.w;
   return r;
-#endif
 }
+template <int ALIGN = 16>
+__device__ __forceinline__ uint4 load_stream_u4(const void* p) {
+  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const typename U4At<ALIGN>::type*>(p));
+  uint4 r;
+  r.x = v.x; r.y = v.y; r.z = v.z; r.w = v.w;
+  return r;
+}
+template <int ALIGN = 16>
 __device__ __forceinline__ void store_stream_u4(void* p, const uint4& q) {
-#ifdef WT_EMULATE
-  *reinterpret_cast<uint4*>(p) = q;
-#else
-  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
   u32x4_t v;
   v.x = q.x; v.y = q.y; v.z = q.z; v.w = q.w;
-  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t*>(p));
-#endif
+  __builtin_nontemporal_store(v, reinterpret_cast<typename U4At<ALIGN>::type*>(p));
 }
+#endif
 
 // Workgroups of a launch are dealt to the eight XCDs of the GPU in turn (workgroup i runs on XCD i % 8, each with an
 // L2 of its own).  Index i of n -> an index such that the workgroups of one XCD hold a contiguous range, neighbours in

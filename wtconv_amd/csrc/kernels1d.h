@@ -1,4 +1,4 @@
-// Tiled WTConv1d kernels for gfx950.
+// Tiled WTConv1d kernels for gfx950: layers of kernel size 1 (every other size runs on kernels1d_row.h).
 //
 // One workgroup owns a tile of T consecutive samples of one (b, c) row plus the halo the
 // cascade needs, so rows of any length are handled.  Maths (reference

@@ -1,6 +1,6 @@
 // Row-resident WTConv1d kernels for gfx950.
 //
-// One workgroup owns a whole (b, c) row; every lane owns S consecutive samples and keeps
+// One workgroup owns a (b, c) row, or a segment of a longer one; every lane owns S consecutive samples and keeps
 // them, their complete Haar pyramid and the outputs in registers.  S is a multiple of 2^L, so
 // the analysis and synthesis butterflies never leave the lane.  The K-tap conv of a level
 // needs R = K/2 coefficients from beyond either end of the lane's array: each lane publishes
@@ -31,14 +31,11 @@
 namespace wt {
 
 // Samples per lane S: a multiple of 2^L (the pyramid of a lane is local) and of 8 (16-byte vectors of either
-// dtype): 16 or 32.  16 wherever the row fits the workgroup with it (twice the lanes per row, half the registers
-// per lane: more waves in flight, which is what these latency-bound kernels need), 32 for longer rows and for
-// five levels.
-constexpr int kRow1dMaxSamples = 32;
-constexpr int kRow1dMaxLanes = 512;      // threads per workgroup
-constexpr bool row1d_built(int K, int L, int S) {
-  return K >= 3 && (S == 16 || S == 32) && S % (1 << L) == 0;
-}
+// dtype): 16 up to four levels (half the registers per lane of 32: more waves in flight, which is what these
+// latency-bound kernels need), 32 for five.
+constexpr int kRow1dMaxLanes = 256;      // threads per workgroup
+constexpr int row1d_samples(int L) { return L <= 4 ? 16 : 32; }
+constexpr bool row1d_built(int K, int L, int S) { return K >= 3 && S == row1d_samples(L); }
 
 // Edge entries a lane publishes of an array of n entries: the first and last R, or all of
 // them when there are fewer than 2R.
@@ -75,34 +72,66 @@ constexpr size_t row1d_region(int K, int L, int S, int block) {
   return static_cast<size_t>(block + 2 * row1d_guard(K, L, S)) * row1d_slot(K, L, S);
 }
 
+// A row longer than a workgroup is cut into `nseg` segments of `use` lanes each.  A segment is staged with `hal` more
+// lanes on either side, whose samples give the convolutions of its own lanes their neighbours (the pyramid of a lane
+// is local, so nothing reaches further than row1d_guard lanes); what the halo lanes compute themselves is dropped.
+// Rows that fit the workgroup are one segment without halo.
 struct Row1D {
   int C, N;
-  int nl;        // lanes that hold samples: ceil(N / S)
-  int vec_ok;    // rows are 16-byte sized and aligned
+  int nl;        // lanes that hold samples of a segment, halo included
+  int hal, use, nseg;
 };
 
-// HBM row -> LDS slots (slot of lane j = samples [j*S, (j+1)*S), zeros past N), in two steps
+// The (batch item, segment) units of a channel, one after the other.
+struct RowUnit {
+  int b, seg;
+  __device__ __forceinline__ RowUnit(int unit, const Row1D& pl) : b(unit / pl.nseg), seg(unit - b * pl.nseg) {}
+  __device__ __forceinline__ void next(const Row1D& pl) {
+    if (++seg == pl.nseg) { seg = 0; ++b; }
+  }
+  // the sample that the segment's first lane holds first (negative in the halo of a row's first segment)
+  __device__ __forceinline__ int first(const Row1D& pl, int S) const { return WT_UNIFORM((seg * pl.use - pl.hal) * S); }
+  template <typename T>
+  __device__ __forceinline__ T* row(T* base, const Row1D& pl, int c) const {
+    return base + (static_cast<size_t>(WT_UNIFORM(b)) * pl.C + c) * pl.N;
+  }
+};
+
+// HBM row -> LDS slots (slot of lane j = samples [p0 + j*S, p0 + (j+1)*S), zeros outside the row), in two steps
 // so that the loads of the next row can be in flight while the current one is computed:
 // row1d_fetch issues every 16-byte load of the thread at once (at most S / EV of them, since
 // the workgroup has at least as many threads as lanes that hold samples), row1d_commit
-// converts and writes them to the slots.  Fast path only: rows are 16-byte sized and aligned,
-// so every vector lies wholly inside or wholly outside the row.
+// converts and writes them to the slots.  The vectors are those of the row, whatever its address: rows of odd length
+// start anywhere, and a 16-byte load at an element's alignment costs one cache line more per wave, where loads of
+// single elements are eight times as many (rows of 20011 bfloat16 samples).  The elements behind the last whole
+// vector are loaded one each by the first lanes.
 // STREAM: the loads are marked non-temporal (measured: pays in the whole-backward kernel, which reads two rows per
 // row it writes, not in the forward kernel).
-template <typename T, int S, bool STREAM = false>
-__device__ __forceinline__ void row1d_fetch(const T* __restrict__ row, int N, int tid, int nth,
-                                            uint4 (&q)[S / (16 / sizeof(T))]) {
-  constexpr int EV = 16 / sizeof(T);
+template <typename T, int S>
+struct RowFetch {
+  static constexpr int EV = 16 / sizeof(T);
+  static constexpr int NQ = S / EV;
+  uint4 q[NQ];
+  float tail;
+
+  template <bool STREAM = false>
+  __device__ __forceinline__ void fetch(const T* __restrict__ row, int p0, int N, int tid, int nth) {
+    const unsigned nvec = static_cast<unsigned>(N / EV * EV);
 #pragma unroll
-  for (int u = 0; u < S / EV; ++u) {
-    const int p = (tid + u * nth) * EV;
-    q[u].x = 0u; q[u].y = 0u; q[u].z = 0u; q[u].w = 0u;
-    if (p < N) {
-      if constexpr (STREAM) q[u] = load_stream_u4(row + p);
-      else q[u] = *reinterpret_cast<const uint4*>(row + p);
+    for (int u = 0; u < NQ; ++u) {
+      const unsigned p = static_cast<unsigned>(p0) + (tid + u * nth) * EV;      // (a negative sample is a large one)
+      q[u].x = 0u; q[u].y = 0u; q[u].z = 0u; q[u].w = 0u;
+      if (p < nvec) {
+        if constexpr (STREAM) q[u] = load_stream_u4<sizeof(T)>(row + p);
+        else q[u] = load_u4<sizeof(T)>(row + p);
+      }
     }
+    if (N % EV != 0) tail = tid < N % EV ? to_f32<T>(row[nvec + tid]) : 0.f;
   }
-}
+
+  template <int SLOT>
+  __device__ __forceinline__ void commit(float* __restrict__ lds, int p0, int N, int nl, int tid, int nth) const;
+};
 
 template <int S, int SLOT, int EV>
 __device__ __forceinline__ void row1d_put(float* __restrict__ lds, int p, const float (&vals)[EV]) {
@@ -116,110 +145,107 @@ __device__ __forceinline__ void row1d_put(float* __restrict__ lds, int p, const 
   }
 }
 
-template <typename T, int S, int SLOT>
-__device__ __forceinline__ void row1d_commit(float* __restrict__ lds, int nl, int tid, int nth,
-                                             const uint4 (&q)[S / (16 / sizeof(T))]) {
-  constexpr int EV = 16 / sizeof(T);
-  const int total = nl * S;
+template <typename T>
+__device__ __forceinline__ void row1d_unpack(const uint4& q, float (&vals)[16 / sizeof(T)]) {
+  if constexpr (sizeof(T) == 4) {
+    vals[0] = __uint_as_float(q.x); vals[1] = __uint_as_float(q.y);
+    vals[2] = __uint_as_float(q.z); vals[3] = __uint_as_float(q.w);
+  } else {
+    const uint32_t qq[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-  for (int u = 0; u < S / EV; ++u) {
-    const int p = (tid + u * nth) * EV;
-    if (p < total) {
-      float vals[EV];
-      if constexpr (sizeof(T) == 4) {
-        vals[0] = __uint_as_float(q[u].x); vals[1] = __uint_as_float(q[u].y);
-        vals[2] = __uint_as_float(q[u].z); vals[3] = __uint_as_float(q[u].w);
-      } else {
-        const uint32_t qq[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          unpack2<T>(qq[k], vals[2 * k], vals[2 * k + 1]);
-        }
-      }
-      row1d_put<S, SLOT, EV>(lds, p, vals);
+    for (int k = 0; k < 4; ++k) {
+      unpack2<T>(qq[k], vals[2 * k], vals[2 * k + 1]);
     }
   }
 }
 
-// Fetch and commit of two rows (x and grad_out) in one call, four vectors of each at a time:
+template <typename T, int S>
+template <int SLOT>
+__device__ __forceinline__ void RowFetch<T, S>::commit(float* __restrict__ lds, int p0, int N, int nl, int tid,
+                                                       int nth) const {
+  const int total = nl * S, nvec = N / EV * EV;
+  const int split = N % EV != 0 ? nvec - p0 : -1;      // the vector that the tail's elements take the place of
+#pragma unroll
+  for (int u = 0; u < NQ; ++u) {
+    const int p = (tid + u * nth) * EV;
+    if (p < total && p != split) {
+      float vals[EV];
+      row1d_unpack<T>(q[u], vals);
+      row1d_put<S, SLOT, EV>(lds, p, vals);
+    }
+  }
+  if (split >= 0 && split < total && tid < EV) {
+    const int owner = split / S;
+    lds[owner * SLOT + (split - owner * S) + tid] = tail;
+  }
+}
+
+// Fetch and commit of two rows (x and grad_out) in one call, at most four vectors of each at a time:
 // bounded register use for the kernel that holds many running sums, and the loads of both
 // rows share their HBM latency.
 template <typename T, int S, int SLOT>
 __device__ __forceinline__ void row1d_stage_pair(const T* __restrict__ row0, const T* __restrict__ row1,
-                                                 float* __restrict__ lds0, float* __restrict__ lds1, int N, int nl,
-                                                 int tid, int nth) {
+                                                 float* __restrict__ lds0, float* __restrict__ lds1, int p0, int N,
+                                                 int nl, int tid, int nth) {
   constexpr int EV = 16 / sizeof(T);
-  constexpr int U = 4;
-  const int total = nl * S;
-  auto unpack = [](const uint4& q, float (&vals)[EV]) {
-    if constexpr (sizeof(T) == 4) {
-      vals[0] = __uint_as_float(q.x); vals[1] = __uint_as_float(q.y);
-      vals[2] = __uint_as_float(q.z); vals[3] = __uint_as_float(q.w);
-    } else {
-      const uint32_t qq[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        unpack2<T>(qq[k], vals[2 * k], vals[2 * k + 1]);
-      }
-    }
-  };
+  constexpr int U = S / EV < 4 ? S / EV : 4;
+  const int total = nl * S, nvec = N / EV * EV;
+  const int split = N % EV != 0 ? nvec - p0 : -1;
+  float t0 = 0.f, t1 = 0.f;
+  if (split >= 0 && tid < N % EV) {
+    t0 = to_f32<T>(row0[nvec + tid]);
+    t1 = to_f32<T>(row1[nvec + tid]);
+  }
   for (int v0 = tid; v0 * EV < total; v0 += U * nth) {
     uint4 q0[U], q1[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int p = (v0 + u * nth) * EV;
+      const unsigned p = static_cast<unsigned>(p0) + (v0 + u * nth) * EV;
       q0[u].x = 0u; q0[u].y = 0u; q0[u].z = 0u; q0[u].w = 0u;
       q1[u] = q0[u];
-      if (p < N) {
-        q0[u] = *reinterpret_cast<const uint4*>(row0 + p);
-        q1[u] = *reinterpret_cast<const uint4*>(row1 + p);
+      if (p < static_cast<unsigned>(nvec)) {
+        q0[u] = load_u4<sizeof(T)>(row0 + p);
+        q1[u] = load_u4<sizeof(T)>(row1 + p);
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int p = (v0 + u * nth) * EV;
-      if (p < total) {
+      if (p < total && p != split) {
         float vals[EV];
-        unpack(q0[u], vals);
+        row1d_unpack<T>(q0[u], vals);
         row1d_put<S, SLOT, EV>(lds0, p, vals);
-        unpack(q1[u], vals);
+        row1d_unpack<T>(q1[u], vals);
         row1d_put<S, SLOT, EV>(lds1, p, vals);
       }
     }
   }
-}
-
-// Element-wise staging for rows that are not 16-byte sized or aligned.
-template <typename T, int S, int SLOT>
-__device__ __forceinline__ void row1d_stage_scalar(const T* __restrict__ row, float* __restrict__ lds, int N,
-                                                   int nl, int tid, int nth) {
-  constexpr int EV = 16 / sizeof(T);
-  const int total = nl * S;
-  for (int v = tid; v * EV < total; v += nth) {
-    const int p = v * EV;
-    float vals[EV];
-#pragma unroll
-    for (int k = 0; k < EV; ++k) vals[k] = p + k < N ? to_f32<T>(row[p + k]) : 0.f;
-    row1d_put<S, SLOT, EV>(lds, p, vals);
+  if (split >= 0 && split < total && tid < EV) {
+    const int owner = split / S, at = owner * SLOT + (split - owner * S) + tid;
+    lds0[at] = t0;
+    lds1[at] = t1;
   }
 }
 
-// LDS slots -> HBM row (entries past N are dropped).
+// LDS slots of a segment's own lanes -> HBM row (entries past N are dropped).  p0: sample of the slot of lane 0.
 template <typename T, int S, int SLOT>
-__device__ __forceinline__ void row1d_unstage(T* __restrict__ row, const float* __restrict__ lds, int N, bool vec,
-                                              int tid, int nth) {
+__device__ __forceinline__ void row1d_unstage(T* __restrict__ row, const float* __restrict__ lds, int p0,
+                                              const Row1D& pl, int tid, int nth) {
   constexpr int EV = 16 / sizeof(T);
-  for (int v = tid; v * EV < N; v += nth) {
-    const int p = v * EV;
-    const int owner = p / S;
-    const float* src = lds + owner * SLOT + (p - owner * S);
+  const int first = p0 + pl.hal * S, N = pl.N;
+  const int end = N - first < pl.use * S ? N - first : pl.use * S;
+  const float* own = lds + pl.hal * SLOT;
+  for (int v = tid; v * EV < end; v += nth) {
+    const int lp = v * EV, p = first + lp;
+    const int owner = lp / S;
+    const float* src = own + owner * SLOT + (lp - owner * S);
     float vals[EV];
 #pragma unroll
     for (int g = 0; g < EV / 4; ++g) {
       const float4 r4 = reinterpret_cast<const float4*>(src)[g];
       vals[4 * g] = r4.x; vals[4 * g + 1] = r4.y; vals[4 * g + 2] = r4.z; vals[4 * g + 3] = r4.w;
     }
-    if (vec && p + EV <= N) {
+    if (lp + EV <= N - first) {
       uint4 q;
       if constexpr (sizeof(T) == 4) {
         q.x = __float_as_uint(vals[0]); q.y = __float_as_uint(vals[1]);
@@ -231,11 +257,11 @@ __device__ __forceinline__ void row1d_unstage(T* __restrict__ row, const float* 
           qq[k] = pack2<T>(vals[2 * k], vals[2 * k + 1]);
         q.x = qq[0]; q.y = qq[1]; q.z = qq[2]; q.w = qq[3];
       }
-      store_stream_u4(row + p, q);       // written once, read by another kernel: non-temporal
+      store_stream_u4<sizeof(T)>(row + p, q);       // written once, read by another kernel: non-temporal
     } else {
 #pragma unroll
       for (int k = 0; k < EV; ++k)
-        if (p + k < N) row[p + k] = from_f32<T>(vals[k]);
+        if (lp + k < N - first) row[p + k] = from_f32<T>(vals[k]);
     }
   }
 }
@@ -656,47 +682,44 @@ __device__ __forceinline__ void row1d_fwd_levels(const RowEdges<K, L>& ed, const
   if constexpr (l < L) row1d_fwd_levels<K, S, SLOT, L, l + 1>(ed, fwc, xlo, o);
 }
 
-// Forward / input-gradient kernel.  grid = (channels, batch chunks), block = lanes (multiple of 64,
-// >= ceil(N / S)), dynamic LDS = one slot region (row1d_region floats).  A workgroup walks the rows (b, c) of
-// its chunk of batch items; the next row is fetched into registers while the current one is computed and
+// Forward / input-gradient kernel.  grid = (channels, chunks of units), block = lanes (multiple of 64,
+// >= Row1D::nl), dynamic LDS = one slot region (row1d_region floats).  A workgroup walks the units (segments of
+// rows (b, c)) of its chunk; the next row is fetched into registers while the current one is computed and
 // committed to the slots once the current outputs have left them.  One region instead of two alternating
 // ones: half the LDS per workgroup, i.e. twice the workgroups per CU, which pays more here than the two
 // barriers per row it costs.  flip != 0: the input gradient (taps reversed, no bias).
+//
+// Measured, forward us (training step us), tiles of 1024 samples in LDS (kernels1d.h) -> this kernel in segments:
+// [8,48,20011] bfloat16, K = 7, five levels 46.3 -> 21.8 (172 -> 75); [8,16,39000] float32, K = 5, four levels
+// 28.4 -> 9.5.  Short rows: [256,64,100] float32, three levels 37.1 -> 17.2, although a wave's lanes are mostly idle.
 template <typename T, int K, int L, int S>
-__global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_kernel(const T* __restrict__ x, T* __restrict__ out,
+__global__ __launch_bounds__(kRow1dMaxLanes, 2) void wt1d_row_kernel(const T* __restrict__ x, T* __restrict__ out,
                                                                    const ParamTable prm, int pdtype, int flip,
-                                                                   Row1D pl, int B, int per_chunk) {
+                                                                   Row1D pl, int units, int per_chunk) {
   WT_SHARED_FLOATS(lds);
   constexpr int R = K / 2;
   constexpr int SLOT = row1d_slot(K, L, S);
-  constexpr int EV = 16 / sizeof(T);
   const int tid = threadIdx.x, nth = blockDim.x;
   const int c = blockIdx.x;
-  const int b_begin = static_cast<int>(blockIdx.y) * per_chunk;
-  const int b_end = b_begin + per_chunk < B ? b_begin + per_chunk : B;
-  const bool fast = pl.vec_ok != 0 && pl.N % EV == 0;
+  const int u_begin = static_cast<int>(blockIdx.y) * per_chunk;
+  const int u_end = u_begin + per_chunk < units ? u_begin + per_chunk : units;
   constexpr int G = row1d_guard(K, L, S);
   float* cur = lds + G * SLOT;                      // (the region points at the slot of lane 0, behind its left guard)
   row1d_zero_guards<K, L, S>(lds, 1, tid, nth);
-  auto row_of = [&](int b) { return (static_cast<size_t>(b) * pl.C + c) * pl.N; };
 
-  uint4 q[S / EV];
-  if (b_begin < b_end && fast) row1d_fetch<T, S>(x + row_of(b_begin), pl.N, tid, nth, q);
+  RowFetch<T, S> rf;
+  RowUnit at(u_begin, pl);
+  if (u_begin < u_end) rf.fetch(at.row(x, pl, c), at.first(pl, S), pl.N, tid, nth);
   RowWeights<K, L> fwc;                 // (its parameter loads share the latency of the first row's)
   row1d_fold<K, L>(prm, pdtype, c, flip, fwc);
   const float bias = (!flip && prm.base_bias != nullptr)
                          ? load_param(prm.base_bias, pdtype, c) * load_param(prm.base_scale, pdtype, c) : 0.f;
-  if (b_begin < b_end) {
-    if (fast)
-      row1d_commit<T, S, SLOT>(cur, pl.nl, tid, nth, q);
-    else
-      row1d_stage_scalar<T, S, SLOT>(x + row_of(b_begin), cur, pl.N, pl.nl, tid, nth);
-  }
+  if (u_begin < u_end) rf.template commit<SLOT>(cur, at.first(pl, S), pl.N, pl.nl, tid, nth);
   WT_LDS_BARRIER();
-  for (int bv = b_begin; bv < b_end; ++bv) {
-    const int b = WT_UNIFORM(bv);
-    const bool more = b + 1 < b_end;
-    const T* xnext = x + row_of(more ? b + 1 : b);
+  for (int u = u_begin; u < u_end; ++u) {
+    const bool more = u + 1 < u_end;
+    RowUnit nx = at;
+    nx.next(pl);
     float* slot = cur + tid * SLOT;
     float xs[S];
     if (tid < pl.nl) {
@@ -705,7 +728,7 @@ __global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_kernel(const T* __res
 #pragma unroll
       for (int e = 0; e < S; ++e) xs[e] = 0.f;
     }
-    if (fast && more) row1d_fetch<T, S>(xnext, pl.N, tid, nth, q);
+    if (more) rf.fetch(nx.row(x, pl, c), nx.first(pl, S), pl.N, tid, nth);
     // the slot held this lane's samples only: it can take the lane's edges right away
     row1d_publish<K, S, 0>(slot, xs);
     row1d_publish_chain<K, S, L, 1>(slot, xs);
@@ -726,27 +749,23 @@ __global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_kernel(const T* __res
     WT_LDS_BARRIER();            // every neighbour has read this lane's edges
     row1d_write_slot<S>(slot, o);
     WT_LDS_BARRIER();
-    row1d_unstage<T, S, SLOT>(out + row_of(b), cur, pl.N, pl.vec_ok != 0, tid, nth);
+    row1d_unstage<T, S, SLOT>(at.row(out, pl, c), cur, at.first(pl, S), pl, tid, nth);
     WT_LDS_BARRIER();            // the outputs have left the slots
-    if (more) {
-      if (fast)
-        row1d_commit<T, S, SLOT>(cur, pl.nl, tid, nth, q);
-      else
-        row1d_stage_scalar<T, S, SLOT>(xnext, cur, pl.N, pl.nl, tid, nth);
-    }
+    if (more) rf.template commit<SLOT>(cur, nx.first(pl, S), pl.N, pl.nl, tid, nth);
+    at = nx;
     WT_LDS_BARRIER();
   }
 }
 
 // Parameter gradients, first stage.  grid = (C, nchunk), block = lanes, dynamic LDS =
-// 2 * block * SLOT floats (x slots, then grad_out slots).  A workgroup walks `per_chunk` rows
+// 2 * block * SLOT floats (x slots, then grad_out slots).  A workgroup walks `per_chunk` units
 // of one channel; every lane keeps K sums per filter in registers.  Output layout as the
 // tiled kernel: partial[chunk][c][(1 + 2L) * K + 1].
 template <typename T, int K, int L, int S>
-__global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_wgrad_kernel(const T* __restrict__ x,
+__global__ __launch_bounds__(kRow1dMaxLanes, 2) void wt1d_row_wgrad_kernel(const T* __restrict__ x,
                                                                          const T* __restrict__ g,
                                                                          float* __restrict__ partial, Row1D pl,
-                                                                         int B, int per_chunk) {
+                                                                         int units, int per_chunk) {
   WT_SHARED_FLOATS(lds);
   constexpr int R = K / 2;
   constexpr int SLOT = row1d_slot(K, L, S);
@@ -761,9 +780,6 @@ __global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_wgrad_kernel(const T*
   const float* gslot = glds + tid * SLOT;
   row1d_zero_guards<K, L, S>(lds, 2, tid, nth);
 
-  constexpr int EV = 16 / sizeof(T);
-  const bool fast = pl.vec_ok != 0 && pl.N % EV == 0;
-
   float acc[NF][K];
   float gsum = 0.f;
 #pragma unroll
@@ -771,24 +787,16 @@ __global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_wgrad_kernel(const T*
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[f][k] = 0.f;
 
-  const int b_end = (chunk + 1) * per_chunk < B ? (chunk + 1) * per_chunk : B;
-  for (int b = chunk * per_chunk; b < b_end; ++b) {
-    const size_t roff = (static_cast<size_t>(b) * pl.C + c) * pl.N;
-    if (fast) {
-      row1d_stage_pair<T, S, SLOT>(x + roff, g + roff, xlds, glds, pl.N, pl.nl, tid, nth);
-    } else {
-      row1d_stage_scalar<T, S, SLOT>(x + roff, xlds, pl.N, pl.nl, tid, nth);
-      row1d_stage_scalar<T, S, SLOT>(g + roff, glds, pl.N, pl.nl, tid, nth);
-    }
+  const int u_end = (chunk + 1) * per_chunk < units ? (chunk + 1) * per_chunk : units;
+  RowUnit at(chunk * per_chunk, pl);
+  for (int u = chunk * per_chunk; u < u_end; ++u, at.next(pl)) {
+    row1d_stage_pair<T, S, SLOT>(at.row(x, pl, c), at.row(g, pl, c), xlds, glds, at.first(pl, S), pl.N, pl.nl, tid, nth);
     WT_LDS_BARRIER();
     float xs[S], gs[S];
-    if (tid < pl.nl) {
-      row1d_read_slot<S>(slot, xs);
-      row1d_read_slot<S>(gslot, gs);
-    } else {
 #pragma unroll
-      for (int q = 0; q < S; ++q) { xs[q] = 0.f; gs[q] = 0.f; }
-    }
+    for (int q = 0; q < S; ++q) { xs[q] = 0.f; gs[q] = 0.f; }
+    if (tid < pl.nl) row1d_read_slot<S>(slot, xs);
+    if (tid >= pl.hal && tid < pl.hal + pl.use) row1d_read_slot<S>(gslot, gs);    // (the halo's sums are its owners')
     RowPyramid<S, L> py;
     row1d_analysis<S, L>(xs, py);
     row1d_publish<K, S, 0>(slot, xs);
@@ -809,7 +817,6 @@ __global__ __launch_bounds__(kRow1dMaxLanes) void wt1d_row_wgrad_kernel(const T*
   row1d_store_partial<K, NF>(acc, gsum, lds, partial + (static_cast<size_t>(chunk) * pl.C + c) * NRED, tid, nth);
 }
 
-constexpr int kRow1dBwdMaxLanes = 256;      // threads per workgroup of the fused backward kernel (register budget)
 // (K, L) pairs the fused backward kernel is built for: its (1 + 2L) * K + 1 running sums per lane must leave room for
 // the rest in 256 registers (beyond 50 sums, 45 with 32 samples per lane, the compiler spills; those pairs run the
 // backward pass as two kernels).
@@ -824,19 +831,18 @@ constexpr bool row1d_bwd_built(int K, int L, int S) {
 // stores its record of sums and draws its channel's ticket; the last one of a channel runs the second stage
 // (wgrad_finish_channel) for it and leaves the ticket zero.  `tickets`: C words, zero at launch.
 template <typename T, int K, int L, int S>
-__global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(const T* __restrict__ x,
+__global__ __launch_bounds__(kRow1dMaxLanes, 2) void wt1d_row_bwd_kernel(const T* __restrict__ x,
                                                                           const T* __restrict__ g,
                                                                           T* __restrict__ gx,
                                                                           float* __restrict__ partial,
                                                                           unsigned* __restrict__ tickets,
                                                                           const ParamTable prm, int pdtype,
-                                                                          const GradTable gt, Row1D pl, int B,
+                                                                          const GradTable gt, Row1D pl, int units,
                                                                           int per_chunk, int nchunk) {
   WT_SHARED_FLOATS(lds);
   constexpr int R = K / 2;
   constexpr int SLOT = row1d_slot(K, L, S);
   constexpr int NF = 1 + 2 * L;
-  constexpr int EV = 16 / sizeof(T);
   const int c = blockIdx.x;
   const int chunk = blockIdx.y;
   const int tid = threadIdx.x, nth = blockDim.x;
@@ -846,7 +852,6 @@ __global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(cons
   float* xslot = xlds + tid * SLOT;
   float* gslot = glds + tid * SLOT;
   row1d_zero_guards<K, L, S>(lds, 2, tid, nth);
-  const bool fast = pl.vec_ok != 0 && pl.N % EV == 0;
 
   RowWeights<K, L> fwc;
   row1d_fold<K, L>(prm, pdtype, c, 1, fwc);
@@ -858,35 +863,28 @@ __global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(cons
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[f][k] = 0.f;
 
-  const int b_end = (chunk + 1) * per_chunk < B ? (chunk + 1) * per_chunk : B;
-  // with 16 samples per lane, rows on the fast path (16-byte sized and aligned) are fetched one row ahead into
-  // registers; with 32 the registers for that are not there, and the rows are staged as the loop reaches them
+  const int u_first = chunk * per_chunk;
+  const int u_end = u_first + per_chunk < units ? u_first + per_chunk : units;
+  // with 16 samples per lane, the rows are fetched one unit ahead into registers; with 32 the registers for that are
+  // not there, and they are staged as the loop reaches them
   constexpr bool kAhead = S <= 16;
-  const bool ahead = kAhead && fast;
-  uint4 qx[kAhead ? S / EV : 1], qg[kAhead ? S / EV : 1];
-  const int b_first = chunk * per_chunk;
-  if (b_first < b_end && ahead) {
-    const size_t r0 = (static_cast<size_t>(b_first) * pl.C + c) * pl.N;
-    if constexpr (kAhead) {
-      row1d_fetch<T, S, true>(x + r0, pl.N, tid, nth, qx);
-      row1d_fetch<T, S, true>(g + r0, pl.N, tid, nth, qg);
-      row1d_commit<T, S, SLOT>(xlds, pl.nl, tid, nth, qx);
-      row1d_commit<T, S, SLOT>(glds, pl.nl, tid, nth, qg);
+  RowFetch<T, kAhead ? S : 8> rx, rg;
+  RowUnit at(u_first, pl);
+  if constexpr (kAhead) {
+    if (u_first < u_end) {
+      const int p0 = at.first(pl, S);
+      rx.template fetch<true>(at.row(x, pl, c), p0, pl.N, tid, nth);
+      rg.template fetch<true>(at.row(g, pl, c), p0, pl.N, tid, nth);
+      rx.template commit<SLOT>(xlds, p0, pl.N, pl.nl, tid, nth);
+      rg.template commit<SLOT>(glds, p0, pl.N, pl.nl, tid, nth);
     }
   }
-  for (int bv = b_first; bv < b_end; ++bv) {
-    const int b = WT_UNIFORM(bv);
-    const size_t roff = (static_cast<size_t>(b) * pl.C + c) * pl.N;
-    const bool more = b + 1 < b_end;
-    const size_t rnext = (static_cast<size_t>(more ? b + 1 : b) * pl.C + c) * pl.N;
-    if (!ahead) {
-      if (fast) {
-        row1d_stage_pair<T, S, SLOT>(x + roff, g + roff, xlds, glds, pl.N, pl.nl, tid, nth);
-      } else {
-        row1d_stage_scalar<T, S, SLOT>(x + roff, xlds, pl.N, pl.nl, tid, nth);
-        row1d_stage_scalar<T, S, SLOT>(g + roff, glds, pl.N, pl.nl, tid, nth);
-      }
-    }
+  for (int u = u_first; u < u_end; ++u) {
+    const bool more = u + 1 < u_end;
+    RowUnit nx = at;
+    nx.next(pl);
+    if constexpr (!kAhead)
+      row1d_stage_pair<T, S, SLOT>(at.row(x, pl, c), at.row(g, pl, c), xlds, glds, at.first(pl, S), pl.N, pl.nl, tid, nth);
     WT_LDS_BARRIER();
     float xs[S], gs[S];
     if (tid < pl.nl) {
@@ -897,9 +895,9 @@ __global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(cons
       for (int q = 0; q < S; ++q) { xs[q] = 0.f; gs[q] = 0.f; }
     }
     if constexpr (kAhead) {
-      if (ahead && more) {
-        row1d_fetch<T, S, true>(x + rnext, pl.N, tid, nth, qx);
-        row1d_fetch<T, S, true>(g + rnext, pl.N, tid, nth, qg);
+      if (more) {
+        rx.template fetch<true>(nx.row(x, pl, c), nx.first(pl, S), pl.N, tid, nth);
+        rg.template fetch<true>(nx.row(g, pl, c), nx.first(pl, S), pl.N, tid, nth);
       }
     }
     row1d_publish<K, S, 0>(xslot, xs);
@@ -911,6 +909,10 @@ __global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(cons
     // the barrier instead of forming them again level by level)
     pin_values(xs);
     pin_values(gs);
+    if (pl.hal != 0 && (tid < pl.hal || tid >= pl.hal + pl.use)) {      // the halo's sums are its owners'
+#pragma unroll
+      for (int q = 0; q < S; ++q) gs[q] = 0.f;
+    }
     // base conv: its correlation sums, and its share of grad_x (the layer on grad_out with the reversed taps)
     float o[S];
 #pragma unroll
@@ -933,14 +935,15 @@ __global__ __launch_bounds__(kRow1dBwdMaxLanes, 2) void wt1d_row_bwd_kernel(cons
     WT_LDS_BARRIER();            // every neighbour has read this lane's edges
     row1d_write_slot<S>(gslot, o);
     WT_LDS_BARRIER();
-    row1d_unstage<T, S, SLOT>(gx + roff, glds, pl.N, pl.vec_ok != 0, tid, nth);
-    WT_LDS_BARRIER();            // the next row's staging overwrites the slots read above
+    row1d_unstage<T, S, SLOT>(at.row(gx, pl, c), glds, at.first(pl, S), pl, tid, nth);
+    WT_LDS_BARRIER();            // the next unit's staging overwrites the slots read above
     if constexpr (kAhead) {
-      if (ahead && more) {
-        row1d_commit<T, S, SLOT>(xlds, pl.nl, tid, nth, qx);
-        row1d_commit<T, S, SLOT>(glds, pl.nl, tid, nth, qg);
+      if (more) {
+        rx.template commit<SLOT>(xlds, nx.first(pl, S), pl.N, pl.nl, tid, nth);
+        rg.template commit<SLOT>(glds, nx.first(pl, S), pl.N, pl.nl, tid, nth);
       }
     }
+    at = nx;
   }
 
   constexpr int NRED = NF * K + 1;

@@ -36,17 +36,17 @@ int launch_stream2d_wgrad(int dtype, int K, const void* x, const void* g, float*
                           const Stream2D& sp, int B, int nchunk, hipStream_t stream, bool have_g_pyramid);
 
 // conv1d.hip: the 1-D layer, by tiles of a row and with rows in registers.
-int launch_tile1d(int dtype, int K, const void* x, void* out, const float* fw, const float* fb, const Plan1D& pl, int B,
+int launch_tile1d(int dtype, const void* x, void* out, const float* fw, const float* fb, const Plan1D& pl, int B,
                   hipStream_t stream);
-int launch_wgrad1d(int dtype, int K, int L, const void* x, const void* g, float* partial, const Plan1D& pl, int B, int per_chunk,
+int launch_wgrad1d(int dtype, int L, const void* x, const void* g, float* partial, const Plan1D& pl, int B, int per_chunk,
                    int nchunk, hipStream_t stream);
-int launch_row1d(int dtype, int K, int L, int S, const void* x, void* out, const wtconv_params* params, int pdtype, int flip,
+int launch_row1d(int dtype, int K, int L, const void* x, void* out, const wtconv_params* params, int pdtype, int flip,
                  const Row1D& pl, int B, int block, hipStream_t stream);
-int launch_row1d_bwd(int dtype, int K, int L, int S, const void* x, const void* g, void* gx, float* partial, unsigned* tickets,
+int launch_row1d_bwd(int dtype, int K, int L, const void* x, const void* g, void* gx, float* partial, unsigned* tickets,
                      const wtconv_params* params, int pdtype, const GradTable& gt, const Row1D& pl, int B, int block,
                      int per_chunk, int nchunk, hipStream_t stream);
-int launch_row1d_wgrad(int dtype, int K, int L, int S, const void* x, const void* g, float* partial, const Row1D& pl, int B,
+int launch_row1d_wgrad(int dtype, int K, int L, const void* x, const void* g, float* partial, const Row1D& pl, int B,
                        int block, int per_chunk, int nchunk, hipStream_t stream);
-void row1d_chunks(int B, int C, int per_cu, int* per_chunk, int* nchunk);
+void row1d_chunks(int units, int C, int per_cu, int* per_chunk, int* nchunk);
 
 }  // namespace wt
