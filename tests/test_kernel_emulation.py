@@ -99,6 +99,8 @@ def test_emulated_2d_fp32(B, C, H, W, K, L, bias):
     (1, 1, 20, 136, 3, 2, False, 1024),  # three column tiles at level 0, two at level 1, no bias
     (1, 1, 18, 24, 7, 1, True, 1024),    # K = 7 halo of 3
     (1, 1, 36, 36, 3, 2, False, 12000),  # plane-resident forward, level-by-level weight gradients
+    (2, 2, 39, 50, 5, 3, True, 14000),   # one step, then plane-resident: two more steps for the weight gradients
+    (1, 2, 64, 36, 7, 4, True, 14000),   # two steps; K = 7, whose correlation sums take two launches
 ])
 def test_emulated_2d_level_by_level(B, C, H, W, K, L, bias, limit):
     x, g, bw, bb, bs, ws, ss = _case2d(B, C, H, W, K, L, bias)
@@ -111,6 +113,7 @@ def test_emulated_2d_level_by_level(B, C, H, W, K, L, bias, limit):
     (1, 1, 24, 48, 3, 2, False, 1024, 2),    # the same on fp16 tensors
     (1, 1, 18, 24, 7, 1, True, 1024, 0),     # a single level: nothing to share, the two passes run as they are
     (1, 1, 36, 36, 3, 2, False, 12000, 0),   # plane-resident input gradient, level-by-level weight gradients: not shared
+    (2, 2, 39, 50, 5, 3, True, 14000, 0),    # steps, then plane-resident kernels with their own second-stage records
     (2, 3, 14, 14, 5, 2, True, None, 0),     # plane-resident both: the plain sequence of the two passes
 ])
 def test_emulated_2d_fused_backward(B, C, H, W, K, L, bias, limit, dtype):

@@ -64,67 +64,132 @@ static int launch_fold(const wtconv_params* params, int pdtype, float* fw, float
 }
 
 // ---- planes that do not fit LDS: level-by-level kernels through an HBM pyramid ----------
-static size_t lds_fit_limit() {
-#ifdef WT_EMULATE   // host emulation only: send small planes through the level-by-level kernels
+static size_t lds_fit_limit(size_t limit) {
+#ifdef WT_EMULATE   // host emulation only: send small planes through the step kernels
   if (const char* e = getenv("WT_EMU_LDS_LIMIT")) return static_cast<size_t>(atol(e));
 #endif
-  return kLdsLimitBytes;
+  return limit;
 }
 
+static size_t plane_lds_bytes(int B, int C, int H, int W, int K, int L) {
+  return static_cast<size_t>(make_plan2d(B, C, H, W, K, L, false, 256, 4, nullptr, nullptr, nullptr).plane_lds_floats) * 4;
+}
+
+// Planes that the plane-resident kernel takes: two of them fit a CU's LDS.  With one, nothing hides its phases' latency,
+// and taking the first level as a step of its own is faster, us forward: 96x96 (16 images of 64 channels, fp32, K = 5,
+// three levels) 81 -> 70, 112x112 (12 images) 83 -> 70, 99x83 (16, fp16) 146 -> 82.  At three to a CU it is not: 80x80
+// 53.5 resident, 56.5 in steps.
 static bool plane_fits_lds(int B, int C, int H, int W, int K, int L) {
-  Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256, 4, nullptr, nullptr, nullptr);
-  return static_cast<size_t>(pl.plane_lds_floats) * 4 <= lds_fit_limit();
+  return plane_lds_bytes(B, C, H, W, K, L) <= lds_fit_limit(kLdsLimitBytes / 2);
 }
 
+// The parameter-gradient kernel (512 threads) keeps planes that fit alone: 128x128 fp32 training step 179 us, 185 with
+// one level more as a step.
 static bool wgrad_fits_lds(int B, int C, int H, int W, int K, int L) {
   Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, 4, nullptr, nullptr, nullptr, 1);
-  return static_cast<size_t>(pl.plane_lds_floats) * 4 <= lds_fit_limit();
+  return static_cast<size_t>(pl.plane_lds_floats) * 4 <= lds_fit_limit(kLdsLimitBytes);
 }
 
 constexpr long long kMaxPlaneElems = 1LL << 28;
 
-static Stream2D make_stream2d(int B, int C, int H, int W, int L) {
+// Workgroups of stream_corr_kernel that run at once (three per CU on 256 CUs; a constant, as workspace sizes must not
+// depend on the device queried): one round of them, at most one per batch item and 16 x 64 tile.
+constexpr int kStreamResident = 768;
+static int stream_chunks(int B, int C, int H, int W) {
+  const long long units = static_cast<long long>(B) * ((H + 31) / 32) * ((W + 127) / 128);
+  long long want = kStreamResident / C;
+  if (want > units) want = units;
+  return static_cast<int>(want < 1 ? 1 : want);
+}
+
+// Planes beyond LDS: how many levels are taken one at a time (kernels2d_stream.h) until what is left fits -- the layer
+// itself (`depth`), its parameter gradients, which need two pyramids (`wdepth`) --, and where the workspace keeps what
+// goes from step to step: LL bands of x (or grad_out) and results of the sub-layers, (B * C, h_d, w_d) each.
+struct Stream2D {
+  int h[kMaxLevels + 1], w[kMaxLevels + 1];
+  int depth, wdepth;
+  size_t ll[kMaxLevels + 1];     // offsets in floats from the start of an area of `floats`
+  size_t floats;
+};
+
+static Stream2D make_stream2d(int B, int C, int H, int W, int K, int L) {
   Stream2D s = {};
-  s.C = C; s.H = H; s.W = W; s.L = L;
-  s.nplanes = B * C;
   s.h[0] = H; s.w[0] = W;
   size_t off = 0;
   for (int l = 1; l <= L; ++l) {
     s.h[l] = (s.h[l - 1] + 1) / 2;
     s.w[l] = (s.w[l - 1] + 1) / 2;
-    s.aoff[l] = off;
-    off += round_up64(static_cast<size_t>(s.nplanes) * 4 * s.h[l] * s.w[l]);
-  }
-  for (int l = 2; l <= L; ++l) {
-    s.zoff[l] = off;
-    off += round_up64(static_cast<size_t>(s.nplanes) * s.h[l - 1] * s.w[l - 1]);
+    s.ll[l] = off;
+    off += round_up64(static_cast<size_t>(B) * C * s.h[l] * s.w[l]);
   }
   s.floats = off;
+  while (s.depth < L && !plane_fits_lds(B, C, s.h[s.depth], s.w[s.depth], K, L - s.depth)) ++s.depth;
+  while (s.wdepth < L && !wgrad_fits_lds(B, C, s.h[s.wdepth], s.w[s.wdepth], K, L - s.wdepth)) ++s.wdepth;
   return s;
 }
 
-// Chunks of the streamed weight-gradient kernels: the (batch item, tile) units of a level are
-// split over `nchunk` workgroups per filter, about 2048 workgroups for the base-conv launch
-// (C filters) and four times that for the sub-band launches, never more chunks than the
-// finest level has units (a constant rule: workspace sizes do not depend on the device).
-static int stream_chunks(int B, int C, int H, int W) {
-  const long units = static_cast<long>(B) * ((H + kStreamTile - 1) / kStreamTile) *
-                     ((W + kStreamTileW - 1) / kStreamTileW);
-  long want = (2048 + C - 1) / C;
-  if (want > 64) want = 64;
-  if (want > units) want = units;
-  if (want < 1) want = 1;
-  return static_cast<int>(want);
+// Partial sums of the steps, then those of the plane-resident sub-layer.
+static size_t stream_records(int B, int C, int H, int W, int K, int L) {
+  return round_up64(static_cast<size_t>(stream_chunks(B, C, H, W)) * C * ((1 + 4 * L) * K * K + 1));
+}
+static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) {
+  if (s.wdepth == L) return 0;
+  int bchunk, nchunk;
+  const int d = s.wdepth;
+  wgrad_chunks(B, C, wgrad_planes_per_iter(B, s.h[d], s.w[d], K, L - d), kWgradResident, &bchunk, &nchunk);
+  return round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * (L - d)) * K * K + 1));
 }
 
-// `shared_pyr` (level-by-level path only): where to build the whole pyramid of x -- detail bands of level 1 included --
-// for a later pass of the same call to reuse; the folded parameters then go to `shared_fw` instead of the workspace start.
+// One launch of the plane-resident kernels on planes that fit LDS; `fw` / `fb` folded parameters, those of a channel
+// `fw_stride` floats from the next one's, the level filters `fw_skip` floats behind their usual place.
+static int resident2d(const char* fn, const void* x, void* out, const float* fw, const float* fb, int B, int C, int H,
+                      int W, int K, int L, int dtype, int fw_stride, int fw_skip, hipStream_t stream) {
+  const size_t esz = dtype == WTCONV_F32 ? 4 : 2;
+  Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256, esz, x, out, nullptr);
+  int tj1 = 4, sg_shift = 8;
+  choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
+  // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
+  while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
+  finish_plane_plan(&pl, sg_shift);
+  pl.fw_stride = fw_stride;
+  pl.fw_skip = fw_skip;
+  if (static_cast<size_t>(pl.lds_floats) * 4 > kLdsLimitBytes)
+    return fail(WTCONV_E_UNSUPPORTED,
+                "%s: a %dx%d plane with %d levels needs %zu B of LDS (limit %d); plane too large for the "
+                "plane-resident kernels", fn, H, W, L, static_cast<size_t>(pl.lds_floats) * 4, kLdsLimitBytes);
+  return launch_plane2d(dtype, K, tj1, x, out, fw, fb, pl, stream);
+}
+
+// The layer on planes beyond LDS.  `ll` and `res`: areas of make_stream2d (LL bands, results of the sub-layers).
+static int stream2d_pass(const char* fn, const Stream2D& sp, const void* x, void* out, const float* fw, const float* fb,
+                         float* ll, float* res, int B, int C, int K, int L, int dtype, hipStream_t stream) {
+  const int KK = K * K, D = sp.depth, fstride = (1 + 4 * L) * KK;
+  auto type_at = [&](int d) { return d == 0 ? dtype : WTCONV_F32; };
+  auto in_at = [&](int d) { return d == 0 ? x : static_cast<const void*>(ll + sp.ll[d]); };
+  auto base_at = [&](int d) { return d == 0 ? 0 : (1 + 4 * (d - 1)) * KK; };     // filter that is step d's base conv
+  for (int d = 0; d < D && d + 1 < L; ++d)
+    if (int e = launch_stream_ll(type_at(d), in_at(d), sp.h[d], sp.w[d], ll + sp.ll[d + 1], B * C, stream)) return e;
+  if (D < L)
+    if (int e = resident2d(fn, in_at(D), res + sp.ll[D], fw + base_at(D), nullptr, B, C, sp.h[D], sp.w[D], K, L - D,
+                           WTCONV_F32, fstride, 3 * KK, stream)) return e;
+  for (int d = D - 1; d >= 0; --d) {
+    const StreamStep st = {B, C, sp.h[d], sp.w[d]};
+    void* to = d == 0 ? out : static_cast<void*>(res + sp.ll[d]);
+    if (int e = launch_stream_final(type_at(d), K, st, in_at(d), to, d + 1 < L ? res + sp.ll[d + 1] : nullptr, fw,
+                                    d == 0 ? fb : nullptr, fstride, base_at(d), (1 + 4 * d) * KK, stream)) return e;
+  }
+  return 0;
+}
+
+// `shared_ll` (planes beyond LDS only): where to leave the LL bands for a later pass of the same call; the folded
+// parameters and the results of the sub-layers then go to `shared_fw` instead of the workspace start.
+// `resident`: planes that fit LDS alone run on the plane-resident kernel, which needs room for the folded parameters only.
 // `tickets` (plane-resident paths only): C words this pass clears on its way, for the parameter-gradient pass that
 // follows it on the stream; they must lie outside the folded parameters at the workspace start.
 static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_params* params, int B, int C,
                         int H, int W, int K, int L, int dtype, int pdtype, void* ws, size_t ws_bytes,
-                        void* stream_, int flip, float* shared_pyr = nullptr, float* shared_fw = nullptr,
-                        unsigned* tickets = nullptr) {
+                        void* stream_, int flip, float* shared_ll = nullptr, float* shared_fw = nullptr,
+                        unsigned* tickets = nullptr, bool resident = false) {
   if (int e = check_common(fn, params, B, C, K, L, dtype, pdtype)) return e;
   if (H <= 0 || W <= 0) return fail(WTCONV_E_ARG, "%s: spatial size must be positive (got %dx%d)", fn, H, W);
   if (static_cast<long long>(H) * W > kMaxPlaneElems)   // 32-bit offsets inside a plane and its four stacked sub-bands
@@ -134,38 +199,27 @@ static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_p
   if ((reinterpret_cast<uintptr_t>(x) % esz) || (reinterpret_cast<uintptr_t>(out) % esz))
     return fail(WTCONV_E_ARG, "%s: tensor pointer not aligned to its element size", fn);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const size_t need = wtconv2d_workspace_bytes(B, C, H, W, K, L, flip ? WTCONV_PASS_BACKWARD_INPUT : WTCONV_PASS_FORWARD);
+  const size_t need = resident ? fold_floats(C, 4, L, K * K) * sizeof(float)
+                               : wtconv2d_workspace_bytes(B, C, H, W, K, L, flip ? WTCONV_PASS_BACKWARD_INPUT : WTCONV_PASS_FORWARD);
   if (ws == nullptr || ws_bytes < need)
     return fail(WTCONV_E_WORKSPACE, "%s: workspace of %zu B needed, %zu given", fn, need, ws_bytes);
   if (static_cast<long long>(B) * C > 0x7fffffffLL / 4)
     return fail(WTCONV_E_UNSUPPORTED, "%s: batch*channels = %lld is too large", fn, static_cast<long long>(B) * C);
   if (mfma2d_query(B, C, H, W, K, L, dtype).ok)
     return mfma2d_pass(fn, x, out, params, B, C, H, W, K, L, dtype, pdtype, stream, flip, tickets, C);
-  if (!plane_fits_lds(B, C, H, W, K, L)) {
-    const Stream2D sp = make_stream2d(B, C, H, W, L);
-    float* fw = shared_pyr != nullptr ? shared_fw : static_cast<float*>(ws);
+  if (!resident && !plane_fits_lds(B, C, H, W, K, L)) {
+    const Stream2D sp = make_stream2d(B, C, H, W, K, L);
+    float* fw = shared_ll != nullptr ? shared_fw : static_cast<float*>(ws);
     float* fb = fw + static_cast<size_t>(C) * (1 + 4 * L) * K * K;
-    float* pyr = shared_pyr != nullptr ? shared_pyr : fw + round_up64(fold_floats(C, 4, L, K * K));
+    float* res = fw + round_up64(fold_floats(C, 4, L, K * K));
+    float* ll = shared_ll != nullptr ? shared_ll : res + sp.floats;
     if (int e = launch_fold(params, pdtype, fw, fb, C, 4, L, K * K, flip, flip ? 0 : 1, stream)) return e;
-    if (shared_pyr != nullptr) {
-      if (int e = launch_stream_analysis(dtype, x, pyr, sp, stream, false)) return e;
-    }
-    return launch_stream2d(dtype, K, x, out, fw, fb, pyr, sp, stream, shared_pyr != nullptr);
+    return stream2d_pass(fn, sp, x, out, fw, fb, ll, res, B, C, K, L, dtype, stream);
   }
-  Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256, esz, x, out, nullptr);
-  int tj1 = 4, sg_shift = 8;
-  choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
-  // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
-  while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
-  finish_plane_plan(&pl, sg_shift);
-  if (static_cast<size_t>(pl.lds_floats) * 4 > kLdsLimitBytes)
-    return fail(WTCONV_E_UNSUPPORTED,
-                "%s: a %dx%d plane with %d levels needs %zu B of LDS (limit %d); plane too large for the "
-                "plane-resident kernels", fn, H, W, L, static_cast<size_t>(pl.lds_floats) * 4, kLdsLimitBytes);
   float* fw = static_cast<float*>(ws);
   float* fb = fw + static_cast<size_t>(C) * (1 + 4 * L) * K * K;
   if (int e = launch_fold(params, pdtype, fw, fb, C, 4, L, K * K, flip, flip ? 0 : 1, stream, tickets, C)) return e;
-  return launch_plane2d(dtype, K, tj1, x, out, fw, fb, pl, stream);
+  return resident2d(fn, x, out, fw, fb, B, C, H, W, K, L, dtype, (1 + 4 * L) * K * K, 0, stream);
 }
 
 // ---- row-resident 1-D kernels ----------------------------------------------------------
@@ -288,8 +342,22 @@ const char* wtconv_last_error(void) { return g_err; }
 
 int wtconv_max_kernel_size(void) { return 7; }
 
+// Whether both passes of a backward call are made of steps (planes beyond LDS): they share the LL bands of grad_out.
+static bool stream2d_backward(int B, int C, int H, int W, int K, int L) {
+  return !plane_fits_lds(B, C, H, W, K, L) && !wgrad_fits_lds(B, C, H, W, K, L);
+}
+
 size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, int pass) {
   if (pass == WTCONV_PASS_BACKWARD) {
+    if (B > 0 && C > 0 && H > 0 && W > 0 && K > 0 && levels > 0 && levels <= kMaxLevels &&
+        static_cast<long long>(H) * W <= kMaxPlaneElems && stream2d_backward(B, C, H, W, K, levels)) {
+      // what the parameter-gradient pass needs (its LL bands of grad_out serve both), folded parameters, sub-layers
+      const size_t extra = round_up64(fold_floats(C, 4, levels, K * K)) + make_stream2d(B, C, H, W, K, levels).floats;
+      const size_t both = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD_PARAMS) +
+                          (extra * sizeof(float) + 255) / 256 * 256;
+      const size_t input = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD_INPUT);
+      return both > input ? both : input;
+    }
     const size_t a = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD_INPUT);
     const size_t b = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD_PARAMS);
     return a > b ? a : b;
@@ -305,10 +373,9 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
     if (wgrad_fits_lds(B, C, H, W, K, levels)) {
       wgrad_chunks(B, C, wgrad_planes_per_iter(B, H, W, K, levels), kWgradResident, &bchunk, &nchunk);
       floats = static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1);
-    } else {      // partial sums, then the pyramids of x and of grad_out
-      nchunk = stream_chunks(B, C, H, W);
-      floats = round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1)) +
-               2 * make_stream2d(B, C, H, W, levels).floats;
+    } else {      // partial sums, then the LL bands of x and of grad_out
+      const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
+      floats = stream_records(B, C, H, W, K, levels) + stream_sub_records(sp, B, C, K, levels) + 2 * sp.floats;
     }
     if (mfloats > floats) floats = mfloats;
     floats = round_up64(floats) + static_cast<size_t>(C);      // one ticket word per channel behind the records
@@ -321,7 +388,17 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
       if (q.ok && q.ws_bytes > mf) mf = q.ws_bytes;
     }
     floats = fold_floats(C, 4, levels, K * K);
-    if (!plane_fits_lds(B, C, H, W, K, levels)) floats = round_up64(floats) + make_stream2d(B, C, H, W, levels).floats;
+    if (!plane_fits_lds(B, C, H, W, K, levels)) {
+      // (planes beyond LDS: never less than the four bands of every level, which these calls once kept here, so that the
+      // shapes refused for want of static scratch are the same)
+      size_t area = 0;
+      const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
+      if (plane_lds_bytes(B, C, H, W, K, levels) > static_cast<size_t>(kLdsLimitBytes))
+        for (int l = 1; l <= levels; ++l)
+          area += round_up64(static_cast<size_t>(B) * C * sp.h[l] * sp.w[l] * (l < levels ? 5 : 4));
+      if (area < 2 * sp.floats) area = 2 * sp.floats;
+      floats = round_up64(floats) + area;
+    }
     if (mf > floats * sizeof(float)) floats = (mf + 3) / 4;
   }
   return (floats * sizeof(float) + 255) / 256 * 256;
@@ -339,15 +416,18 @@ size_t wtconv_static_scratch_bytes(void) { return kStaticScratchBytes; }
 int wtconv2d_forward_static(const void* x, void* out, const wtconv_params* params, int B, int C, int H, int W,
                             int K, int levels, int dtype, int param_dtype, void* stream) {
   const char* fn = "wtconv2d_forward_static";
-  const size_t need = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_FORWARD);
-  if (need > kStaticScratchBytes)
+  size_t need = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_FORWARD);
+  // (planes that are faster in steps, but not with this much scratch, stay in LDS where they fit)
+  const bool resident = need > kStaticScratchBytes && fold_floats(C, 4, levels, K * K) * sizeof(float) <= kStaticScratchBytes &&
+                        plane_lds_bytes(B, C, H, W, K, levels) <= static_cast<size_t>(kLdsLimitBytes);
+  if (need > kStaticScratchBytes && !resident)
     return fail(WTCONV_E_UNSUPPORTED,
                 "%s: this shape needs %zu B of scratch, the static buffer holds %zu B; use wtconv2d_forward with a "
                 "caller-supplied workspace", fn, need, kStaticScratchBytes);
   void* ptr = nullptr;
   if (int e = static_scratch(fn, &ptr)) return e;
   return plane2d_pass(fn, x, out, params, B, C, H, W, K, levels, dtype, param_dtype, ptr, kStaticScratchBytes,
-                      stream, 0);
+                      stream, 0, nullptr, nullptr, nullptr, resident);
 }
 
 int wtconv2d_backward_input(const void* grad_out, void* grad_x, const wtconv_params* params, int B, int C,
@@ -363,12 +443,12 @@ static unsigned* wgrad2d_tickets(void* workspace, int B, int C, int H, int W, in
   return reinterpret_cast<unsigned*>(static_cast<char*>(workspace) + need) - C;
 }
 
-// have_g_pyramid (level-by-level path only): the pyramid of grad_out is in its place in the workspace already.
+// have_g_ll (planes beyond LDS only): the LL bands of grad_out that the layer itself needs are in the workspace already.
 // tickets_zeroed (plane-resident paths only): an earlier kernel on the stream has cleared the channel tickets.
 static int backward_params2d(const char* fn, const void* x, const void* grad_out, const wtconv_params* params,
                              const wtconv_param_grads* grads, int B, int C, int H, int W, int K, int levels,
                              int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
-                             void* stream_, bool have_g_pyramid, bool tickets_zeroed = false) {
+                             void* stream_, bool have_g_ll, bool tickets_zeroed = false) {
   const int L = levels;
   if (int e = check_common(fn, params, B, C, K, L, dtype, param_dtype)) return e;
   if (H <= 0 || W <= 0) return fail(WTCONV_E_ARG, "%s: spatial size must be positive (got %dx%d)", fn, H, W);
@@ -393,6 +473,7 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
   int bchunk, nchunk;
   float* partial = static_cast<float*>(workspace);
   int e;
+  SubRecords sub = {};
   const Mfma2dWgradQuery mq = mfma2d_wgrad_query(B, C, H, W, K, L, dtype);
   const bool resident = mq.ok || wgrad_fits_lds(B, C, H, W, K, L);
   // The plane-resident first-stage kernels finish their channels themselves (last workgroup of a channel): one ticket
@@ -418,18 +499,42 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
     wgrad_chunks(B, C, pb, kWgradResident, &bchunk, &nchunk);
     e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream);
   } else {
-    const Stream2D sp = make_stream2d(B, C, H, W, L);
+    const Stream2D sp = make_stream2d(B, C, H, W, K, L);
     nchunk = stream_chunks(B, C, H, W);
-    if (nchunk > 65535 || C > 0x7fffffff / 4) return fail(WTCONV_E_UNSUPPORTED, "%s: too many chunks (%d)", fn, nchunk);
-    float* pyr_x = partial + round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * L) * K * K + 1));
-    float* pyr_g = pyr_x + sp.floats;
-    e = launch_stream2d_wgrad(dtype, K, x, grad_out, partial, pyr_x, pyr_g, sp, B, nchunk, stream, have_g_pyramid);
+    float* sub_partial = partial + stream_records(B, C, H, W, K, L);
+    float* gll = sub_partial + stream_sub_records(sp, B, C, K, L);
+    float* xll = gll + sp.floats;
+    const int D = sp.wdepth;
+    e = 0;
+    for (int d = 0; d <= D && d <= L && !e; ++d) {
+      const int dt = d == 0 ? dtype : WTCONV_F32;
+      const void* xd = d == 0 ? x : static_cast<const void*>(xll + sp.ll[d]);
+      const void* gd = d == 0 ? grad_out : static_cast<const void*>(gll + sp.ll[d]);
+      if (d == D && d < L) {       // the rest fits LDS
+        const int Ls = L - d, pb = wgrad_planes_per_iter(B, sp.h[d], sp.w[d], K, Ls);
+        Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, 4, xd, gd, nullptr, pb);
+        finish_wgrad_plan(&pl, K);
+        int sub_chunk;
+        wgrad_chunks(B, C, pb, kWgradResident, &sub_chunk, &sub.nchunk);
+        sub.partial = sub_partial;
+        sub.depth = d;
+        e = launch_wgrad2d(WTCONV_F32, K, Ls, xd, gd, sub_partial, pl, B, sub_chunk, sub.nchunk, FinishArgs{}, stream);
+        break;
+      }
+      // a step; at d == L only the LL band's own filter is left, the base conv of a layer without levels
+      const StreamStep st = {B, C, sp.h[d], sp.w[d]};
+      const bool more = d < L;
+      const bool g_there = have_g_ll && d + 1 <= sp.depth && d + 1 < L;
+      const StreamCorrOut o = {partial, (1 + 4 * L) * K * K + 1, d == 0 ? 0 : 1 + 4 * (d - 1), 2 + 4 * d, d == 0 ? 1 : 0};
+      e = launch_stream_corr(dt, K, st, xd, gd, more ? xll + sp.ll[d + 1] : nullptr,
+                             more && !g_there ? gll + sp.ll[d + 1] : nullptr, more, o, nchunk, stream);
+    }
   }
   if (e || resident) return e;
   const GradTable gt = to_grad_table(grads, L);
   const int nrec = (1 + 4 * L) * K * K + 1;
   WT_LAUNCH(wgrad_finish_kernel, dim3(C), dim3(finish_threads(nrec)), static_cast<size_t>(nrec) * sizeof(float),
-            stream, partial, nchunk, to_table(params, L), param_dtype, gt, C, 4, L, K * K);
+            stream, partial, nchunk, to_table(params, L), param_dtype, gt, C, 4, L, K * K, sub);
   return check_launch("wgrad_finish_kernel");
 }
 
@@ -444,28 +549,25 @@ int wtconv2d_backward_params(const void* x, const void* grad_out, const wtconv_p
 int wtconv2d_backward(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
                       const wtconv_param_grads* grads, int B, int C, int H, int W, int K, int levels, int dtype,
                       int param_dtype, void* workspace, size_t workspace_bytes, void* stream) {
-  // Planes beyond LDS (both passes level by level): the pyramid of grad_out is built once, in the place the
-  // parameter-gradient pass keeps it, and serves both passes; the folded parameters of the input-gradient pass sit
-  // where the pyramid of x goes afterwards.
+  // Planes beyond LDS (both passes in steps): the LL bands of grad_out are built once, in the place where the
+  // parameter-gradient pass keeps them, and serve both passes.
   const bool sizes_ok = B > 0 && C > 0 && H > 0 && W > 0 && K >= 1 && K % 2 == 1 && K <= wtconv_max_kernel_size() &&
-                        levels >= 2 && levels <= kMaxLevels && static_cast<long long>(H) * W <= kMaxPlaneElems;
-  if (sizes_ok && !mfma2d_query(B, C, H, W, K, levels, dtype).ok && !plane_fits_lds(B, C, H, W, K, levels) &&
-      !mfma2d_wgrad_query(B, C, H, W, K, levels, dtype).ok && !wgrad_fits_lds(B, C, H, W, K, levels)) {
+                        levels >= 1 && levels <= kMaxLevels && static_cast<long long>(H) * W <= kMaxPlaneElems;
+  if (sizes_ok && !mfma2d_query(B, C, H, W, K, levels, dtype).ok && !mfma2d_wgrad_query(B, C, H, W, K, levels, dtype).ok &&
+      stream2d_backward(B, C, H, W, K, levels)) {
     const size_t need = wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD);
     if (workspace == nullptr || workspace_bytes < need)
       return fail(WTCONV_E_WORKSPACE, "wtconv2d_backward: workspace of %zu B needed, %zu given", need, workspace_bytes);
-    const Stream2D sp = make_stream2d(B, C, H, W, levels);
-    const int nchunk = stream_chunks(B, C, H, W);
-    float* partial = static_cast<float*>(workspace);
-    float* pyr_x = partial + round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1));
-    float* pyr_g = pyr_x + sp.floats;
-    if (fold_floats(C, 4, levels, K * K) <= sp.floats) {
-      if (int e = plane2d_pass("wtconv2d_backward", grad_out, grad_x, params, B, C, H, W, K, levels, dtype, param_dtype,
-                               workspace, workspace_bytes, stream, 1, pyr_g, pyr_x))
-        return e;
-      return backward_params2d("wtconv2d_backward", x, grad_out, params, grads, B, C, H, W, K, levels, dtype,
-                               param_dtype, workspace, workspace_bytes, stream, true);
-    }
+    const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
+    float* gll = static_cast<float*>(workspace) + stream_records(B, C, H, W, K, levels) +
+                 stream_sub_records(sp, B, C, K, levels);
+    float* fw = static_cast<float*>(workspace) +
+                wtconv2d_workspace_bytes(B, C, H, W, K, levels, WTCONV_PASS_BACKWARD_PARAMS) / sizeof(float);
+    if (int e = plane2d_pass("wtconv2d_backward", grad_out, grad_x, params, B, C, H, W, K, levels, dtype, param_dtype,
+                             workspace, workspace_bytes, stream, 1, gll, fw))
+      return e;
+    return backward_params2d("wtconv2d_backward", x, grad_out, params, grads, B, C, H, W, K, levels, dtype,
+                             param_dtype, workspace, workspace_bytes, stream, true);
   }
   // Otherwise the two passes run one after the other on the stream and share the workspace.  Plane-resident shapes:
   // the input-gradient pass clears the channel tickets of the parameter-gradient pass on its way (one launch fewer),
@@ -575,7 +677,7 @@ int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_p
   for (int l = 0; l < L; ++l) { gt.wt_weight[l] = grads->wt_weight[l]; gt.wt_scale[l] = grads->wt_scale[l]; }
   const int nrec = (1 + 2 * L) * K + 1;
   WT_LAUNCH(wgrad_finish_kernel, dim3(C), dim3(finish_threads(nrec)), static_cast<size_t>(nrec) * sizeof(float),
-            stream, partial, nchunk, to_table(params, L), param_dtype, gt, C, 2, L, K);
+            stream, partial, nchunk, to_table(params, L), param_dtype, gt, C, 2, L, K, SubRecords{});
   return check_launch("wgrad_finish_kernel");
 }
 

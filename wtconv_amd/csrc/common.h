@@ -313,6 +313,14 @@ __device__ __forceinline__ uint4 load_u4(const void* p) {
   memcpy(&r, p, sizeof(r));
   return r;
 }
+template <int ALIGN = 8>
+__device__ __forceinline__ uint2 load_u2(const void* p) {
+  uint2 r;
+  memcpy(&r, p, sizeof(r));
+  return r;
+}
+template <int ALIGN = 16>
+__device__ __forceinline__ void store_u4(void* p, const uint4& q) { memcpy(p, &q, sizeof(q)); }
 template <int ALIGN = 16>
 __device__ __forceinline__ uint4 load_stream_u4(const void* p) { return load_u4<ALIGN>(p); }
 template <int ALIGN = 16>
@@ -322,12 +330,28 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 template <int ALIGN> struct U4At { typedef u32x4_t type; };
 template <> struct U4At<4> { typedef u32x4_t type __attribute__((aligned(4))); };
 template <> struct U4At<2> { typedef u32x4_t type __attribute__((aligned(2))); };
+typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+template <int ALIGN> struct U2At { typedef u32x2_t type; };
+template <> struct U2At<2> { typedef u32x2_t type __attribute__((aligned(2))); };
 template <int ALIGN = 16>
 __device__ __forceinline__ uint4 load_u4(const void* p) {
   const u32x4_t v = *reinterpret_cast<const typename U4At<ALIGN>::type*>(p);
   uint4 r;
   r.x = v.x; r.y = v.y; r.z = v.z; r.w = v.w;
   return r;
+}
+template <int ALIGN = 8>
+__device__ __forceinline__ uint2 load_u2(const void* p) {
+  const u32x2_t v = *reinterpret_cast<const typename U2At<ALIGN>::type*>(p);
+  uint2 r;
+  r.x = v.x; r.y = v.y;
+  return r;
+}
+template <int ALIGN = 16>
+__device__ __forceinline__ void store_u4(void* p, const uint4& q) {
+  u32x4_t v;
+  v.x = q.x; v.y = q.y; v.z = q.z; v.w = q.w;
+  *reinterpret_cast<typename U4At<ALIGN>::type*>(p) = v;
 }
 template <int ALIGN = 16>
 __device__ __forceinline__ uint4 load_stream_u4(const void* p) {

@@ -50,6 +50,9 @@ struct Plan2D {
   int block;                   // plane kernel: threads per workgroup (256, or 512 = two whole-workgroup planes)
   int pb;                      // weight-gradient kernel: planes of one channel stacked per iteration
   int slot_shift;              //   log2 of the threads that load/analyse one of them
+  int fw_stride;               // plane kernel: folded filters of a channel to the next channel's (floats)
+  int fw_skip;                 //   floats between where the level filters would follow the base filter and where they
+                               //   are (a sub-layer's base filter is the LL filter of the level above it)
 };
 
 // ------------------------------------------------------------------ parameter folding
@@ -650,7 +653,8 @@ __global__ __launch_bounds__(512, 4) void wt2d_plane_kernel(const T* __restrict_
   const Plan2D& pl = Geo::kStatic ? kGeo : plarg;
   const int nB = plarg.B, nC = plarg.C, nplanes = plarg.nplanes, gpc = plarg.groups_per_channel;
   constexpr int KK = K * K;
-  const int NF = 1 + 4 * pl.L;
+  const int fw_stride = Geo::kStatic ? (1 + 4 * pl.L) * KK : plarg.fw_stride;
+  const int fw_skip = Geo::kStatic ? 0 : plarg.fw_skip;
   const size_t plane_elems = static_cast<size_t>(pl.H) * pl.W;
   const int tid = threadIdx.x;
   const int sg = 1 << pl.sg_shift;
@@ -732,7 +736,7 @@ __global__ __launch_bounds__(512, 4) void wt2d_plane_kernel(const T* __restrict_
     const int c = WT_UNIFORM(channel_of(nxt));
     const bool live = plane >= 0;
     advance(nxt);
-    wt_uniform_ptr fwc = (wt_uniform_ptr)(fw + static_cast<size_t>(c) * NF * KK);
+    wt_uniform_ptr fwc = (wt_uniform_ptr)(fw + static_cast<size_t>(c) * fw_stride);
     const size_t plane_off = static_cast<size_t>(live ? plane : 0) * plane_elems;
     int l0 = 2;
     WT_WAVE_PRIORITY(3);
@@ -768,12 +772,13 @@ __global__ __launch_bounds__(512, 4) void wt2d_plane_kernel(const T* __restrict_
     }
     for (int lv = pl.L; lv >= 2; --lv) {
       const int l = WT_UNIFORM(lv);
-      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + (1 + 4 * (l - 1)) * KK, ltid, sg);
+      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + fw_skip + (1 + 4 * (l - 1)) * KK, ltid, sg);
       plane_sync(wave_local);
     }
     WT_WAIT_VMEM();     // next plane's loads have landed; the stores below are not waited for
     WT_WAVE_PRIORITY(0);
-    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + KK, fb[c], out + plane_off, ltid, sg);
+    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, fb != nullptr ? fb[c] : 0.f, out + plane_off,
+                                        ltid, sg);
     plane_sync(wave_local);   // the next plane overwrites the buffers read above
   }
 }
@@ -1081,9 +1086,9 @@ __global__ __launch_bounds__(512, 4) void wt2d_wgrad_kernel(const T* __restrict_
 // The second stage as a launch of its own (one workgroup per channel, dynamic LDS NF*KK + 1 floats): after a first
 // stage that does not finish its channels itself.
 static __global__ void wgrad_finish_kernel(const float* __restrict__ partial, int nchunk, ParamTable p,
-                                    int pdtype, GradTable gt, int C, int S, int L, int KK) {
+                                    int pdtype, GradTable gt, int C, int S, int L, int KK, SubRecords sub) {
   WT_SHARED_FLOATS(prod);
-  wgrad_finish_channel<false>(partial, nchunk, p, pdtype, gt, C, static_cast<int>(blockIdx.x), S, L, KK, prod);
+  wgrad_finish_channel<false>(partial, nchunk, p, pdtype, gt, C, static_cast<int>(blockIdx.x), S, L, KK, prod, sub);
 }
 
 // Clears the ticket words of a first stage that finishes its channels itself (a kernel rather than a memset, so

@@ -27,13 +27,14 @@ int launch_plane2d(int dtype, int K, int tj1, const void* x, void* out, const fl
 int launch_wgrad2d(int dtype, int K, int L, const void* x, const void* g, float* partial, const Plan2D& pl, int B, int bchunk,
                    int nchunk, const FinishArgs& fin, hipStream_t stream);
 
-// stream2d.hip: both, level by level, for planes beyond LDS.
-struct Stream2D;
-int launch_stream_analysis(int dtype, const void* src, float* pyr, const Stream2D& sp, hipStream_t stream, bool ll_only);
-int launch_stream2d(int dtype, int K, const void* x, void* out, const float* fw, const float* fb, float* pyr, const Stream2D& sp,
-                    hipStream_t stream, bool have_pyramid);
-int launch_stream2d_wgrad(int dtype, int K, const void* x, const void* g, float* partial, float* pyr_x, float* pyr_g,
-                          const Stream2D& sp, int B, int nchunk, hipStream_t stream, bool have_g_pyramid);
+// stream2d.hip: the steps that both are made of on planes beyond LDS.
+struct StreamStep { int B, C, H, W; };
+struct StreamCorrOut;
+int launch_stream_ll(int dtype, const void* src, int hs, int ws, float* dst, int nplanes, hipStream_t stream);
+int launch_stream_final(int dtype, int K, const StreamStep& st, const void* x, void* out, const float* sub, const float* fw,
+                        const float* fb, int fstride, int fbase, int fband, hipStream_t stream);
+int launch_stream_corr(int dtype, int K, const StreamStep& st, const void* x, const void* g, float* xll, float* gll,
+                       bool bands, const StreamCorrOut& outp, int nchunk, hipStream_t stream);
 
 // conv1d.hip: the 1-D layer, by tiles of a row and with rows in registers.
 int launch_tile1d(int dtype, const void* x, void* out, const float* fw, const float* fb, const Plan1D& pl, int B,

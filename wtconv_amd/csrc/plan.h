@@ -87,6 +87,7 @@ constexpr Plan2D make_plan2d_geometry(int B, int C, int H, int W, int K, int L, 
   pl.slot_shift = log2_int(nthreads);
   pl.lds_floats = pl.plane_lds_floats;
   pl.groups_per_channel = 1;
+  pl.fw_stride = (1 + 4 * L) * K * K;
   pl.vec_ok = W % 4 == 0;                         // (and aligned pointers: make_plan2d)
   return pl;
 }
@@ -148,7 +149,7 @@ struct PlaneGeoStatic {
 inline bool same_plane_geometry(const Plan2D& a, const Plan2D& b) {
   if (a.H != b.H || a.W != b.W || a.L != b.L || a.P != b.P || a.lds_floats != b.lds_floats || a.vec_ok != b.vec_ok ||
       a.prefetch != b.prefetch || a.sg_shift != b.sg_shift || a.plane_lds_floats != b.plane_lds_floats ||
-      a.fuse != b.fuse || a.block != b.block)
+      a.fuse != b.fuse || a.block != b.block || a.fw_stride != b.fw_stride || a.fw_skip != b.fw_skip)
     return false;
   for (int l = 0; l <= a.L; ++l)
     if (a.h[l] != b.h[l] || a.w[l] != b.w[l] || a.aoff[l] != b.aoff[l] || a.astr[l] != b.astr[l] ||

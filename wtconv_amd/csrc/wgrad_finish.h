@@ -16,10 +16,19 @@ namespace wt {
 // runs this, so the result does not depend on the order in which the first stage finished.  SHARED: called by the
 // last workgroup of a first stage that finishes its channels itself: the records of the other workgroups are read
 // with load_shared_f32.
+// Records of a sub-layer that starts `depth` levels down (0: none): its base filter is the LL filter of level `depth`,
+// its levels are the layer's below that.
+struct SubRecords {
+  const float* partial;
+  int nchunk;
+  int depth;
+};
+
 template <bool SHARED>
 __device__ __forceinline__ void wgrad_finish_channel(const float* __restrict__ partial, int nchunk,
                                                      const ParamTable& p, int pdtype, const GradTable& gt, int C,
-                                                     int c, int S, int L, int KK, float* __restrict__ prod) {
+                                                     int c, int S, int L, int KK, float* __restrict__ prod,
+                                                     const SubRecords& sub = SubRecords{}) {
   const int NF = 1 + S * L;
   const int stride = NF * KK + 1;
   // table entries of a level picked with constant indices (a per-lane index into the argument structs would send
@@ -44,9 +53,21 @@ __device__ __forceinline__ void wgrad_finish_channel(const float* __restrict__ p
     const float gam = load_param(f == 0 ? p.base_scale : level_s(l), pdtype, chn);
     const float wv = load_param(f == 0 ? p.base_weight : level_w(l), pdtype, chn * KK + t);
     float sum = 0.f;
+    const float* rec = partial + static_cast<size_t>(c) * stride + o;
+    size_t step = static_cast<size_t>(C) * stride;
+    int nrec = nchunk;
+    if constexpr (!SHARED) {
+      const int fsub = 1 + S * (sub.depth - 1);
+      if (sub.depth > 0 && tap && (f == fsub || f >= fsub + S)) {
+        const int sstride = (1 + S * (L - sub.depth)) * KK + 1;
+        rec = sub.partial + static_cast<size_t>(c) * sstride + (f == fsub ? 0 : f - S * sub.depth) * KK + t;
+        step = static_cast<size_t>(C) * sstride;
+        nrec = sub.nchunk;
+      }
+    }
 #pragma unroll 8                       // several chunk loads in flight; the order of the adds is unchanged
-    for (int ch = 0; ch < nchunk; ++ch) {
-      const float* src = partial + (static_cast<size_t>(ch) * C + c) * stride + o;
+    for (int ch = 0; ch < nrec; ++ch) {
+      const float* src = rec + ch * step;
       sum += SHARED ? load_shared_f32(src) : *src;
     }
     if (tap) {
