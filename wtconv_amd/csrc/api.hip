@@ -150,6 +150,8 @@ static int resident2d(const char* fn, const void* x, void* out, const float* fw,
   choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
   // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
   while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
+  if (!plane_shape_is_static(K, H, W, L))
+    widen_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, pl.nplanes, &tj1, &sg_shift);
   finish_plane_plan(&pl, sg_shift);
   pl.fw_stride = fw_stride;
   pl.fw_skip = fw_skip;

@@ -47,7 +47,7 @@ struct Plan2D {
   int plane_lds_floats;        // LDS of one plane slot; lds_floats = slots * this
   int groups_per_channel;      // sg < 64: a wave holds 64/sg planes of one channel; number of such groups per channel
   int fuse;                    // deepest analysis level produced from registers at commit (1..3)
-  int block;                   // plane kernel: threads per workgroup (256, or 512 = two whole-workgroup planes)
+  int block;                   // plane kernel: threads per workgroup (256; 512 or 1024 = one plane)
   int pb;                      // weight-gradient kernel: planes of one channel stacked per iteration
   int slot_shift;              //   log2 of the threads that load/analyse one of them
   int fw_stride;               // plane kernel: folded filters of a channel to the next channel's (floats)
@@ -630,10 +630,10 @@ __device__ __forceinline__ void zero_lds(float* lds, int nfloats) {
 }
 
 // Forward (and, with flipped folded weights and zero fb, input-gradient) kernel.
-// Persistent: grid.x = min(work units, resident workgroups), block = 256 or 512 threads.
+// Persistent: grid.x = min(work units, resident workgroups), block = 256 threads, or 512 or 1024 that share one plane
+// where few planes run on a CU at once (widen_plane_shape).
 // 2^sg_shift threads share a plane, so a workgroup holds blockDim >> sg_shift planes, each in
-// its own LDS slot (small planes: up to 16 per workgroup; planes that take 256 threads run
-// two to a workgroup, which halves the barrier-bound cost of their small coarse levels).  When a plane takes less than a wave,
+// its own LDS slot (small planes: up to 16 per workgroup).  When a plane takes less than a wave,
 // the planes of one wave are the same channel of consecutive batch items, so the folded
 // weights stay wave-uniform (SGPRs).  The zero halos written once stay valid for every plane
 // (only interiors are rewritten).
@@ -645,7 +645,7 @@ __device__ __forceinline__ void zero_lds(float* lds, int nfloats) {
 // instruction immediates, loops over levels unroll), or the run-time plan of the argument for any other shape;
 // batch, channels and what follows from them always come from the argument.
 template <typename T, int K, int TJ1, int TJC, int MODE, typename Geo>
-__global__ __launch_bounds__(512, 4) void wt2d_plane_kernel(const T* __restrict__ x, T* __restrict__ out,
+__global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict__ x, T* __restrict__ out,
                                                          const float* __restrict__ fw,
                                                          const float* __restrict__ fb, const Plan2D plarg) {
   WT_SHARED_FLOATS(lds_all);

@@ -105,7 +105,7 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
 constexpr void finish_plane_plan(Plan2D* pl, int tj1_sg_shift) {
   pl->sg_shift = tj1_sg_shift;
   const int sg = 1 << pl->sg_shift;
-  pl->block = 256;   // (two whole planes per 512-thread workgroup measured slower: lockstep phases)
+  pl->block = sg > 256 ? sg : 256;   // (two whole planes per 512-thread workgroup measured slower: lockstep phases)
   const int slots = pl->block / sg;
   pl->lds_floats = pl->plane_lds_floats * slots;
   const int ppw = sg < kWave ? kWave / sg : 1;
@@ -135,6 +135,35 @@ constexpr Plan2D static_plane_plan(int H, int W, int K, int L, int* tj1_out) {
   if (tj1_out != nullptr) *tj1_out = tj1;
   return pl;
 }
+// Shapes with a compile-time plan of the plane kernel (plane2d.hip): the WTConvNeXt stages.
+constexpr bool plane_shape_is_static(int K, int H, int W, int L) {
+  return K == 5 && H == W && ((H == 56 && L == 3) || (H == 28 && L == 3) || (H == 14 && L == 2) || (H == 7 && L == 2));
+}
+
+// More threads for a plane, when the workgroups a CU can hold at once -- by LDS, or for want of planes -- leave it with
+// fewer than twelve waves: the phases of a plane are bound by the latency of LDS then, and halving what a thread does
+// shortens them.  The level-1 strip is the one that gets most done at a time (narrower ones read more LDS per FMA).
+// Forward us, fp32, K = 5, three levels, 256 threads -> widened: [16,64,80,80] (two by LDS) 53.6 -> 43.6, [16,64,72,72]
+// (K = 3, two levels) 35.7 -> 26.4, [16,64,68,68] (five levels) 67.2 -> 49.6; [1,64,40,40] (64 planes) 19.2 -> 17.7,
+// [8,32,64,64] 19.2 -> 18.6.  Planes with a compile-time plan stay with it: [2,96,56,56] 15.2, widened 18.4.
+inline void widen_plane_shape(int h1, int w1, size_t plane_lds_bytes, int nplanes, int* tj1, int* sg_shift) {
+  if (*sg_shift != 8) return;
+  int wgs = plane_lds_bytes ? static_cast<int>(kLdsLimitBytes / plane_lds_bytes) : 1;
+  if (wgs > (nplanes + 255) / 256) wgs = (nplanes + 255) / 256;
+  while (*sg_shift < 10 && (wgs << *sg_shift) < 768) ++*sg_shift;
+  if (*sg_shift == 8) return;
+  const int sg = 1 << *sg_shift;
+  double best = -1.0;
+  for (int tj = 4; tj >= 1; tj /= 2) {
+    const int gs = pow2_ceil((w1 + tj - 1) / tj);
+    const int rpp = sg / gs > 0 ? sg / gs : 1;
+    const int passes = (h1 + rpp - 1) / rpp;
+    const double eff = static_cast<double>(h1) * w1 / (static_cast<double>(sg) * passes * tj) *
+                       (tj == 4 ? 1.0 : tj == 2 ? 0.85 : 0.65);
+    if (eff > best + 1e-9) { best = eff; *tj1 = tj; }
+  }
+}
+
 template <int H, int W, int K, int L>
 struct PlaneGeoStatic {
   static constexpr bool kStatic = true;
