@@ -891,8 +891,10 @@ __device__ __forceinline__ void corr_level(const float* __restrict__ A, int astr
 constexpr int wgrad_sets(int L) { return L >= 4 ? 3 : (L >= 2 ? 2 : 1); }
 constexpr int kStripMinWidth = 12;   // coarse levels of the weight-gradient kernel: strips from this width on
 
+// Registers: with up to three sets of 49 sums K = 7 needs more than the 128 that two workgroups a CU leave each lane (it
+// spilled 300 to 640 bytes a lane): [16,64,56,56] fp32, three levels, training step 154 -> 128.5 us with 256.
 template <typename T, int K, int L, int TJ, typename Geo>
-__global__ __launch_bounds__(512, 4) void wt2d_wgrad_kernel(const T* __restrict__ x, const T* __restrict__ g,
+__global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T* __restrict__ x, const T* __restrict__ g,
                                                          float* __restrict__ partial, const Plan2D plarg,
                                                          int B, int bchunk, const FinishArgs fin) {
   WT_SHARED_FLOATS(lds);
