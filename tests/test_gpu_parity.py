@@ -221,6 +221,28 @@ def test_1d_rows_at_any_address(hip_device, dtype, N, K, L):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("H,W,K,L", [(5, 3, 3, 1), (6, 4, 5, 2), (14, 13, 5, 2), (31, 30, 7, 3), (45, 37, 3, 3), (66, 67, 5, 4),
+                                     (98, 101, 5, 3)])
+def test_2d_planes_at_any_address(hip_device, dtype, H, W, K, L):
+    """Planes that start at any element's address give, bit for bit, what planes at a 16-byte boundary give."""
+    W2, _ = _mods()
+    torch.manual_seed(0)
+    mod = W2(3, 3, K, wt_levels=L).to(hip_device)
+    n, got = 2 * 3 * H * W, []
+    for off in (0, 1, 3):
+        x, g = (torch.empty(n + off, device=hip_device, dtype=dtype)[off:].view(2, 3, H, W) for _ in range(2))
+        gen = torch.Generator(device=hip_device).manual_seed(5)
+        x.normal_(generator=gen)
+        g.normal_(generator=gen)
+        x.requires_grad_(True)
+        out = mod(x)
+        got.append([out.detach()] + list(torch.autograd.grad(out, [x] + [p for p in mod.parameters() if p.requires_grad], g)))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert torch.equal(a, b)
+
+
 def test_1d_bf16(hip_device):
     _, W1 = _mods()
     ref, x, g = U.seeded_case("1d", 16, 5, 4, (4, 16, 1024))

@@ -72,7 +72,7 @@ static size_t lds_fit_limit(size_t limit) {
 }
 
 static size_t plane_lds_bytes(int B, int C, int H, int W, int K, int L) {
-  return static_cast<size_t>(make_plan2d(B, C, H, W, K, L, false, 256, 4, nullptr, nullptr, nullptr).plane_lds_floats) * 4;
+  return static_cast<size_t>(make_plan2d(B, C, H, W, K, L, false, 256).plane_lds_floats) * 4;
 }
 
 // Planes that the plane-resident kernel takes: two of them fit a CU's LDS.  With one, nothing hides its phases' latency,
@@ -86,7 +86,7 @@ static bool plane_fits_lds(int B, int C, int H, int W, int K, int L) {
 // The parameter-gradient kernel (512 threads) keeps planes that fit alone: 128x128 fp32 training step 179 us, 185 with
 // one level more as a step.
 static bool wgrad_fits_lds(int B, int C, int H, int W, int K, int L) {
-  Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, 4, nullptr, nullptr, nullptr, 1);
+  Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512);
   return static_cast<size_t>(pl.plane_lds_floats) * 4 <= lds_fit_limit(kLdsLimitBytes);
 }
 
@@ -144,8 +144,7 @@ static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) 
 // `fw_stride` floats from the next one's, the level filters `fw_skip` floats behind their usual place.
 static int resident2d(const char* fn, const void* x, void* out, const float* fw, const float* fb, int B, int C, int H,
                       int W, int K, int L, int dtype, int fw_stride, int fw_skip, hipStream_t stream) {
-  const size_t esz = dtype == WTCONV_F32 ? 4 : 2;
-  Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256, esz, x, out, nullptr);
+  Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256);
   int tj1 = 4, sg_shift = 8;
   choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
   // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
@@ -496,7 +495,7 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
     e = mfma2d_wgrad_pass(fn, x, grad_out, partial, B, C, H, W, K, L, fin, stream);
   } else if (resident) {
     const int pb = wgrad_planes_per_iter(B, H, W, K, L);
-    Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, esz, x, grad_out, nullptr, pb);
+    Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, pb);
     finish_wgrad_plan(&pl, K);
     wgrad_chunks(B, C, pb, kWgradResident, &bchunk, &nchunk);
     e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream);
@@ -514,7 +513,7 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
       const void* gd = d == 0 ? grad_out : static_cast<const void*>(gll + sp.ll[d]);
       if (d == D && d < L) {       // the rest fits LDS
         const int Ls = L - d, pb = wgrad_planes_per_iter(B, sp.h[d], sp.w[d], K, Ls);
-        Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, 4, xd, gd, nullptr, pb);
+        Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, pb);
         finish_wgrad_plan(&pl, K);
         int sub_chunk;
         wgrad_chunks(B, C, pb, kWgradResident, &sub_chunk, &sub.nchunk);

@@ -319,6 +319,8 @@ __device__ __forceinline__ uint2 load_u2(const void* p) {
   memcpy(&r, p, sizeof(r));
   return r;
 }
+template <int ALIGN = 8>
+__device__ __forceinline__ void store_u2(void* p, const uint2& q) { memcpy(p, &q, sizeof(q)); }
 template <int ALIGN = 16>
 __device__ __forceinline__ void store_u4(void* p, const uint4& q) { memcpy(p, &q, sizeof(q)); }
 template <int ALIGN = 16>
@@ -346,6 +348,12 @@ __device__ __forceinline__ uint2 load_u2(const void* p) {
   uint2 r;
   r.x = v.x; r.y = v.y;
   return r;
+}
+template <int ALIGN = 8>
+__device__ __forceinline__ void store_u2(void* p, const uint2& q) {
+  u32x2_t v;
+  v.x = q.x; v.y = q.y;
+  *reinterpret_cast<typename U2At<ALIGN>::type*>(p) = v;
 }
 template <int ALIGN = 16>
 __device__ __forceinline__ void store_u4(void* p, const uint4& q) {

@@ -37,8 +37,7 @@ struct Plan2D {
   int gstr[kMaxLevels + 1];    //   zero padded on the right/bottom, no halo
   int gpl[kMaxLevels + 1];
   int lds_floats;              // total, including slack
-  int vec_ok;                  // W % 4 == 0 and every tensor pointer aligned to 4 elements:
-                               //   rows can be moved as 4-element vectors
+  int vec_ok;                  // W >= 4: rows are moved in pieces of 4 elements
   int prefetch;                // vec_ok and a plane is at most kFetchPasses pieces per thread:
                                //   the next plane is fetched into registers during compute
   int nplanes;                 // B * C
@@ -124,23 +123,37 @@ __device__ __forceinline__ int group_shift(int nitem) {
   return nitem <= 1 ? 0 : 32 - __clz(nitem - 1);
 }
 
-// Four consecutive elements from HBM (address aligned to 4 elements).
+// Four consecutive elements from any element address.
 template <typename T>
-__device__ __forceinline__ void load4(const T* __restrict__ p, float (&v)[4]) {
+__device__ __forceinline__ void load4_any(const T* __restrict__ p, float (&v)[4]) {
   if constexpr (sizeof(T) == 4) {
-    const float4 q = *reinterpret_cast<const float4*>(p);
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    const uint4 q = load_u4<4>(p);
+    v[0] = __uint_as_float(q.x); v[1] = __uint_as_float(q.y); v[2] = __uint_as_float(q.z); v[3] = __uint_as_float(q.w);
   } else {
-    const uint2 q = *reinterpret_cast<const uint2*>(p);
+    const uint2 q = load_u2<2>(p);
     unpack2<T>(q.x, v[0], v[1]);
     unpack2<T>(q.y, v[2], v[3]);
   }
 }
 
-// Fused plane load + first analysis level for planes whose width is a multiple of 4:
-// a work item owns 2 input rows x 4 input columns (2 level-1 positions); it copies them
+// A row of W >= 4 elements in pieces of four.  The last piece of a row whose width is no multiple of four is read from
+// the row's last four elements (nothing beyond the row is touched) and moved into place afterwards, zeros behind it.
+// Rows of other widths, or at other addresses, than four elements' were once moved one element at a time and without the
+// fetch ahead: [16,64,70,77] bf16 forward 65.8 -> 42.2 us, [16,64,63,50] fp32 41.3 -> 33.9, [64,256,7,7] fp32 18.3 -> 13.9.
+// piece_start gives where the piece at column c0 is read from, piece_shift (when the values have arrived) moves them.
+__device__ __forceinline__ int piece_start(int c0, int W) { return c0 + 4 <= W ? c0 : W - 4; }
+__device__ __forceinline__ void piece_shift(float (&v)[4], int c0, int W) {
+  if ((W & 3) == 0) return;
+  const int sh = c0 + 4 - W;
+  const bool s1 = sh > 0 && (sh & 1) != 0, s2 = sh > 0 && (sh & 2) != 0;
+  v[0] = s1 ? v[1] : v[0]; v[1] = s1 ? v[2] : v[1]; v[2] = s1 ? v[3] : v[2]; v[3] = s1 ? 0.f : v[3];
+  v[0] = s2 ? v[2] : v[0]; v[1] = s2 ? v[3] : v[1]; v[2] = s2 ? 0.f : v[2]; v[3] = s2 ? 0.f : v[3];
+}
+
+// Fused plane load + first analysis level for planes at least 4 wide: a work item owns 2 input rows x 4 input columns (2 level-1 positions); it copies them
 // into the level-0 buffer and writes the four level-1 sub-bands, so the plane is read from
-// HBM with 16-byte (fp32) / 8-byte (bf16) loads and never re-read from LDS for level 1.
+// HBM with 16-byte (fp32) / 8-byte (bf16) loads and never re-read from LDS for level 1.  What the last piece of a row
+// writes behind a width that is no multiple of 4 are zeros, on cells that hold zeros (halo, padding).
 // Odd H: the missing bottom row is the zero padding of wtconv2d.py:49-51.
 template <typename T>
 __device__ __forceinline__ void load_analysis1(const T* __restrict__ src, int H, int W,
@@ -148,7 +161,7 @@ __device__ __forceinline__ void load_analysis1(const T* __restrict__ src, int H,
                                                float* __restrict__ d1, int str1, int pl1, int P1,
                                                int tid, int nthreads, bool valid = true) {
   const int h1 = (H + 1) >> 1;
-  const int nitem = W >> 2;                     // 4-column pieces per row
+  const int nitem = (W + 3) >> 2;               // 4-column pieces per row
   const int gsh = group_shift(nitem);
   const int s = tid & ((1 << gsh) - 1);
   if (s >= nitem) return;
@@ -157,8 +170,10 @@ __device__ __forceinline__ void load_analysis1(const T* __restrict__ src, int H,
     float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
     const bool has_b = 2 * i + 1 < H;
     if (valid) {
-      load4<T>(src + imul(2 * i, W) + c0, a);
-      if (has_b) load4<T>(src + imul(2 * i + 1, W) + c0, b);
+      load4_any<T>(src + imul(2 * i, W) + piece_start(c0, W), a);
+      if (has_b) load4_any<T>(src + imul(2 * i + 1, W) + piece_start(c0, W), b);
+      piece_shift(a, c0, W);
+      piece_shift(b, c0, W);
     }
     float* x0 = d0 + imul(2 * i + P0, str0) + c0 + P0;
 #pragma unroll
@@ -186,7 +201,7 @@ template <typename T, int NP>
 __device__ __forceinline__ void plane_fetch(const T* __restrict__ src, int H, int W, int tid, int nthreads,
                                             float (&a)[NP][4], float (&b)[NP][4]) {
   const int h1 = (H + 1) >> 1;
-  const int nitem = W >> 2;
+  const int nitem = (W + 3) >> 2;
   const int gsh = group_shift(nitem);
   const int s = tid & ((1 << gsh) - 1);
   if (s >= nitem) return;
@@ -198,8 +213,8 @@ __device__ __forceinline__ void plane_fetch(const T* __restrict__ src, int H, in
       // both loads unconditional (no merge with constants, hence no wait right behind the
       // load); a missing bottom row re-reads the top one and is zeroed in plane_commit
       const int rb = 2 * i + 1 < H ? 2 * i + 1 : 2 * i;
-      load4<T>(src + imul(2 * i, W) + c0, a[p]);
-      load4<T>(src + imul(rb, W) + c0, b[p]);
+      load4_any<T>(src + imul(2 * i, W) + piece_start(c0, W), a[p]);
+      load4_any<T>(src + imul(rb, W) + piece_start(c0, W), b[p]);
     }
   }
 }
@@ -210,7 +225,7 @@ __device__ __forceinline__ void plane_commit(const float (&a)[NP][4], const floa
                                              float* __restrict__ d1, int str1, int pl1, int P1,
                                              int tid, int nthreads, bool valid = true) {
   const int h1 = (H + 1) >> 1;
-  const int nitem = W >> 2;
+  const int nitem = (W + 3) >> 2;
   const int gsh = group_shift(nitem);
   const int s = tid & ((1 << gsh) - 1);
   if (s >= nitem) return;
@@ -226,6 +241,8 @@ __device__ __forceinline__ void plane_commit(const float (&a)[NP][4], const floa
         aa[k] = valid ? a[p][k] : 0.f;
         bb[k] = (valid && has_b) ? b[p][k] : 0.f;
       }
+      piece_shift(aa, c0, W);
+      piece_shift(bb, c0, W);
       float* x0 = d0 + imul(2 * i + P0, str0) + c0 + P0;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -262,7 +279,7 @@ __device__ __forceinline__ void plane_commit_fused(const float (&a)[NP][4], cons
                                                    float* __restrict__ d3, int str3, int pl3, int P1,
                                                    int fuse, int tid, int nthreads) {
   const int h1 = (H + 1) >> 1;
-  const int nitem = W >> 2;
+  const int nitem = (W + 3) >> 2;
   const int gsh = group_shift(nitem);
   const int s = tid & ((1 << gsh) - 1);
   const int c0 = 4 * s;
@@ -278,6 +295,8 @@ __device__ __forceinline__ void plane_commit_fused(const float (&a)[NP][4], cons
       aa[k] = valid ? a[p][k] : 0.f;
       bb[k] = (valid && has_b) ? b[p][k] : 0.f;
     }
+    piece_shift(aa, c0, W);
+    piece_shift(bb, c0, W);
     if (valid) {
       float* x0 = d0 + imul(2 * i + P0, str0) + c0 + P0;
 #pragma unroll
@@ -518,23 +537,23 @@ __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2
   }
 }
 
-// Store up to N consecutive outputs (`nvalid` of them lie inside the row): 4-element vectors
-// when the whole strip is inside, the destination is aligned to 4 elements and vec4 is set.
+// Store up to N consecutive outputs (`nvalid` of them lie inside the row): 4-element vectors when the whole strip is.
 template <typename T, int N>
-__device__ __forceinline__ void store_row(T* __restrict__ dst, const float (&v)[N], int nvalid, bool vec4) {
+__device__ __forceinline__ void store_row(T* __restrict__ dst, const float (&v)[N], int nvalid) {
   if constexpr (N % 4 == 0) {
-    if (vec4 && nvalid == N) {           // the common case: whole strip inside the row, 16-byte stores
+    if (nvalid == N) {           // the common case: whole strip inside the row, 16-byte stores
 #pragma unroll
       for (int k = 0; k < N / 4; ++k) {
         if constexpr (sizeof(T) == 4) {
-          float4 q;
-          q.x = v[4 * k]; q.y = v[4 * k + 1]; q.z = v[4 * k + 2]; q.w = v[4 * k + 3];
-          *reinterpret_cast<float4*>(dst + 4 * k) = q;
+          uint4 q;
+          q.x = __float_as_uint(v[4 * k]); q.y = __float_as_uint(v[4 * k + 1]);
+          q.z = __float_as_uint(v[4 * k + 2]); q.w = __float_as_uint(v[4 * k + 3]);
+          store_u4<4>(dst + 4 * k, q);
         } else {
           uint2 q;
           q.x = pack2<T>(v[4 * k], v[4 * k + 1]);
           q.y = pack2<T>(v[4 * k + 2], v[4 * k + 3]);
-          *reinterpret_cast<uint2*>(dst + 4 * k) = q;
+          store_u2<2>(dst + 4 * k, q);
         }
       }
       return;
@@ -615,8 +634,8 @@ __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2
     pin_values(o0);      // all outputs computed before the stores: keeps the compiler from sinking
     pin_values(o1);      // the last FMAs behind the store branches and splitting the 16-byte stores
     if (nvalid > 0) {
-      store_row<T, NO>(out_plane + imul(r0, W) + c0, o0, nvalid, pl.vec_ok != 0);
-      if (r0 + 1 < H) store_row<T, NO>(out_plane + imul(r0 + 1, W) + c0, o1, nvalid, pl.vec_ok != 0);
+      store_row<T, NO>(out_plane + imul(r0, W) + c0, o0, nvalid);
+      if (r0 + 1 < H) store_row<T, NO>(out_plane + imul(r0 + 1, W) + c0, o1, nvalid);
     }
   }
 }
@@ -638,8 +657,8 @@ __device__ __forceinline__ void zero_lds(float* lds, int nfloats) {
 // weights stay wave-uniform (SGPRs).  The zero halos written once stay valid for every plane
 // (only interiors are rewritten).
 // MODE selects the loader at compile time (0: register prefetch of the next plane, 3: the same
-// with levels 2-3 produced at the commit, 1: fused vector load without prefetch, 2: element-wise
-// load), so that the hot variant does not carry
+// with levels 2-3 produced at the commit, 1: fused vector load without prefetch, 2: element-wise, planes less than 4 wide),
+// so that the hot variant does not carry
 // the registers of the others.
 // Geo: the plan's geometry as a compile-time constant for the common shapes (LDS offsets and strides fold into
 // instruction immediates, loops over levels unroll), or the run-time plan of the argument for any other shape;

@@ -29,19 +29,7 @@ namespace wt {
 constexpr int kStreamPad = 4;       // column halo of the LDS tiles in coefficients (>= K/2, keeps rows 16-byte aligned)
 constexpr int kStreamThreads = 256;
 
-// Four consecutive elements from / eight to any element address.
-template <typename T>
-__device__ __forceinline__ void load4_any(const T* __restrict__ p, float (&v)[4]) {
-  if constexpr (sizeof(T) == 4) {
-    const uint4 q = load_u4<4>(p);
-    v[0] = __uint_as_float(q.x); v[1] = __uint_as_float(q.y); v[2] = __uint_as_float(q.z); v[3] = __uint_as_float(q.w);
-  } else {
-    const uint2 q = load_u2<2>(p);
-    unpack2<T>(q.x, v[0], v[1]);
-    unpack2<T>(q.y, v[2], v[3]);
-  }
-}
-
+// Eight elements to any element address.
 template <typename T>
 __device__ __forceinline__ void store8_any(T* __restrict__ p, const float (&v)[8]) {
   uint4 q;

@@ -88,17 +88,12 @@ constexpr Plan2D make_plan2d_geometry(int B, int C, int H, int W, int K, int L, 
   pl.lds_floats = pl.plane_lds_floats;
   pl.groups_per_channel = 1;
   pl.fw_stride = (1 + 4 * L) * K * K;
-  pl.vec_ok = W % 4 == 0;                         // (and aligned pointers: make_plan2d)
+  pl.vec_ok = W >= 4;
   return pl;
 }
 
-inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_grad_pyramid, int nthreads,
-                          size_t elem_size, const void* p0, const void* p1, const void* p2, int pb = 1) {
-  Plan2D pl = make_plan2d_geometry(B, C, H, W, K, L, with_grad_pyramid, nthreads, pb);
-  const uintptr_t mask = 4 * elem_size - 1;       // 4-element vectors: 16 B (fp32) / 8 B (bf16)
-  auto aligned = [mask](const void* p) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) & mask) == 0; };
-  pl.vec_ok = (W % 4 == 0) && aligned(p0) && aligned(p1) && aligned(p2);
-  return pl;
+inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_grad_pyramid, int nthreads, int pb = 1) {
+  return make_plan2d_geometry(B, C, H, W, K, L, with_grad_pyramid, nthreads, pb);
 }
 
 // Completes a plan for the plane kernel: threads per plane, slots per workgroup, prefetch.
@@ -113,7 +108,7 @@ constexpr void finish_plane_plan(Plan2D* pl, int tj1_sg_shift) {
   pl->prefetch = 0;
   pl->fuse = 1;
   if (pl->vec_ok) {
-    const int gs = pow2_ceil(pl->W / 4);       // 2x4 pieces per row pair, one lane each
+    const int gs = pow2_ceil((pl->W + 3) / 4);       // 2x4 pieces per row pair, one lane each
     const int rows_per_pass = sg / gs;
     pl->prefetch = rows_per_pass >= 1 && (pl->h[1] + rows_per_pass - 1) / rows_per_pass <= kFetchPasses;
     if (pl->prefetch && sg == pl->block && gs <= 16 && pl->L >= 2) pl->fuse = pl->L >= 3 ? 3 : 2;
@@ -215,7 +210,7 @@ constexpr void finish_wgrad_plan(Plan2D* pl, int K) {
   pl->prefetch = 0;
   pl->fuse = 1;
   if (pl->vec_ok) {
-    const int gs = pow2_ceil(pl->W / 4);
+    const int gs = pow2_ceil((pl->W + 3) / 4);
     pl->prefetch = nps / gs >= pl->h[1];       // one 2x4 piece per thread covers the plane
     if (pl->prefetch && pl->pb == 1 && gs <= 16 && pl->L >= 2) pl->fuse = pl->L >= 3 ? 3 : 2;
   }
