@@ -109,6 +109,9 @@ template <> struct Quad<bf16_t> {
 };
 
 constexpr int kQuadBatch = 6;      // vector loads a thread keeps in flight before it writes them to LDS
+// Rows that move element by element: loads in flight.  One at a time, a tile's channels were a chain of memory latencies,
+// us a launch at 768 channels of 7 x 7, bf16: residual 28.4 -> 10.4 for one image and 37.1 -> 16.6 for 256, norm 16.1 -> 15.2.
+constexpr int kElemBatch = 12;
 
 // tile element from / to fp32 (LT = float or the tensor's type)
 template <typename LT> __device__ __forceinline__ float tile_get(LT v) { return to_f32<LT>(v); }
@@ -147,10 +150,21 @@ __device__ __forceinline__ void tile_from_nchw(const T* __restrict__ img, LT* ld
   } else {
     const int p = tid & (t.tp - 1), c0 = tid >> t.tp_shift, cstep = kBlockThreads >> t.tp_shift;
     if (p0 + p < t.HW)
-      for (int c = c0; c < t.C; c += cstep) {
-        const T v = img[static_cast<size_t>(c) * t.HW + p0 + p];
-        if constexpr (std::is_same<LT, T>::value) lds[c * pitch + p] = v;
-        else lds[c * pitch + p] = to_f32<T>(v);
+      for (int cb = c0; cb < t.C; cb += kElemBatch * cstep) {
+        T v[kElemBatch];
+#pragma unroll
+        for (int k = 0; k < kElemBatch; ++k) {
+          const int c = cb + k * cstep < t.C ? cb + k * cstep : t.C - 1;      // (a channel past the end: read, not used)
+          v[k] = img[static_cast<size_t>(c) * t.HW + p0 + p];
+        }
+#pragma unroll
+        for (int k = 0; k < kElemBatch; ++k) {
+          const int c = cb + k * cstep;
+          if (c < t.C) {
+            if constexpr (std::is_same<LT, T>::value) lds[c * pitch + p] = v[k];
+            else lds[c * pitch + p] = to_f32<T>(v[k]);
+          }
+        }
       }
   }
 }
@@ -433,13 +447,22 @@ block_residual_kernel(const T* __restrict__ y, const T* __restrict__ shortcut, c
   const int np = t.HW - p0 < t.tp ? t.HW - p0 : t.tp;
   const T* src = y + (static_cast<size_t>(b) * t.HW + p0) * C;
   const int npair = (np * C) >> 1;
-  for (int i = tid; i < npair; i += kBlockThreads) {
-    const int e = 2 * i;
-    const int pp = div_c(e, t.mg_c), c = e - pp * C;
-    T a, bb;
-    load_pair_raw<T>(src + e, a, bb);
-    lds[c * pitch + pp] = a;
-    lds[(c + 1) * pitch + pp] = bb;
+  for (int i0 = tid; i0 < npair; i0 += kElemBatch * kBlockThreads) {
+    T a[kElemBatch], bb[kElemBatch];
+#pragma unroll
+    for (int k = 0; k < kElemBatch; ++k) {
+      const int i = i0 + k * kBlockThreads < npair ? i0 + k * kBlockThreads : npair - 1;
+      load_pair_raw<T>(src + 2 * i, a[k], bb[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < kElemBatch; ++k) {
+      const int e = 2 * (i0 + k * kBlockThreads);
+      if (e < 2 * npair) {
+        const int pp = div_c(e, t.mg_c), c = e - pp * C;
+        lds[c * pitch + pp] = a[k];
+        lds[(c + 1) * pitch + pp] = bb[k];
+      }
+    }
   }
   __syncthreads();
   if constexpr (VEC) {
@@ -474,10 +497,30 @@ block_residual_kernel(const T* __restrict__ y, const T* __restrict__ shortcut, c
     const int p = tid & (t.tp - 1), c0 = tid >> t.tp_shift, cstep = kBlockThreads >> t.tp_shift;
     if (p < np) {
       const size_t base = static_cast<size_t>(b) * C * t.HW + p0 + p;
-      for (int c = c0; c < C; c += cstep) {
-        const float g = gamma != nullptr ? load_param(gamma, pdtype, c) : 1.f;
-        const size_t o = base + static_cast<size_t>(c) * t.HW;
-        out[o] = from_f32<T>(to_f32<T>(shortcut[o]) + g * to_f32<T>(lds[c * pitch + p]));
+      for (int cb = c0; cb < C; cb += kElemBatch * cstep) {
+        T s[kElemBatch];
+        float g[kElemBatch];
+#pragma unroll
+        for (int k = 0; k < kElemBatch; ++k) {
+          const int c = cb + k * cstep < C ? cb + k * cstep : C - 1;
+          s[k] = shortcut[base + static_cast<size_t>(c) * t.HW];
+          g[k] = 1.f;
+        }
+        auto scales = [&](auto* tag) {      // (one branch on the type for all: a branch for each would wait for each)
+          using P = std::remove_pointer_t<decltype(tag)>;
+#pragma unroll
+          for (int k = 0; k < kElemBatch; ++k)
+            g[k] = to_f32<P>(static_cast<const P*>(gamma)[cb + k * cstep < C ? cb + k * cstep : C - 1]);
+        };
+        if (gamma != nullptr) {
+          if (pdtype == WTCONV_F32) scales(static_cast<float*>(nullptr));
+          else scales(static_cast<bf16_t*>(nullptr));
+        }
+#pragma unroll
+        for (int k = 0; k < kElemBatch; ++k) {
+          const int c = cb + k * cstep;
+          if (c < C) out[base + static_cast<size_t>(c) * t.HW] = from_f32<T>(to_f32<T>(s[k]) + g[k] * to_f32<T>(lds[c * pitch + p]));
+        }
       }
     }
   }
