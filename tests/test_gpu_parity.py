@@ -71,6 +71,10 @@ def test_stage_shapes_fp32_small_batch(hip_device, C, H, L):
     ((1, 2, 144, 136), 1, 2, False),   # K = 1 on a large plane
     ((1, 1, 3, 3), 7, 4, True),        # one tiny plane, K = 7: the final weight-gradient reduction needs more LDS than the pyramids
     ((1, 1, 1, 1), 7, 1, True),
+    ((8, 64, 9, 10), 5, 2, True),      # 512 planes: the forward launch folds the parameters itself, several channels a workgroup
+    ((9, 57, 9, 10), 5, 2, True),      # one more: a fold launch
+    ((1, 3, 72, 70), 5, 3, False),     # 1024 threads a plane, no bias
+    ((1, 2, 112, 96), 5, 3, True),     # one level as a step, then plane-resident
 ])
 def test_edge_shapes_fp32(hip_device, shape, K, L, bias):
     _run_fp32("2d", shape[1], K, L, shape, hip_device, bias=bias, seed=3)

@@ -52,6 +52,10 @@ constexpr int kWgradResident = 512;
 
 static size_t fold_floats(int C, int S, int L, int KK) { return static_cast<size_t>(C) * (1 + S * L) * KK + C; }
 
+// Folded filters as the plane kernel writes them itself (PlaneFold): each channel's table on cache lines of its own.
+constexpr int kFoldInsidePlanes = 512;
+static size_t folded_tables(int C, int L, int KK) { return static_cast<size_t>(C) * (((1 + 4 * L) * KK + 31) / 32 * 32); }
+
 static int launch_fold(const wtconv_params* params, int pdtype, float* fw, float* fb, int C, int S, int L,
                        int KK, int flip, int use_bias, hipStream_t stream, unsigned* zero_words = nullptr,
                        int nzero = 0) {
@@ -143,7 +147,8 @@ static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) 
 // One launch of the plane-resident kernels on planes that fit LDS; `fw` / `fb` folded parameters, those of a channel
 // `fw_stride` floats from the next one's, the level filters `fw_skip` floats behind their usual place.
 static int resident2d(const char* fn, const void* x, void* out, const float* fw, const float* fb, int B, int C, int H,
-                      int W, int K, int L, int dtype, int fw_stride, int fw_skip, hipStream_t stream) {
+                      int W, int K, int L, int dtype, int fw_stride, int fw_skip, hipStream_t stream,
+                      const PlaneFold& fold = PlaneFold{}) {
   Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256);
   int tj1 = 4, sg_shift = 8;
   choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
@@ -158,7 +163,7 @@ static int resident2d(const char* fn, const void* x, void* out, const float* fw,
     return fail(WTCONV_E_UNSUPPORTED,
                 "%s: a %dx%d plane with %d levels needs %zu B of LDS (limit %d); plane too large for the "
                 "plane-resident kernels", fn, H, W, L, static_cast<size_t>(pl.lds_floats) * 4, kLdsLimitBytes);
-  return launch_plane2d(dtype, K, tj1, x, out, fw, fb, pl, stream);
+  return launch_plane2d(dtype, K, tj1, x, out, fw, fb, pl, fold, stream);
 }
 
 // The layer on planes beyond LDS.  `ll` and `res`: areas of make_stream2d (LL bands, results of the sub-layers).
@@ -219,6 +224,14 @@ static int plane2d_pass(const char* fn, const void* x, void* out, const wtconv_p
   }
   float* fw = static_cast<float*>(ws);
   float* fb = fw + static_cast<size_t>(C) * (1 + 4 * L) * K * K;
+  // A small forward launch folds its parameters itself: the fold kernel and the gap behind it are a quarter of it, us
+  // [8,32,64,64] fp32, K = 5, three levels 18.1 -> 13.9.  With more planes than one for a CU the launch is the cheaper way.
+  if (!flip && tickets == nullptr && static_cast<long long>(B) * C <= kFoldInsidePlanes && !plane_shape_is_static(K, H, W, L) &&
+      reinterpret_cast<uintptr_t>(ws) % 128 == 0 && ws_bytes >= folded_tables(C, L, K * K) * sizeof(float)) {
+    const PlaneFold fold = {static_cast<float*>(ws), to_table(params, L), pdtype};
+    return resident2d(fn, x, out, fw, nullptr, B, C, H, W, K, L, dtype, static_cast<int>(folded_tables(1, L, K * K)), 0,
+                      stream, fold);
+  }
   if (int e = launch_fold(params, pdtype, fw, fb, C, 4, L, K * K, flip, flip ? 0 : 1, stream, tickets, C)) return e;
   return resident2d(fn, x, out, fw, fb, B, C, H, W, K, L, dtype, (1 + 4 * L) * K * K, 0, stream);
 }
@@ -389,6 +402,9 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
       if (q.ok && q.ws_bytes > mf) mf = q.ws_bytes;
     }
     floats = fold_floats(C, 4, levels, K * K);
+    if (pass == WTCONV_PASS_FORWARD && static_cast<long long>(B) * C <= kFoldInsidePlanes &&
+        folded_tables(C, levels, K * K) > floats)
+      floats = folded_tables(C, levels, K * K);
     if (!plane_fits_lds(B, C, H, W, K, levels)) {
       // (planes beyond LDS: never less than the four bands of every level, which these calls once kept here, so that the
       // shapes refused for want of static scratch are the same)

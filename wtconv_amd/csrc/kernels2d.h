@@ -86,6 +86,35 @@ static __global__ void fold_params_kernel(ParamTable p, int pdtype, float* __res
   }
 }
 
+// The same for one channel, by `nth` lanes of the plane kernel that is about to use it, into dst[0 .. NF * KK): vector
+// stores, read back through the scalar cache.  That is sound because the stores have reached the L2 that both share when
+// the lanes have waited for them (the caller does), because the table starts a cache line of its own (nothing else
+// brings one of its lines into the scalar cache before), and because every workgroup writes the table before it reads it
+// -- workgroups with the same channel write the same values.
+struct PlaneFold {
+  float* dst;        // tables of plarg.fw_stride floats, a multiple of 32, 128-byte aligned; nullptr: `fw` is folded already
+  ParamTable prm;
+  int pdtype;
+};
+struct NoFold {};
+__device__ __forceinline__ void fold_channel(const PlaneFold& p, float* __restrict__ dst, int c, int NF, int KK, int tid,
+                                             int nth) {
+  for (int i = tid; i < NF * KK; i += nth) {
+    const int f = i / KK, t = i - f * KK;
+    const void* w = p.prm.base_weight;
+    const void* g = p.prm.base_scale;
+    int ch = c;
+    if (f > 0) {
+      const int l = (f - 1) >> 2;
+      ch = 4 * c + ((f - 1) & 3);
+#pragma unroll
+      for (int k = 0; k < kMaxLevels; ++k)      // (constant indices: the table stays in scalar registers)
+        if (l == k) { w = p.prm.wt_weight[k]; g = p.prm.wt_scale[k]; }
+    }
+    dst[i] = load_param(w, p.pdtype, ch * KK + t) * load_param(g, p.pdtype, ch);
+  }
+}
+
 // Synchronisation between the phases of a plane: workgroup barrier, or only the ordering of
 // one wave's LDS traffic when every plane belongs to the lanes of a single wave.
 __device__ __forceinline__ void plane_sync(bool wave_local) {
@@ -662,11 +691,14 @@ __device__ __forceinline__ void zero_lds(float* lds, int nfloats) {
 // the registers of the others.
 // Geo: the plan's geometry as a compile-time constant for the common shapes (LDS offsets and strides fold into
 // instruction immediates, loops over levels unroll), or the run-time plan of the argument for any other shape;
-// batch, channels and what follows from them always come from the argument.
+// batch, channels and what follows from them always come from the argument.  Geo::kFold: the run-time plan, and the kernel
+// folds the parameters itself (a variant of its own: the code in the others cost them up to a fifth, 33 -> 40 us on
+// [16,72,45,37] fp16, K = 7).
 template <typename T, int K, int TJ1, int TJC, int MODE, typename Geo>
 __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict__ x, T* __restrict__ out,
                                                          const float* __restrict__ fw,
-                                                         const float* __restrict__ fb, const Plan2D plarg) {
+                                                         const float* __restrict__ fb, const Plan2D plarg,
+                                                         const typename Geo::Fold fold) {
   WT_SHARED_FLOATS(lds_all);
   static constexpr Plan2D kGeo = Geo::plan();
   const Plan2D& pl = Geo::kStatic ? kGeo : plarg;
@@ -734,6 +766,14 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
   // the channel used for the weights (clamped: a thread without a plane still runs uniform code)
   auto channel_of = [&](const Loc& s) { return s.c < nC ? s.c : nC - 1; };
 
+  auto bias_of = [&](int c) {
+    if constexpr (Geo::kFold) {
+      return fold.prm.base_bias == nullptr ? 0.f : load_param(fold.prm.base_bias, fold.pdtype, c) *
+                                                         load_param(fold.prm.base_scale, fold.pdtype, c);
+    } else {
+      return fb != nullptr ? fb[c] : 0.f;
+    }
+  };
   constexpr bool kPrefetch = MODE == 0 || MODE == 3;
   float fa[kFetchPasses][4], fbuf[kFetchPasses][4];
   Loc nxt;
@@ -759,6 +799,12 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
     const size_t plane_off = static_cast<size_t>(live ? plane : 0) * plane_elems;
     int l0 = 2;
     WT_WAVE_PRIORITY(3);
+    if constexpr (Geo::kFold) {      // (by the lanes that share a table: those of the plane, or of the wave)
+      float* to = fold.dst + static_cast<size_t>(c) * fw_stride;
+      if (sg > kWave) fold_channel(fold, to, c, 1 + 4 * pl.L, KK, ltid, sg);
+      else fold_channel(fold, to, c, 1 + 4 * pl.L, KK, tid & (kWave - 1), kWave);
+      WT_WAIT_VMEM();
+    }
     if constexpr (MODE == 0) {
       if (live)
         plane_commit<kFetchPasses>(fa, fbuf, pl.H, pl.W, lds + pl.aoff[0], pl.astr[0], pl.P,
@@ -780,6 +826,7 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
       l0 = 1;
     }
     plane_sync(wave_local);
+    if constexpr (Geo::kFold) WT_LAUNDER_UNIFORM_PTR(fwc);      // (no weight is read before the table is there)
     if (kPrefetch && u + static_cast<int>(gridDim.x) < nunits && nxt.plane >= 0)
       plane_fetch<T, kFetchPasses>(x + nxt.plane * plane_elems, pl.H, pl.W, ltid, sg, fa, fbuf);
     for (int lv = l0; lv <= pl.L; ++lv) {
@@ -796,8 +843,7 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
     }
     WT_WAIT_VMEM();     // next plane's loads have landed; the stores below are not waited for
     WT_WAVE_PRIORITY(0);
-    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, fb != nullptr ? fb[c] : 0.f, out + plane_off,
-                                        ltid, sg);
+    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, bias_of(c), out + plane_off, ltid, sg);
     plane_sync(wave_local);   // the next plane overwrites the buffers read above
   }
 }

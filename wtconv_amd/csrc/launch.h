@@ -21,7 +21,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // plane2d.hip: the layer on planes that fit LDS.
 int launch_plane2d(int dtype, int K, int tj1, const void* x, void* out, const float* fw, const float* fb, const Plan2D& pl,
-                   hipStream_t stream);
+                   const PlaneFold& fold, hipStream_t stream);
 
 // wgrad2d.hip: its parameter gradients.
 int launch_wgrad2d(int dtype, int K, int L, const void* x, const void* g, float* partial, const Plan2D& pl, int B, int bchunk,

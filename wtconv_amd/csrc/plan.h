@@ -118,8 +118,13 @@ constexpr void finish_plane_plan(Plan2D* pl, int tj1_sg_shift) {
 // Geometry of the plane kernel's plan: the run-time plan of the launch, or a compile-time constant for a shape
 // whose rows are whole aligned vectors (the launcher checks that the two agree before it picks the constant).
 struct PlaneGeoRuntime {
-  static constexpr bool kStatic = false;
+  static constexpr bool kStatic = false, kFold = false;
+  using Fold = NoFold;
   static constexpr Plan2D plan() { return Plan2D{}; }
+};
+struct PlaneGeoFold : PlaneGeoRuntime {
+  static constexpr bool kFold = true;
+  using Fold = PlaneFold;
 };
 constexpr Plan2D static_plane_plan(int H, int W, int K, int L, int* tj1_out) {
   Plan2D pl = make_plan2d_geometry(1, 1, H, W, K, L, false, 256, 1);
@@ -161,7 +166,8 @@ inline void widen_plane_shape(int h1, int w1, size_t plane_lds_bytes, int nplane
 
 template <int H, int W, int K, int L>
 struct PlaneGeoStatic {
-  static constexpr bool kStatic = true;
+  static constexpr bool kStatic = true, kFold = false;
+  using Fold = NoFold;
   static constexpr Plan2D plan() { return static_plane_plan(H, W, K, L, nullptr); }
   static constexpr int tj1() { int t = 4; static_plane_plan(H, W, K, L, &t); return t; }
   static constexpr int mode() {
