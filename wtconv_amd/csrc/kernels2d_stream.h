@@ -14,7 +14,7 @@
 // from the pixels of x and grad_out, and the sub-layer's filters are its parameter gradients on X_1 and G_1.
 // Nothing of a level but its LL band goes through memory.
 //
-// Measured, us a training step (forward): [8,96,160,160] fp32 523 -> 391 (167 -> 126) against one launch per level and
+// Measured, us a training step (forward): [8,96,160,160] fp32 523 -> 380 (167 -> 118) against one launch per level and
 // pass with every band in memory; [8,64,141,155] fp16, K = 7 1018 -> 556 (350 -> 156); [4,64,199,230] fp32, five levels
 // 443 -> 325 (138 -> 109).
 //
