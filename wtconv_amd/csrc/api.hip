@@ -132,6 +132,16 @@ static Stream2D make_stream2d(int B, int C, int H, int W, int K, int L) {
   return s;
 }
 
+// Planes beyond LDS: the four bands of every level, which calls once kept in their workspace.  The sizes they ask for are
+// never less, so that the shapes refused for want of static scratch are the same.
+static size_t four_band_floats(int B, int C, int H, int W, int K, int L) {
+  if (plane_lds_bytes(B, C, H, W, K, L) <= static_cast<size_t>(kLdsLimitBytes)) return 0;
+  const Stream2D s = make_stream2d(B, C, H, W, K, L);
+  size_t area = 0;
+  for (int l = 1; l <= L; ++l) area += round_up64(static_cast<size_t>(B) * C * s.h[l] * s.w[l] * (l < L ? 5 : 4));
+  return area;
+}
+
 // Partial sums of the steps, then those of the plane-resident sub-layer.
 static size_t stream_records(int B, int C, int H, int W, int K, int L) {
   return round_up64(static_cast<size_t>(stream_chunks(B, C, H, W)) * C * ((1 + 4 * L) * K * K + 1));
@@ -389,7 +399,9 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
       floats = static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1);
     } else {      // partial sums, then the LL bands of x and of grad_out
       const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
-      floats = stream_records(B, C, H, W, K, levels) + stream_sub_records(sp, B, C, K, levels) + 2 * sp.floats;
+      floats = stream_records(B, C, H, W, K, levels) + stream_sub_records(sp, B, C, K, levels);
+      const size_t area = four_band_floats(B, C, H, W, K, levels);
+      floats += 2 * (area > sp.floats ? area : sp.floats);
     }
     if (mfloats > floats) floats = mfloats;
     floats = round_up64(floats) + static_cast<size_t>(C);      // one ticket word per channel behind the records
@@ -406,13 +418,8 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
         folded_tables(C, levels, K * K) > floats)
       floats = folded_tables(C, levels, K * K);
     if (!plane_fits_lds(B, C, H, W, K, levels)) {
-      // (planes beyond LDS: never less than the four bands of every level, which these calls once kept here, so that the
-      // shapes refused for want of static scratch are the same)
-      size_t area = 0;
+      size_t area = four_band_floats(B, C, H, W, K, levels);
       const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
-      if (plane_lds_bytes(B, C, H, W, K, levels) > static_cast<size_t>(kLdsLimitBytes))
-        for (int l = 1; l <= levels; ++l)
-          area += round_up64(static_cast<size_t>(B) * C * sp.h[l] * sp.w[l] * (l < levels ? 5 : 4));
       if (area < 2 * sp.floats) area = 2 * sp.floats;
       floats = round_up64(floats) + area;
     }
