@@ -1,0 +1,41 @@
+/*
+ * wtconv_ops.h -- C ABI of libwtconv_hip.so, second part: what a WTConvNeXt does around its WTConv layers beyond the two
+ * passes of wtconv_hip.h.  Conventions (error codes, dtypes, streams, caller-owned memory) are those of wtconv_hip.h;
+ * this part is versioned by itself, so that programs of the layer alone keep theirs.
+ */
+#ifndef WTCONV_OPS_H
+#define WTCONV_OPS_H
+
+#include "wtconv_hip.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+#define WTCONV_OPS_VERSION 1
+
+/* Version of this part in the loaded library (== WTCONV_OPS_VERSION). */
+int wtconv_ops_version(void);
+
+/* ---- the convolutions that change resolution, with the LayerNorm beside them, for inference in bfloat16:
+ *   stem != 0:  out = LayerNorm_c(conv 4x4 stride 4 (x) + bias), norm parameters of `cout` values;
+ *   stem == 0:  out = conv 2x2 stride 2 (LayerNorm_c(x)) + bias, norm parameters of `C` values
+ * (wtconvnext/wtconvnext.py:170-181, :294-297 of the reference).  x (B, C, H, W), out (B, cout, H / P, W / P), conv_weight
+ * (cout, C, P, P); everything 16-byte aligned.  Sums and LayerNorm in float; normalised values are rounded to bfloat16
+ * once, as are the results.  wtconv_patch_conv_supported says whether a size has a kernel; the workspace (16-byte aligned)
+ * takes the weights in the order of the products. */
+typedef struct {
+  const void *conv_weight, *conv_bias;
+  const void *norm_weight, *norm_bias;
+} wtconv_patch_params;
+
+int wtconv_patch_conv_supported(int stem, int B, int C, int H, int W, int cout);
+size_t wtconv_patch_conv_workspace_bytes(int stem, int B, int C, int H, int W, int cout);
+int wtconv_patch_conv(int stem, const void* x, void* out, const wtconv_patch_params* params, int B, int C, int H, int W,
+                      int cout, float eps, int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
+                      void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* WTCONV_OPS_H */

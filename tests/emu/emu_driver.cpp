@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/wtconv_hip.h"
+#include "../../include/wtconv_ops.h"
 #include "../../wtconv_amd/csrc/common.h"      // only for the half conversions of the dims == 0 mode
 
 static uint16_t to_bf16(float f) {
@@ -135,6 +136,28 @@ int main(int argc, char** argv) {
     const wtconv_mlp_params prm = {nw.ptr(), nb.ptr(), w1.ptr(), b1.ptr(), w2.ptr(), b2.ptr(), L ? gm.ptr() : nullptr};
     const int rc = wtconv_block_mlp(bx.ptr(), sc.ptr(), o.ptr(), &prm, B, C, H * W, hidden, eps, 1, 1, ws.data(), ws.size(), nullptr);
     if (rc) { fprintf(stderr, "block_mlp: %s\n", wtconv_last_error()); return 3; }
+    o.unpack();
+    FILE* fo = fopen(argv[2], "wb");
+    if (!fo) { perror("open out"); return 2; }
+    fwrite(o.f.data(), 4, P, fo);
+    fclose(fo);
+    return 0;
+  }
+  if (dims == 6) {
+    // stem or downsample: header {6, B, C, H, W, cout (K slot), stem (L slot), 1, 1, unused}, eps;
+    //   in x, convolution weight and bias, norm weight and bias -> out
+    const int cout = K, stem = L, side = stem ? 4 : 2, normed = stem ? cout : C;
+    float eps;
+    if (fread(&eps, 4, 1, fp) != 1) return 2;
+    Buf bx = read_buf(fp, static_cast<size_t>(B) * C * H * W, 1), cw = read_buf(fp, static_cast<size_t>(cout) * C * side * side, 1);
+    Buf cb = read_buf(fp, cout, 1), nw = read_buf(fp, normed, 1), nb = read_buf(fp, normed, 1);
+    fclose(fp);
+    const size_t P = static_cast<size_t>(B) * cout * (H / side) * (W / side);
+    Buf o = out_buf(P, 1);
+    std::vector<char> ws(wtconv_patch_conv_workspace_bytes(stem, B, C, H, W, cout));
+    const wtconv_patch_params prm = {cw.ptr(), cb.ptr(), nw.ptr(), nb.ptr()};
+    const int rc = wtconv_patch_conv(stem, bx.ptr(), o.ptr(), &prm, B, C, H, W, cout, eps, 1, 1, ws.data(), ws.size(), nullptr);
+    if (rc) { fprintf(stderr, "patch_conv: %s\n", wtconv_last_error()); return 3; }
     o.unpack();
     FILE* fo = fopen(argv[2], "wb");
     if (!fo) { perror("open out"); return 2; }

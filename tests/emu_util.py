@@ -14,11 +14,12 @@ BUILD_DIR = os.path.join(EMU_DIR, "_build")
 EXE = os.path.join(BUILD_DIR, "emu_driver")
 SOURCES = [os.path.join(ROOT, "wtconv_amd", "csrc", "api.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "mfma2d.hip"),
            os.path.join(ROOT, "wtconv_amd", "csrc", "block.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "haar.hip"),
-           os.path.join(ROOT, "wtconv_amd", "csrc", "mlp.hip"),
+           os.path.join(ROOT, "wtconv_amd", "csrc", "mlp.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "patch.hip"),
            os.path.join(EMU_DIR, "emu_driver.cpp")]
 # api.hip includes the other translation units here, and every one of them its headers: all of csrc
 DEPS = sorted(set(SOURCES + [f for ext in ("h", "hip") for f in glob.glob(os.path.join(ROOT, "wtconv_amd", "csrc", "*." + ext))] + [
-    os.path.join(EMU_DIR, "emu_runtime.h"), os.path.join(ROOT, "include", "wtconv_hip.h")]))
+    os.path.join(EMU_DIR, "emu_runtime.h"), os.path.join(ROOT, "include", "wtconv_hip.h"),
+    os.path.join(ROOT, "include", "wtconv_ops.h")]))
 
 
 def build(force=False):
@@ -170,3 +171,22 @@ def run_block_mlp(x, shortcut, nw, nb, w1, b1, w2, b2, gamma, eps=1e-6, timeout=
         if r.returncode != 0:
             raise RuntimeError(f"emu_driver failed ({r.returncode}):\n{r.stderr[-4000:]}")
         return np.fromfile(fout, dtype=np.float32).reshape(x.shape)
+
+
+def run_patch_conv(stem, x, cw, cb, nw, nb, eps=1e-6, timeout=600):
+    """wtconv_patch_conv on the host; x (B,C,H,W), bf16 values in float32 arrays."""
+    exe = build()
+    B, C, H, W = x.shape
+    P = 4 if stem else 2
+    hdr = np.array([6, B, C, H, W, cw.shape[0], int(stem), 1, 1, 0], dtype=np.int32)
+    parts = [hdr.tobytes(), np.float32(eps).tobytes()] + [np.ascontiguousarray(a, dtype=np.float32).tobytes() for a in (x, cw, cb, nw, nb)]
+    with tempfile.TemporaryDirectory() as td:
+        fin, fout = os.path.join(td, "in.bin"), os.path.join(td, "out.bin")
+        with open(fin, "wb") as f:
+            f.write(b"".join(parts))
+        env = dict(os.environ)
+        env["ASAN_OPTIONS"] = "detect_leaks=0"
+        r = subprocess.run([exe, fin, fout], capture_output=True, text=True, timeout=timeout, env=env)
+        if r.returncode != 0:
+            raise RuntimeError(f"emu_driver failed ({r.returncode}):\n{r.stderr[-4000:]}")
+        return np.fromfile(fout, dtype=np.float32).reshape(B, cw.shape[0], H // P, W // P)

@@ -452,3 +452,30 @@ def test_emulated_block_mlp(B, C, H, W, hidden, layer_scale):
     # operands and result are rounded to bfloat16 (2^-9 relative each): the norm of the errors, and the largest
     assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
     assert np.abs(got - want).max() < 6e-2 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("stem,B,C,H,W,cout", [
+    (0, 1, 96, 6, 10, 32),      # 15 output pixels of one tile, pixel by pixel
+    (0, 2, 96, 8, 6, 64),       # 24: a tile and a half; K in parts
+    (0, 2, 96, 8, 12, 192),     # laid-out weights; the many-pixel split (two compute units are assumed here)
+    (0, 1, 192, 6, 16, 128),    # the middle one
+    (1, 1, 3, 4, 16, 96),       # four output pixels
+    (1, 2, 3, 20, 32, 96),      # two groups of 64 pixels, the second a part
+    (1, 3, 2, 16, 16, 128),     # groups of 32; two input channels: half of K
+])
+def test_emulated_patch_conv(stem, B, C, H, W, cout):
+    """wtconv_patch_conv on the host under the sanitizers, against float64 on the same bfloat16 values."""
+    rng = np.random.default_rng(C + H)
+    f = lambda *s, k=1.0: _bf16_round((rng.standard_normal(s) * k).astype(np.float32))
+    P, normed = (4, cout) if stem else (2, C)
+    x, cw, cb = f(B, C, H, W), f(cout, C, P, P, k=(C * P * P) ** -.5), f(cout, k=.3)
+    nw, nb = _bf16_round(1 + f(normed, k=.2)), f(normed, k=.2)
+    got = emu_util.run_patch_conv(stem, x, cw, cb, nw, nb)
+    d = lambda a: torch.from_numpy(a).double()
+    F = torch.nn.functional
+    norm = lambda t: F.layer_norm(t.permute(0, 2, 3, 1), (normed,), d(nw), d(nb), 1e-6).permute(0, 3, 1, 2)
+    y = F.conv2d(d(x) if stem else norm(d(x)), d(cw), d(cb), stride=P)
+    want = (norm(y) if stem else y).numpy()
+    # operands and result are rounded to bfloat16 (2^-9 relative each): the norm of the errors, and the largest
+    assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
+    assert np.abs(got - want).max() < 6e-2 * np.abs(want).max()

@@ -1,4 +1,4 @@
-"""ctypes binding of libwtconv_hip.so (C ABI declared in include/wtconv_hip.h)."""
+"""ctypes binding of libwtconv_hip.so (C ABI declared in include/wtconv_hip.h and include/wtconv_ops.h)."""
 import ctypes
 import os
 import threading
@@ -8,7 +8,8 @@ from . import _build
 MAX_LEVELS = 5
 F32, BF16, F16 = 0, 1, 2
 PASS_FORWARD, PASS_BACKWARD_INPUT, PASS_BACKWARD_PARAMS, PASS_BACKWARD = 0, 1, 2, 3
-ABI_VERSION = 6
+ABI_VERSION = 6      # of wtconv_hip.h
+OPS_VERSION = 1      # of wtconv_ops.h
 
 
 class Params(ctypes.Structure):
@@ -24,6 +25,10 @@ class ParamGrads(ctypes.Structure):
 class MlpParams(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in ("norm_weight", "norm_bias", "fc1_weight", "fc1_bias", "fc2_weight",
                                                "fc2_bias", "gamma")]
+
+
+class PatchParams(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("conv_weight", "conv_bias", "norm_weight", "norm_bias")]
 
 
 EXPORTS = {
@@ -64,6 +69,13 @@ EXPORTS["wtconv_haar1d"] = (_i, [_p, _p, _ll, _i, _i, _i, _p])
 EXPORTS["wtconv_haar2d_checked"] = (_i, [_p, _p, _ll, _i, _i, _i, _i, _p, _i, _p, _p])
 EXPORTS["wtconv_haar1d_checked"] = (_i, [_p, _p, _ll, _i, _i, _i, _p, _i, _p, _p])
 
+OPS_EXPORTS = {
+    "wtconv_ops_version": (_i, []),
+    "wtconv_patch_conv_supported": (_i, [_i] * 6),
+    "wtconv_patch_conv_workspace_bytes": (_z, [_i] * 6),
+    "wtconv_patch_conv": (_i, [_i, _p, _p, ctypes.POINTER(PatchParams)] + [_i] * 5 + [_f, _i, _i, _p, _z, _p]),
+}
+
 _lib = None
 _lock = threading.Lock()
 
@@ -94,7 +106,11 @@ def load():
         if version != ABI_VERSION:
             raise WTConvLibraryError(f"{path}: ABI version {version} != {ABI_VERSION}; build it again with "
                                      "`python -m wtconv_amd._build`")
-        for name, (res, args) in EXPORTS.items():
+        ops = lib.wtconv_ops_version() if hasattr(lib, "wtconv_ops_version") else 0
+        if ops != OPS_VERSION:
+            raise WTConvLibraryError(f"{path}: version {ops} of the block operators != {OPS_VERSION}; build it again with "
+                                     "`python -m wtconv_amd._build`")
+        for name, (res, args) in {**EXPORTS, **OPS_EXPORTS}.items():
             fn = getattr(lib, name)          # AttributeError if a declared symbol is not exported
             fn.restype, fn.argtypes = res, args
         _lib = lib

@@ -91,6 +91,25 @@ def block_mlp(x, shortcut, norm, mlp, gamma):
     return ext.block_mlp(x, shortcut, *args)
 
 
+def patch_conv(x, seq, conv, norm, stem):
+    """The stem (`conv` 4 x 4 with stride 4, then `norm` over the channels) or a downsample layer (`norm`, then `conv` 2 x 2
+    with stride 2) of a WTConvNeXt, the two modules of `seq`, in one kernel; None where it does not apply: autograd records,
+    another dtype than bfloat16, sizes without a kernel, another kind of convolution, observers that expect to see the
+    modules called, or tensors of a subclass."""
+    ext = _ext.get()
+    if ext is None or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+        return None
+    size = (4, 4) if stem else (2, 2)
+    if (type(conv) is not torch.nn.Conv2d or conv.kernel_size != size or conv.stride != size or conv.dilation != (1, 1)
+            or conv.groups != 1 or conv.padding not in ((0, 0), "valid") or _watched(seq, conv, norm)):
+        return None
+    args = (_param(conv), _param(conv, "bias"), _param(norm), _param(norm, "bias"))
+    for t in (x, *args):
+        if t is None or type(t) not in _PLAIN:
+            return None
+    return ext.patch_conv(x, *args, norm.eps, stem)
+
+
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 

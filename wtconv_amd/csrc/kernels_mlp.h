@@ -26,7 +26,7 @@
 // 917 -> 243 (490 TFLOP/s), 28 x 28 x 192 455 -> 187, 14 x 14 x 384 295 -> 182 (650 TFLOP/s); 56 x 56 x 128 1059 -> 350, 28 x 28 x 256 609 -> 346.
 #pragma once
 
-#include "common.h"
+#include "matrix.h"
 
 namespace wt {
 
@@ -62,19 +62,6 @@ __device__ __forceinline__ float gelu_erf(float x) {
   p = fmaf(a, p, -1.00000798f);
   return fmaf(fabsf(x), 0.5f - __builtin_amdgcn_exp2f(p), 0.5f * x);
 }
-
-#ifdef WT_EMULATE
-typedef ::emu::bf16x8 mlp_frag;
-typedef ::emu::f32x4 mlp_acc;
-typedef unsigned char* mlp_lds_addr;
-#define WT_MLP_LDS_ADDR(p) (p)
-#else
-typedef __bf16 mlp_frag __attribute__((ext_vector_type(8)));
-typedef float mlp_acc __attribute__((ext_vector_type(4)));
-typedef uint32_t mlp_lds_addr;
-#define WT_MLP_LDS_ADDR(p) \
-  static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)(p)))
-#endif
 
 // C channels, NT pixel tiles a wave, WAVES waves a workgroup, at least PER_SIMD waves a SIMD, slices of HC hidden units,
 // RING stages in LDS.
@@ -112,17 +99,6 @@ struct MlpShape {
   }
 };
 
-// 64 granules straight from memory (a uniform base and a byte offset per lane) into LDS: lane i's go to dst + 16 i.
-// (Issued as one instruction; the caller counts it in vmcnt.)
-__device__ __forceinline__ void granules_to_lds(const void* base, uint32_t offset, mlp_lds_addr lds_dst) {
-#ifdef WT_EMULATE
-  memcpy(lds_dst + 16 * (threadIdx.x & (kWave - 1)), static_cast<const unsigned char*>(base) + offset, 16);
-#else
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_dst), "v"(offset), "s"(base)
-               : "memory", "m0");
-#endif
-}
-
 // ROOM: there are HC floats of LDS behind the bias (which S::lds_bytes does not count).
 template <typename S, bool ROOM>
 __global__ void __launch_bounds__(S::kThreads, S::PER_SIMD)
@@ -150,11 +126,11 @@ block_mlp_kernel(MlpArgs a) {
     const int r2 = p / S::G2, g2 = S::swz2(r2, p - r2 * S::G2);
     src2[i] = static_cast<uint32_t>(r2 * a.hidden + g2 * 8) * 2;
   }
-  const mlp_lds_addr lds0 = WT_MLP_LDS_ADDR(mlp_lds);
+  const lds_addr lds0 = WT_LDS_ADDR(mlp_lds);
   auto holds = [&](int k) { return (k + 1) * S::kThreads <= S::kGranules || k * S::kThreads + wave * 64 < S::kGranules; };
   // stage i of the ring: W1's slice i and W2's slice i - 1, as far as they exist (slices counted from s_begin)
   auto load_stage = [&](int i, int at) {
-    const mlp_lds_addr dst = WT_UNIFORM(lds0 + at * S::kStageBytes + wave * 1024);
+    const lds_addr dst = WT_UNIFORM(lds0 + at * S::kStageBytes + wave * 1024);
     if (i < nsl) {
       const bf16_t* w1 = a.w1 + static_cast<size_t>(h0 + i * HC) * C;
 #pragma unroll
@@ -292,13 +268,13 @@ block_mlp_kernel(MlpArgs a) {
 
   load_stage(0, 0);
   load_stage(1, 1);
-  auto frag = [](const uint32_t (&v)[4]) { return __builtin_bit_cast(mlp_frag, uint4{v[0], v[1], v[2], v[3]}); };
+  auto frag = [](const uint32_t (&v)[4]) { return frag_of(uint4{v[0], v[1], v[2], v[3]}); };
 
-  mlp_acc acc[MT][NT];
+  mat_acc acc[MT][NT];
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = mlp_acc{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NT; ++t) acc[m][t] = mat_acc{0.f, 0.f, 0.f, 0.f};
 
   // this lane's part of the fragment addresses (bytes): its row, and the granule of each step in it (the permutations
   // do not depend on what is added to the row below)
@@ -318,23 +294,23 @@ block_mlp_kernel(MlpArgs a) {
   // iteration start before this one ends.
   constexpr int NG = HC / 32, N1 = NG * KS * 2, N2 = NG * MT, kAhead = N1 % 4 == 0 && N2 % 4 == 0 ? 4 : 3, PACKS = NG * NT * 4;
   static_assert(N1 % kAhead == 0 && N2 % kAhead == 0, "the fragments in flight keep their places");
-  mlp_acc h[NG][2][NT], hn[NG][2][NT];            // slice i - 1 and slice i before GELU
-  mlp_frag w[kAhead];                             // fragments in flight
+  mat_acc h[NG][2][NT], hn[NG][2][NT];            // slice i - 1 and slice i before GELU
+  mat_frag w[kAhead];                             // fragments in flight
   uint32_t hf[NG][NT][4];                         // slice i - 1 behind GELU
   const unsigned char* stage = mlp_lds;           // this iteration's
   int fill = 2;                                   // where stage i + 2 goes
   auto fetch1 = [&](const unsigned char* st, int j) {
-    return *reinterpret_cast<const mlp_frag*>(st + at1 + go1[j / 2 % KS] + (32 * (j / (2 * KS)) + 4 * (j & 1)) * S::G1 * 16);
+    return *reinterpret_cast<const mat_frag*>(st + at1 + go1[j / 2 % KS] + (32 * (j / (2 * KS)) + 4 * (j & 1)) * S::G1 * 16);
   };
   auto fetch2 = [&](const unsigned char* st, int j) {
-    return *reinterpret_cast<const mlp_frag*>(st + S::kSliceBytes + at2 + go2[j % NG] + 16 * (j / NG) * S::G2 * 16);
+    return *reinterpret_cast<const mat_frag*>(st + S::kSliceBytes + at2 + go2[j % NG] + 16 * (j / NG) * S::G2 * 16);
   };
   auto start = [&](const unsigned char* st, int i) {      // first reads of iteration i
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        const mlp_acc b = *reinterpret_cast<const mlp_acc*>(bias_lds + i * HC + 32 * g + 8 * q + 4 * m);
+        const mat_acc b = *reinterpret_cast<const mat_acc*>(bias_lds + i * HC + 32 * g + 8 * q + 4 * m);
 #pragma unroll
         for (int t = 0; t < NT; ++t) hn[g][m][t] = b;
       }
@@ -360,7 +336,7 @@ block_mlp_kernel(MlpArgs a) {
     for (int j = 0; j < N1; ++j) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        mlp_acc& d = hn[j / (2 * KS)][j & 1][t];
+        mat_acc& d = hn[j / (2 * KS)][j & 1][t];
         d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j % kAhead], frag(xf[t][j / 2 % KS]), d, 0, 0, 0);
       }
       if (j + kAhead < N1) w[j % kAhead] = fetch1(stage, j + kAhead);
@@ -377,7 +353,7 @@ block_mlp_kernel(MlpArgs a) {
     for (int j = 0; j < N2; ++j) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        mlp_acc& d = acc[j / NG][t];
+        mat_acc& d = acc[j / NG][t];
         d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j % kAhead], frag(hf[j % NG][t]), d, 0, 0, 0);
       }
       if (j + kAhead < N2) w[j % kAhead] = fetch2(stage, j + kAhead);

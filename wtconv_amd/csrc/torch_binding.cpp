@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/wtconv_hip.h"
+#include "../../include/wtconv_ops.h"
 
 namespace {
 
@@ -60,6 +61,10 @@ struct Abi {
   size_t (*mlp_ws)(int, int, int, int);
   int (*mlp)(const void*, const void*, void*, const wtconv_mlp_params*, int, int, int, int, float, int, int, void*, size_t,
              void*);
+  int (*patch_ok)(int, int, int, int, int, int);
+  size_t (*patch_ws)(int, int, int, int, int, int);
+  int (*patch)(int, const void*, void*, const wtconv_patch_params*, int, int, int, int, int, float, int, int, void*, size_t,
+               void*);
   bool bound = false;
 } abi;
 
@@ -68,12 +73,13 @@ void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 18, "bind: expected 18 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 21, "bind: expected 21 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
   take(abi.haar2, a[11]); take(abi.haar1, a[12]); take(abi.haar2c, a[13]); take(abi.haar1c, a[14]);
   take(abi.mlp_ok, a[15]); take(abi.mlp_ws, a[16]); take(abi.mlp, a[17]);
+  take(abi.patch_ok, a[18]); take(abi.patch_ws, a[19]); take(abi.patch, a[20]);
   abi.bound = true;
 }
 
@@ -530,6 +536,38 @@ py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm
   return py::cast(out);
 }
 
+// Stem (convolution, then LayerNorm over the channels) or downsample (LayerNorm, then convolution) in one kernel
+// (inference): None if no kernel takes these arguments or autograd would record the call.
+py::object patch_conv(const Tensor& x, const Tensor& conv_w, const Tensor& conv_b, const Tensor& norm_w, const Tensor& norm_b,
+                      double eps, bool stem) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (x.dim() != 4 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || x.numel() == 0) return py::none();
+  const int64_t B = x.size(0), C = x.size(1), H = x.size(2), W = x.size(3), P = stem ? 4 : 2;
+  if (conv_w.dim() != 4 || conv_w.size(1) != C || conv_w.size(2) != P || conv_w.size(3) != P) return py::none();
+  const int64_t cout = conv_w.size(0), normed = stem ? cout : C;
+  if (conv_b.numel() != cout || norm_w.numel() != normed || norm_b.numel() != normed) return py::none();
+  const bool grad = at::GradMode::is_enabled();
+  if (grad && x.requires_grad()) return py::none();
+  uintptr_t bits = reinterpret_cast<uintptr_t>(x.const_data_ptr());
+  for (const Tensor* t : {&conv_w, &conv_b, &norm_w, &norm_b}) {
+    if (!canonical(*t, x.device(), at::kBFloat16) || (grad && t->requires_grad())) return py::none();
+    bits |= reinterpret_cast<uintptr_t>(t->const_data_ptr());
+  }
+  if (bits % 16 || x.numel() > (1LL << 40) || !abi.patch_ok(stem, B, C, H, W, cout)) return py::none();
+  for (const Tensor* t : {&x, &conv_w, &conv_b, &norm_w, &norm_b})
+    if (t->_fw_grad(0).defined()) return py::none();      // forward-mode differentiation: PyTorch's own operators
+  const c10::DeviceGuard guard(x.device());
+  Tensor out = at::empty({B, cout, H / P, W / P}, x.options());
+  const size_t wsz = abi.patch_ws(stem, B, C, H, W, cout);
+  c10::DataPtr ws;
+  if (wsz) ws = scratch(x, wsz);
+  const wtconv_patch_params p = {conv_w.const_data_ptr(), conv_b.const_data_ptr(), norm_w.const_data_ptr(), norm_b.const_data_ptr()};
+  const int rc = abi.patch(stem, x.const_data_ptr(), out.mutable_data_ptr(), &p, B, C, H, W, cout, static_cast<float>(eps),
+                           WTCONV_BF16, WTCONV_BF16, ws.get(), wsz, c10::hip::getCurrentHIPStream(x.device().index()).stream());
+  if (rc) fail(rc, "wtconv patch conv");
+  return py::cast(out);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -540,5 +578,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       {nullptr, nullptr, 0, nullptr}};
   if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
   m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
+  m.def("patch_conv", &patch_conv, "stem or downsample of a WTConvNeXt in one kernel; None if not taken");
   m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }

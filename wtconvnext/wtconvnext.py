@@ -48,6 +48,18 @@ class LayerNorm2d(nn.LayerNorm):
         return x.permute(0, 3, 1, 2)
 
 
+def _resample(seq, x, stem):
+    """The stem's or a downsample layer's two modules; at inference on the GPU as one kernel."""
+    ops = _block_ops()
+    if ops is not None and type(seq) is nn.Sequential and len(seq) == 2:
+        conv, norm = seq if stem else (seq[1], seq[0])
+        if type(norm) is LayerNorm2d:
+            out = ops.patch_conv(x, seq, conv, norm, stem)
+            if out is not None:
+                return out
+    return seq(x)
+
+
 class Mlp(nn.Module):
     def __init__(self, dim, hidden):
         super().__init__()
@@ -145,7 +157,7 @@ class WTConvNeXtStage(nn.Module):
             for i in range(depth)])
 
     def forward(self, x):
-        x = self.downsample(x)
+        x = _resample(self.downsample, x, stem=False)
         if self.grad_checkpointing and torch.is_grad_enabled():
             from torch.utils.checkpoint import checkpoint
             for blk in self.blocks:
@@ -233,7 +245,7 @@ class WTConvNeXt(nn.Module):
             s.grad_checkpointing = enable
 
     def forward_features(self, x):
-        return self.stages(self.stem(x))
+        return self.stages(_resample(self.stem, x, stem=True))
 
     def forward_head(self, x, pre_logits: bool = False):
         return self.head(x, pre_logits=pre_logits)
