@@ -35,6 +35,28 @@ int wtconv_patch_conv(int stem, const void* x, void* out, const wtconv_patch_par
                       int cout, float eps, int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
                       void* stream);
 
+/* ---- a block's MLP in training, bfloat16: y = fc2(gelu(fc1(x))) with x, y (pixels, C), exact (erf) GELU, fc1_weight
+ * (hidden, C), fc2_weight (C, hidden) (wtconvnext/wtconvnext.py:125-136; the norm and gamma of wtconv_mlp_params are not
+ * read).  Everything 16-byte aligned.  Sums and GELU in float; each result is rounded to bfloat16 once.
+ * The forward call writes act = gelu(h) and, unless h is NULL, h = fc1(x), both (pixels, hidden); the backward call takes
+ * them and dy = dL/dy, and writes what is not NULL of dx and the parameters' gradients (a bias gradient only together
+ * with its weight's).  `want` says the same to the workspace query.  wtconv_mlp_supported: whether a size has kernels. */
+typedef struct {
+  void *fc1_weight, *fc1_bias, *fc2_weight, *fc2_bias;
+} wtconv_mlp_grads;
+
+#define WTCONV_MLP_DX 1
+#define WTCONV_MLP_FC1 2
+#define WTCONV_MLP_FC2 4
+
+int wtconv_mlp_supported(long long pixels, int C, int hidden);
+int wtconv_mlp_forward(const void* x, void* h, void* act, void* y, const wtconv_mlp_params* params, long long pixels, int C,
+                       int hidden, int dtype, int param_dtype, void* stream);
+size_t wtconv_mlp_backward_workspace_bytes(long long pixels, int C, int hidden, int want);
+int wtconv_mlp_backward(const void* x, const void* h, const void* act, const void* dy, const wtconv_mlp_params* params,
+                        void* dx, const wtconv_mlp_grads* grads, long long pixels, int C, int hidden, int dtype,
+                        int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -165,6 +165,28 @@ int main(int argc, char** argv) {
     fclose(fo);
     return 0;
   }
+  if (dims == 7) {
+    // a block's MLP in training: header {7, pixels, C, 1, 1, hidden (K slot), 0, 1, 1, unused};
+    //   in x, dy, fc1 weight and bias, fc2 weight and bias -> y, dx, gradients in that order
+    const int hidden = K;
+    const size_t P = static_cast<size_t>(B) * C, Q = static_cast<size_t>(B) * hidden, M = static_cast<size_t>(hidden) * C;
+    Buf bx = read_buf(fp, P, 1), dy = read_buf(fp, P, 1), w1 = read_buf(fp, M, 1), b1 = read_buf(fp, hidden, 1);
+    Buf w2 = read_buf(fp, M, 1), b2 = read_buf(fp, C, 1);
+    fclose(fp);
+    Buf h = out_buf(Q, 1), act = out_buf(Q, 1), y = out_buf(P, 1), dx = out_buf(P, 1);
+    Buf g1 = out_buf(M, 1), gb1 = out_buf(hidden, 1), g2 = out_buf(M, 1), gb2 = out_buf(C, 1);
+    std::vector<char> ws(wtconv_mlp_backward_workspace_bytes(B, C, hidden, WTCONV_MLP_DX | WTCONV_MLP_FC1 | WTCONV_MLP_FC2));
+    const wtconv_mlp_params prm = {nullptr, nullptr, w1.ptr(), b1.ptr(), w2.ptr(), b2.ptr(), nullptr};
+    const wtconv_mlp_grads gr = {g1.ptr(), gb1.ptr(), g2.ptr(), gb2.ptr()};
+    int rc = wtconv_mlp_forward(bx.ptr(), h.ptr(), act.ptr(), y.ptr(), &prm, B, C, hidden, 1, 1, nullptr);
+    if (!rc) rc = wtconv_mlp_backward(bx.ptr(), h.ptr(), act.ptr(), dy.ptr(), &prm, dx.ptr(), &gr, B, C, hidden, 1, 1, ws.data(), ws.size(), nullptr);
+    if (rc) { fprintf(stderr, "mlp: %s\n", wtconv_last_error()); return 3; }
+    FILE* fo = fopen(argv[2], "wb");
+    if (!fo) { perror("open out"); return 2; }
+    for (Buf* b : {&y, &dx, &g1, &gb1, &g2, &gb2}) { b->unpack(); fwrite(b->f.data(), 4, b->f.size(), fo); }
+    fclose(fo);
+    return 0;
+  }
   const int S = dims == 2 ? 4 : 2;
   const size_t KK = dims == 2 ? static_cast<size_t>(K) * K : K;
   const size_t P = static_cast<size_t>(B) * C * H * W;   // 1-D: H == 1, W == N

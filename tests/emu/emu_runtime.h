@@ -106,6 +106,20 @@ inline f32x4 mfma_16x16x32_bf16(const bf16x8& a, const bf16x8& b, f32x4 c, int, 
   mfma_16x16x32_bf16(a.v, b.v, c.v);
   return c;
 }
+// What ds_read_b64_tr_b16 gives: in each group of 16 lanes, lane i names four 16-bit values; lane i gets value i % 4 of
+// the lanes i / 4, 4 + i / 4, 8 + i / 4 and 12 + i / 4.
+inline uint2 column_of_4(const uint16_t* p) {
+  BlockState* st = tls_block;
+  const unsigned t = threadIdx.x, base = t / 16 * 16, i = t % 16;
+  std::memcpy(&st->mfma_a[t * 8], p, 8);
+  wave_barrier();
+  uint16_t v[4];
+  for (unsigned j = 0; j < 4; ++j) v[j] = st->mfma_a[(base + 4 * j + i / 4) * 8 + i % 4];
+  wave_barrier();
+  uint2 r;
+  std::memcpy(&r, v, 8);
+  return r;
+}
 // Byte i of the result is byte sel[i] of the eight bytes of `lo` (0-3) and `hi` (4-7).
 inline uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
   const uint64_t both = static_cast<uint64_t>(hi) << 32 | lo;

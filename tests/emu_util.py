@@ -15,6 +15,7 @@ EXE = os.path.join(BUILD_DIR, "emu_driver")
 SOURCES = [os.path.join(ROOT, "wtconv_amd", "csrc", "api.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "mfma2d.hip"),
            os.path.join(ROOT, "wtconv_amd", "csrc", "block.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "haar.hip"),
            os.path.join(ROOT, "wtconv_amd", "csrc", "mlp.hip"), os.path.join(ROOT, "wtconv_amd", "csrc", "patch.hip"),
+           os.path.join(ROOT, "wtconv_amd", "csrc", "mlp_train.hip"),
            os.path.join(EMU_DIR, "emu_driver.cpp")]
 # api.hip includes the other translation units here, and every one of them its headers: all of csrc
 DEPS = sorted(set(SOURCES + [f for ext in ("h", "hip") for f in glob.glob(os.path.join(ROOT, "wtconv_amd", "csrc", "*." + ext))] + [
@@ -190,3 +191,27 @@ def run_patch_conv(stem, x, cw, cb, nw, nb, eps=1e-6, timeout=600):
         if r.returncode != 0:
             raise RuntimeError(f"emu_driver failed ({r.returncode}):\n{r.stderr[-4000:]}")
         return np.fromfile(fout, dtype=np.float32).reshape(B, cw.shape[0], H // P, W // P)
+
+
+def run_mlp(x, dy, w1, b1, w2, b2, timeout=600):
+    """wtconv_mlp_forward and wtconv_mlp_backward on the host; x, dy (pixels, C), bf16 values in float32 arrays.  Returns
+    y, dx and the gradients of the parameters in the order of the arguments."""
+    exe = build()
+    M, C = x.shape
+    hdr = np.array([7, M, C, 1, 1, w1.shape[0], 0, 1, 1, 0], dtype=np.int32)
+    parts = [hdr.tobytes()] + [np.ascontiguousarray(a, dtype=np.float32).tobytes() for a in (x, dy, w1, b1, w2, b2)]
+    with tempfile.TemporaryDirectory() as td:
+        fin, fout = os.path.join(td, "in.bin"), os.path.join(td, "out.bin")
+        with open(fin, "wb") as f:
+            f.write(b"".join(parts))
+        env = dict(os.environ)
+        env["ASAN_OPTIONS"] = "detect_leaks=0"
+        r = subprocess.run([exe, fin, fout], capture_output=True, text=True, timeout=timeout, env=env)
+        if r.returncode != 0:
+            raise RuntimeError(f"emu_driver failed ({r.returncode}):\n{r.stderr[-4000:]}")
+        raw = np.fromfile(fout, dtype=np.float32)
+    res = []
+    for a in (x, x, w1, b1, w2, b2):
+        res.append(raw[:a.size].reshape(a.shape))
+        raw = raw[a.size:]
+    return res

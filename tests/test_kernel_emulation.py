@@ -479,3 +479,25 @@ def test_emulated_patch_conv(stem, B, C, H, W, cout):
     # operands and result are rounded to bfloat16 (2^-9 relative each): the norm of the errors, and the largest
     assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
     assert np.abs(got - want).max() < 6e-2 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("M,C,hidden", [
+    (70, 96, 128),       # 96 channels: steps of 32 and tiles of 96 outputs; 64 pixels and six
+    (130, 128, 256),     # shares of the pixels; the last stage holds two pixels
+    (33, 192, 128),      # tiles of 64 outputs, of 192 channels in the weight gradients; a part of the only tile
+])
+def test_emulated_mlp_training(M, C, hidden):
+    """wtconv_mlp_forward / _backward on the host under the sanitizers, against float64 on the same bfloat16 values."""
+    rng = np.random.default_rng(C + M)
+    f = lambda *s, k=1.0: _bf16_round((rng.standard_normal(s) * k).astype(np.float32))
+    args = f(M, C), f(M, C), f(hidden, C, k=C ** -.5), f(hidden), f(C, hidden, k=hidden ** -.5), f(C)
+    got = emu_util.run_mlp(*args)
+    x, dy, w1, b1, w2, b2 = [torch.from_numpy(a).double() for a in args]
+    par = [t.requires_grad_() for t in (x, w1, b1, w2, b2)]
+    F = torch.nn.functional
+    y = F.linear(F.gelu(F.linear(x, w1, b1)), w2, b2)
+    want = [y.detach()] + list(torch.autograd.grad(y, par, dy))
+    for a, w in zip(got, want):
+        # operands, hidden values and results are rounded to bfloat16 (2^-9 relative each)
+        w = w.numpy()
+        assert np.linalg.norm(a - w) < 6e-3 * np.linalg.norm(w)

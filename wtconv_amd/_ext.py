@@ -16,7 +16,8 @@ _ENTRY_POINTS = ("wtconv2d_forward", "wtconv2d_backward", "wtconv2d_backward_inp
                  "wtconv1d_workspace_bytes", "wtconv_last_error",
                  "wtconv_haar2d", "wtconv_haar1d", "wtconv_haar2d_checked", "wtconv_haar1d_checked",
                  "wtconv_block_mlp_supported", "wtconv_block_mlp_workspace_bytes", "wtconv_block_mlp",
-                 "wtconv_patch_conv_supported", "wtconv_patch_conv_workspace_bytes", "wtconv_patch_conv")
+                 "wtconv_patch_conv_supported", "wtconv_patch_conv_workspace_bytes", "wtconv_patch_conv",
+                 "wtconv_mlp_supported", "wtconv_mlp_forward", "wtconv_mlp_backward_workspace_bytes", "wtconv_mlp_backward")
 
 _mod = None
 _tried = False

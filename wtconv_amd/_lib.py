@@ -27,6 +27,10 @@ class MlpParams(ctypes.Structure):
                                                "fc2_bias", "gamma")]
 
 
+class MlpGrads(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("fc1_weight", "fc1_bias", "fc2_weight", "fc2_bias")]
+
+
 class PatchParams(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in ("conv_weight", "conv_bias", "norm_weight", "norm_bias")]
 
@@ -73,6 +77,10 @@ OPS_EXPORTS = {
     "wtconv_ops_version": (_i, []),
     "wtconv_patch_conv_supported": (_i, [_i] * 6),
     "wtconv_patch_conv_workspace_bytes": (_z, [_i] * 6),
+    "wtconv_mlp_supported": (_i, [_ll, _i, _i]),
+    "wtconv_mlp_forward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _ll] + [_i] * 4 + [_p]),
+    "wtconv_mlp_backward_workspace_bytes": (_z, [_ll, _i, _i, _i]),
+    "wtconv_mlp_backward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _p, ctypes.POINTER(MlpGrads), _ll] + [_i] * 4 + [_p, _z, _p]),
     "wtconv_patch_conv": (_i, [_i, _p, _p, ctypes.POINTER(PatchParams)] + [_i] * 5 + [_f, _i, _i, _p, _z, _p]),
 }
 

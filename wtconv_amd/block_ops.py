@@ -66,6 +66,12 @@ def _watched(*modules):
     return False
 
 
+def _watched_backward(*modules):
+    """Whether something expects to see gradients at the borders of these modules."""
+    return bool(_nn._global_backward_hooks or _nn._global_backward_pre_hooks
+                or any(m.__dict__["_backward_hooks"] or m.__dict__["_backward_pre_hooks"] for m in modules))
+
+
 _PLAIN = (torch.Tensor, torch.nn.Parameter, type(None))
 
 
@@ -108,6 +114,23 @@ def patch_conv(x, seq, conv, norm, stem):
         if t is None or type(t) not in _PLAIN:
             return None
     return ext.patch_conv(x, *args, norm.eps, stem)
+
+
+def mlp_fn(x, mlp):
+    """A block's `mlp` (fc1, exact GELU, fc2) on x (B, H, W, C) where autograd records it, products, GELU and bias sums as
+    kernels of this library; None where that does not apply (see block_mlp)."""
+    ext = _ext.get()
+    if ext is None or not torch.is_grad_enabled() or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+        return None
+    fc1, act, fc2 = mlp.fc1, mlp.act, mlp.fc2
+    if (type(fc1) is not torch.nn.Linear or type(fc2) is not torch.nn.Linear or type(act) is not torch.nn.GELU
+            or act.approximate != "none" or _watched(mlp, fc1, act, fc2) or _watched_backward(mlp, fc1, act, fc2)):
+        return None
+    args = (_param(fc1), _param(fc1, "bias"), _param(fc2), _param(fc2, "bias"))
+    for t in (x, *args):
+        if t is None or type(t) not in _PLAIN:
+            return None
+    return ext.mlp(x, *args)
 
 
 def _stream():

@@ -26,6 +26,7 @@
 // 917 -> 243 (490 TFLOP/s), 28 x 28 x 192 455 -> 187, 14 x 14 x 384 295 -> 182 (650 TFLOP/s); 56 x 56 x 128 1059 -> 350, 28 x 28 x 256 609 -> 346.
 #pragma once
 
+#include "gelu.h"
 #include "matrix.h"
 
 namespace wt {
@@ -46,22 +47,6 @@ struct MlpArgs {
   int splits;
   int vec;                            // pixels moved at once: 8, 4 or 1 (they share an image and an aligned word)
 };
-
-// erf form of GELU: x * Phi(x) = x / 2 + |x| * (1 / 2 - Phi(-|x|)).  log2 of Phi(-a) is a smooth, nearly quadratic function, so
-// Phi(-a) is 2 to a polynomial in a (degree 7, fitted to the error of the result weighted by a * Phi(-a)): |error| <=
-// 3.9e-7 over all x (x / 2 * (1 + erf) in float32: 1.2e-6), for 28 cycles of the vector pipe a value instead of the 44 of
-// a rational times an exponential.  (The last two terms see x itself: infinities and NaNs come out as they do of erf.)
-__device__ __forceinline__ float gelu_erf(float x) {
-  const float a = fminf(fabsf(x), 16.f);      // (Phi(-16) is 0 in float32; an infinity must not meet that 0)
-  float p = fmaf(a, -1.09032517e-06f, 4.60320700e-05f);
-  p = fmaf(a, p, -8.13045196e-04f);
-  p = fmaf(a, p, 8.10905740e-03f);
-  p = fmaf(a, p, -5.33128628e-02f);
-  p = fmaf(a, p, -4.58948432e-01f);
-  p = fmaf(a, p, -1.15110632f);
-  p = fmaf(a, p, -1.00000798f);
-  return fmaf(fabsf(x), 0.5f - __builtin_amdgcn_exp2f(p), 0.5f * x);
-}
 
 // C channels, NT pixel tiles a wave, WAVES waves a workgroup, at least PER_SIMD waves a SIMD, slices of HC hidden units,
 // RING stages in LDS.

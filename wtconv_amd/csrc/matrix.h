@@ -31,4 +31,27 @@ __device__ __forceinline__ void granules_to_lds(const void* base, uint32_t offse
 #endif
 }
 
+// Four values of one column of a row-major tile of 16-bit values in LDS: the 16 lanes that share lane / 16 each name four
+// neighbouring values, lane i those of row i / 4 of four and of the columns 4 (i % 4) ... of sixteen; lane i gets column i,
+// rows 0 to 3.  (ds_read_b64_tr_b16.)
+__device__ __forceinline__ uint2 column_of_4(const bf16_t* p) {
+#ifdef WT_EMULATE
+  return ::emu::column_of_4(p);
+#else
+  typedef short four __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) four*)(p)));
+#endif
+}
+
+// Waits until at most N of this wave's loads are on their way and its LDS reads have arrived, then for the workgroup.
+template <int N>
+__device__ __forceinline__ void arrive_and_wait() {
+#ifdef WT_EMULATE
+  __syncthreads();
+#else
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+#endif
+}
+
 }  // namespace wt

@@ -65,6 +65,11 @@ struct Abi {
   size_t (*patch_ws)(int, int, int, int, int, int);
   int (*patch)(int, const void*, void*, const wtconv_patch_params*, int, int, int, int, int, float, int, int, void*, size_t,
                void*);
+  int (*mlpt_ok)(long long, int, int);
+  int (*mlpt_fwd)(const void*, void*, void*, void*, const wtconv_mlp_params*, long long, int, int, int, int, void*);
+  size_t (*mlpt_ws)(long long, int, int, int);
+  int (*mlpt_bwd)(const void*, const void*, const void*, const void*, const wtconv_mlp_params*, void*, const wtconv_mlp_grads*,
+                  long long, int, int, int, int, void*, size_t, void*);
   bool bound = false;
 } abi;
 
@@ -73,13 +78,14 @@ void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 21, "bind: expected 21 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 25, "bind: expected 25 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
   take(abi.haar2, a[11]); take(abi.haar1, a[12]); take(abi.haar2c, a[13]); take(abi.haar1c, a[14]);
   take(abi.mlp_ok, a[15]); take(abi.mlp_ws, a[16]); take(abi.mlp, a[17]);
   take(abi.patch_ok, a[18]); take(abi.patch_ws, a[19]); take(abi.patch, a[20]);
+  take(abi.mlpt_ok, a[21]); take(abi.mlpt_fwd, a[22]); take(abi.mlpt_ws, a[23]); take(abi.mlpt_bwd, a[24]);
   abi.bound = true;
 }
 
@@ -159,6 +165,17 @@ Tensor layer_forward(const Tensor& x, const LayerParams& lp, int dims, int K) {
                                       ws.get(), wsz, stream);
   if (rc) fail(rc, "wtconv forward");
   return out;
+}
+
+// Results that come from raw pointers and carry no graph: a derivative of theirs is refused.
+void refuse_second_derivatives(variable_list& res, const char* what) {
+  for (Tensor& t : res)
+    if (t.defined()) {
+      auto err = std::make_shared<torch::autograd::Error>(
+          std::string("the backward pass of ") + what + " is not differentiable (double backward / create_graph=True through "
+          "this layer is not supported)", torch::autograd::edge_list());
+      torch::autograd::create_gradient_edge(t, err);
+    }
 }
 
 // Gradients of x and of the parameters: edges 0 and 1..count() of the node.
@@ -250,14 +267,7 @@ struct WTConvNode : public torch::autograd::Node {
       for (int i = 0; i < n; ++i)
         if (lp.t[i].defined() && task_should_compute_output(1 + i)) res[1 + i] = part_of(src, pos[i], lp.t[i].sizes());
     }
-    if (twice)
-      for (Tensor& t : res)
-        if (t.defined()) {
-          auto err = std::make_shared<torch::autograd::Error>(
-              "the backward pass of the WTConv layer is not differentiable (double backward / create_graph=True through "
-              "this layer is not supported)", torch::autograd::edge_list());
-          torch::autograd::create_gradient_edge(t, err);
-        }
+    if (twice) refuse_second_derivatives(res, "the WTConv layer");
     return res;
   }
 };
@@ -536,6 +546,115 @@ py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm
   return py::cast(out);
 }
 
+// ---- a block's MLP in training: fc2(gelu(fc1(x))) over the last extent of x.
+
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
+
+// Gradients of x, fc1's weight and bias, fc2's weight and bias: edges 0..4 of the node.
+struct MlpNode : public torch::autograd::Node {
+  torch::autograd::SavedVariable x_, w1_, w2_, h_, act_;
+
+  std::string name() const override { return "WTConvMlpBackward"; }
+
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    for (auto* v : {&x_, &w1_, &w2_, &h_, &act_}) v->reset_data();
+  }
+
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const Tensor x = x_.unpack(), w1 = w1_.unpack(), w2 = w2_.unpack(), h = h_.unpack(), act = act_.unpack();
+    variable_list res(5);
+    if (!grads[0].defined()) return res;
+    const bool need_x = task_should_compute_output(0);
+    const bool need_1 = task_should_compute_output(1) || task_should_compute_output(2);
+    const bool need_2 = task_should_compute_output(3) || task_should_compute_output(4);
+    if (!need_x && !need_1 && !need_2) return res;
+    const bool twice = at::GradMode::is_enabled() &&
+                       (grads[0].requires_grad() || x.requires_grad() || w1.requires_grad() || w2.requires_grad());
+    const at::NoGradGuard no_grad;
+    Tensor g = grads[0];
+    if (g.scalar_type() != x.scalar_type()) g = g.to(x.scalar_type());
+    if (!g.is_contiguous()) g = g.contiguous();
+    if (!aligned16(g)) g = g.clone();
+    const c10::DeviceGuard guard(x.device());
+    const int64_t C = w1.size(1), hidden = w1.size(0), pixels = x.numel() / C;
+    const int want = (need_x ? WTCONV_MLP_DX : 0) | (need_1 ? WTCONV_MLP_FC1 : 0) | (need_2 ? WTCONV_MLP_FC2 : 0);
+    const size_t wsz = abi.mlpt_ws(pixels, C, hidden, want);
+    const c10::DataPtr ws = scratch(x, wsz);
+    if (need_x) res[0] = at::empty(x.sizes(), x.options().requires_grad(false));
+    // (one allocation for the parameters' gradients; their sizes are multiples of 32)
+    const int64_t sizes[4] = {hidden * C, hidden, C * hidden, C};
+    Tensor flat = at::empty({(need_1 ? sizes[0] + sizes[1] : 0) + (need_2 ? sizes[2] + sizes[3] : 0)}, x.options().requires_grad(false));
+    void* to[4] = {nullptr, nullptr, nullptr, nullptr};
+    int64_t pos[4], at_elem = 0;
+    for (int i = 0; i < 4; ++i) {
+      pos[i] = at_elem;
+      if (i < 2 ? !need_1 : !need_2) continue;
+      to[i] = static_cast<at::BFloat16*>(flat.mutable_data_ptr()) + at_elem;
+      at_elem += sizes[i];
+    }
+    const wtconv_mlp_params p = {nullptr, nullptr, w1.const_data_ptr(), nullptr, w2.const_data_ptr(), nullptr, nullptr};
+    const wtconv_mlp_grads gt = {to[0], to[1], to[2], to[3]};
+    const int rc = abi.mlpt_bwd(x.const_data_ptr(), h.const_data_ptr(), act.const_data_ptr(), g.const_data_ptr(), &p,
+                                need_x ? res[0].mutable_data_ptr() : nullptr, &gt, pixels, C, hidden, WTCONV_BF16, WTCONV_BF16,
+                                ws.get(), wsz, c10::hip::getCurrentHIPStream(x.device().index()).stream());
+    if (rc) fail(rc, "wtconv mlp backward");
+    for (int i = 0; i < 4; ++i)
+      if (task_should_compute_output(1 + i))
+        res[1 + i] = i == 0 ? part_of(flat, pos[0], {hidden, C}) : i == 2 ? part_of(flat, pos[2], {C, hidden}) : part_of(flat, pos[i], {sizes[i]});
+    if (twice) refuse_second_derivatives(res, "the block's MLP");
+    return res;
+  }
+};
+
+// The MLP with its C++ autograd node, where autograd records it: None otherwise, or if there are no kernels for these arguments.
+py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (!at::GradMode::is_enabled() || x.dim() < 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || x.numel() == 0)
+    return py::none();
+  if (w1.dim() != 2 || w2.dim() != 2 || w1.size(1) != x.size(-1) || w2.size(0) != x.size(-1) || w1.size(0) != w2.size(1)) return py::none();
+  const int64_t C = w1.size(1), hidden = w1.size(0), pixels = x.numel() / C;
+  if (b1.numel() != hidden || b2.numel() != C || !abi.mlpt_ok(pixels, C, hidden)) return py::none();
+  bool any = x.requires_grad();
+  for (const Tensor* t : {&w1, &b1, &w2, &b2}) {
+    if (!canonical(*t, x.device(), at::kBFloat16) || !aligned16(*t) || t->_fw_grad(0).defined()) return py::none();
+    any = any || t->requires_grad();
+  }
+  if (!any || !aligned16(x) || x._fw_grad(0).defined()) return py::none();
+  Tensor y;
+  {
+    py::gil_scoped_release nogil;
+    const c10::DeviceGuard guard(x.device());
+    Tensor h, act;
+    {
+      const at::NoGradGuard no_grad;
+      std::vector<int64_t> wide = x.sizes().vec();
+      wide.back() = hidden;
+      const at::TensorOptions opt = x.options().requires_grad(false);
+      y = at::empty(x.sizes(), opt);
+      h = at::empty(wide, opt);
+      act = at::empty(wide, opt);
+    }
+    const wtconv_mlp_params p = {nullptr, nullptr, w1.const_data_ptr(), b1.const_data_ptr(), w2.const_data_ptr(), b2.const_data_ptr(), nullptr};
+    const int rc = abi.mlpt_fwd(x.const_data_ptr(), h.mutable_data_ptr(), act.mutable_data_ptr(), y.mutable_data_ptr(), &p, pixels, C,
+                                hidden, WTCONV_BF16, WTCONV_BF16, c10::hip::getCurrentHIPStream(x.device().index()).stream());
+    if (rc) fail(rc, "wtconv mlp forward");
+    const std::shared_ptr<MlpNode> node(new MlpNode(), torch::autograd::deleteNode);
+    torch::autograd::edge_list next;
+    next.reserve(5);
+    for (const Tensor* t : {&x, &w1, &b1, &w2, &b2}) next.push_back(torch::autograd::impl::gradient_edge(*t));
+    node->set_next_edges(std::move(next));
+    node->x_ = torch::autograd::SavedVariable(x, false);
+    node->w1_ = torch::autograd::SavedVariable(w1, false);
+    node->w2_ = torch::autograd::SavedVariable(w2, false);
+    node->h_ = torch::autograd::SavedVariable(h, false);
+    node->act_ = torch::autograd::SavedVariable(act, false);
+    torch::autograd::set_history(y, node);
+  }
+  return py::cast(y);
+}
+
 // Stem (convolution, then LayerNorm over the channels) or downsample (LayerNorm, then convolution) in one kernel
 // (inference): None if no kernel takes these arguments or autograd would record the call.
 py::object patch_conv(const Tensor& x, const Tensor& conv_w, const Tensor& conv_b, const Tensor& norm_w, const Tensor& norm_b,
@@ -578,6 +697,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       {nullptr, nullptr, 0, nullptr}};
   if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
   m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
+  m.def("mlp", &mlp, "a block's MLP with a C++ autograd node; None if not taken");
   m.def("patch_conv", &patch_conv, "stem or downsample of a WTConvNeXt in one kernel; None if not taken");
   m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }
