@@ -17,6 +17,28 @@ extern "C" {
 /* Version of this part in the loaded library (== WTCONV_OPS_VERSION). */
 int wtconv_ops_version(void);
 
+/* ---- the backward passes of wtconv_hip.h with the parameters' gradients in a dtype of the caller's choice (float, bfloat16 or
+ * half: `dtype` of the table).  Sums are in float; the results are rounded once. */
+typedef struct {
+  void *base_weight, *base_bias, *base_scale;
+  void* wt_weight[WTCONV_MAX_LEVELS];
+  void* wt_scale[WTCONV_MAX_LEVELS];
+  int dtype;
+} wtconv_typed_grads;
+
+int wtconv2d_backward_params_typed(const void* x, const void* grad_out, const wtconv_params* params,
+                                   const wtconv_typed_grads* grads, int B, int C, int H, int W, int K, int levels,
+                                   int dtype, int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+int wtconv2d_backward_typed(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
+                            const wtconv_typed_grads* grads, int B, int C, int H, int W, int K, int levels, int dtype,
+                            int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+int wtconv1d_backward_params_typed(const void* x, const void* grad_out, const wtconv_params* params,
+                                   const wtconv_typed_grads* grads, int B, int C, int N, int K, int levels, int dtype,
+                                   int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+int wtconv1d_backward_typed(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
+                            const wtconv_typed_grads* grads, int B, int C, int N, int K, int levels, int dtype,
+                            int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- the convolutions that change resolution, with the LayerNorm beside them, for inference in bfloat16:
  *   stem != 0:  out = LayerNorm_c(conv 4x4 stride 4 (x) + bias), norm parameters of `cout` values;
  *   stem == 0:  out = conv 2x2 stride 2 (LayerNorm_c(x)) + bias, norm parameters of `C` values

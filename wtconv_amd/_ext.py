@@ -10,9 +10,9 @@ import os
 from . import _build, _lib
 
 # order of the addresses bind() takes (torch_binding.cpp)
-_ENTRY_POINTS = ("wtconv2d_forward", "wtconv2d_backward", "wtconv2d_backward_input", "wtconv2d_backward_params",
+_ENTRY_POINTS = ("wtconv2d_forward", "wtconv2d_backward_typed", "wtconv2d_backward_input", "wtconv2d_backward_params_typed",
                  "wtconv2d_workspace_bytes",
-                 "wtconv1d_forward", "wtconv1d_backward", "wtconv1d_backward_input", "wtconv1d_backward_params",
+                 "wtconv1d_forward", "wtconv1d_backward_typed", "wtconv1d_backward_input", "wtconv1d_backward_params_typed",
                  "wtconv1d_workspace_bytes", "wtconv_last_error",
                  "wtconv_haar2d", "wtconv_haar1d", "wtconv_haar2d_checked", "wtconv_haar1d_checked",
                  "wtconv_block_mlp_supported", "wtconv_block_mlp_workspace_bytes", "wtconv_block_mlp",

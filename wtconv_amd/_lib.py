@@ -27,6 +27,10 @@ class MlpParams(ctypes.Structure):
                                                "fc2_bias", "gamma")]
 
 
+class TypedGrads(ctypes.Structure):
+    _fields_ = Params._fields_ + [("dtype", ctypes.c_int)]
+
+
 class MlpGrads(ctypes.Structure):
     _fields_ = [(n, ctypes.c_void_p) for n in ("fc1_weight", "fc1_bias", "fc2_weight", "fc2_bias")]
 
@@ -77,6 +81,10 @@ OPS_EXPORTS = {
     "wtconv_ops_version": (_i, []),
     "wtconv_patch_conv_supported": (_i, [_i] * 6),
     "wtconv_patch_conv_workspace_bytes": (_z, [_i] * 6),
+    "wtconv2d_backward_params_typed": (_i, [_p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 8 + [_p, _z, _p]),
+    "wtconv2d_backward_typed": (_i, [_p, _p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 8 + [_p, _z, _p]),
+    "wtconv1d_backward_params_typed": (_i, [_p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 7 + [_p, _z, _p]),
+    "wtconv1d_backward_typed": (_i, [_p, _p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 7 + [_p, _z, _p]),
     "wtconv_mlp_supported": (_i, [_ll, _i, _i]),
     "wtconv_mlp_forward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _ll] + [_i] * 4 + [_p]),
     "wtconv_mlp_backward_workspace_bytes": (_z, [_ll, _i, _i, _i]),

@@ -8,6 +8,7 @@
 #include "common.h"
 #include "host_util.h"
 #include "launch.h"
+#include "../../include/wtconv_ops.h"
 #include "mfma2d.h"
 #include "kernels1d.h"
 #include "kernels1d_row.h"
@@ -339,8 +340,28 @@ static unsigned char scratch[kStaticScratchBytes];
 static int static_scratch(const char*, void** ptr) { *ptr = scratch; return 0; }
 #endif
 
-static int check_grad_table(const char* fn, const wtconv_params* params, const wtconv_param_grads* grads, int L) {
+static int check_grad_dtype(const char* fn, const wtconv_typed_grads* grads) {
+  if (grads->dtype != WTCONV_F32 && grads->dtype != WTCONV_BF16 && grads->dtype != WTCONV_F16)
+    return fail(WTCONV_E_ARG, "%s: unknown gradient dtype %d", fn, grads->dtype);
+  return 0;
+}
+
+// The gradients of the untyped entry points: float.
+struct FloatGrads {
+  wtconv_typed_grads t = {};
+  const wtconv_typed_grads* ptr = nullptr;
+  FloatGrads(const wtconv_param_grads* g, int levels) {
+    if (g == nullptr) return;
+    t.dtype = WTCONV_F32;
+    t.base_weight = g->base_weight; t.base_bias = g->base_bias; t.base_scale = g->base_scale;
+    for (int l = 0; l < levels && l < kMaxLevels; ++l) { t.wt_weight[l] = g->wt_weight[l]; t.wt_scale[l] = g->wt_scale[l]; }
+    ptr = &t;
+  }
+};
+
+static int check_grad_table(const char* fn, const wtconv_params* params, const wtconv_typed_grads* grads, int L) {
   if (grads == nullptr) return fail(WTCONV_E_ARG, "%s: null tensor pointer", fn);
+  if (int e = check_grad_dtype(fn, grads)) return e;
   if (grads->base_weight == nullptr || grads->base_scale == nullptr ||
       (params->base_bias != nullptr && grads->base_bias == nullptr))
     return fail(WTCONV_E_ARG, "%s: null gradient pointer", fn);
@@ -350,8 +371,9 @@ static int check_grad_table(const char* fn, const wtconv_params* params, const w
   return 0;
 }
 
-static GradTable to_grad_table(const wtconv_param_grads* grads, int L) {
+static GradTable to_grad_table(const wtconv_typed_grads* grads, int L) {
   GradTable gt = {};
+  gt.dtype = grads->dtype;
   gt.base_weight = grads->base_weight;
   gt.base_bias = grads->base_bias;
   gt.base_scale = grads->base_scale;
@@ -476,7 +498,7 @@ static unsigned* wgrad2d_tickets(void* workspace, int B, int C, int H, int W, in
 // have_g_ll (planes beyond LDS only): the LL bands of grad_out that the layer itself needs are in the workspace already.
 // tickets_zeroed (plane-resident paths only): an earlier kernel on the stream has cleared the channel tickets.
 static int backward_params2d(const char* fn, const void* x, const void* grad_out, const wtconv_params* params,
-                             const wtconv_param_grads* grads, int B, int C, int H, int W, int K, int levels,
+                             const wtconv_typed_grads* grads, int B, int C, int H, int W, int K, int levels,
                              int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
                              void* stream_, bool have_g_ll, bool tickets_zeroed = false) {
   const int L = levels;
@@ -485,6 +507,7 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
   if (static_cast<long long>(H) * W > kMaxPlaneElems)   // 32-bit offsets inside a plane and its four stacked sub-bands
     return fail(WTCONV_E_UNSUPPORTED, "%s: a plane of %dx%d exceeds 2^28 elements", fn, H, W);
   if (x == nullptr || grad_out == nullptr || grads == nullptr) return fail(WTCONV_E_ARG, "%s: null tensor pointer", fn);
+  if (int e = check_grad_dtype(fn, grads)) return e;
   if (grads->base_weight == nullptr || grads->base_scale == nullptr ||
       (params->base_bias != nullptr && grads->base_bias == nullptr))
     return fail(WTCONV_E_ARG, "%s: null gradient pointer", fn);
@@ -572,6 +595,14 @@ int wtconv2d_backward_params(const void* x, const void* grad_out, const wtconv_p
                              const wtconv_param_grads* grads, int B, int C, int H, int W, int K, int levels,
                              int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
                              void* stream) {
+  return wtconv2d_backward_params_typed(x, grad_out, params, FloatGrads(grads, levels).ptr, B, C, H, W, K, levels, dtype,
+                                        param_dtype, workspace, workspace_bytes, stream);
+}
+
+int wtconv2d_backward_params_typed(const void* x, const void* grad_out, const wtconv_params* params,
+                                   const wtconv_typed_grads* grads, int B, int C, int H, int W, int K, int levels,
+                                   int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
   return backward_params2d("wtconv2d_backward_params", x, grad_out, params, grads, B, C, H, W, K, levels, dtype,
                            param_dtype, workspace, workspace_bytes, stream, false);
 }
@@ -579,6 +610,13 @@ int wtconv2d_backward_params(const void* x, const void* grad_out, const wtconv_p
 int wtconv2d_backward(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
                       const wtconv_param_grads* grads, int B, int C, int H, int W, int K, int levels, int dtype,
                       int param_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  return wtconv2d_backward_typed(x, grad_out, grad_x, params, FloatGrads(grads, levels).ptr, B, C, H, W, K, levels, dtype,
+                                 param_dtype, workspace, workspace_bytes, stream);
+}
+
+int wtconv2d_backward_typed(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
+                            const wtconv_typed_grads* grads, int B, int C, int H, int W, int K, int levels, int dtype,
+                            int param_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   // Planes beyond LDS (both passes in steps): the LL bands of grad_out are built once, in the place where the
   // parameter-gradient pass keeps them, and serve both passes.
   const bool sizes_ok = B > 0 && C > 0 && H > 0 && W > 0 && K >= 1 && K % 2 == 1 && K <= wtconv_max_kernel_size() &&
@@ -619,8 +657,8 @@ int wtconv2d_backward(const void* x, const void* grad_out, void* grad_x, const w
   if (int e = wtconv2d_backward_input(grad_out, grad_x, params, B, C, H, W, K, levels, dtype, param_dtype, workspace,
                                       workspace_bytes, stream))
     return e;
-  return wtconv2d_backward_params(x, grad_out, params, grads, B, C, H, W, K, levels, dtype, param_dtype, workspace,
-                                  workspace_bytes, stream);
+  return wtconv2d_backward_params_typed(x, grad_out, params, grads, B, C, H, W, K, levels, dtype, param_dtype, workspace,
+                                        workspace_bytes, stream);
 }
 
 size_t wtconv1d_workspace_bytes(int B, int C, int N, int K, int levels, int pass) {
@@ -664,12 +702,21 @@ int wtconv1d_backward_input(const void* grad_out, void* grad_x, const wtconv_par
 int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_params* params,
                              const wtconv_param_grads* grads, int B, int C, int N, int K, int levels,
                              int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
-                             void* stream_) {
+                             void* stream) {
+  return wtconv1d_backward_params_typed(x, grad_out, params, FloatGrads(grads, levels).ptr, B, C, N, K, levels, dtype,
+                                        param_dtype, workspace, workspace_bytes, stream);
+}
+
+int wtconv1d_backward_params_typed(const void* x, const void* grad_out, const wtconv_params* params,
+                                   const wtconv_typed_grads* grads, int B, int C, int N, int K, int levels,
+                                   int dtype, int param_dtype, void* workspace, size_t workspace_bytes,
+                                   void* stream_) {
   const char* fn = "wtconv1d_backward_params";
   const int L = levels;
   if (int e = check_common(fn, params, B, C, K, L, dtype, param_dtype)) return e;
   if (N <= 0) return fail(WTCONV_E_ARG, "%s: length must be positive (got %d)", fn, N);
   if (x == nullptr || grad_out == nullptr || grads == nullptr) return fail(WTCONV_E_ARG, "%s: null tensor pointer", fn);
+  if (int e = check_grad_dtype(fn, grads)) return e;
   if (grads->base_weight == nullptr || grads->base_scale == nullptr ||
       (params->base_bias != nullptr && grads->base_bias == nullptr))
     return fail(WTCONV_E_ARG, "%s: null gradient pointer", fn);
@@ -700,11 +747,7 @@ int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_p
     e = launch_wgrad1d(dtype, L, x, grad_out, partial, pl, B, per_chunk, nchunk, stream);
   }
   if (e) return e;
-  GradTable gt = {};
-  gt.base_weight = grads->base_weight;
-  gt.base_bias = grads->base_bias;
-  gt.base_scale = grads->base_scale;
-  for (int l = 0; l < L; ++l) { gt.wt_weight[l] = grads->wt_weight[l]; gt.wt_scale[l] = grads->wt_scale[l]; }
+  const GradTable gt = to_grad_table(grads, L);
   const int nrec = (1 + 2 * L) * K + 1;
   WT_LAUNCH(wgrad_finish_kernel, dim3(C), dim3(finish_threads(nrec)), static_cast<size_t>(nrec) * sizeof(float),
             stream, partial, nchunk, to_table(params, L), param_dtype, gt, C, 2, L, K, SubRecords{});
@@ -714,6 +757,13 @@ int wtconv1d_backward_params(const void* x, const void* grad_out, const wtconv_p
 int wtconv1d_backward(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
                       const wtconv_param_grads* grads, int B, int C, int N, int K, int levels, int dtype,
                       int param_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+  return wtconv1d_backward_typed(x, grad_out, grad_x, params, FloatGrads(grads, levels).ptr, B, C, N, K, levels, dtype,
+                                 param_dtype, workspace, workspace_bytes, stream);
+}
+
+int wtconv1d_backward_typed(const void* x, const void* grad_out, void* grad_x, const wtconv_params* params,
+                            const wtconv_typed_grads* grads, int B, int C, int N, int K, int levels, int dtype,
+                            int param_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   const char* fn = "wtconv1d_backward";
   // rows that the register-resident kernels take run the whole backward pass as one kernel -- with the lanes, chunks
   // and workspace layout of the separate parameter-gradient pass, so the two share wtconv1d_workspace_bytes
@@ -744,8 +794,8 @@ int wtconv1d_backward(const void* x, const void* grad_out, void* grad_x, const w
   if (int e = wtconv1d_backward_input(grad_out, grad_x, params, B, C, N, K, levels, dtype, param_dtype, workspace,
                                       workspace_bytes, stream))
     return e;
-  return wtconv1d_backward_params(x, grad_out, params, grads, B, C, N, K, levels, dtype, param_dtype, workspace,
-                                  workspace_bytes, stream);
+  return wtconv1d_backward_params_typed(x, grad_out, params, grads, B, C, N, K, levels, dtype, param_dtype, workspace,
+                                        workspace_bytes, stream);
 }
 
 }  // extern "C"

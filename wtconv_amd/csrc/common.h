@@ -210,13 +210,20 @@ struct ParamTable {
   const void* wt_scale[kMaxLevels];
 };
 
+// The parameters' gradients, all of one dtype.
 struct GradTable {
-  float* base_weight;
-  float* base_bias;
-  float* base_scale;
-  float* wt_weight[kMaxLevels];
-  float* wt_scale[kMaxLevels];
+  void* base_weight;
+  void* base_bias;
+  void* base_scale;
+  void* wt_weight[kMaxLevels];
+  void* wt_scale[kMaxLevels];
+  int dtype;
 };
+
+__device__ __forceinline__ void store_grad(void* p, int dtype, int idx, float v) {
+  if (dtype == WTCONV_F32) static_cast<float*>(p)[idx] = v;
+  else static_cast<uint16_t*>(p)[idx] = dtype == WTCONV_F16 ? f32_to_f16_bits(v) : f32_to_bf16(v);
+}
 
 // Value of lane `src` (a constant) of the calling wavefront, as a wave-uniform value (v_readlane_b32: the result lives
 // in an SGPR, so an FMA takes it as its scalar operand).  The host emulation has no lanes to read from: there every

@@ -39,17 +39,17 @@ using torch::autograd::variable_list;
 // The C ABI as function pointers (filled once by bind()).
 struct Abi {
   int (*fwd2)(const void*, void*, const wtconv_params*, int, int, int, int, int, int, int, int, void*, size_t, void*);
-  int (*bwd2)(const void*, const void*, void*, const wtconv_params*, const wtconv_param_grads*, int, int, int, int, int,
+  int (*bwd2)(const void*, const void*, void*, const wtconv_params*, const wtconv_typed_grads*, int, int, int, int, int,
               int, int, int, void*, size_t, void*);
   int (*bwdin2)(const void*, void*, const wtconv_params*, int, int, int, int, int, int, int, int, void*, size_t, void*);
-  int (*bwdpar2)(const void*, const void*, const wtconv_params*, const wtconv_param_grads*, int, int, int, int, int, int,
+  int (*bwdpar2)(const void*, const void*, const wtconv_params*, const wtconv_typed_grads*, int, int, int, int, int, int,
                  int, int, void*, size_t, void*);
   size_t (*ws2)(int, int, int, int, int, int, int);
   int (*fwd1)(const void*, void*, const wtconv_params*, int, int, int, int, int, int, int, void*, size_t, void*);
-  int (*bwd1)(const void*, const void*, void*, const wtconv_params*, const wtconv_param_grads*, int, int, int, int, int,
+  int (*bwd1)(const void*, const void*, void*, const wtconv_params*, const wtconv_typed_grads*, int, int, int, int, int,
               int, int, void*, size_t, void*);
   int (*bwdin1)(const void*, void*, const wtconv_params*, int, int, int, int, int, int, int, void*, size_t, void*);
-  int (*bwdpar1)(const void*, const void*, const wtconv_params*, const wtconv_param_grads*, int, int, int, int, int, int,
+  int (*bwdpar1)(const void*, const void*, const wtconv_params*, const wtconv_typed_grads*, int, int, int, int, int, int,
                  int, void*, size_t, void*);
   size_t (*ws1)(int, int, int, int, int, int);
   const char* (*last_error)();
@@ -227,25 +227,26 @@ struct WTConvNode : public torch::autograd::Node {
     const int dt = dtype_code(x.scalar_type()), pdt = dtype_code(lp.t[0].scalar_type());
     Tensor grad_x;
     if (need_x) grad_x = at::empty(x.sizes(), x.options().requires_grad(false));
-    // parameter gradients are written as fp32 into one flat buffer (one allocation for the 3 + 2 L tensors): fp32
-    // parameters get parts of it in their own shapes, others parts of one cast of it
-    const bool f32 = lp.t[0].scalar_type() == at::kFloat;
+    // parameter gradients are written, in the parameters' type, into one flat buffer (one allocation for the 3 + 2 L
+    // tensors), of which each parameter gets its part
     int64_t pos[kMaxTensors], total = 0;
     Tensor flat;
-    wtconv_param_grads gt = {};
+    wtconv_typed_grads gt = {};
+    gt.dtype = pdt;
     if (need_params) {
       for (int i = 0; i < n; ++i) {
         pos[i] = total;
         if (lp.t[i].defined()) total += lp.t[i].numel();
       }
-      flat = at::empty({total}, x.options().dtype(at::kFloat).requires_grad(false));
-      float* f = flat.mutable_data_ptr<float>();
-      gt.base_weight = f + pos[0];
-      gt.base_bias = lp.t[1].defined() ? f + pos[1] : nullptr;
-      gt.base_scale = f + pos[2];
+      flat = at::empty({total}, x.options().dtype(lp.t[0].scalar_type()).requires_grad(false));
+      char* f = static_cast<char*>(flat.mutable_data_ptr());
+      const size_t size = flat.element_size();
+      gt.base_weight = f + pos[0] * size;
+      gt.base_bias = lp.t[1].defined() ? f + pos[1] * size : nullptr;
+      gt.base_scale = f + pos[2] * size;
       for (int l = 0; l < L; ++l) {
-        gt.wt_weight[l] = f + pos[3 + l];
-        gt.wt_scale[l] = f + pos[3 + L + l];
+        gt.wt_weight[l] = f + pos[3 + l] * size;
+        gt.wt_scale[l] = f + pos[3 + L + l] * size;
       }
     }
     const void *xp = x.const_data_ptr(), *gp = g.const_data_ptr();
@@ -263,9 +264,8 @@ struct WTConvNode : public torch::autograd::Node {
     if (rc) fail(rc, "wtconv backward");
     res[0] = std::move(grad_x);
     if (need_params) {
-      const Tensor src = f32 ? flat : flat.to(lp.t[0].scalar_type());
       for (int i = 0; i < n; ++i)
-        if (lp.t[i].defined() && task_should_compute_output(1 + i)) res[1 + i] = part_of(src, pos[i], lp.t[i].sizes());
+        if (lp.t[i].defined() && task_should_compute_output(1 + i)) res[1 + i] = part_of(flat, pos[i], lp.t[i].sizes());
     }
     if (twice) refuse_second_derivatives(res, "the WTConv layer");
     return res;

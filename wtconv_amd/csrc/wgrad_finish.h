@@ -13,7 +13,9 @@ namespace wt {
 // for one channel, by the threads of one workgroup: one thread per (filter, tap) plus one for sumG where the
 // workgroup has that many (else strided); the per-filter dot products go through `prod` (NF*KK + 1 floats of
 // LDS).  S = 4 (2-D) or 2 (1-D).  blockDim.x >= NF.  The chunks are summed in index order whichever workgroup
-// runs this, so the result does not depend on the order in which the first stage finished.  SHARED: called by the
+// runs this, so the result does not depend on the order in which the first stage finished.  The sums are in float whatever the
+// type of the gradients, which are rounded once, here: a pass of their own for that took 4 us behind the kernels of a 16-bit
+// layer (training step of 7 x 7 x 768 bf16 90.5 -> 85.8 us, of 56 x 56 x 96 205.4 -> 203.2).  SHARED: called by the
 // last workgroup of a first stage that finishes its channels itself: the records of the other workgroups are read
 // with load_shared_f32.
 // Records of a sub-layer that starts `depth` levels down (0: none): its base filter is the LL filter of level `depth`,
@@ -39,10 +41,10 @@ __device__ __forceinline__ void wgrad_finish_channel(const float* __restrict__ p
   auto level_s = [&](int l) { const void* q = p.wt_scale[0];
 #pragma unroll
     for (int i = 1; i < kMaxLevels; ++i) q = l == i ? p.wt_scale[i] : q; return q; };
-  auto grad_w = [&](int l) { float* q = gt.wt_weight[0];
+  auto grad_w = [&](int l) { void* q = gt.wt_weight[0];
 #pragma unroll
     for (int i = 1; i < kMaxLevels; ++i) q = l == i ? gt.wt_weight[i] : q; return q; };
-  auto grad_s = [&](int l) { float* q = gt.wt_scale[0];
+  auto grad_s = [&](int l) { void* q = gt.wt_scale[0];
 #pragma unroll
     for (int i = 1; i < kMaxLevels; ++i) q = l == i ? gt.wt_scale[i] : q; return q; };
   for (int o = threadIdx.x; o <= NF * KK; o += blockDim.x) {      // (the last index is the sumG slot of the records)
@@ -71,8 +73,7 @@ __device__ __forceinline__ void wgrad_finish_channel(const float* __restrict__ p
       sum += SHARED ? load_shared_f32(src) : *src;
     }
     if (tap) {
-      float* dst = f == 0 ? gt.base_weight : grad_w(l);
-      dst[chn * KK + t] = gam * sum;
+      store_grad(f == 0 ? gt.base_weight : grad_w(l), gt.dtype, chn * KK + t, gam * sum);
       prod[o] = wv * sum;
     } else {
       prod[o] = sum;
@@ -87,12 +88,12 @@ __device__ __forceinline__ void wgrad_finish_channel(const float* __restrict__ p
       const float sg = prod[NF * KK];
       if (p.base_bias != nullptr) {
         dot = fmaf(load_param(p.base_bias, pdtype, c), sg, dot);
-        if (gt.base_bias != nullptr) gt.base_bias[c] = load_param(p.base_scale, pdtype, c) * sg;
+        if (gt.base_bias != nullptr) store_grad(gt.base_bias, gt.dtype, c, load_param(p.base_scale, pdtype, c) * sg);
       }
-      gt.base_scale[c] = dot;
+      store_grad(gt.base_scale, gt.dtype, c, dot);
     } else {
       const int l = (o - 1) / S, chn = c * S + (o - 1) % S;
-      grad_s(l)[chn] = dot;
+      store_grad(grad_s(l), gt.dtype, chn, dot);
     }
   }
 }
