@@ -1,0 +1,42 @@
+"""Parameter gradients and results of the vector kernels at the shapes where their plans change: planes of which LDS holds one
+pair of pyramids or two, K = 7 with one and with more planes an iteration."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,K,L,dtype", [
+    ((16, 24, 45, 37), 7, 2, torch.float16),      # three planes an iteration, one workgroup a CU
+    ((5, 7, 40, 39), 7, 4, torch.float32),        # fewer workgroups than compute units: one plane
+    ((33, 16, 11, 13), 7, 2, torch.float32),      # eleven instead of sixteen, so that the last iteration is full
+    ((40, 3, 6, 7), 7, 2, torch.float32),         # as many as the kernel takes
+    ((9, 12, 30, 25), 7, 1, torch.bfloat16),      # one level: two workgroups a CU
+    ((7, 6, 58, 66), 5, 3, torch.float32),        # one pair of pyramids takes more than half of the LDS
+    ((3, 5, 75, 60), 5, 2, torch.float16),
+    ((2, 4, 100, 85), 5, 1, torch.float32),
+    ((4, 10, 33, 41), 5, 3, torch.float32),       # rows a little above a power of two
+    ((3, 10, 35, 33), 5, 4, torch.float16),
+])
+def test_layer_against_fp64(hip_device, shape, K, L, dtype):
+    import wtconv
+    from oracle import wtconv_ref as R
+    torch.manual_seed(K + L)
+    C = shape[1]
+    ref = R.RefWTConv2d(C, C, K, wt_levels=L).double()
+    mod = wtconv.WTConv2d(C, C, kernel_size=K, wt_levels=L).float()
+    mod.load_state_dict({k: v.float() for k, v in ref.state_dict().items()})
+    ref.load_state_dict({k: v.double() for k, v in mod.state_dict().items()})
+    mod = mod.to(hip_device)
+    x, g = torch.randn(shape).to(dtype), torch.randn(shape).to(dtype)
+    out64, dx64, grads64 = R.layer_grads(ref, x.double(), g.double())
+    xd = x.to(hip_device).requires_grad_()
+    out = mod(xd)
+    out.backward(g.to(hip_device))
+    rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
+    # results are rounded to their type once; float sums of up to 1e5 products in float
+    eps = {torch.float32: 2e-6, torch.float16: 4e-4, torch.bfloat16: 3e-3}[dtype]
+    assert rel(out.detach(), out64) < eps and rel(xd.grad, dx64) < eps
+    for n, p in mod.named_parameters():
+        if p.grad is not None:
+            assert rel(p.grad, grads64[n]) < 5e-6, n

@@ -47,12 +47,6 @@ static int check_common(const char* fn, const wtconv_params* params, int B, int 
   return 0;
 }
 
-// Workgroups of the weight-gradient kernel assumed resident when chunking the batch (2 per
-// CU on 256 CUs).  A constant, so that workspace sizes do not depend on the device queried.
-// (K = 7 asks for 256 registers a lane and runs one workgroup a CU, so its chunks take two rounds where one is planned;
-// a plan of its own has not been measured.)
-constexpr int kWgradResident = 512;
-
 static size_t fold_floats(int C, int S, int L, int KK) { return static_cast<size_t>(C) * (1 + S * L) * KK + C; }
 
 // Folded filters as the plane kernel writes them itself (PlaneFold): each channel's table on cache lines of its own.
@@ -153,8 +147,8 @@ static size_t stream_records(int B, int C, int H, int W, int K, int L) {
 static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) {
   if (s.wdepth == L) return 0;
   int bchunk, nchunk;
-  const int d = s.wdepth;
-  wgrad_chunks(B, C, wgrad_planes_per_iter(B, s.h[d], s.w[d], K, L - d), kWgradResident, &bchunk, &nchunk);
+  const int d = s.wdepth, pb = wgrad_planes_per_iter(B, C, s.h[d], s.w[d], K, L - d);
+  wgrad_chunks(B, C, pb, wgrad_resident(pb, s.h[d], s.w[d], K, L - d), &bchunk, &nchunk);
   return round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * (L - d)) * K * K + 1));
 }
 
@@ -422,7 +416,8 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
     const Mfma2dWgradQuery mq = mfma2d_wgrad_query(B, C, H, W, K, levels, WTCONV_BF16);
     const size_t mfloats = mq.ok ? mq.ws_bytes / sizeof(float) : 0;
     if (wgrad_fits_lds(B, C, H, W, K, levels)) {
-      wgrad_chunks(B, C, wgrad_planes_per_iter(B, H, W, K, levels), kWgradResident, &bchunk, &nchunk);
+      const int pb = wgrad_planes_per_iter(B, C, H, W, K, levels);
+      wgrad_chunks(B, C, pb, wgrad_resident(pb, H, W, K, levels), &bchunk, &nchunk);
       floats = static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1);
     } else {      // partial sums, then the LL bands of x and of grad_out
       const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
@@ -546,10 +541,10 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
     nchunk = mq.nchunk;
     e = mfma2d_wgrad_pass(fn, x, grad_out, partial, B, C, H, W, K, L, fin, stream);
   } else if (resident) {
-    const int pb = wgrad_planes_per_iter(B, H, W, K, L);
+    const int pb = wgrad_planes_per_iter(B, C, H, W, K, L);
     Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, pb);
     finish_wgrad_plan(&pl, K);
-    wgrad_chunks(B, C, pb, kWgradResident, &bchunk, &nchunk);
+    wgrad_chunks(B, C, pb, wgrad_resident(pb, H, W, K, L), &bchunk, &nchunk);
     e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream);
   } else {
     const Stream2D sp = make_stream2d(B, C, H, W, K, L);
@@ -564,11 +559,11 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
       const void* xd = d == 0 ? x : static_cast<const void*>(xll + sp.ll[d]);
       const void* gd = d == 0 ? grad_out : static_cast<const void*>(gll + sp.ll[d]);
       if (d == D && d < L) {       // the rest fits LDS
-        const int Ls = L - d, pb = wgrad_planes_per_iter(B, sp.h[d], sp.w[d], K, Ls);
+        const int Ls = L - d, pb = wgrad_planes_per_iter(B, C, sp.h[d], sp.w[d], K, Ls);
         Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, pb);
         finish_wgrad_plan(&pl, K);
         int sub_chunk;
-        wgrad_chunks(B, C, pb, kWgradResident, &sub_chunk, &sub.nchunk);
+        wgrad_chunks(B, C, pb, wgrad_resident(pb, sp.h[d], sp.w[d], K, Ls), &sub_chunk, &sub.nchunk);
         sub.partial = sub_partial;
         sub.depth = d;
         e = launch_wgrad2d(WTCONV_F32, K, Ls, xd, gd, sub_partial, pl, B, sub_chunk, sub.nchunk, FinishArgs{}, stream);
