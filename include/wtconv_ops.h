@@ -39,6 +39,14 @@ int wtconv1d_backward_typed(const void* x, const void* grad_out, void* grad_x, c
                             const wtconv_typed_grads* grads, int B, int C, int N, int K, int levels, int dtype,
                             int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
+/* wtconv_channel_norm_backward and wtconv_block_residual_backward likewise. */
+int wtconv_channel_norm_backward_typed(const void* x, const void* dy, const void* weight, void* dx, void* dweight, void* dbias,
+                                       int grad_dtype, int B, int C, int HW, float eps, int dtype, int param_dtype,
+                                       int dy_nhwc, void* workspace, size_t workspace_bytes, void* stream);
+int wtconv_block_residual_backward_typed(const void* dout, const void* y, const void* gamma, void* dy, void* dgamma,
+                                         int grad_dtype, int B, int C, int HW, int dtype, int param_dtype, void* workspace,
+                                         size_t workspace_bytes, void* stream);
+
 /* ---- the convolutions that change resolution, with the LayerNorm beside them, for inference in bfloat16:
  *   stem != 0:  out = LayerNorm_c(conv 4x4 stride 4 (x) + bias), norm parameters of `cout` values;
  *   stem == 0:  out = conv 2x2 stride 2 (LayerNorm_c(x)) + bias, norm parameters of `C` values

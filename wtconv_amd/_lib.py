@@ -85,6 +85,8 @@ OPS_EXPORTS = {
     "wtconv2d_backward_typed": (_i, [_p, _p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 8 + [_p, _z, _p]),
     "wtconv1d_backward_params_typed": (_i, [_p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 7 + [_p, _z, _p]),
     "wtconv1d_backward_typed": (_i, [_p, _p, _p, ctypes.POINTER(Params), ctypes.POINTER(TypedGrads)] + [_i] * 7 + [_p, _z, _p]),
+    "wtconv_channel_norm_backward_typed": (_i, [_p] * 6 + [_i] * 4 + [_f] + [_i] * 3 + [_p, _z, _p]),
+    "wtconv_block_residual_backward_typed": (_i, [_p] * 5 + [_i] * 6 + [_p, _z, _p]),
     "wtconv_mlp_supported": (_i, [_ll, _i, _i]),
     "wtconv_mlp_forward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _ll] + [_i] * 4 + [_p]),
     "wtconv_mlp_backward_workspace_bytes": (_z, [_ll, _i, _i, _i]),

@@ -133,12 +133,26 @@ def mlp_fn(x, mlp):
     return ext.mlp(x, *args)
 
 
+def _native(name, *args):
+    """The function of the C++ binding: None where it is not built, does not take the arguments, or they are of a subclass."""
+    ext = _ext.get()
+    if ext is None:
+        return None
+    for t in args:
+        if isinstance(t, torch.Tensor) and type(t) not in _PLAIN:
+            return None
+    return getattr(ext, name)(*args)
+
+
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
 def channel_norm(x, weight, bias, eps, nhwc):
-    """LayerNorm over the channels of x (B, C, H, W); returns (B, H, W, C) if `nhwc` else (B, C, H, W)."""
+    """LayerNorm over the channels of x (B, C, H, W); returns (B, H, W, C) if `nhwc` else (B, C, H, W).  Not recorded."""
+    out = _native("channel_norm", x, weight, bias, eps, nhwc) if not records(x, weight, bias) else None
+    if out is not None:
+        return out
     lib = _lib.load()
     B, C, H, W = x.shape
     with torch.cuda.device(x.device):
@@ -151,7 +165,10 @@ def channel_norm(x, weight, bias, eps, nhwc):
 
 
 def block_residual(y, shortcut, gamma):
-    """shortcut (B, C, H, W) + gamma[c] * y, with y (B, H, W, C); gamma may be None.  Returns (B, C, H, W)."""
+    """shortcut (B, C, H, W) + gamma[c] * y, with y (B, H, W, C); gamma may be None.  Returns (B, C, H, W).  Not recorded."""
+    out = _native("block_residual", y, shortcut, gamma) if not records(y, shortcut, gamma) else None
+    if out is not None:
+        return out
     lib = _lib.load()
     B, C, H, W = shortcut.shape
     if tuple(y.shape) != (B, H, W, C) or y.dtype != shortcut.dtype or not y.is_contiguous():
@@ -242,9 +259,11 @@ class _BlockResidualFn(torch.autograd.Function):
 
 def channel_norm_fn(x, weight, bias, eps, nhwc):
     """channel_norm that autograd can differentiate (gradients of x, weight and bias from the backward kernel)."""
-    return _ChannelNormFn.apply(x, weight, bias, eps, nhwc)
+    out = _native("channel_norm", x, weight, bias, eps, nhwc)
+    return out if out is not None else _ChannelNormFn.apply(x, weight, bias, eps, nhwc)
 
 
 def block_residual_fn(y, shortcut, gamma):
     """block_residual (with a layer scale) that autograd can differentiate (gradients of y, shortcut and gamma)."""
-    return _BlockResidualFn.apply(y, shortcut, gamma)
+    out = _native("block_residual", y, shortcut, gamma)
+    return out if out is not None else _BlockResidualFn.apply(y, shortcut, gamma)

@@ -6,6 +6,7 @@
 
 #include "common.h"
 #include "host_util.h"
+#include "../../include/wtconv_ops.h"
 #include "kernels_block.h"
 
 namespace wt {
@@ -280,27 +281,38 @@ static unsigned* sum_tickets(float* partial, size_t rec_floats, int C) {
   return reinterpret_cast<unsigned*>(partial + rec_floats + static_cast<size_t>(kSumSlices) * 2 * C);
 }
 
-static int launch_column_sum_sliced(float* partial, size_t rec_floats, int C, int nrec, int ncol, float* out0,
-                                    float* out1, int split, hipStream_t stream) {
+static int launch_column_sum_sliced(float* partial, size_t rec_floats, int C, int nrec, int ncol, void* out0,
+                                    void* out1, int split, int out_dtype, hipStream_t stream) {
   int ns = nrec / 16;                          // at least 16 records per slice
   if (ns > kSumSlices) ns = kSumSlices;
   if (ns < 1) ns = 1;
   WT_LAUNCH(column_sum_sliced_kernel, dim3((ncol + 63) / 64, ns), dim3(kBlockThreads), 0, stream, partial, nrec, ncol,
-            partial + rec_floats, sum_tickets(partial, rec_floats, C), out0, out1, split);
+            partial + rec_floats, sum_tickets(partial, rec_floats, C), out0, out1, split, out_dtype);
   return check_launch("column_sum_sliced_kernel");
 }
 
-static int launch_column_sum(const float* partial, int nrec, int ncol, float* out0, float* out1, int split,
-                             hipStream_t stream) {
+static int launch_column_sum(const float* partial, int nrec, int ncol, void* out0, void* out1, int split,
+                             int out_dtype, hipStream_t stream) {
   WT_LAUNCH(column_sum_kernel, dim3((ncol + 63) / 64), dim3(kBlockThreads), 0, stream, partial, nrec, ncol, out0, out1,
-            split);
+            split, out_dtype);
   return check_launch("column_sum_kernel");
 }
 
 extern "C" int wtconv_channel_norm_backward(const void* x, const void* dy, const void* weight, void* dx, float* dweight,
                                             float* dbias, int B, int C, int HW, float eps, int dtype, int param_dtype,
-                                            int dy_nhwc, void* workspace, size_t workspace_bytes, void* stream_) {
+                                            int dy_nhwc, void* workspace, size_t workspace_bytes, void* stream) {
+  return wtconv_channel_norm_backward_typed(x, dy, weight, dx, dweight, dbias, WTCONV_F32, B, C, HW, eps, dtype, param_dtype,
+                                            dy_nhwc, workspace, workspace_bytes, stream);
+}
+
+static bool known_grad_dtype(int d) { return d == WTCONV_F32 || d == WTCONV_BF16 || d == WTCONV_F16; }
+
+extern "C" int wtconv_channel_norm_backward_typed(const void* x, const void* dy, const void* weight, void* dx, void* dweight,
+                                                  void* dbias, int grad_dtype, int B, int C, int HW, float eps, int dtype,
+                                                  int param_dtype, int dy_nhwc, void* workspace, size_t workspace_bytes,
+                                                  void* stream_) {
   const char* fn = "wtconv_channel_norm_backward";
+  if (!known_grad_dtype(grad_dtype)) return fail(WTCONV_E_ARG, "%s: unknown gradient dtype %d", fn, grad_dtype);
   const TileVal* tv = nullptr;
   if (int e = check_block_args(fn, B, C, HW, dtype, param_dtype, &tv, false, 2)) return e;
   if (x == nullptr || dy == nullptr || weight == nullptr || dx == nullptr || dweight == nullptr || dbias == nullptr)
@@ -340,7 +352,7 @@ extern "C" int wtconv_channel_norm_backward(const void* x, const void* dy, const
       };
       const int e = dtype == WTCONV_F32 ? by_layout(static_cast<float*>(nullptr)) : by_layout(static_cast<bf16_t*>(nullptr));
       if (e) return e;
-      return launch_column_sum_sliced(partial, rec_floats, C, B * nv.t.tiles, 2 * C, dweight, dbias, C, stream);
+      return launch_column_sum_sliced(partial, rec_floats, C, B * nv.t.tiles, 2 * C, dweight, dbias, C, grad_dtype, stream);
     }
   }
   auto launch = [&](auto kern, auto* tag) {
@@ -358,13 +370,21 @@ extern "C" int wtconv_channel_norm_backward(const void* x, const void* dy, const
     e = vec ? launch(channel_norm_bwd_kernel<bf16_t, true>, static_cast<bf16_t*>(nullptr))
             : launch(channel_norm_bwd_kernel<bf16_t, false>, static_cast<bf16_t*>(nullptr));
   if (e) return e;
-  return launch_column_sum(partial, B * tv->t.tiles, 2 * C, dweight, dbias, C, stream);
+  return launch_column_sum(partial, B * tv->t.tiles, 2 * C, dweight, dbias, C, grad_dtype, stream);
 }
 
 extern "C" int wtconv_block_residual_backward(const void* dout, const void* y, const void* gamma, void* dy, float* dgamma,
                                               int B, int C, int HW, int dtype, int param_dtype, void* workspace,
-                                              size_t workspace_bytes, void* stream_) {
+                                              size_t workspace_bytes, void* stream) {
+  return wtconv_block_residual_backward_typed(dout, y, gamma, dy, dgamma, WTCONV_F32, B, C, HW, dtype, param_dtype, workspace,
+                                              workspace_bytes, stream);
+}
+
+extern "C" int wtconv_block_residual_backward_typed(const void* dout, const void* y, const void* gamma, void* dy, void* dgamma,
+                                                    int grad_dtype, int B, int C, int HW, int dtype, int param_dtype,
+                                                    void* workspace, size_t workspace_bytes, void* stream_) {
   const char* fn = "wtconv_block_residual_backward";
+  if (!known_grad_dtype(grad_dtype)) return fail(WTCONV_E_ARG, "%s: unknown gradient dtype %d", fn, grad_dtype);
   const TileVal* tv = nullptr;
   if (int e = check_block_args(fn, B, C, HW, dtype, param_dtype, &tv, false, 2)) return e;
   if (dout == nullptr || y == nullptr || gamma == nullptr || dy == nullptr || dgamma == nullptr)
@@ -399,7 +419,7 @@ extern "C" int wtconv_block_residual_backward(const void* dout, const void* y, c
       };
       const int e = dtype == WTCONV_F32 ? by_rows(static_cast<float*>(nullptr)) : by_rows(static_cast<bf16_t*>(nullptr));
       if (e) return e;
-      return launch_column_sum_sliced(partial, rec_floats, C, B * nv.t.tiles, C, dgamma, dgamma, C, stream);
+      return launch_column_sum_sliced(partial, rec_floats, C, B * nv.t.tiles, C, dgamma, dgamma, C, grad_dtype, stream);
     }
   }
   auto launch = [&](auto kern, auto* tag) {
@@ -417,5 +437,5 @@ extern "C" int wtconv_block_residual_backward(const void* dout, const void* y, c
     e = vec ? launch(block_residual_bwd_kernel<bf16_t, true>, static_cast<bf16_t*>(nullptr))
             : launch(block_residual_bwd_kernel<bf16_t, false>, static_cast<bf16_t*>(nullptr));
   if (e) return e;
-  return launch_column_sum(partial, B * tv->t.tiles, C, dgamma, dgamma, C, stream);
+  return launch_column_sum(partial, B * tv->t.tiles, C, dgamma, dgamma, C, grad_dtype, stream);
 }

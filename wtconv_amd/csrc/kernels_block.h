@@ -1089,8 +1089,8 @@ block_residual_bwd_reg_kernel(const T* __restrict__ dout, const T* __restrict__ 
 // out[v] = sum over the `nrec` records of partial[r][v], v < ncol, added in record order (grid = ceil(ncol / 64)
 // workgroups of 256 threads: four row groups per column, joined through LDS in a fixed order).
 __global__ void __launch_bounds__(kBlockThreads) column_sum_kernel(const float* __restrict__ partial, int nrec, int ncol,
-                                                                   float* __restrict__ out0, float* __restrict__ out1,
-                                                                   int split) {
+                                                                   void* __restrict__ out0, void* __restrict__ out1,
+                                                                   int split, int out_dtype) {
   __shared__ float red[kBlockThreads];
   const int col = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;
   float s = 0.f;
@@ -1104,8 +1104,8 @@ __global__ void __launch_bounds__(kBlockThreads) column_sum_kernel(const float* 
   __syncthreads();
   if (grp == 0 && col < ncol) {
     const float v = (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]);
-    if (col < split) out0[col] = v;
-    else out1[col - split] = v;
+    if (col < split) store_grad(out0, out_dtype, col, v);
+    else store_grad(out1, out_dtype, col - split, v);
   }
 }
 
@@ -1115,7 +1115,8 @@ __global__ void __launch_bounds__(kBlockThreads) column_sum_kernel(const float* 
 // one zeroed word per column block (left zero again).
 __global__ void __launch_bounds__(kBlockThreads)
 column_sum_sliced_kernel(const float* __restrict__ partial, int nrec, int ncol, float* __restrict__ slices,
-                         unsigned* __restrict__ tickets, float* __restrict__ out0, float* __restrict__ out1, int split) {
+                         unsigned* __restrict__ tickets, void* __restrict__ out0, void* __restrict__ out1, int split,
+                         int out_dtype) {
   __shared__ float red[kBlockThreads];
   __shared__ unsigned flag;
   const int col = blockIdx.x * 64 + (threadIdx.x & 63), grp = threadIdx.x >> 6;
@@ -1145,8 +1146,8 @@ column_sum_sliced_kernel(const float* __restrict__ partial, int nrec, int ncol, 
 #pragma unroll
         for (int u = 0; u < 8; ++u) v += w[u];
       }
-      if (col < split) out0[col] = v;
-      else out1[col - split] = v;
+      if (col < split) store_grad(out0, out_dtype, col, v);
+      else store_grad(out1, out_dtype, col - split, v);
     }
     if (threadIdx.x == 0) tickets[blockIdx.x] = 0u;
   }

@@ -70,6 +70,12 @@ struct Abi {
   size_t (*mlpt_ws)(long long, int, int, int);
   int (*mlpt_bwd)(const void*, const void*, const void*, const void*, const wtconv_mlp_params*, void*, const wtconv_mlp_grads*,
                   long long, int, int, int, int, void*, size_t, void*);
+  int (*norm)(const void*, void*, const void*, const void*, int, int, int, float, int, int, int, void*);
+  int (*residual)(const void*, const void*, const void*, void*, int, int, int, int, int, void*);
+  size_t (*block_ws)(int, int, int, int);
+  int (*norm_bwd)(const void*, const void*, const void*, void*, void*, void*, int, int, int, int, float, int, int, int, void*,
+                  size_t, void*);
+  int (*residual_bwd)(const void*, const void*, const void*, void*, void*, int, int, int, int, int, int, void*, size_t, void*);
   bool bound = false;
 } abi;
 
@@ -78,7 +84,7 @@ void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 25, "bind: expected 25 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 30, "bind: expected 30 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
@@ -86,6 +92,7 @@ void bind(const std::vector<uintptr_t>& a) {
   take(abi.mlp_ok, a[15]); take(abi.mlp_ws, a[16]); take(abi.mlp, a[17]);
   take(abi.patch_ok, a[18]); take(abi.patch_ws, a[19]); take(abi.patch, a[20]);
   take(abi.mlpt_ok, a[21]); take(abi.mlpt_fwd, a[22]); take(abi.mlpt_ws, a[23]); take(abi.mlpt_bwd, a[24]);
+  take(abi.norm, a[25]); take(abi.residual, a[26]); take(abi.block_ws, a[27]); take(abi.norm_bwd, a[28]); take(abi.residual_bwd, a[29]);
   abi.bound = true;
 }
 
@@ -655,6 +662,185 @@ py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor
   return py::cast(y);
 }
 
+// ---- the two passes a block makes around its WTConv layer: LayerNorm over the channels of x (B, C, H, W), to (B, H, W, C) or
+// (B, C, H, W), and shortcut (B, C, H, W) + gamma * y (B, H, W, C).
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+bool block_dtype(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
+
+c10::DataPtr block_workspace(const Tensor& x, size_t* bytes) {
+  *bytes = abi.block_ws(x.size(0), x.size(1), x.size(2) * x.size(3), dtype_code(x.scalar_type()));
+  TORCH_CHECK(*bytes > 0, "block backward: no tile plan for C=", x.size(1), ", HW=", x.size(2) * x.size(3));
+  return scratch(x, *bytes);
+}
+
+// The upstream gradient as the kernels take it (zeros where there is none).
+Tensor upstream(const Tensor& g, at::IntArrayRef sizes, const at::TensorOptions& opt) {
+  if (!g.defined()) return at::zeros(sizes, opt);
+  const Tensor t = g.scalar_type() == c10::typeMetaToScalarType(opt.dtype()) ? g : g.to(opt.dtype());
+  return t.contiguous();
+}
+
+// Gradients of x, weight and bias: edges 0..2 of the node.
+struct NormNode : public torch::autograd::Node {
+  torch::autograd::SavedVariable x_, weight_;
+  double eps_ = 0;
+  bool nhwc_ = false;
+
+  std::string name() const override { return "WTConvChannelNormBackward"; }
+
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    x_.reset_data();
+    weight_.reset_data();
+  }
+
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const Tensor x = x_.unpack(), weight = weight_.unpack();
+    const bool twice = at::GradMode::is_enabled() &&
+                       ((grads[0].defined() && grads[0].requires_grad()) || x.requires_grad() || weight.requires_grad());
+    const at::NoGradGuard no_grad;
+    const c10::DeviceGuard guard(x.device());
+    const at::TensorOptions opt = x.options().requires_grad(false);
+    const int64_t B = x.size(0), C = x.size(1), H = x.size(2), W = x.size(3);
+    const Tensor g = nhwc_ ? upstream(grads[0], {B, H, W, C}, opt) : upstream(grads[0], {B, C, H, W}, opt);
+    Tensor dx = at::empty(x.sizes(), opt), flat = at::empty({2 * C}, weight.options().requires_grad(false));
+    size_t wsz;
+    const c10::DataPtr ws = block_workspace(x, &wsz);
+    char* f = static_cast<char*>(flat.mutable_data_ptr());
+    const int pdt = dtype_code(weight.scalar_type());
+    const int rc = abi.norm_bwd(x.const_data_ptr(), g.const_data_ptr(), weight.const_data_ptr(), dx.mutable_data_ptr(), f,
+                                f + C * flat.element_size(), pdt, B, C, H * W, static_cast<float>(eps_),
+                                dtype_code(x.scalar_type()), pdt, nhwc_, ws.get(), wsz, stream_of(x));
+    if (rc) fail(rc, "wtconv channel norm backward");
+    variable_list res(3);
+    if (task_should_compute_output(0)) res[0] = std::move(dx);
+    for (int i = 0; i < 2; ++i)
+      if (task_should_compute_output(1 + i)) res[1 + i] = part_of(flat, i * C, weight.sizes());
+    if (twice) refuse_second_derivatives(res, "the channel norm");
+    return res;
+  }
+};
+
+// LayerNorm over the channels; None if the kernels do not take these arguments.
+py::object channel_norm(const Tensor& x, const Tensor& weight, const Tensor& bias, double eps, bool nhwc) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (!x.is_cuda() || x.dim() != 4 || !block_dtype(x.scalar_type()) || !x.is_contiguous() || x.numel() == 0) return py::none();
+  const int64_t B = x.size(0), C = x.size(1), H = x.size(2), W = x.size(3);
+  for (const Tensor* t : {&weight, &bias})
+    if (!canonical(*t, x.device(), weight.scalar_type()) || !block_dtype(t->scalar_type()) || t->numel() != C || t->dim() != 1 ||
+        t->_fw_grad(0).defined())
+      return py::none();
+  if (x._fw_grad(0).defined()) return py::none();
+  const bool record = at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad() || bias.requires_grad());
+  Tensor out;
+  {
+    py::gil_scoped_release nogil;
+    const c10::DeviceGuard guard(x.device());
+    const at::TensorOptions opt = x.options().requires_grad(false);
+    out = nhwc ? at::empty({B, H, W, C}, opt) : at::empty({B, C, H, W}, opt);
+    const int rc = abi.norm(x.const_data_ptr(), out.mutable_data_ptr(), weight.const_data_ptr(), bias.const_data_ptr(), B, C, H * W,
+                            static_cast<float>(eps), dtype_code(x.scalar_type()), dtype_code(weight.scalar_type()), nhwc, stream_of(x));
+    if (rc) fail(rc, "wtconv channel norm");
+    if (record) {
+      const std::shared_ptr<NormNode> node(new NormNode(), torch::autograd::deleteNode);
+      torch::autograd::edge_list next;
+      next.reserve(3);
+      for (const Tensor* t : {&x, &weight, &bias}) next.push_back(torch::autograd::impl::gradient_edge(*t));
+      node->set_next_edges(std::move(next));
+      node->x_ = torch::autograd::SavedVariable(x, false);
+      node->weight_ = torch::autograd::SavedVariable(weight, false);
+      node->eps_ = eps;
+      node->nhwc_ = nhwc;
+      torch::autograd::set_history(out, node);
+    }
+  }
+  return py::cast(out);
+}
+
+// Gradients of y, shortcut and gamma: edges 0..2 of the node.
+struct ResidualNode : public torch::autograd::Node {
+  torch::autograd::SavedVariable y_, gamma_;
+
+  std::string name() const override { return "WTConvBlockResidualBackward"; }
+
+  void release_variables() override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    y_.reset_data();
+    gamma_.reset_data();
+  }
+
+  variable_list apply(variable_list&& grads) override {
+    const std::lock_guard<std::mutex> lock(mutex_);
+    const Tensor y = y_.unpack(), gamma = gamma_.unpack();
+    const bool twice = at::GradMode::is_enabled() &&
+                       ((grads[0].defined() && grads[0].requires_grad()) || y.requires_grad() || gamma.requires_grad());
+    const at::NoGradGuard no_grad;
+    const c10::DeviceGuard guard(y.device());
+    const at::TensorOptions opt = y.options().requires_grad(false);
+    const int64_t B = y.size(0), H = y.size(1), W = y.size(2), C = y.size(3);
+    Tensor g = upstream(grads[0], {B, C, H, W}, opt);
+    variable_list res(3);
+    if (task_should_compute_output(0) || task_should_compute_output(2)) {
+      Tensor dy = at::empty(y.sizes(), opt), dgamma = at::empty(gamma.sizes(), gamma.options().requires_grad(false));
+      size_t wsz;
+      const c10::DataPtr ws = block_workspace(g, &wsz);
+      const int pdt = dtype_code(gamma.scalar_type());
+      const int rc = abi.residual_bwd(g.const_data_ptr(), y.const_data_ptr(), gamma.const_data_ptr(), dy.mutable_data_ptr(),
+                                      dgamma.mutable_data_ptr(), pdt, B, C, H * W, dtype_code(y.scalar_type()), pdt, ws.get(), wsz,
+                                      stream_of(y));
+      if (rc) fail(rc, "wtconv block residual backward");
+      if (task_should_compute_output(0)) res[0] = std::move(dy);
+      if (task_should_compute_output(2)) res[2] = std::move(dgamma);
+    }
+    if (task_should_compute_output(1)) res[1] = std::move(g);
+    if (twice) refuse_second_derivatives(res, "the block's layer scale and shortcut");
+    return res;
+  }
+};
+
+// shortcut + gamma * y; None if the kernels do not take these arguments, or autograd records and there is no gamma.
+py::object block_residual(const Tensor& y, const Tensor& shortcut, const std::optional<Tensor>& gamma) {
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  if (!y.is_cuda() || y.dim() != 4 || shortcut.dim() != 4 || !block_dtype(y.scalar_type()) || y.numel() == 0) return py::none();
+  const int64_t B = y.size(0), H = y.size(1), W = y.size(2), C = y.size(3);
+  if (!y.is_contiguous() || !canonical(shortcut, y.device(), y.scalar_type()) || shortcut.sizes() != at::IntArrayRef({B, C, H, W}))
+    return py::none();
+  if (y._fw_grad(0).defined() || shortcut._fw_grad(0).defined()) return py::none();
+  bool record = at::GradMode::is_enabled(), any = y.requires_grad() || shortcut.requires_grad();
+  if (gamma.has_value()) {
+    if (!canonical(*gamma, y.device(), gamma->scalar_type()) || !block_dtype(gamma->scalar_type()) || gamma->numel() != C ||
+        gamma->_fw_grad(0).defined())
+      return py::none();
+    any = any || gamma->requires_grad();
+  }
+  record = record && any;
+  if (record && !gamma.has_value()) return py::none();
+  Tensor out;
+  {
+    py::gil_scoped_release nogil;
+    const c10::DeviceGuard guard(y.device());
+    out = at::empty(shortcut.sizes(), shortcut.options().requires_grad(false));
+    const int rc = abi.residual(y.const_data_ptr(), shortcut.const_data_ptr(), gamma.has_value() ? gamma->const_data_ptr() : nullptr,
+                                out.mutable_data_ptr(), B, C, H * W, dtype_code(y.scalar_type()),
+                                gamma.has_value() ? dtype_code(gamma->scalar_type()) : WTCONV_F32, stream_of(y));
+    if (rc) fail(rc, "wtconv block residual");
+    if (record) {
+      const std::shared_ptr<ResidualNode> node(new ResidualNode(), torch::autograd::deleteNode);
+      torch::autograd::edge_list next;
+      next.reserve(3);
+      for (const Tensor* t : {&y, &shortcut, &*gamma}) next.push_back(torch::autograd::impl::gradient_edge(*t));
+      node->set_next_edges(std::move(next));
+      node->y_ = torch::autograd::SavedVariable(y, false);
+      node->gamma_ = torch::autograd::SavedVariable(*gamma, false);
+      torch::autograd::set_history(out, node);
+    }
+  }
+  return py::cast(out);
+}
+
 // Stem (convolution, then LayerNorm over the channels) or downsample (LayerNorm, then convolution) in one kernel
 // (inference): None if no kernel takes these arguments or autograd would record the call.
 py::object patch_conv(const Tensor& x, const Tensor& conv_w, const Tensor& conv_b, const Tensor& norm_w, const Tensor& norm_b,
@@ -698,6 +884,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
   m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
   m.def("mlp", &mlp, "a block's MLP with a C++ autograd node; None if not taken");
+  m.def("channel_norm", &channel_norm, "LayerNorm over the channels with a C++ autograd node; None if not taken");
+  m.def("block_residual", &block_residual, "layer scale and shortcut with a C++ autograd node; None if not taken");
   m.def("patch_conv", &patch_conv, "stem or downsample of a WTConvNeXt in one kernel; None if not taken");
   m.def("haar", &haar, "single-level Haar transform with a C++ autograd node, and the check of the bank it is handed");
 }
