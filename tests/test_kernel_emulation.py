@@ -501,3 +501,13 @@ def test_emulated_mlp_training(M, C, hidden):
         # operands, hidden values and results are rounded to bfloat16 (2^-9 relative each)
         w = w.numpy()
         assert np.linalg.norm(a - w) < 6e-3 * np.linalg.norm(w)
+
+
+@pytest.mark.parametrize("B,C,H,W,hidden,layer_scale", [
+    (1, 96, 5, 7, 64, True),        # 35 pixels: a tile and three pixels, pixel by pixel
+    (1, 384, 8, 5, 192, False),     # a tile and eight pixels; hidden units in six steps over four waves
+    (2, 768, 4, 4, 1024, True),     # a tile exactly; eight waves
+])
+def test_emulated_block_mlp_few_pixels(B, C, H, W, hidden, layer_scale):
+    """The two-kernel form of wtconv_block_mlp on the host under the sanitizers."""
+    test_emulated_block_mlp(B, C, H, W, hidden, layer_scale)

@@ -10,7 +10,7 @@ SOURCES = [os.path.join(CSRC, "api.hip"), os.path.join(CSRC, "mfma2d.hip"), os.p
            os.path.join(CSRC, "haar.hip"), os.path.join(CSRC, "mlp.hip"), os.path.join(CSRC, "plane2d.hip"),
            os.path.join(CSRC, "wgrad2d.hip"), os.path.join(CSRC, "stream2d.hip"), os.path.join(CSRC, "conv1d.hip"),
            os.path.join(CSRC, "patch.hip"), os.path.join(CSRC, "mlp_train.hip")]
-HEADERS = [os.path.join(CSRC, f) for f in ("common.h", "host_util.h", "kernels1d.h", "kernels1d_row.h", "kernels2d.h", "kernels2d_mfma.h", "kernels2d_mfma_wgrad.h", "kernels_block.h", "kernels_haar.h", "kernels_mlp.h", "kernels_patch.h", "kernels_product.h", "gelu.h", "matrix.h", "wgrad_finish.h",
+HEADERS = [os.path.join(CSRC, f) for f in ("common.h", "host_util.h", "kernels1d.h", "kernels1d_row.h", "kernels2d.h", "kernels2d_mfma.h", "kernels2d_mfma_wgrad.h", "kernels_block.h", "kernels_haar.h", "kernels_mlp.h", "kernels_mlp_few.h", "kernels_patch.h", "kernels_product.h", "gelu.h", "matrix.h", "wgrad_finish.h",
                                          "kernels2d_stream.h", "launch.h", "mfma2d.h", "plan.h")] + [
     os.path.join(os.path.dirname(PKG_DIR), "include", f) for f in ("wtconv_hip.h", "wtconv_ops.h")]
 
