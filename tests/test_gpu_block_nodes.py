@@ -60,3 +60,14 @@ def test_what_the_nodes_refuse(hip_device):
         gy.sum().backward()
     with torch.autograd.forward_ad.dual_level(), pytest.raises(RuntimeError):      # no tangents, as before
         ops.channel_norm_fn(torch.autograd.forward_ad.make_dual(x.detach(), r(2, 8, 4, 4)), w.requires_grad_(), b, 1e-6, True)
+
+
+def test_upstream_gradient_keeps_its_own_history(hip_device):
+    from wtconv_amd import block_ops as ops
+    r = lambda *s: torch.randn(*s, device=hip_device)
+    y, x, w = r(2, 4, 4, 8), r(2, 8, 4, 4).requires_grad_(), r(8)
+    g = r(2, 8, 4, 4).requires_grad_()
+    gx, = torch.autograd.grad(ops.block_residual_fn(y, x, w), x, g, create_graph=True)
+    assert torch.equal(gx, g) and g.is_leaf and g.grad_fn is None      # the shortcut's gradient is g's values, not g
+    with pytest.raises(RuntimeError, match="not differentiable"):
+        gx.sum().backward()

@@ -174,10 +174,12 @@ Tensor layer_forward(const Tensor& x, const LayerParams& lp, int dims, int K) {
   return out;
 }
 
-// Results that come from raw pointers and carry no graph: a derivative of theirs is refused.
+// Results that come from raw pointers and carry no graph: a derivative of theirs is refused.  (Detached: a result may be the
+// caller's own upstream gradient, passed on, whose history is not ours to write.)
 void refuse_second_derivatives(variable_list& res, const char* what) {
   for (Tensor& t : res)
     if (t.defined()) {
+      t = t.detach();
       auto err = std::make_shared<torch::autograd::Error>(
           std::string("the backward pass of ") + what + " is not differentiable (double backward / create_graph=True through "
           "this layer is not supported)", torch::autograd::edge_list());
