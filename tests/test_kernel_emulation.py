@@ -435,6 +435,10 @@ def test_emulated_block_residual(B, C, H, W, dtype):
     (5, 96, 8, 12, 64, True),      # four tiles: unsplit
     (1, 128, 6, 6, 64, True),      # 4-pixel vectors
     (1, 256, 6, 6, 128, True),     # a pixel tile a wave, eight waves
+    # (up to 320000 / C pixels take the two kernels below: these are the one kernel's)
+    (1, 384, 29, 29, 64, True),    # pixel by pixel, part of a last tile
+    (1, 256, 36, 36, 64, False),   # 8-pixel vectors
+    (1, 96, 58, 58, 128, True),    # 4-pixel vectors, two pixel tiles a wave
 ])
 def test_emulated_block_mlp(B, C, H, W, hidden, layer_scale):
     """wtconv_block_mlp on the host under the sanitizers, against float64 on the same bfloat16 values."""
