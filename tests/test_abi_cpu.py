@@ -4,6 +4,8 @@ device, and the Python modules keep the reference's constructor/state-dict surfa
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -90,6 +92,32 @@ def test_static_scratch_refuses_rows_longer_than_a_workgroup_takes(lib):
     that takes it instead needs more than the static scratch."""
     rc = lib.wtconv2d_forward_static(0x1000, 0x2000, ctypes.byref(_params(1)), 2000, 64, 1, 5000, 1, 1, 0, 0, None)
     assert rc == -2 and "scratch" in lib.wtconv_last_error().decode()
+
+
+def test_size_queries_answer_for_sizes_that_do_not_exist(lib):
+    """0 for extents of zero and below, in every position, and an error code from the calls (in a process of their own: a
+    division by zero would end it)."""
+    code = """
+import itertools
+from wtconv_amd import _lib
+lib = _lib.load()
+for c in (0, -1, -96):
+    assert lib.wtconv_block_mlp_supported(1, c, 196, 64) == 0 and lib.wtconv_block_mlp_workspace_bytes(1, c, 196, 64) == 0
+    p = _lib.MlpParams(*[0x1000] * 7)
+    assert lib.wtconv_block_mlp(0x1000, 0x2000, 0x3000, p, 1, c, 196, 64, 1e-6, 1, 1, 0x4000, 1 << 20, None) < 0
+queries = [(lib.wtconv_block_mlp_supported, (1, 96, 196, 64)), (lib.wtconv_block_mlp_workspace_bytes, (1, 96, 196, 64)),
+           (lib.wtconv_patch_conv_supported, (0, 1, 96, 8, 8, 192)), (lib.wtconv_patch_conv_workspace_bytes, (0, 1, 96, 8, 8, 192)),
+           (lib.wtconv_patch_conv_supported, (1, 1, 3, 16, 16, 96)), (lib.wtconv_patch_conv_workspace_bytes, (1, 1, 3, 16, 16, 96)),
+           (lib.wtconv_mlp_supported, (196, 96, 384)), (lib.wtconv_mlp_backward_workspace_bytes, (196, 96, 384, 7)),
+           (lib.wtconv_block_workspace_bytes, (1, 96, 196, 1))]
+for fn, sizes in queries:
+    first = 1 if fn in (lib.wtconv_patch_conv_supported, lib.wtconv_patch_conv_workspace_bytes) else 0
+    for i, bad in itertools.product(range(first, first + 3), (0, -1, -2 ** 31)):
+        assert fn(*sizes[:i], bad, *sizes[i + 1:]) == 0, (fn.__name__, i, bad)
+print("answered")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT, timeout=300)
+    assert r.returncode == 0 and "answered" in r.stdout, (r.returncode, r.stderr[-2000:])
 
 
 def test_null_parameter_pointer_rejected(lib):

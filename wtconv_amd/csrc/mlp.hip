@@ -95,7 +95,7 @@ int few_tiles(int pixels) { return (pixels + 16 * kFewTiles - 1) / (16 * kFewTil
 size_t few_workspace(int pixels, int hidden) { return sizeof(bf16_t) * 16 * kFewTiles * static_cast<size_t>(few_tiles(pixels)) * hidden; }
 
 bool takes_few(int B, int C, int HW, int hidden) {
-  if (B <= 0 || HW <= 0 || hidden <= 0 || hidden % 64 != 0 || hidden > kMaxHidden) return false;
+  if (B <= 0 || C <= 0 || HW <= 0 || hidden <= 0 || hidden % 64 != 0 || hidden > kMaxHidden) return false;
   // (fewer pixels than a tile: most of every product would be padding)
   const long long pixels = static_cast<long long>(B) * HW;
   if (pixels < 16 * kFewTiles || pixels > kFewPixelChannels / C) return false;
