@@ -511,6 +511,7 @@ def test_emulated_mlp_training(M, C, hidden):
     (1, 96, 5, 7, 64, True),        # 35 pixels: a tile and three pixels, pixel by pixel
     (1, 384, 8, 5, 192, False),     # a tile and eight pixels; hidden units in six steps over four waves
     (2, 768, 4, 4, 1024, True),     # a tile exactly; eight waves
+    (1, 1024, 4, 8, 64, True),      # more than 64 KB of LDS
 ])
 def test_emulated_block_mlp_few_pixels(B, C, H, W, hidden, layer_scale):
     """The two-kernel form of wtconv_block_mlp on the host under the sanitizers."""

@@ -5,6 +5,7 @@
 
 #include <stdarg.h>
 #include <stdio.h>
+#include <stdlib.h>
 
 #include <functional>
 #include <mutex>
@@ -25,10 +26,22 @@ inline int fail(int code, const char* fmt, ...) {
 }
 
 #ifdef WT_EMULATE
-#define WT_LAUNCH(kernel, grid, block, lds_bytes, stream, ...) \
-  ::emu::launch((grid), (block), (lds_bytes), [&]() { kernel(__VA_ARGS__); })
+// (here a launch that the opt-in of allow_lds is missing for ends the process, whatever a runtime lets pass)
+inline std::unordered_map<const void*, size_t> g_lds_allowed;
+inline void need_lds(const void* kernel, const char* name, size_t bytes) {
+  if (bytes <= 64 * 1024 || (g_lds_allowed.count(kernel) && g_lds_allowed[kernel] >= bytes)) return;
+  fprintf(stderr, "%s: %zu bytes of LDS without allow_lds\n", name, bytes);
+  abort();
+}
+#define WT_LAUNCH(kernel, grid, block, lds_bytes, stream, ...)                       \
+  (::wt::need_lds(reinterpret_cast<const void*>(kernel), #kernel, (lds_bytes)), \
+   ::emu::launch((grid), (block), (lds_bytes), [&]() { kernel(__VA_ARGS__); }))
 inline int check_launch(const char*) { return 0; }
-template <typename F> inline int allow_lds(F, size_t) { return 0; }
+template <typename F> inline int allow_lds(F kernel, size_t bytes) {
+  size_t& most = g_lds_allowed[reinterpret_cast<const void*>(kernel)];
+  if (bytes > most) most = bytes;
+  return 0;
+}
 #else
 #define WT_LAUNCH(kernel, grid, block, lds_bytes, stream, ...) \
   hipLaunchKernelGGL(kernel, (grid), (block), (lds_bytes), (stream), __VA_ARGS__)

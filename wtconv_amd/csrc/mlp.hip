@@ -122,8 +122,10 @@ int launch_few(const MlpArgs& m, int C, size_t workspace_bytes, hipStream_t stre
   const int tiles = few_tiles(a.pixels);
 #define WT_CASE(c, ng, kg)                                                                             \
   if (C == c) {                                                                                        \
-    using S = FewShape<c, kFewTiles, ng, kg>;                                                                     \
-    WT_LAUNCH(few_hidden_kernel<S>, dim3(tiles, a.hidden / (16 * ng)), dim3(S::kThreads), S::kLdsBytes, stream, a);                    \
+    using S = FewShape<c, kFewTiles, ng, kg>;                                                          \
+    auto kern = few_hidden_kernel<S>;                                                                  \
+    if (int e = allow_lds(kern, S::kLdsBytes)) return e;                                               \
+    WT_LAUNCH(kern, dim3(tiles, a.hidden / (16 * ng)), dim3(S::kThreads), S::kLdsBytes, stream, a);    \
   }
   WT_FEW_SHAPES(WT_CASE)
 #undef WT_CASE
