@@ -120,6 +120,15 @@ print("answered")
     assert r.returncode == 0 and "answered" in r.stdout, (r.returncode, r.stderr[-2000:])
 
 
+def test_mlp_sizes_beyond_32_bit_indices_are_refused(lib):
+    """Threads of a launch and values of a weight gradient are counted in 32 bits."""
+    ws = lib.wtconv_mlp_backward_workspace_bytes
+    assert ws(64, 65536, 65536, 7) == 0 and lib.wtconv_mlp_supported(64, 65536, 65536) == 0      # 2^31 threads add up the weight gradients
+    assert ws(64, 32768, 65536, 7) > 2 ** 33
+    assert ws(1 << 27, 384, 1536, 7) == 0 and ws(1 << 30, 96, 128, 7) == 0                       # 2^33 threads of a product
+    assert ws(1 << 24, 384, 1536, 7) > 2 ** 35
+
+
 def test_null_parameter_pointer_rejected(lib):
     from wtconv_amd import _lib
     p = _lib.Params()

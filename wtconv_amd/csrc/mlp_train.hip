@@ -51,8 +51,10 @@ int product_to_channels(const ProductArgs& a, hipStream_t stream) {
 
 bool takes(long long M, int C, int hidden) {
   if (M <= 0 || C <= 0 || hidden <= 0 || hidden % 128 != 0 || (C % 96 != 0 && C % 128 != 0)) return false;
-  // pixel indices and the offsets inside a tile are 32-bit
-  return M <= (1 << 30) && hidden <= (1 << 16) && C <= (1 << 16);
+  // 32-bit: pixel indices, the offsets inside a tile, the threads that add up the weight gradients (half as many as they have
+  // values), and the threads of a product (four per 64 values)
+  if (M > (1 << 30) || hidden > (1 << 16) || C > (1 << 16)) return false;
+  return static_cast<long long>(C) * hidden <= (1LL << 31) && M * (C > hidden ? C : hidden) <= (1LL << 35);
 }
 
 struct GradPlan {
