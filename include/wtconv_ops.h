@@ -70,7 +70,9 @@ int wtconv_patch_conv(int stem, const void* x, void* out, const wtconv_patch_par
  * read).  Everything 16-byte aligned.  Sums and GELU in float; each result is rounded to bfloat16 once.
  * The forward call writes act = gelu(h) and, unless h is NULL, h = fc1(x), both (pixels, hidden); the backward call takes
  * them and dy = dL/dy, and writes what is not NULL of dx and the parameters' gradients (a bias gradient only together
- * with its weight's).  `want` says the same to the workspace query.  wtconv_mlp_supported: whether a size has kernels. */
+ * with its weight's).  `want` says the same to the workspace query.  wtconv_mlp_supported: whether a
+ * size has kernels that are faster than a library's products with passes between them; the calls take every size with kernels,
+ * those for which the workspace query is not 0. */
 typedef struct {
   void *fc1_weight, *fc1_bias, *fc2_weight, *fc2_bias;
 } wtconv_mlp_grads;

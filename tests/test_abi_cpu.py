@@ -129,6 +129,20 @@ def test_mlp_sizes_beyond_32_bit_indices_are_refused(lib):
     assert ws(1 << 24, 384, 1536, 7) > 2 ** 35
 
 
+@pytest.mark.parametrize("C,hidden,faster,slower", [
+    (96, 384, (1, 401408), ()), (384, 1536, (1, 200704), ()), (512, 2048, (1, 100352), ()), (1024, 2048, (1, 100352), ()),
+    (768, 3072, (1, 49, 12544, 25088), (50176, 200704)), (1536, 1536, (25088,), (50176,)),
+    (896, 3584, (784, 6272), (12544, 50176)), (768, 4096, (784, 6272), (25088,)),
+    (1024, 4096, (1, 784, 2048), (3136, 6272, 12544, 50176)), (2048, 2048, (1024,), (6272,)),
+    (1536, 6144, (), (784, 12544)), (2048, 8192, (), (1, 200, 12544)), (4096, 4096, (), (200, 12544)),
+])
+def test_mlp_training_kernels_are_offered_where_they_are_faster(lib, C, hidden, faster, slower):
+    """Sizes on both sides of the line (measured as faster or slower than the library's passes); the calls take all of them."""
+    for pixels in faster + slower:
+        assert lib.wtconv_mlp_supported(pixels, C, hidden) == (pixels in faster), pixels
+        assert lib.wtconv_mlp_backward_workspace_bytes(pixels, C, hidden, 7) > 0
+
+
 def test_null_parameter_pointer_rejected(lib):
     from wtconv_amd import _lib
     p = _lib.Params()

@@ -57,6 +57,30 @@ bool takes(long long M, int C, int hidden) {
   return static_cast<long long>(C) * hidden <= (1LL << 31) && M * (C > hidden ? C : hidden) <= (1LL << 35);
 }
 
+// Whether the kernels are the faster way, and not the library's products with passes for biases, GELU and its derivative between
+// them.  What they save grows with the pixels, what they lose with the weights: their tiles reach about half of the rate of
+// the library's on large products.  Measured, time of a forward and backward pass over that of the library's passes (graph
+// replay), by pixels:
+//                             1    49   256  1024  2048  3136  6272 12544 25088 50176
+//   384 -> 1536   (0.6 M)  0.83  0.77        0.55        0.49        0.50        0.58
+//   512 -> 2048   (1.0 M)  1.03  0.94  0.70  0.62  0.56  0.57  0.67  0.64  0.70  0.73
+//  1024 -> 2048   (2.1 M)  1.16        0.72  0.67  0.66  0.79  0.84  0.87  0.88  0.93
+//   768 -> 3072   (2.4 M)  1.12  0.94  0.75  0.68  0.67  0.81  0.82  0.88  0.92  1.05
+//  1536 -> 1536   (2.4 M)  1.02        0.75  0.67  0.70  0.77  0.77  0.77  0.93  1.07
+//   896 -> 3584   (3.2 M)  1.08        0.79  0.79  0.82  0.86  0.85  1.01  1.03  1.11
+//   768 -> 4096   (3.1 M)  1.21        0.83  0.75  0.79  0.93  0.98  0.96  1.03  1.19
+//  1024 -> 4096   (4.2 M)  1.24  1.08  0.85  0.80  0.85  0.98  1.08  1.15  1.14  1.26
+//  1536 -> 6144   (9.4 M)  1.56  1.26  1.00  1.04        1.20        1.51
+//  2048 -> 8192    (17 M)  2.20  1.85  1.32  1.40        1.64        1.76
+// (Fewer pixels than about 48 are a little slower from a million weights on, but for as long as launching the library's eleven
+// passes takes the host three times as long as either takes the device, which a caller without a graph waits for: 79 us
+// against 225 with one pixel of 512 channels.)
+bool pays(long long M, int C, int hidden) {
+  const long long weights = static_cast<long long>(C) * hidden;
+  const long long most = weights <= (2LL << 20) ? 1LL << 30 : weights <= (5LL << 19) ? 1 << 15 : weights <= (13LL << 18) ? 6500 : 2048;
+  return weights <= (4LL << 20) && M <= most;
+}
+
 struct GradPlan {
   int tiles = 0, shares = 0, stages = 0;
   size_t partial = 0, bias = 0;
@@ -138,7 +162,9 @@ bool aligned(std::initializer_list<const void*> ptrs) {
 
 }  // namespace
 
-extern "C" int wtconv_mlp_supported(long long pixels, int C, int hidden) { return takes(pixels, C, hidden) ? 1 : 0; }
+extern "C" int wtconv_mlp_supported(long long pixels, int C, int hidden) {
+  return takes(pixels, C, hidden) && pays(pixels, C, hidden) ? 1 : 0;
+}
 
 extern "C" int wtconv_mlp_forward(const void* x, void* h, void* act, void* y, const wtconv_mlp_params* w, long long pixels,
                                   int C, int hidden, int dtype, int param_dtype, void* stream) {
