@@ -206,7 +206,8 @@ int wtconv_block_residual_backward(const void* dout, const void* y, const void* 
  * GELU, fc1_weight (hidden, C) and fc2_weight (C, hidden) as nn.Linear keeps them.  bfloat16 tensors and parameters, the
  * latter 16-byte aligned; gamma may be NULL.  out may be the shortcut, but not x.  Products, sums, LayerNorm and GELU in
  * float; the normalised values and the hidden activations are rounded to bfloat16 once.
- * wtconv_block_mlp_supported says whether a size has a kernel; the workspace takes partial sums of small batches. */
+ * wtconv_block_mlp_supported says whether a size has a kernel that is faster than the separate passes; the workspace takes
+ * partial sums of small batches, or the hidden values of a few pixels. */
 typedef struct {
   const void *norm_weight, *norm_bias;      /* (C) */
   const void *fc1_weight, *fc1_bias;        /* (hidden, C), (hidden) */

@@ -143,6 +143,26 @@ def test_mlp_training_kernels_are_offered_where_they_are_faster(lib, C, hidden, 
         assert lib.wtconv_mlp_backward_workspace_bytes(pixels, C, hidden, 7) > 0
 
 
+@pytest.mark.parametrize("C,two,one", [
+    (96, ((32, 64), (3332, 384), (1664, 768), (488, 2048)), ((96, 2048), (64, 4096), (560, 2048), (1666, 4096))),
+    (128, ((32, 64), (2340, 256), (256, 512), (1952, 512)), ((64, 512), (2500, 512), (192, 2048), (1120, 1024), (1250, 4096))),
+    (192, ((32, 192), (1664, 768), (312, 4096)), ((833, 4096), (1666, 4096))),
+    (256, ((32, 256), (1250, 1024), (244, 4096)), ((625, 4096),)),
+    (384, ((196, 1536), (832, 1536), (312, 4096)), ((833, 4096), (834, 1536))),
+    (512, ((624, 2048), (312, 4096)), ((625, 4096), (626, 64))), (768, ((49, 3072), (416, 3072)), ((416, 4096),)),
+    (1024, ((49, 4096), (256, 4096), (312, 1024)), ((312, 4096),)),
+])
+def test_few_pixels_take_the_kernels_that_are_faster(lib, C, two, one):
+    """Pixels x hidden units on both sides of the line between the two kernels for few pixels and the one kernel (from 512
+    channels: the separate passes), each side measured.  The two kernels' workspace holds the hidden values of whole tiles."""
+    for pixels, hidden in two + one:
+        hid = 2 * ((pixels + 31) // 32 * 32) * hidden
+        few = lib.wtconv_block_mlp_workspace_bytes(1, C, pixels, hidden) == hid
+        if (pixels, hidden) in two or C < 512:
+            assert few == ((pixels, hidden) in two), (pixels, hidden)
+        assert lib.wtconv_block_mlp_supported(1, C, pixels, hidden) == (C < 512 or (pixels, hidden) in two)
+
+
 def test_null_parameter_pointer_rejected(lib):
     from wtconv_amd import _lib
     p = _lib.Params()

@@ -13,6 +13,8 @@ namespace {
 #define WT_MLP_SHAPES(X) X(96, 2, 4, 3, 32, 3) X(128, 2, 4, 2, 32, 3) X(192, 2, 4, 2, 32, 3) X(256, 1, 8, 2, 32, 3) \
                          X(384, 1, 8, 2, 32, 3)
 
+constexpr int kMaxHidden = 4096;
+
 struct MlpPlan {
   int tiles = 0, splits = 0, padded = 0;
 };
@@ -32,7 +34,6 @@ MlpPlan plan_of(int pixels, int hidden) {
   return p;
 }
 
-constexpr int kMaxHidden = 4096;
 template <typename S> constexpr size_t kRoomBytes = S::HC * sizeof(float);
 
 // Whether LDS has room for one more slice of bias, with as many workgroups a CU as without.
@@ -80,26 +81,43 @@ int launch(MlpArgs a, size_t workspace_bytes, hipStream_t stream) {
   return check_launch(fn);
 }
 
-// ---- few pixels: two kernels (kernels_mlp_few.h), for these channel counts and as many pixels as make them the faster way.
-// Each tile of 32 pixels goes through all weights, 8 C^2 of them, on its own, while the one kernel's time hardly depends on the
-// pixels before its workgroups fill the chip; the lines of equal time lie near a constant pixels * C.  Measured (graph
-// replay), us, two kernels / one kernel with its combination, from 512 channels the separate passes:
-//   96 channels, 3136 pixels 12.4/13.5, 6272 16.0/16.1     128, 3136 17.6/17.5          192, 784 11.2/20.1, 3136 24.3/25.1
-//   256, 784 16.8/23.3, 3136 43/27.6                       384, 196 11.3/22.6, 784 24.3/28.5, 1568 38.4/31.5
-//   512, 196 17.0/29.6, 784 41.1/37.2                      768, 49 15.3/41.0, 392 38.3/52.6      1024, 49 19.9/55.5, 392 66/63
-#define WT_FEW_SHAPES(X) X(96, 2, 1) X(128, 2, 1) X(192, 2, 2) X(256, 2, 2) X(384, 4, 2) X(512, 4, 2) X(768, 4, 2) X(1024, 4, 2)
+// ---- few pixels: two kernels (kernels_mlp_few.h), for these channel counts.  (Behind the shape: few_pays's limits, the hidden
+// units up to which the pixels do not matter, and the most pixels times hidden units.)
+#define WT_FEW_SHAPES(X) X(96, 2, 1, 768, 1280000) X(128, 2, 1, 256, 1280000) X(192, 2, 2, kMaxHidden, 1280000)         \
+                         X(256, 2, 2, kMaxHidden, 1280000) X(384, 4, 2, kMaxHidden, 1280000) X(512, 4, 2, kMaxHidden, 1280000) \
+                         X(768, 4, 2, kMaxHidden, 1280000) X(1024, 4, 2, kMaxHidden, 1 << 20)
 constexpr long long kFewPixelChannels = 320000;
 constexpr int kFewTiles = 2;
 
 int few_tiles(int pixels) { return (pixels + 16 * kFewTiles - 1) / (16 * kFewTiles); }
 size_t few_workspace(int pixels, int hidden) { return sizeof(bf16_t) * 16 * kFewTiles * static_cast<size_t>(few_tiles(pixels)) * hidden; }
 
-bool takes_few(int B, int C, int HW, int hidden) {
+bool has_few(int B, int C, int HW, int hidden) {
   if (B <= 0 || C <= 0 || HW <= 0 || hidden <= 0 || hidden % 64 != 0 || hidden > kMaxHidden) return false;
   // (fewer pixels than a tile: most of every product would be padding)
   const long long pixels = static_cast<long long>(B) * HW;
   if (pixels < 16 * kFewTiles || pixels > kFewPixelChannels / C) return false;
 #define WT_CASE(c, ...) if (C == c) return true;
+  WT_FEW_SHAPES(WT_CASE)
+#undef WT_CASE
+  return false;
+}
+
+// Whether the two kernels are the faster way.  Each tile of 32 pixels goes through all weights on its own, 2 C times the hidden
+// units, while the one kernel's time hardly depends on the pixels before its workgroups fill the chip: the lines of equal time
+// lie near a constant number of pixels * hidden units.  Where the one kernel needs no second launch (few channels), a second
+// launch pays from some hundred pixels on.  Measured (graph replay), us, two kernels / one kernel with its combination, from
+// 512 channels the separate passes, pixels by hidden units:
+//    96   32 x 64 5.9/7.9    3332 x 384 13.0/13.8   1664 x 768 10.1/15.2  | 96 x 2048 10.7/10.1  488 x 2048 10.6/15.4  1666 x 4096 39.9/21.3
+//   128   32 x 64 8.3/8.7    2340 x 256 13.1/15.2   | 64 x 512 9.5/9.0   256 x 512 9.1/9.9   1952 x 512 13.8/19.9   2500 x 512 17.4/16.2   1120 x 1024 16.5/14.6
+//   192   196 x 768 8.0/14.7   1664 x 768 13.3/21.5   312 x 4096 19.4/20.5   833 x 4096 38.4/24.8
+//   256   196 x 1024 11.6/15.7   976 x 1024 18.2/27.6   312 x 4096 23.2/23.1   625 x 4096 38.9/28.7
+//   384   196 x 1536 11.6/22.7   832 x 1536 22.0/28.3   312 x 4096 23.1/28.6   833 x 4096 54.1/36.3
+//   512   196 x 2048 16.9/29.7   624 x 2048 29.6/37.3   768   49 x 3072 15.6/40.7   416 x 3072 36.2/44.2   416 x 4096 47.8/44.2
+//  1024   49 x 4096 20.4/55.8   256 x 4096 36.9/39.8   312 x 4096 49.9/44.6
+bool few_pays(int pixels, int C, int hidden) {
+  const long long work = static_cast<long long>(pixels) * hidden;
+#define WT_CASE(c, ng, kg, any, most) if (C == c) return hidden <= any ? work <= most : pixels >= 224 && work <= (1 << 20);
   WT_FEW_SHAPES(WT_CASE)
 #undef WT_CASE
   return false;
@@ -120,7 +138,7 @@ int launch_few(const MlpArgs& m, int C, size_t workspace_bytes, hipStream_t stre
   const uintptr_t bits = reinterpret_cast<uintptr_t>(a.shortcut) | reinterpret_cast<uintptr_t>(a.out);
   a.vec = a.HW % 4 == 0 && bits % 8 == 0;
   const int tiles = few_tiles(a.pixels);
-#define WT_CASE(c, ng, kg)                                                                             \
+#define WT_CASE(c, ng, kg, ...)                                                                        \
   if (C == c) {                                                                                        \
     using S = FewShape<c, kFewTiles, ng, kg>;                                                          \
     auto kern = few_hidden_kernel<S>;                                                                  \
@@ -155,14 +173,19 @@ bool takes(int B, int C, int HW, int hidden) {
   return false;
 }
 
+// (The calls take every size with a kernel, also one at which the separate passes are faster.)
+bool uses_few(int B, int C, int HW, int hidden) {
+  return has_few(B, C, HW, hidden) && (few_pays(B * HW, C, hidden) || !takes(B, C, HW, hidden));
+}
+
 }  // namespace
 
 extern "C" int wtconv_block_mlp_supported(int B, int C, int HW, int hidden) {
-  return takes_few(B, C, HW, hidden) || takes(B, C, HW, hidden) ? 1 : 0;
+  return (has_few(B, C, HW, hidden) && few_pays(B * HW, C, hidden)) || takes(B, C, HW, hidden) ? 1 : 0;
 }
 
 extern "C" size_t wtconv_block_mlp_workspace_bytes(int B, int C, int HW, int hidden) {
-  if (takes_few(B, C, HW, hidden)) return few_workspace(B * HW, hidden);
+  if (uses_few(B, C, HW, hidden)) return few_workspace(B * HW, hidden);
   if (!takes(B, C, HW, hidden)) return 0;
   MlpPlan p;
 #define WT_CASE(c, ...) if (C == c) p = plan_of<MlpShape<c, __VA_ARGS__>>(B * HW, hidden);
@@ -180,7 +203,7 @@ extern "C" int wtconv_block_mlp(const void* x, const void* shortcut, void* out, 
     return fail(WTCONV_E_ARG, "%s: null parameter", fn);
   if (out == x) return fail(WTCONV_E_ARG, "%s: in-place use is not supported", fn);
   if (dtype != WTCONV_BF16 || param_dtype != WTCONV_BF16) return fail(WTCONV_E_UNSUPPORTED, "%s: bfloat16 only", fn);
-  const bool few = takes_few(B, C, HW, hidden);
+  const bool few = uses_few(B, C, HW, hidden);
   if (!few && !takes(B, C, HW, hidden)) return fail(WTCONV_E_UNSUPPORTED, "%s: no kernel for C=%d, hidden=%d", fn, C, hidden);
   uintptr_t bits = 0;
   for (const void* p : {w->norm_weight, w->norm_bias, w->fc1_weight, w->fc1_bias, w->fc2_weight, w->fc2_bias, w->gamma})
