@@ -52,8 +52,10 @@ int wtconv_block_residual_backward_typed(const void* dout, const void* y, const 
  *   stem == 0:  out = conv 2x2 stride 2 (LayerNorm_c(x)) + bias, norm parameters of `C` values
  * (wtconvnext/wtconvnext.py:170-181, :294-297 of the reference).  x (B, C, H, W), out (B, cout, H / P, W / P), conv_weight
  * (cout, C, P, P); everything 16-byte aligned.  Sums and LayerNorm in float; normalised values are rounded to bfloat16
- * once, as are the results.  wtconv_patch_conv_supported says whether a size has a kernel; the workspace (16-byte aligned)
- * takes the weights in the order of the products. */
+ * once, as are the results.  wtconv_patch_conv_supported says whether a size has a kernel that is faster than a library's
+ * convolution with passes around it (the call takes every size with a kernel: cout in multiples of 32 for C of 96, 128, 192, 256,
+ * 384 and 512, cout of 96 or 128 for a stem of up to 4 channels whose rows are multiples of 16); the workspace (16-byte aligned) takes
+ * the weights in the order of the products. */
 typedef struct {
   const void *conv_weight, *conv_bias;
   const void *norm_weight, *norm_bias;

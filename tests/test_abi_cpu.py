@@ -163,6 +163,20 @@ def test_few_pixels_take_the_kernels_that_are_faster(lib, C, two, one):
         assert lib.wtconv_block_mlp_supported(1, C, pixels, hidden) == (C < 512 or (pixels, hidden) in two)
 
 
+@pytest.mark.parametrize("C,cout,faster,slower", [
+    (96, 192, (1, 512), ()), (384, 768, (1, 64, 2048), ()), (512, 1024, (1, 64, 2048), ()), (512, 6144, (64, 512), ()),
+    (96, 480, (1, 64, 512), (2048,)), (96, 992, (1, 64), (170, 512)), (128, 480, (170, 512), (2048,)),
+    (192, 224, (64, 512, 2048), ()), (192, 480, (64,), (170, 512)), (256, 224, (512, 2048), ()), (256, 736, (), (64, 170)),
+    (384, 224, (64, 170, 512), (2048,)), (384, 416, (16,), (64, 170)), (512, 224, (170, 512), (2048,)), (512, 544, (1, 16), (64, 256)),
+    (256, 3200, (64, 512), ()), (384, 640, (64, 512), ()), (384, 2048, (16, 32), (64, 256)), (512, 640, (64, 512), (2048,)),
+    (512, 896, (64, 170), (256, 2048)), (512, 1152, (32, 100), (256,)),
+])
+def test_downsample_kernels_are_offered_where_they_are_faster(lib, C, cout, faster, slower):
+    """Images of 14 x 14 on both sides of the lines for output channels that the many-pixel split does not divide."""
+    for images in faster + slower:
+        assert lib.wtconv_patch_conv_supported(0, images, C, 14, 14, cout) == (images in faster), images
+
+
 def test_null_parameter_pointer_rejected(lib):
     from wtconv_amd import _lib
     p = _lib.Params()
