@@ -71,3 +71,47 @@ def test_upstream_gradient_keeps_its_own_history(hip_device):
     assert torch.equal(gx, g) and g.is_leaf and g.grad_fn is None      # the shortcut's gradient is g's values, not g
     with pytest.raises(RuntimeError, match="not differentiable"):
         gx.sum().backward()
+
+
+def _spread(t):
+    return torch.stack([t, torch.full_like(t, float("nan"))], -1)[..., 0] if t.is_floating_point() else t
+
+
+def _shifted(t):
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    flat[1:] = t.reshape(-1)
+    return flat[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("back", [_spread, _shifted])
+@pytest.mark.parametrize("which", ["layer", "norm", "mlp", "residual"])
+def test_saved_tensors_may_come_back_otherwise(hip_device, which, back):
+    """Hooks on saved tensors that give them back with other strides or at an odd address: the same bits.  Another type, size or
+    device is refused before anything is launched."""
+    from wtconv import WTConv2d
+    from wtconv_amd import _ext
+    ext = _ext.get()
+    gen = torch.Generator().manual_seed(0)
+    r = lambda *s: torch.randn(*s, generator=gen).bfloat16().to(hip_device)
+    B, C, H, W = 2, 96, 14, 14
+    x, y, g = r(B, C, H, W), r(B, H, W, C), r(B, C, H, W)
+    conv = WTConv2d(C, C, kernel_size=5, wt_levels=2).to(hip_device).bfloat16()
+    params = [p for p in conv.parameters() if p.requires_grad]
+    fn, tensors, g = {
+        "layer": (lambda a, *p: torch.func.functional_call(conv, dict(zip(names, p)), (a,)), (x, *params), g),
+        "norm": (lambda *a: ext.channel_norm(*a, 1e-6, True), (x, r(C), r(C)), y),
+        "mlp": (ext.mlp, (y, r(4 * C, C), r(4 * C), r(C, 4 * C), r(C)), r(B, H, W, C)),
+        "residual": (ext.block_residual, (y, x, r(C)), g)}[which]
+    names = [n for n, p in conv.named_parameters() if p.requires_grad]
+
+    def grads(unpack):
+        leaves = [t.detach().clone().requires_grad_() for t in tensors]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = fn(*leaves)
+        return torch.autograd.grad(out, leaves, g)
+
+    for a, b in zip(grads(lambda t: t), grads(back)):
+        assert torch.equal(a, b)
+    for other in (lambda t: t.float(), lambda t: t.cpu(), lambda t: t.reshape(-1)[:-1]):
+        with pytest.raises(RuntimeError, match="came back"):
+            grads(other)

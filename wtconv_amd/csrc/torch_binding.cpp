@@ -148,6 +148,11 @@ struct LayerParams {
   Tensor t[kMaxTensors];
   int L = 0;
   int count() const { return 3 + 2 * L; }
+  // values of tensor i
+  int64_t numel(int i, int64_t C, int dims, int64_t K) const {
+    const int64_t taps = dims == 2 ? K * K : K, S = dims == 2 ? 4 : 2;
+    return i == 0 ? C * taps : i < 3 ? C : i < 3 + L ? S * C * taps : S * C;
+  }
   at::TensorList levels() const { return at::TensorList(t + 3, 2 * L); }
 };
 
@@ -174,6 +179,23 @@ Tensor layer_forward(const Tensor& x, const LayerParams& lp, int dims, int K) {
   return out;
 }
 
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
+
+// A tensor that a node saved, as the kernels read it: hooks on saved tensors may give it back with other strides, at an
+// address of less alignment, or as another tensor altogether.
+Tensor readable(const torch::autograd::SavedVariable& v, const torch::autograd::Node& node, at::ScalarType type, int64_t numel) {
+  Tensor t = v.unpack();
+  if (!t.defined()) return t;
+  const at::Device dev = node.input_metadata(0).device();
+  TORCH_CHECK(t.device() == dev && t.scalar_type() == type && t.numel() == numel, "wtconv backward: ", numel, " values of type ", type,
+              " on ", dev, " were saved, and ", t.numel(), " of type ", t.scalar_type(), " on ", t.device(), " came back");
+  if (!t.is_contiguous()) t = t.contiguous();
+  return aligned16(t) ? t : t.clone();
+}
+
+// The type of a node's results: that of the activations.
+at::ScalarType made_type(const torch::autograd::Node& node) { return c10::typeMetaToScalarType(node.input_metadata(0).dtype()); }
+
 // Results that come from raw pointers and carry no graph: a derivative of theirs is refused.  (Detached: a result may be the
 // caller's own upstream gradient, passed on, whose history is not ours to write.)
 void refuse_second_derivatives(variable_list& res, const char* what) {
@@ -191,6 +213,8 @@ void refuse_second_derivatives(variable_list& res, const char* what) {
 struct WTConvNode : public torch::autograd::Node {
   torch::autograd::SavedVariable x_, p_[kMaxTensors];
   int dims_ = 0, K_ = 0, L_ = 0;
+  Shape shape_ = {};
+  at::ScalarType ptype_ = at::kFloat;
 
   std::string name() const override { return "WTConvLayerBackward"; }
 
@@ -203,11 +227,12 @@ struct WTConvNode : public torch::autograd::Node {
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
     const int dims = dims_, K = K_, L = L_;
-    const Tensor x = x_.unpack();
+    const Shape s = shape_;
+    const Tensor x = readable(x_, *this, made_type(*this), static_cast<int64_t>(s.B) * s.C * s.H * s.W);
     LayerParams lp;
     lp.L = L;
     const int n = lp.count();
-    for (int i = 0; i < n; ++i) lp.t[i] = p_[i].unpack();
+    for (int i = 0; i < n; ++i) lp.t[i] = readable(p_[i], *this, ptype_, lp.numel(i, s.C, dims, K));
     variable_list res(1 + n);
     if (!grads[0].defined()) return res;
     const bool need_x = task_should_compute_output(0);
@@ -226,7 +251,6 @@ struct WTConvNode : public torch::autograd::Node {
     if (g.scalar_type() != x.scalar_type()) g = g.to(x.scalar_type());
     if (!g.is_contiguous()) g = g.contiguous();
     const c10::DeviceGuard guard(x.device());
-    const Shape s = shape_of(x, dims);
     const int pass = need_x && need_params ? 3 : (need_x ? 1 : 2);
     const size_t wsz = workspace_bytes(dims, s, K, L, pass);
     const c10::DataPtr ws = scratch(x, wsz);
@@ -323,13 +347,12 @@ PyObject* layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::ScalarType pd = lp.t[0].scalar_type();
   const at::Device dev = x_in.device();
   if (dtype_code(pd) < 0) Py_RETURN_NONE;
-  const int64_t C = x_in.size(1), taps = dims == 2 ? K * K : K, S = dims == 2 ? 4 : 2;
+  const int64_t C = x_in.size(1);
   bool record = at::GradMode::is_enabled(), any = x_in.requires_grad();
   for (int i = 0; i < lp.count(); ++i) {
     const Tensor& t = lp.t[i];
     if (!t.defined()) continue;
-    const int64_t want = i == 0 ? C * taps : i < 3 ? C : i < 3 + L ? S * C * taps : S * C;
-    if (!canonical(t, dev, pd) || t.numel() != want || t._fw_grad(0).defined()) Py_RETURN_NONE;
+    if (!canonical(t, dev, pd) || t.numel() != lp.numel(i, C, dims, K) || t._fw_grad(0).defined()) Py_RETURN_NONE;
     any = any || t.requires_grad();
   }
   if (x_in._fw_grad(0).defined()) Py_RETURN_NONE;      // forward-mode differentiation: refused by the Python function
@@ -358,6 +381,8 @@ PyObject* layer(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       node->dims_ = dims;
       node->K_ = static_cast<int>(K);
       node->L_ = lp.L;
+      node->shape_ = shape_of(x, dims);
+      node->ptype_ = pd;
       torch::autograd::set_history(out, node);
     }
   }
@@ -557,11 +582,10 @@ py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm
 
 // ---- a block's MLP in training: fc2(gelu(fc1(x))) over the last extent of x.
 
-bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
-
 // Gradients of x, fc1's weight and bias, fc2's weight and bias: edges 0..4 of the node.
 struct MlpNode : public torch::autograd::Node {
   torch::autograd::SavedVariable x_, w1_, w2_, h_, act_;
+  int64_t pixels_ = 0, C_ = 0, hidden_ = 0;
 
   std::string name() const override { return "WTConvMlpBackward"; }
 
@@ -572,7 +596,10 @@ struct MlpNode : public torch::autograd::Node {
 
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
-    const Tensor x = x_.unpack(), w1 = w1_.unpack(), w2 = w2_.unpack(), h = h_.unpack(), act = act_.unpack();
+    const int64_t C = C_, hidden = hidden_, pixels = pixels_;
+    auto saved = [&](const torch::autograd::SavedVariable& v, int64_t numel) { return readable(v, *this, at::kBFloat16, numel); };
+    const Tensor x = saved(x_, pixels * C), w1 = saved(w1_, hidden * C), w2 = saved(w2_, C * hidden), h = saved(h_, pixels * hidden),
+                 act = saved(act_, pixels * hidden);
     variable_list res(5);
     if (!grads[0].defined()) return res;
     const bool need_x = task_should_compute_output(0);
@@ -587,7 +614,6 @@ struct MlpNode : public torch::autograd::Node {
     if (!g.is_contiguous()) g = g.contiguous();
     if (!aligned16(g)) g = g.clone();
     const c10::DeviceGuard guard(x.device());
-    const int64_t C = w1.size(1), hidden = w1.size(0), pixels = x.numel() / C;
     const int want = (need_x ? WTCONV_MLP_DX : 0) | (need_1 ? WTCONV_MLP_FC1 : 0) | (need_2 ? WTCONV_MLP_FC2 : 0);
     const size_t wsz = abi.mlpt_ws(pixels, C, hidden, want);
     const c10::DataPtr ws = scratch(x, wsz);
@@ -659,6 +685,9 @@ py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor
     node->w2_ = torch::autograd::SavedVariable(w2, false);
     node->h_ = torch::autograd::SavedVariable(h, false);
     node->act_ = torch::autograd::SavedVariable(act, false);
+    node->pixels_ = pixels;
+    node->C_ = C;
+    node->hidden_ = hidden;
     torch::autograd::set_history(y, node);
   }
   return py::cast(y);
@@ -687,6 +716,8 @@ Tensor upstream(const Tensor& g, at::IntArrayRef sizes, const at::TensorOptions&
 // Gradients of x, weight and bias: edges 0..2 of the node.
 struct NormNode : public torch::autograd::Node {
   torch::autograd::SavedVariable x_, weight_;
+  int64_t B_ = 0, C_ = 0, H_ = 0, W_ = 0;
+  at::ScalarType ptype_ = at::kFloat;
   double eps_ = 0;
   bool nhwc_ = false;
 
@@ -700,13 +731,13 @@ struct NormNode : public torch::autograd::Node {
 
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
-    const Tensor x = x_.unpack(), weight = weight_.unpack();
+    const int64_t B = B_, C = C_, H = H_, W = W_;
+    const Tensor x = readable(x_, *this, made_type(*this), B * C * H * W), weight = readable(weight_, *this, ptype_, C);
     const bool twice = at::GradMode::is_enabled() &&
                        ((grads[0].defined() && grads[0].requires_grad()) || x.requires_grad() || weight.requires_grad());
     const at::NoGradGuard no_grad;
     const c10::DeviceGuard guard(x.device());
     const at::TensorOptions opt = x.options().requires_grad(false);
-    const int64_t B = x.size(0), C = x.size(1), H = x.size(2), W = x.size(3);
     const Tensor g = nhwc_ ? upstream(grads[0], {B, H, W, C}, opt) : upstream(grads[0], {B, C, H, W}, opt);
     Tensor dx = at::empty(x.sizes(), opt), flat = at::empty({2 * C}, weight.options().requires_grad(false));
     size_t wsz;
@@ -754,6 +785,11 @@ py::object channel_norm(const Tensor& x, const Tensor& weight, const Tensor& bia
       node->set_next_edges(std::move(next));
       node->x_ = torch::autograd::SavedVariable(x, false);
       node->weight_ = torch::autograd::SavedVariable(weight, false);
+      node->B_ = B;
+      node->C_ = C;
+      node->H_ = H;
+      node->W_ = W;
+      node->ptype_ = weight.scalar_type();
       node->eps_ = eps;
       node->nhwc_ = nhwc;
       torch::autograd::set_history(out, node);
@@ -765,6 +801,8 @@ py::object channel_norm(const Tensor& x, const Tensor& weight, const Tensor& bia
 // Gradients of y, shortcut and gamma: edges 0..2 of the node.
 struct ResidualNode : public torch::autograd::Node {
   torch::autograd::SavedVariable y_, gamma_;
+  int64_t B_ = 0, C_ = 0, H_ = 0, W_ = 0;
+  at::ScalarType ptype_ = at::kFloat;
 
   std::string name() const override { return "WTConvBlockResidualBackward"; }
 
@@ -776,13 +814,13 @@ struct ResidualNode : public torch::autograd::Node {
 
   variable_list apply(variable_list&& grads) override {
     const std::lock_guard<std::mutex> lock(mutex_);
-    const Tensor y = y_.unpack(), gamma = gamma_.unpack();
+    const int64_t B = B_, C = C_, H = H_, W = W_;
+    const Tensor y = readable(y_, *this, made_type(*this), B * C * H * W), gamma = readable(gamma_, *this, ptype_, C);
     const bool twice = at::GradMode::is_enabled() &&
                        ((grads[0].defined() && grads[0].requires_grad()) || y.requires_grad() || gamma.requires_grad());
     const at::NoGradGuard no_grad;
     const c10::DeviceGuard guard(y.device());
     const at::TensorOptions opt = y.options().requires_grad(false);
-    const int64_t B = y.size(0), H = y.size(1), W = y.size(2), C = y.size(3);
     Tensor g = upstream(grads[0], {B, C, H, W}, opt);
     variable_list res(3);
     if (task_should_compute_output(0) || task_should_compute_output(2)) {
@@ -837,6 +875,11 @@ py::object block_residual(const Tensor& y, const Tensor& shortcut, const std::op
       node->set_next_edges(std::move(next));
       node->y_ = torch::autograd::SavedVariable(y, false);
       node->gamma_ = torch::autograd::SavedVariable(*gamma, false);
+      node->B_ = B;
+      node->C_ = C;
+      node->H_ = H;
+      node->W_ = W;
+      node->ptype_ = gamma->scalar_type();
       torch::autograd::set_history(out, node);
     }
   }
