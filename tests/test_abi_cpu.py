@@ -355,3 +355,12 @@ def test_cpp_autograd_node_builds_loads_and_declines_host_tensors(lib):
             [torch.randn(1, 4 * C, 1, 1)])
     assert ext.layer(x, *args, 2, K, 1) is None
     assert ext.layer(x, args[0], None, *args[2:], 2, K, 1) is None
+
+
+def test_planes_of_one_round_stay_in_one_round(lib):
+    """K = 7 runs one workgroup a CU: up to 128 channels their chunks make no more workgroups than there are compute units (a
+    few more take a second round), and at least two thirds of that where there are planes enough."""
+    for B, C, H, W, L in [(52, 86, 20, 22, 4), (45, 102, 24, 19, 2), (132, 55, 12, 10, 2), (256, 96, 11, 10, 2), (20, 56, 63, 47, 5),
+                          (45, 50, 15, 12, 2), (16, 72, 45, 37, 2), (128, 116, 15, 16, 2)]:
+        records = lib.wtconv2d_workspace_bytes(B, C, H, W, 7, L, 2) // 4 - C
+        assert 170 <= records // ((1 + 4 * L) * 49 + 1) <= 256, (B, C, H, W, L)

@@ -9,8 +9,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("shape,K,L,dtype", [
     ((16, 24, 45, 37), 7, 2, torch.float16),      # three planes an iteration, one workgroup a CU
     ((5, 7, 40, 39), 7, 4, torch.float32),        # fewer workgroups than compute units: one plane
-    ((33, 16, 11, 13), 7, 2, torch.float32),      # eleven instead of sixteen, so that the last iteration is full
-    ((40, 3, 6, 7), 7, 2, torch.float32),         # as many as the kernel takes
+    ((33, 16, 11, 13), 7, 2, torch.float32),      # one iteration a workgroup, the last workgroup's not full
+    ((40, 3, 6, 7), 7, 2, torch.float32),         # one iteration of as many planes as there are places
+    ((53, 86, 20, 22), 7, 4, torch.float32),      # two workgroups a channel with several iterations each, the last one short
+    ((37, 270, 8, 9), 7, 2, torch.float16),       # more channels than compute units
     ((9, 12, 30, 25), 7, 1, torch.bfloat16),      # one level: two workgroups a CU
     ((7, 6, 58, 66), 5, 3, torch.float32),        # one pair of pyramids takes more than half of the LDS
     ((3, 5, 75, 60), 5, 2, torch.float16),

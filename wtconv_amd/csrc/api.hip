@@ -47,6 +47,45 @@ static int check_common(const char* fn, const wtconv_params* params, int B, int 
   return 0;
 }
 
+// How the plane-resident parameter-gradient kernel walks a channel's B planes: pb an iteration, `bchunk` a workgroup, which
+// makes `nchunk` workgroups a channel.
+struct WgradSplit { int pb, bchunk, nchunk; };
+
+static WgradSplit wgrad_split(int B, int C, int H, int W, int K, int L) {
+  constexpr int kPlannedCUs = 256;      // a constant, so that workspace sizes do not depend on the device queried
+  WgradSplit s = {wgrad_planes_that_fit(B, H, W, K, L), 0, 0};
+  if (!wgrad_is_alone(K, L)) {
+    // Two workgroups a CU, one where an iteration's planes take more than half of the LDS.  (Planned for two while one ran, the
+    // chunks made two rounds, and each workgroup's fixed parts were paid twice: [23,29,75,60] fp16, K = 5, two levels
+    // 43 -> 31 us, [16,40,61,69] fp32 48 -> 37, [6,58,100,85] one level 36 -> 30, [4,368,79,98] K = 3, five levels 99 -> 84.)
+    const Plan2D t = make_plan2d_geometry(s.pb, 1, H, W, K, L, true, 512, s.pb);
+    const bool one = static_cast<size_t>(t.plane_lds_floats) * 4 > static_cast<size_t>(kLdsLimitBytes) / 2;
+    wgrad_chunks(B, C, s.pb, kPlannedCUs * (one ? 1 : 2), &s.bchunk, &s.nchunk);
+    return s;
+  }
+  // One workgroup a CU, with as many planes an iteration as suit the chunks, of up to four rounds of the chip: the split of
+  // least time by a model of it, in microseconds 13 a round (clearing LDS, a first load with nothing beside it, the
+  // reduction), 4 an iteration and 1.6 per 1000 pixels in it (a third of that goes by the places for planes, a power of two,
+  // of which the kernel deals each the same threads), 0.2 a chunk for the last workgroup's sums.  Of 90 drawn shapes, each
+  // measured with every number of planes and one to four rounds, it takes 0.4 % longer than the best split at the geometric
+  // mean and up to 5 %, once 11.  Of the time with planes for 80 KB and chunks for two workgroups a CU it takes 0.86 over 400 other
+  // drawn shapes, at most 1.10 ([46,10,16,18], three levels, 24 -> 27 us; [256,270,6,5] 164 -> 180): [16,72,45,37] fp16, two levels, 59 -> 46, [41,89,13,13] three
+  // levels 57 -> 34, [52,86,20,22] four 87 -> 68, [103,44,39,48] fp32, three 147 -> 117, [34,350,31,27] four 245 -> 181.
+  const int fit = s.pb, most = B < 64 ? B : 64, four = 4 * kPlannedCUs / C;
+  float best = 0.f;
+  for (int n = 1; n <= (four < most ? four : most) || n == 1; ++n) {
+    const int planes = (B + n - 1) / n, iters = (planes + fit - 1) / fit, even = (planes + iters - 1) / iters, slots = pow2_ceil(even);
+    for (int pb = even;; pb = slots / 2) {
+      const int its = (planes + pb - 1) / pb, nn = (B + its * pb - 1) / (its * pb), rounds = (C * nn + kPlannedCUs - 1) / kPlannedCUs;
+      const float places = 0.65f * pb + 0.35f * pow2_ceil(pb);
+      const float cost = rounds * (13.f + its * (4.f + places * 0.0016f * H * W)) + 0.2f * nn;
+      if (s.nchunk == 0 || cost < best) { best = cost; s = {pb, its * pb, nn}; }
+      if (pb != even || even == slots) break;
+    }
+  }
+  return s;
+}
+
 static size_t fold_floats(int C, int S, int L, int KK) { return static_cast<size_t>(C) * (1 + S * L) * KK + C; }
 
 // Folded filters as the plane kernel writes them itself (PlaneFold): each channel's table on cache lines of its own.
@@ -146,10 +185,8 @@ static size_t stream_records(int B, int C, int H, int W, int K, int L) {
 }
 static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) {
   if (s.wdepth == L) return 0;
-  int bchunk, nchunk;
-  const int d = s.wdepth, pb = wgrad_planes_per_iter(B, C, s.h[d], s.w[d], K, L - d);
-  wgrad_chunks(B, C, pb, wgrad_resident(pb, s.h[d], s.w[d], K, L - d), &bchunk, &nchunk);
-  return round_up64(static_cast<size_t>(nchunk) * C * ((1 + 4 * (L - d)) * K * K + 1));
+  const int d = s.wdepth;
+  return round_up64(static_cast<size_t>(wgrad_split(B, C, s.h[d], s.w[d], K, L - d).nchunk) * C * ((1 + 4 * (L - d)) * K * K + 1));
 }
 
 // One launch of the plane-resident kernels on planes that fit LDS; `fw` / `fb` folded parameters, those of a channel
@@ -411,14 +448,11 @@ size_t wtconv2d_workspace_bytes(int B, int C, int H, int W, int K, int levels, i
   if (static_cast<long long>(H) * W > kMaxPlaneElems) return 0;
   size_t floats;
   if (pass == WTCONV_PASS_BACKWARD_PARAMS) {
-    int bchunk, nchunk;
     // the dtype is not an argument here: room for the bf16 matrix-core kernel's partial sums as well
     const Mfma2dWgradQuery mq = mfma2d_wgrad_query(B, C, H, W, K, levels, WTCONV_BF16);
     const size_t mfloats = mq.ok ? mq.ws_bytes / sizeof(float) : 0;
     if (wgrad_fits_lds(B, C, H, W, K, levels)) {
-      const int pb = wgrad_planes_per_iter(B, C, H, W, K, levels);
-      wgrad_chunks(B, C, pb, wgrad_resident(pb, H, W, K, levels), &bchunk, &nchunk);
-      floats = static_cast<size_t>(nchunk) * C * ((1 + 4 * levels) * K * K + 1);
+      floats = static_cast<size_t>(wgrad_split(B, C, H, W, K, levels).nchunk) * C * ((1 + 4 * levels) * K * K + 1);
     } else {      // partial sums, then the LL bands of x and of grad_out
       const Stream2D sp = make_stream2d(B, C, H, W, K, levels);
       floats = stream_records(B, C, H, W, K, levels) + stream_sub_records(sp, B, C, K, levels);
@@ -518,7 +552,7 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
   if (static_cast<long long>(B) * C > 0x7fffffffLL / 4)
     return fail(WTCONV_E_UNSUPPORTED, "%s: batch*channels = %lld is too large", fn, static_cast<long long>(B) * C);
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  int bchunk, nchunk;
+  int nchunk;
   float* partial = static_cast<float*>(workspace);
   int e;
   SubRecords sub = {};
@@ -541,11 +575,11 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
     nchunk = mq.nchunk;
     e = mfma2d_wgrad_pass(fn, x, grad_out, partial, B, C, H, W, K, L, fin, stream);
   } else if (resident) {
-    const int pb = wgrad_planes_per_iter(B, C, H, W, K, L);
-    Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, pb);
+    const WgradSplit split = wgrad_split(B, C, H, W, K, L);
+    Plan2D pl = make_plan2d(B, C, H, W, K, L, true, 512, split.pb);
     finish_wgrad_plan(&pl, K);
-    wgrad_chunks(B, C, pb, wgrad_resident(pb, H, W, K, L), &bchunk, &nchunk);
-    e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, bchunk, nchunk, fin, stream);
+    nchunk = split.nchunk;
+    e = launch_wgrad2d(dtype, K, L, x, grad_out, partial, pl, B, split.bchunk, nchunk, fin, stream);
   } else {
     const Stream2D sp = make_stream2d(B, C, H, W, K, L);
     nchunk = stream_chunks(B, C, H, W);
@@ -559,14 +593,14 @@ static int backward_params2d(const char* fn, const void* x, const void* grad_out
       const void* xd = d == 0 ? x : static_cast<const void*>(xll + sp.ll[d]);
       const void* gd = d == 0 ? grad_out : static_cast<const void*>(gll + sp.ll[d]);
       if (d == D && d < L) {       // the rest fits LDS
-        const int Ls = L - d, pb = wgrad_planes_per_iter(B, C, sp.h[d], sp.w[d], K, Ls);
-        Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, pb);
+        const int Ls = L - d;
+        const WgradSplit split = wgrad_split(B, C, sp.h[d], sp.w[d], K, Ls);
+        Plan2D pl = make_plan2d(B, C, sp.h[d], sp.w[d], K, Ls, true, 512, split.pb);
         finish_wgrad_plan(&pl, K);
-        int sub_chunk;
-        wgrad_chunks(B, C, pb, wgrad_resident(pb, sp.h[d], sp.w[d], K, Ls), &sub_chunk, &sub.nchunk);
+        sub.nchunk = split.nchunk;
         sub.partial = sub_partial;
         sub.depth = d;
-        e = launch_wgrad2d(WTCONV_F32, K, Ls, xd, gd, sub_partial, pl, B, sub_chunk, sub.nchunk, FinishArgs{}, stream);
+        e = launch_wgrad2d(WTCONV_F32, K, Ls, xd, gd, sub_partial, pl, B, split.bchunk, sub.nchunk, FinishArgs{}, stream);
         break;
       }
       // a step; at d == L only the LL band's own filter is left, the base conv of a layer without levels

@@ -209,40 +209,18 @@ inline bool same_plane_geometry(const Plan2D& a, const Plan2D& b) {
 // 7x7 148 -> 137 us); a 56x56 plane fills the budget by itself.  The threads are dealt to the
 // planes of an iteration, so planes with long rows share them with fewer others.
 //
-// K = 7 with two levels or more takes over 128 registers a lane, so that one workgroup runs on a CU: it gets all of the LDS.
-// Measured, us, planes for 80 KB and chunks for two workgroups a CU -> for 160 KB and one: [16,72,45,37] fp16, two levels
-// 59 -> 46, [103,44,39,48] fp32, three levels 147 -> 116, [34,350,31,27] four levels 245 -> 181, [256,23,14,11] three
-// 58 -> 37.  Where that leaves fewer workgroups than compute units, or would leave most of a last iteration empty, an
-// iteration takes fewer planes ([26,28,29,26] four planes 29.3, two 24.0; [33,437,11,13] sixteen 78, twelve 67).
+// K = 7 with two levels or more takes over 128 registers a lane, so that one workgroup runs on a CU: it may have all of the LDS.
 constexpr bool wgrad_is_alone(int K, int L) { return K == 7 && L >= 2; }
-constexpr int kPlannedCUs = 256;      // a constant, so that workspace sizes do not depend on the device queried
 
-constexpr int wgrad_planes_per_iter(int B, int C, int H, int W, int K, int L) {
-  const bool alone = wgrad_is_alone(K, L);
+constexpr int wgrad_planes_that_fit(int B, int H, int W, int K, int L) {
   int pb = B < 16 ? B : 16;
   if (pb < 1) pb = 1;
   while (pb > 1) {
     const Plan2D t = make_plan2d_geometry(B, 1, H, W, K, L, true, 512, pb);
-    if (static_cast<size_t>(t.plane_lds_floats) * 4 <= (alone ? 160 : 80) * 1024 && 512 / pow2_ceil(pb) >= row_lanes(W)) break;
+    if (static_cast<size_t>(t.plane_lds_floats) * 4 <= (wgrad_is_alone(K, L) ? 160 : 80) * 1024 && 512 / pow2_ceil(pb) >= row_lanes(W)) break;
     --pb;
   }
-  if (alone && pb > 1) {
-    int iters = (B + pb - 1) / pb;
-    const int fill = (kPlannedCUs + C - 1) / C;
-    if (iters < fill) iters = fill < B ? fill : B;
-    pb = (B + iters - 1) / iters;
-  }
   return pb;
-}
-
-// Workgroups of the parameter-gradient kernel that run at once, with iterations of pb planes: one a CU where the registers allow no more or an iteration's
-// planes take more than half of the LDS, else two.  (Planned for two while one ran, the chunks made two rounds, and each
-// workgroup's fixed parts were paid twice: [23,29,75,60] fp16, K = 5, two levels 43 -> 31 us, [16,40,61,69] fp32 48 -> 37,
-// [6,58,100,85] one level 36 -> 30, [4,368,79,98] K = 3, five levels 99 -> 84.)
-constexpr int wgrad_resident(int pb, int H, int W, int K, int L) {
-  const Plan2D t = make_plan2d_geometry(pb, 1, H, W, K, L, true, 512, pb);
-  const bool one = wgrad_is_alone(K, L) || static_cast<size_t>(t.plane_lds_floats) * 4 > static_cast<size_t>(kLdsLimitBytes) / 2;
-  return kPlannedCUs * (one ? 1 : 2);
 }
 
 // Completes a plan for the weight-gradient kernel: threads per stacked plane, prefetch.

@@ -23,7 +23,7 @@ static int run_wgrad2d_static(int K, int L, const void* x, const void* g, float*
   if (K != 5 || pl.H != pl.W) return 1;
 #define WT_TRY(H_, L_)                                                                                   \
   if (pl.H == H_ && L == L_) {                                                                           \
-    constexpr int PB = wgrad_planes_per_iter(128, 1, H_, H_, 5, L_);                                        \
+    constexpr int PB = wgrad_planes_that_fit(128, H_, H_, 5, L_);                                        \
     using G = WgradGeoStatic<H_, H_, 5, L_, PB>;                                                         \
     constexpr Plan2D gp = G::plan();                                                                     \
     if (same_wgrad_geometry(gp, pl))                                                                     \
