@@ -103,6 +103,29 @@ def test_calls_without_kernels_are_left_alone(hip_device):
         gx.float().sum().backward()
 
 
+def test_second_derivatives_of_a_block_without_layer_scale(hip_device):
+    """Those that do not lead through the gradients of the layer or the norm, against the separate passes (an observer)."""
+    from wtconvnext.wtconvnext import WTConvNeXtBlock
+    torch.manual_seed(0)
+    blk = WTConvNeXtBlock(96, wt_levels=2, ls_init_value=None).to(hip_device).bfloat16()
+    x = torch.randn(2, 96, 14, 14, device=hip_device).bfloat16()
+    leaves = [blk.mlp.fc1.weight, blk.mlp.fc1.bias, blk.mlp.fc2.weight]
+
+    def second():
+        first = torch.autograd.grad(blk(x).float().square().sum(), leaves, create_graph=True)
+        return torch.autograd.grad(sum(t.float().square().sum() for t in first), leaves)
+
+    got = second()
+    handle = blk.mlp.fc1.register_forward_hook(lambda m, i, o: None)
+    want = second()
+    handle.remove()
+    for a, b in zip(got, want):      # products of bfloat16 values in another order, four deep
+        assert _rel(a, b.double()) < 2e-2
+    blk.gamma = torch.nn.Parameter(torch.ones(96, device=hip_device).bfloat16())
+    with pytest.raises(RuntimeError):
+        second()
+
+
 @pytest.mark.parametrize("C,side", [(96, 14), (384, 14), (768, 7)])
 def test_block_step_with_and_without_the_kernels(hip_device, C, side):
     """Observers make the block take the separate passes: the same gradients within bfloat16 rounding, strided upstream

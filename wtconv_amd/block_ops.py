@@ -116,9 +116,11 @@ def patch_conv(x, seq, conv, norm, stem):
     return ext.patch_conv(x, *args, norm.eps, stem)
 
 
-def mlp_fn(x, mlp):
+def mlp_fn(x, mlp, twice=True):
     """A block's `mlp` (fc1, exact GELU, fc2) on x (B, H, W, C) where autograd records it, products, GELU and bias sums as
-    kernels of this library; None where that does not apply (see block_mlp)."""
+    kernels of this library; None where that does not apply (see block_mlp).  Second derivatives are PyTorch's; with
+    `twice` False they are refused (for a caller whose upstream gradient comes without a history, so that an answer
+    would lack what goes through it)."""
     ext = _ext.get()
     if ext is None or not torch.is_grad_enabled() or torch.compiler.is_compiling() or torch.is_autocast_enabled():
         return None
@@ -130,7 +132,7 @@ def mlp_fn(x, mlp):
     for t in (x, *args):
         if t is None or type(t) not in _PLAIN:
             return None
-    return ext.mlp(x, *args)
+    return ext.mlp(x, *args, twice)
 
 
 def _native(name, *args):

@@ -584,14 +584,15 @@ py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm
 
 // Gradients of x, fc1's weight and bias, fc2's weight and bias: edges 0..4 of the node.
 struct MlpNode : public torch::autograd::Node {
-  torch::autograd::SavedVariable x_, w1_, w2_, h_, act_;
+  torch::autograd::SavedVariable x_, w1_, b1_, w2_, h_, act_;
   int64_t pixels_ = 0, C_ = 0, hidden_ = 0;
+  bool twice_ = false;      // whether second derivatives are answered
 
   std::string name() const override { return "WTConvMlpBackward"; }
 
   void release_variables() override {
     const std::lock_guard<std::mutex> lock(mutex_);
-    for (auto* v : {&x_, &w1_, &w2_, &h_, &act_}) v->reset_data();
+    for (auto* v : {&x_, &w1_, &b1_, &w2_, &h_, &act_}) v->reset_data();
   }
 
   variable_list apply(variable_list&& grads) override {
@@ -608,6 +609,7 @@ struct MlpNode : public torch::autograd::Node {
     if (!need_x && !need_1 && !need_2) return res;
     const bool twice = at::GradMode::is_enabled() &&
                        (grads[0].requires_grad() || x.requires_grad() || w1.requires_grad() || w2.requires_grad());
+    if (twice && twice_) return recorded(grads[0].to(x.scalar_type()), x, w1, b1_.unpack(), w2);
     const at::NoGradGuard no_grad;
     Tensor g = grads[0];
     if (g.scalar_type() != x.scalar_type()) g = g.to(x.scalar_type());
@@ -641,10 +643,24 @@ struct MlpNode : public torch::autograd::Node {
     if (twice) refuse_second_derivatives(res, "the block's MLP");
     return res;
   }
+
+  // The gradients by operators that autograd records, all of them products of two matrices.
+  variable_list recorded(const Tensor& g_in, const Tensor& x_in, const Tensor& w1, const Tensor& b1, const Tensor& w2) {
+    const Tensor g = g_in.reshape({pixels_, C_}), x = x_in.reshape({pixels_, C_});
+    const Tensor h = at::addmm(b1, x, w1.t()), dh = at::gelu_backward(at::mm(g, w2), h);
+    variable_list res(5);
+    if (task_should_compute_output(0)) res[0] = at::mm(dh, w1).reshape(x_in.sizes());
+    if (task_should_compute_output(1)) res[1] = at::mm(dh.t(), x);
+    if (task_should_compute_output(2)) res[2] = dh.sum(0);
+    if (task_should_compute_output(3)) res[3] = at::mm(g.t(), at::gelu(h));
+    if (task_should_compute_output(4)) res[4] = g.sum(0);
+    return res;
+  }
 };
 
 // The MLP with its C++ autograd node, where autograd records it: None otherwise, or if there are no kernels for these arguments.
-py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
+// `twice`: second derivatives are answered, not refused.
+py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2, bool twice) {
   TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
   if (!at::GradMode::is_enabled() || x.dim() < 2 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || x.numel() == 0)
     return py::none();
@@ -682,9 +698,11 @@ py::object mlp(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor
     node->set_next_edges(std::move(next));
     node->x_ = torch::autograd::SavedVariable(x, false);
     node->w1_ = torch::autograd::SavedVariable(w1, false);
+    if (twice) node->b1_ = torch::autograd::SavedVariable(b1, false);
     node->w2_ = torch::autograd::SavedVariable(w2, false);
     node->h_ = torch::autograd::SavedVariable(h, false);
     node->act_ = torch::autograd::SavedVariable(act, false);
+    node->twice_ = twice;
     node->pixels_ = pixels;
     node->C_ = C;
     node->hidden_ = hidden;
@@ -928,7 +946,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       {nullptr, nullptr, 0, nullptr}};
   if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
   m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
-  m.def("mlp", &mlp, "a block's MLP with a C++ autograd node; None if not taken");
+  m.def("mlp", &mlp, "a block's MLP with a C++ autograd node; None if not taken", py::arg("x"), py::arg("fc1_weight"), py::arg("fc1_bias"),
+        py::arg("fc2_weight"), py::arg("fc2_bias"), py::arg("twice") = false);
   m.def("channel_norm", &channel_norm, "LayerNorm over the channels with a C++ autograd node; None if not taken");
   m.def("block_residual", &block_residual, "layer scale and shortcut with a C++ autograd node; None if not taken");
   m.def("patch_conv", &patch_conv, "stem or downsample of a WTConvNeXt in one kernel; None if not taken");

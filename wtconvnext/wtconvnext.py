@@ -119,7 +119,8 @@ class WTConvNeXtBlock(nn.Module):
                 y = ops.channel_norm_fn(x, self.norm.weight, self.norm.bias, self.norm.eps, True)
             else:
                 y = ops.channel_norm(x, self.norm.weight, self.norm.bias, self.norm.eps, nhwc=True)
-            z = ops.mlp_fn(y, self.mlp) if type(self.mlp) is Mlp else None
+            # (the gradient of block_residual_fn has no second derivative)
+            z = ops.mlp_fn(y, self.mlp, twice=self.gamma is None) if type(self.mlp) is Mlp else None
             y = self.mlp(y) if z is None else z
             # the MLP may change the dtype; the residual kernels take a tensor of the shortcut's type
             if ops.usable_nhwc(y, shortcut):
