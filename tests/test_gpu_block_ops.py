@@ -321,20 +321,21 @@ def test_autocast_keeps_the_plain_passes(hip_device):
 
 
 @pytest.mark.parametrize("shape,hidden", [
-    ((2, 96, 8, 8), 384),        # one tile exactly, rows of whole 8-pixel vectors
-    ((5, 96, 7, 9), 384),        # odd pixel count: pixel by pixel, tile over several images, remainder
-    ((3, 128, 6, 6), 512),       # 4-pixel vectors
-    ((1, 192, 11, 3), 768),      # one pixel more than the smallest taken
-    ((70, 192, 28, 28), 64),     # a single slice of hidden units, many tiles
-    ((2, 256, 14, 14), 1024),    # hidden units dealt to several workgroups
+    ((2, 96, 8, 8), 384),        # (two kernels:) whole tiles, rows of whole 4-pixel vectors
+    ((5, 96, 7, 9), 384),        # (two kernels:) odd pixel count: pixel by pixel, tile over several images, remainder
+    ((3, 128, 6, 6), 512),       # one kernel: part of a tile, a slice of hidden units a workgroup, 4-pixel vectors
+    ((1, 192, 11, 3), 768),      # (two kernels:) one pixel more than the smallest taken
+    ((70, 192, 28, 28), 64),     # one kernel: a single slice of hidden units, many tiles
+    ((2, 256, 14, 14), 1024),    # (two kernels)
     ((2, 384, 14, 14), 1536),
-    ((168, 384, 14, 14), 1536),  # enough tiles to go unsplit
-    ((1, 384, 13, 11), 192),
-    ((168, 384, 14, 14), 4096),  # the bias of all hidden units ends where the LDS does
+    ((168, 384, 14, 14), 1536),  # one kernel: enough tiles to go unsplit
+    ((1, 384, 13, 11), 192),     # (two kernels)
+    ((168, 384, 14, 14), 4096),  # one kernel: the bias of all hidden units ends where the LDS does
 ])
 @pytest.mark.parametrize("layer_scale", [True, False])
 def test_fused_block_against_fp64(hip_device, shape, hidden, layer_scale):
-    """LayerNorm, MLP, layer scale and shortcut in one kernel against float64 on the same bfloat16 values."""
+    """LayerNorm, MLP, layer scale and shortcut, in the one kernel or the two for few pixels, against float64 on the same
+    bfloat16 values."""
     import torch.nn.functional as F
     from wtconv_amd import _ext
     B, C, H, W = shape
@@ -355,6 +356,21 @@ def test_fused_block_against_fp64(hip_device, shape, hidden, layer_scale):
     assert rel < 4e-3, rel
     rms = want.pow(2).mean().sqrt()
     assert ((d(got) - want).abs() / torch.maximum(want.abs(), rms)).max().item() < 6e-2
+
+
+@pytest.mark.parametrize("shape,hidden", [
+    ((5, 96, 29, 31), 384), ((20, 128, 14, 14), 512), ((10, 192, 15, 13), 768), ((3, 256, 25, 27), 1024), ((8, 384, 14, 14), 1536),
+    ((4, 384, 16, 24), 1536), ((7, 128, 16, 24), 512),      # 8-pixel vectors
+    ((1, 96, 8, 24), 2048),                                 # a slice a workgroup
+])
+@pytest.mark.parametrize("layer_scale", [True, False])
+def test_one_kernel_block_with_hidden_units_dealt_to_workgroups(hip_device, shape, hidden, layer_scale):
+    """The sums of several workgroups meet in a second launch."""
+    from wtconv_amd import _lib
+    B, C, H, W = shape
+    padded = (B * H * W + 127) // 128 * 128
+    assert _lib.load().wtconv_block_mlp_workspace_bytes(B, C, H * W, hidden) in [4 * n * C * padded for n in range(2, hidden // 32 + 1)]
+    test_fused_block_against_fp64(hip_device, shape, hidden, layer_scale)
 
 
 def test_fused_block_keeps_infinities_and_nans_to_their_pixels(hip_device):

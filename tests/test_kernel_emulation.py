@@ -430,12 +430,14 @@ def test_emulated_block_residual(B, C, H, W, dtype):
 
 
 @pytest.mark.parametrize("B,C,H,W,hidden,layer_scale", [
-    (2, 96, 8, 8, 64, True),       # a tile exactly, rows of whole 8-pixel vectors; two slices, one a workgroup
-    (1, 96, 11, 3, 192, False),    # pixel by pixel, part of a tile; three slices a workgroup
-    (5, 96, 8, 12, 64, True),      # four tiles: unsplit
-    (1, 128, 6, 6, 64, True),      # 4-pixel vectors
-    (1, 256, 6, 6, 128, True),     # a pixel tile a wave, eight waves
-    # (up to 320000 / C pixels take the two kernels below: these are the one kernel's)
+    (2, 96, 8, 8, 64, True),       # (two kernels:) whole tiles, 4-pixel vectors
+    (1, 96, 11, 3, 192, False),    # (two kernels:) pixel by pixel, a tile and a pixel
+    (5, 96, 8, 12, 64, True),      # (two kernels:) many tiles
+    (1, 128, 6, 6, 64, True),
+    (1, 256, 6, 6, 128, True),
+    # the one kernel's, with the hidden units dealt to two workgroups (two compute units are assumed here) and without
+    (1, 96, 7, 11, 832, True),     # pixel by pixel, part of a tile
+    (1, 128, 8, 8, 320, False),    # 8-pixel vectors
     (1, 384, 29, 29, 64, True),    # pixel by pixel, part of a last tile
     (1, 256, 36, 36, 64, False),   # 8-pixel vectors
     (1, 96, 58, 58, 128, True),    # 4-pixel vectors, two pixel tiles a wave
