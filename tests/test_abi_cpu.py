@@ -33,6 +33,34 @@ def test_header_symbols_are_exported(lib):
     assert lib.wtconv_max_kernel_size() == 7
 
 
+def _prototypes(header):
+    """name -> (result, argument types) of a header's functions, as ctypes types; enums and pointers by their kind."""
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", header)).read(), flags=re.S)
+    text = re.sub(r"typedef struct \{.*?\} \w+;", "", text, flags=re.S)
+    scalar = {"int": ctypes.c_int, "long long": ctypes.c_longlong, "size_t": ctypes.c_size_t, "float": ctypes.c_float}
+
+    def kind(t):
+        return "pointer" if "*" in t else scalar[" ".join(t.split()[:-1]) if t.split()[-1] not in ("int", "long", "float", "size_t") else t]
+    out = {}
+    for res, name, args in re.findall(r"^(int|size_t|const char\*) (wtconv\w*)\(([^)]*)\);", text, flags=re.M):
+        args = [a.strip() for a in args.split(",") if a.strip() not in ("", "void")]
+        out[name] = ("pointer" if "*" in res else scalar[res], [kind(a) for a in args])
+    return out
+
+
+def test_second_header_is_exported_and_bound_as_declared(lib):
+    from wtconv_amd import _lib
+    of = lambda t: t if t in (ctypes.c_int, ctypes.c_longlong, ctypes.c_size_t, ctypes.c_float) else "pointer"
+    for header, exports in (("wtconv_ops.h", _lib.OPS_EXPORTS), ("wtconv_hip.h", _lib.EXPORTS)):
+        declared = _prototypes(header)
+        assert set(declared) == set(exports), set(declared) ^ set(exports)
+        for name, (res, args) in exports.items():
+            assert hasattr(lib, name), name
+            assert (of(res), [of(a) for a in args]) == declared[name], name
+    define = re.search(r"#define WTCONV_OPS_VERSION (\d+)", open(os.path.join(ROOT, "include", "wtconv_ops.h")).read())
+    assert lib.wtconv_ops_version() == _lib.OPS_VERSION == int(define.group(1))
+
+
 def test_workspace_sizes(lib):
     C, K, L = 96, 5, 3
     fwd = lib.wtconv2d_workspace_bytes(128, C, 56, 56, K, L, 0)

@@ -49,7 +49,7 @@ def test_mlp_against_fp64(hip_device, M, C, hidden):
 
 
 def test_a_frozen_part_is_not_computed(hip_device):
-    """Every subset of what may need a gradient: the same bits as in the full pass, None elsewhere."""
+    """Every subset of what may need a gradient: the full pass's gradients to rounding, None elsewhere."""
     from wtconv_amd import _ext
     x, dy, *params = _inputs(hip_device, 300, 192, 768)
     full = _call(x, dy, *params)[1:]
