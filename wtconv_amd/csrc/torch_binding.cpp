@@ -182,15 +182,21 @@ Tensor layer_forward(const Tensor& x, const LayerParams& lp, int dims, int K) {
 bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
 
 // A tensor that a node saved, as the kernels read it: hooks on saved tensors may give it back with other strides, at an
-// address of less alignment, or as another tensor altogether.
-Tensor readable(const torch::autograd::SavedVariable& v, const torch::autograd::Node& node, at::ScalarType type, int64_t numel) {
-  Tensor t = v.unpack();
-  if (!t.defined()) return t;
-  const at::Device dev = node.input_metadata(0).device();
-  TORCH_CHECK(t.device() == dev && t.scalar_type() == type && t.numel() == numel, "wtconv backward: ", numel, " values of type ", type,
-              " on ", dev, " were saved, and ", t.numel(), " of type ", t.scalar_type(), " on ", t.device(), " came back");
+// address of less alignment (`align`: copied then, too), or as another tensor altogether.
+[[gnu::noinline, gnu::cold]] void another_came_back(const Tensor& t, const at::Device& dev, at::ScalarType type, int64_t numel) {
+  TORCH_CHECK(false, "wtconv backward: ", numel, " values of type ", type, " on ", dev, " were saved, and ", t.numel(), " of type ",
+              t.scalar_type(), " on ", t.device(), " came back");
+}
+inline void make_readable(Tensor& t, const at::Device& dev, at::ScalarType type, int64_t numel, bool align) {
+  if (!t.defined()) return;
+  if (t.device() != dev || t.scalar_type() != type || t.numel() != numel) another_came_back(t, dev, type, numel);
   if (!t.is_contiguous()) t = t.contiguous();
-  return aligned16(t) ? t : t.clone();
+  if (align && !aligned16(t)) t = t.clone();
+}
+inline Tensor readable(const torch::autograd::SavedVariable& v, const torch::autograd::Node& node, at::ScalarType type, int64_t numel) {
+  Tensor t = v.unpack();
+  make_readable(t, node.input_metadata(0).device(), type, numel, true);
+  return t;
 }
 
 // The type of a node's results: that of the activations.
@@ -228,11 +234,16 @@ struct WTConvNode : public torch::autograd::Node {
     const std::lock_guard<std::mutex> lock(mutex_);
     const int dims = dims_, K = K_, L = L_;
     const Shape s = shape_;
-    const Tensor x = readable(x_, *this, made_type(*this), static_cast<int64_t>(s.B) * s.C * s.H * s.W);
+    const at::Device dev = input_metadata(0).device();
+    Tensor x = x_.unpack();
+    make_readable(x, dev, made_type(*this), static_cast<int64_t>(s.B) * s.C * s.H * s.W, false);
     LayerParams lp;
     lp.L = L;
     const int n = lp.count();
-    for (int i = 0; i < n; ++i) lp.t[i] = readable(p_[i], *this, ptype_, lp.numel(i, s.C, dims, K));
+    for (int i = 0; i < n; ++i) {
+      lp.t[i] = p_[i].unpack();
+      make_readable(lp.t[i], dev, ptype_, lp.numel(i, s.C, dims, K), false);
+    }
     variable_list res(1 + n);
     if (!grads[0].defined()) return res;
     const bool need_x = task_should_compute_output(0);
