@@ -170,3 +170,17 @@ def test_one_kernel_block_is_not_taken_while_its_modules_are_observed(one_kernel
         with torch.device("cpu"):          # a default device is no observer
             blk(x)
     assert len(one_kernel) == 2
+
+
+def test_compiling_comes_before_the_binding(monkeypatch):
+    """While a model is being compiled the fused passes step aside before they ask for the C++ binding: loading it is not
+    traceable, and a model may be compiled before its first call."""
+    from wtconv_amd import block_ops
+    from wtconvnext.wtconvnext import WTConvNeXt
+    model = WTConvNeXt(depths=(1, 1, 1, 1), dims=(8, 16, 24, 32), num_classes=2)
+    blk, x = model.stages[0].blocks[0], torch.zeros(1, 3, 8, 8)
+    monkeypatch.setattr(block_ops._ext, "get", lambda: pytest.fail("asked for"))
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert block_ops.block_mlp(x, x, blk.norm, blk.mlp, blk.gamma) is None
+    assert block_ops.patch_conv(x, model.stem, model.stem[0], model.stem[1], True) is None
+    assert block_ops.mlp_fn(x, blk.mlp) is None

@@ -80,8 +80,10 @@ def block_mlp(x, shortcut, norm, mlp, gamma):
     None where it does not apply: autograd records, another dtype than bfloat16, a channel count without a kernel, an
     activation other than the exact GELU, observers that expect to see the modules called, or tensors of a subclass
     (quantised or sharded weights bring their own product, and often no memory that a kernel could read)."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled():      # (first: loading the binding is not traceable)
+        return None
     ext = _ext.get()
-    if ext is None or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+    if ext is None:
         return None
     fc1, act, fc2 = mlp.fc1, mlp.act, mlp.fc2
     if (type(fc1) is not torch.nn.Linear or type(fc2) is not torch.nn.Linear or type(act) is not torch.nn.GELU
@@ -102,8 +104,10 @@ def patch_conv(x, seq, conv, norm, stem):
     with stride 2) of a WTConvNeXt, the two modules of `seq`, in one kernel; None where it does not apply: autograd records,
     another dtype than bfloat16, sizes without a kernel, another kind of convolution, observers that expect to see the
     modules called, or tensors of a subclass."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled():      # (first: loading the binding is not traceable)
+        return None
     ext = _ext.get()
-    if ext is None or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+    if ext is None:
         return None
     size = (4, 4) if stem else (2, 2)
     if (type(conv) is not torch.nn.Conv2d or conv.kernel_size != size or conv.stride != size or conv.dilation != (1, 1)
@@ -121,8 +125,10 @@ def mlp_fn(x, mlp, twice=True):
     kernels of this library; None where that does not apply (see block_mlp).  Second derivatives are PyTorch's; with
     `twice` False they are refused (for a caller whose upstream gradient comes without a history, so that an answer
     would lack what goes through it)."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled() or not torch.is_grad_enabled():
+        return None
     ext = _ext.get()
-    if ext is None or not torch.is_grad_enabled() or torch.compiler.is_compiling() or torch.is_autocast_enabled():
+    if ext is None:
         return None
     fc1, act, fc2 = mlp.fc1, mlp.act, mlp.fc2
     if (type(fc1) is not torch.nn.Linear or type(fc2) is not torch.nn.Linear or type(act) is not torch.nn.GELU
