@@ -16,7 +16,8 @@ namespace wt {
 // runs this, so the result does not depend on the order in which the first stage finished.  The sums are in float whatever the
 // type of the gradients, which are rounded once, here: a pass of their own for that took 4 us of kernel time behind those of a
 // 16-bit layer (training step of 56 x 56 x 96 205.6 -> 203.7 us; of 7 x 7 x 768, whose runs differ by up to 8 % among themselves, between
-// 86.5 -> 85.0 and 91.7 -> 84.4 in three pairs).  SHARED: called by the
+// 86.5 -> 85.0 and 91.7 -> 84.4 in three pairs).  Float gradients pay 0.3 us a launch for the choice (median of 120 shapes; with the
+// type beside the parameters' in the arguments, the same).  SHARED: called by the
 // last workgroup of a first stage that finishes its channels itself: the records of the other workgroups are read
 // with load_shared_f32.
 // Records of a sub-layer that starts `depth` levels down (0: none): its base filter is the LL filter of level `depth`,
