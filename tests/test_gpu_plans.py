@@ -1,5 +1,5 @@
 """Parameter gradients and results of the vector kernels at the shapes where their plans change: planes of which LDS holds one
-pair of pyramids or two, K = 7 with one and with more planes an iteration."""
+pair of pyramids or two, K = 7 with one and with more planes an iteration, rows whose strips divide no thread count."""
 import pytest
 import torch
 
@@ -19,6 +19,11 @@ pytestmark = pytest.mark.gpu
     ((2, 4, 100, 85), 5, 1, torch.float32),
     ((4, 10, 33, 41), 5, 3, torch.float32),       # rows a little above a power of two
     ((3, 10, 35, 33), 5, 4, torch.float16),
+    ((16, 9, 17, 19), 5, 1, torch.float16),       # rows of 5 strips or 10 over 64 threads: the last pass is not full
+    ((6, 20, 12, 10), 7, 1, torch.float32),       # two strips a row, four planes a wave
+    ((40, 9, 45, 50), 3, 2, torch.float32),       # K = 3: strips of two, odd rows a pass
+    ((300, 1, 87, 66), 7, 1, torch.float32),      # 512 threads a plane, rows of 17 strips
+    ((2, 130, 5, 77), 7, 2, torch.float32),       # three rows of 39 coefficients
 ])
 def test_layer_against_fp64(hip_device, shape, K, L, dtype):
     import wtconv

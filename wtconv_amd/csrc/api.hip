@@ -196,12 +196,12 @@ static int resident2d(const char* fn, const void* x, void* out, const float* fw,
                       const PlaneFold& fold = PlaneFold{}) {
   Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256);
   int tj1 = 4, sg_shift = 8;
-  choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
+  choose_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
   // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
   while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
   if (!plane_shape_is_static(K, H, W, L))
-    widen_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, pl.nplanes, &tj1, &sg_shift);
-  finish_plane_plan(&pl, sg_shift);
+    widen_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, pl.nplanes, &tj1, &sg_shift);
+  finish_plane_plan(&pl, tj1, sg_shift);
   pl.fw_stride = fw_stride;
   pl.fw_skip = fw_skip;
   if (static_cast<size_t>(pl.lds_floats) * 4 > kLdsLimitBytes)

@@ -22,6 +22,16 @@ namespace wt {
 
 constexpr int kFetchPasses = 2;  // 2x4 pieces of the next plane a thread may hold in registers
 
+// How a plane's threads walk a level: thread t takes item t % per_row of rows t / per_row, + rows, ...  The quotient comes
+// from a reciprocal (exact below 1024 threads and 512 items: the error of v * magic is under v * per_row < 2^20).
+struct RowSplit {
+  int per_row, rows;           // work items of a row; rows that the threads take at once
+  unsigned magic;              // ceil(2^20 / per_row)
+};
+__device__ __forceinline__ int row_of(const RowSplit& s, int t) {
+  return static_cast<int>((static_cast<unsigned>(t) * s.magic) >> 20);
+}
+
 // LDS layout of one plane, computed on the host (plan.h).
 struct Plan2D {
   int C, H, W, L;
@@ -52,6 +62,8 @@ struct Plan2D {
   int fw_stride;               // plane kernel: folded filters of a channel to the next channel's (floats)
   int fw_skip;                 //   floats between where the level filters would follow the base filter and where they
                                //   are (a sub-layer's base filter is the LL filter of the level above it)
+  RowSplit strips1;            // plane kernel: the strips of level 1 over the threads of a plane
+  RowSplit coefs[kMaxLevels + 1];      // and the single coefficients of level l >= 2 (analysis and synthesis)
 };
 
 // ------------------------------------------------------------------ parameter folding
@@ -531,15 +543,14 @@ __device__ __forceinline__ void ihaar4(float ll, float lh, float hl, float hh,
 // inverse Haar, cropped store into Z_l.
 template <int K, int TJ>
 __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2D& pl, int l,
-                                            wt_uniform_ptr wl_f, int ltid, int nth) {
+                                            wt_uniform_ptr wl_f, int ltid) {
   constexpr int R = K / 2;
   constexpr int VW = (R >= 1) ? TJ : 1;   // window starts at column j0 when the halo equals R
-  const int hl = pl.h[l], wl = pl.w[l];
-  const int nstrip = (wl + TJ - 1) / TJ;
-  const int gsh = group_shift(nstrip);
-  const int strip = ltid & ((1 << gsh) - 1);
-  if (strip >= nstrip) return;
-  const int j0 = strip * TJ;
+  const int hl = pl.h[l];
+  const RowSplit split = pl.coefs[l];
+  const int row = row_of(split, ltid);
+  if (row >= split.rows) return;
+  const int j0 = (ltid - imul(row, split.per_row)) * TJ;
   const int astr = pl.astr[l], apl = pl.apl[l], P = pl.P;
   const float* A = lds + pl.aoff[l];
   const bool has_carry = l < pl.L;
@@ -548,9 +559,7 @@ __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2
   float* Zout = lds + pl.zoff[l];
   const int zout_str = pl.zstr[l];
   const int ho = pl.h[l - 1], wo = pl.w[l - 1];
-  const int rpp = (nth >> gsh) > 0 ? (nth >> gsh) : 1;
-  if ((ltid >> gsh) >= rpp) return;            // (a row never has more strips than lanes: row_lanes, plan.h)
-  for (int i = ltid >> gsh; i < hl; i += rpp) {
+  for (int i = row; i < hl; i += split.rows) {
     float o0[2 * TJ], o1[2 * TJ];
     subband_chunks<K, TJ, VW>(A + imul(i - R + P, astr) + (j0 - R + P), astr, apl, wl_f,
                                  has_carry ? Zin + imul(i, zin_str) + j0 : nullptr, o0, o1);
@@ -598,17 +607,16 @@ __device__ __forceinline__ void store_row(T* __restrict__ dst, const float (&v)[
 template <typename T, int K, int TJ>
 __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2D& pl,
                                             wt_uniform_ptr wb_f, wt_uniform_ptr w1_f, float bias,
-                                            T* __restrict__ out_plane, int ltid, int nth) {
+                                            T* __restrict__ out_plane, int ltid) {
   constexpr int R = K / 2;
   constexpr int NO = 2 * TJ;
   constexpr int VW = (R >= 1) ? TJ : 1;
   constexpr int VWX = (R >= 1) ? (NO >= 4 ? 4 : NO) : 1;
-  const int hl = pl.h[1], wl = pl.w[1];
-  const int nstrip = (wl + TJ - 1) / TJ;
-  const int gsh = group_shift(nstrip);
-  const int strip = ltid & ((1 << gsh) - 1);
-  if (strip >= nstrip) return;
-  const int j0 = strip * TJ;
+  const int hl = pl.h[1];
+  const RowSplit split = pl.strips1;
+  const int row = row_of(split, ltid);
+  if (row >= split.rows) return;
+  const int j0 = (ltid - imul(row, split.per_row)) * TJ;
   const int astr = pl.astr[1], apl = pl.apl[1], P = pl.P;
   const float* A = lds + pl.aoff[1];
   const float* X = lds + pl.aoff[0];
@@ -617,9 +625,7 @@ __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2
   const float* Zin = lds + pl.zoff[2];
   const int zin_str = pl.zstr[2];
   const int H = pl.H, W = pl.W;
-  const int rpp = (nth >> gsh) > 0 ? (nth >> gsh) : 1;
-  if ((ltid >> gsh) >= rpp) return;
-  for (int i = ltid >> gsh; i < hl; i += rpp) {
+  for (int i = row; i < hl; i += split.rows) {
     float o0[NO], o1[NO];
     subband_chunks<K, TJ, VW>(A + imul(i - R + P, astr) + (j0 - R + P), astr, apl, w1_f,
                                  has_carry ? Zin + imul(i, zin_str) + j0 : nullptr, o0, o1);
@@ -843,12 +849,12 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
     }
     for (int lv = pl.L; lv >= 2; --lv) {
       const int l = WT_UNIFORM(lv);
-      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + fw_skip + (1 + 4 * (l - 1)) * KK, ltid, sg);
+      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + fw_skip + (1 + 4 * (l - 1)) * KK, ltid);
       plane_sync(wave_local);
     }
     WT_WAIT_VMEM();     // next plane's loads have landed; the stores below are not waited for
     WT_WAVE_PRIORITY(0);
-    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, bias_of(c), out + plane_off, ltid, sg);
+    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, bias_of(c), out + plane_off, ltid);
     plane_sync(wave_local);   // the next plane overwrites the buffers read above
   }
 }

@@ -30,29 +30,41 @@ static_assert(kTJC == 1, "row_lanes counts single coefficients of level 2");
 // Widest plane of the weight-gradient kernel: a wave sums strips of kTJW pixels of whole rows.
 constexpr int kMaxWgradWidth = kWave * kTJW;
 
-// Level-1 strip width and threads per plane of the plane kernel: the pair that keeps most
-// lanes busy in the level-1 phase (ties: the wider strip, which reads less LDS per FMA),
-// discounted when the slots of a workgroup (256 / threads-per-plane planes of
+// What level 1 costs in strips of `tj` over `threads` threads, in lane-instructions: the lanes that are taken up -- half of
+// it counted by the waves that have any strip, half by whole passes (an idle wave costs no issue slots, but its workgroup
+// waits) -- times a strip's 8 K^2 tj multiply-adds, divided by what its LDS reads leave of them (a 5 x 5 window does 1.7, 0.9
+// or 0.6 multiply-adds for a float it reads), and 100 instructions a thread in the plane's other phases.
+// Fitted to every width and thread count on 308 shapes (fp32, 6 to 110 pixels, K = 3 to 7): the pick is 2 % slower than the
+// best pair at the geometric mean, picks by busy lanes alone 5 %, up to half slower.  Those took (forward, us)
+// [16,72,45,37], K = 7, two levels 33.9, now 27.5; [17,140,87,66], K = 7, one level 129 -> 90; [148,168,19,17], K = 5, one
+// level 64 -> 46; [20,252,44,43], K = 7, two levels 100 -> 77.
+constexpr double strip_cost(int K, int h1, int w1, int tj, int threads) {
+  const int per_row = (w1 + tj - 1) / tj, rows = threads / per_row, full = h1 / rows, rest = h1 - full * rows;
+  auto waves_of = [](int lanes) { return (lanes + kWave - 1) / kWave * kWave; };
+  const double passes = static_cast<double>(threads) * (full + (rest > 0 ? 1 : 0));
+  const double busy = threads >= kWave ? static_cast<double>(full) * waves_of(rows * per_row) + waves_of(rest * per_row) : passes;
+  return 0.5 * (passes + busy) * 8 * K * K * tj / (tj == 1 ? (K > 5 ? 0.4 : 0.65) : tj == 2 && K > 3 ? 0.9 : 1.0) + 100.0 * threads;
+}
+
+// Level-1 strip width and threads per plane of the plane kernel: the cheaper pair (ties: the
+// wider strip), which counts for more when the slots of a workgroup (256 / threads-per-plane planes of
 // `plane_lds_bytes` each) leave room for fewer than three workgroups per CU: with two, the
 // phases of a plane are latency bound (measured on 14x14 planes: 88 -> 76 us with 32 instead
 // of 16 threads per plane, i.e. half the slots).
-constexpr void choose_plane_shape(int h1, int w1, size_t plane_lds_bytes, int* tj1, int* sg_shift) {
-  double best = -1.0;
+constexpr void choose_plane_shape(int K, int h1, int w1, size_t plane_lds_bytes, int* tj1, int* sg_shift) {
+  double best = 0.0;
   const int lanes = row_lanes(2 * w1), most = lanes > 256 ? lanes : 256;
   for (int tj = 4; tj >= 1; tj /= 2) {
-    const int gs = pow2_ceil((w1 + tj - 1) / tj);
-    if (gs > most) continue;
-    int sg = pow2_ceil(gs * h1);
+    const int per_row = (w1 + tj - 1) / tj;
+    if (per_row > most) continue;
+    int sg = per_row * h1 < most ? pow2_ceil(per_row * h1) : most;
     if (sg < 16) sg = 16;
     if (sg < lanes) sg = lanes;
-    if (sg > most) sg = most;
-    const int rpp = sg / gs;
-    const int passes = (h1 + rpp - 1) / rpp;
-    double eff = static_cast<double>(h1) * w1 / (static_cast<double>(sg) * passes * tj);
+    double cost = strip_cost(K, h1, w1, tj, sg);
     const size_t wg_lds = plane_lds_bytes * (256 / sg);
     const int resident = wg_lds ? static_cast<int>(kLdsLimitBytes / wg_lds) : 3;
-    if (resident < 3) eff *= (resident > 0 ? resident : 0.5) / 3.0;
-    if (eff > best + 1e-9) { best = eff; *tj1 = tj; *sg_shift = log2_int(sg); }
+    if (resident < 3) cost *= 3.0 / (resident > 0 ? resident : 0.5);
+    if (best == 0.0 || cost < best - 1e-9) { best = cost; *tj1 = tj; *sg_shift = log2_int(sg); }
   }
 }
 
@@ -109,10 +121,16 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
   return make_plan2d_geometry(B, C, H, W, K, L, with_grad_pyramid, nthreads, pb);
 }
 
+constexpr RowSplit row_split(int per_row, int threads) {
+  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row};
+}
+
 // Completes a plan for the plane kernel: threads per plane, slots per workgroup, prefetch.
-constexpr void finish_plane_plan(Plan2D* pl, int tj1_sg_shift) {
-  pl->sg_shift = tj1_sg_shift;
+constexpr void finish_plane_plan(Plan2D* pl, int tj1, int sg_shift) {
+  pl->sg_shift = sg_shift;
   const int sg = 1 << pl->sg_shift;
+  pl->strips1 = row_split((pl->w[1] + tj1 - 1) / tj1, sg);
+  for (int l = 2; l <= pl->L; ++l) pl->coefs[l] = row_split(pl->w[l], sg);
   pl->block = sg > 256 ? sg : 256;   // (two whole planes per 512-thread workgroup measured slower: lockstep phases)
   const int slots = pl->block / sg;
   pl->lds_floats = pl->plane_lds_floats * slots;
@@ -142,9 +160,9 @@ struct PlaneGeoFold : PlaneGeoRuntime {
 constexpr Plan2D static_plane_plan(int H, int W, int K, int L, int* tj1_out) {
   Plan2D pl = make_plan2d_geometry(1, 1, H, W, K, L, false, 256, 1);
   int tj1 = 4, sg_shift = 8;
-  choose_plane_shape(pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
+  choose_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
   while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
-  finish_plane_plan(&pl, sg_shift);
+  finish_plane_plan(&pl, tj1, sg_shift);
   if (tj1_out != nullptr) *tj1_out = tj1;
   return pl;
 }
@@ -155,26 +173,21 @@ constexpr bool plane_shape_is_static(int K, int H, int W, int L) {
 
 // More threads for a plane, when the workgroups a CU can hold at once -- by LDS, or for want of planes -- leave it with
 // fewer than twelve waves: the phases of a plane are bound by the latency of LDS then, and halving what a thread does
-// shortens them.  The level-1 strip is the one that gets most done at a time (narrower ones read more LDS per FMA).
+// shortens them.  The level-1 strip is the cheapest one.
 // Forward us, fp32, K = 5, three levels, 256 threads -> widened: [16,64,80,80] (two by LDS) 53.6 -> 43.6, [16,64,72,72]
 // (K = 3, two levels) 35.7 -> 26.4, [16,64,68,68] (five levels) 67.2 -> 49.6; [1,64,40,40] (64 planes) 19.2 -> 17.7,
 // [8,32,64,64] 19.2 -> 18.6.  Planes with a compile-time plan stay with it: [2,96,56,56] 15.2, widened 18.4.
-inline void widen_plane_shape(int h1, int w1, size_t plane_lds_bytes, int nplanes, int* tj1, int* sg_shift) {
+inline void widen_plane_shape(int K, int h1, int w1, size_t plane_lds_bytes, int nplanes, int* tj1, int* sg_shift) {
   if (*sg_shift != 8) return;
   int wgs = plane_lds_bytes ? static_cast<int>(kLdsLimitBytes / plane_lds_bytes) : 1;
   if (wgs > (nplanes + 255) / 256) wgs = (nplanes + 255) / 256;
   while (*sg_shift < 10 && (wgs << *sg_shift) < 768) ++*sg_shift;
   if (*sg_shift == 8) return;
-  const int sg = 1 << *sg_shift;
-  double best = -1.0;
+  double best = 0.0;
   for (int tj = 4; tj >= 1; tj /= 2) {
-    const int gs = pow2_ceil((w1 + tj - 1) / tj);
-    if (gs > sg) continue;
-    const int rpp = sg / gs;
-    const int passes = (h1 + rpp - 1) / rpp;
-    const double eff = static_cast<double>(h1) * w1 / (static_cast<double>(sg) * passes * tj) *
-                       (tj == 4 ? 1.0 : tj == 2 ? 0.85 : 0.65);
-    if (eff > best + 1e-9) { best = eff; *tj1 = tj; }
+    if ((w1 + tj - 1) / tj > 1 << *sg_shift) continue;
+    const double cost = strip_cost(K, h1, w1, tj, 1 << *sg_shift);
+    if (best == 0.0 || cost < best - 1e-9) { best = cost; *tj1 = tj; }
   }
 }
 
