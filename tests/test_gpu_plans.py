@@ -47,3 +47,34 @@ def test_layer_against_fp64(hip_device, shape, K, L, dtype):
     for n, p in mod.named_parameters():
         if p.grad is not None:
             assert rel(p.grad, grads64[n]) < 5e-6, n
+
+
+@pytest.mark.parametrize("shape,K,L", [
+    ((3, 5, 9, 33), 5, 2), ((2, 7, 10, 18), 5, 1), ((5, 3, 13, 43), 3, 3), ((4, 6, 12, 20), 5, 2),      # 1 to 7 columns past whole
+    ((3, 4, 11, 29), 5, 3), ((2, 3, 7, 22), 5, 2), ((6, 5, 15, 15), 5, 3),                              # pairs of 4 x 4 blocks
+    ((40, 3, 17, 17), 5, 4),      # eight tiles of level-1 blocks for four waves
+    ((9, 2, 64, 40), 5, 5),       # as wide and deep as the kernel takes, five tiles
+    ((37, 9, 4, 4), 1, 1), ((70, 4, 7, 7), 5, 2), ((1, 1, 5, 6), 3, 2),      # many planes a unit; one plane, the tensor's last
+    ((26, 4, 14, 14), 5, 3),      # a compile-time plan, the last unit not full
+])
+def test_matrix_core_layer_against_fp64(hip_device, shape, K, L):
+    import wtconv
+    from oracle import wtconv_ref as R
+    torch.manual_seed(shape[3] + L)
+    C = shape[1]
+    mod = wtconv.WTConv2d(C, C, kernel_size=K, wt_levels=L).bfloat16()
+    with torch.no_grad():
+        for p in mod.parameters():
+            if p.requires_grad:
+                p.copy_(torch.randn(p.shape) * 0.4)
+    ref = R.RefWTConv2d(C, C, K, wt_levels=L).double()
+    ref.load_state_dict({k: v.double() for k, v in mod.state_dict().items()})
+    mod = mod.to(hip_device)
+    x, g = torch.randn(shape).bfloat16(), torch.randn(shape).bfloat16()
+    out64, dx64, _ = R.layer_grads(ref, x.double(), g.double())
+    xd = x.to(hip_device).requires_grad_()
+    out = mod(xd)
+    out.backward(g.to(hip_device))
+    rel = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
+    # each product has a coefficient and a folded weight rounded to 8 bits (at most 2^-9 of them each), the result is once more
+    assert rel(out.detach(), out64) < 3 * 2 ** -9 and rel(xd.grad, dx64) < 3 * 2 ** -9

@@ -230,6 +230,13 @@ def test_emulated_2d_mfma_bf16_random_shapes(B, C, H, W, K, L, bias):
     _compare(got, _oracle(2, x, g, bw, bb, bs, ws, ss), rtol=2e-2, atol_scale=2e-2)
 
 
+@pytest.mark.parametrize("B,C,H,W,K,L", [(1, 3, 1, 5, 5, 1), (1, 3, 2, 7, 3, 1), (2, 2, 5, 1, 5, 1), (1, 5, 1, 1, 3, 1), (3, 2, 3, 6, 5, 2)])
+def test_emulated_2d_mfma_loads_stay_inside_the_tensor(B, C, H, W, K, L):
+    x, g, bw, bb, bs, ws, ss = _case2d(B, C, H, W, K, L, True, dtype=1, pdtype=1)
+    got = emu_util.run(2, x, g, bw, bb, bs, ws, ss, K, dtype=1, pdtype=1, mfma=1)
+    _compare(got, _oracle(2, x, g, bw, bb, bs, ws, ss), rtol=2e-2, atol_scale=2e-2)
+
+
 def test_emulated_2d_bf16_vector_alu_kernels():
     """bf16 tensors on the vector-ALU kernels (what K = 7 or planes wider than 64 take)."""
     x, g, bw, bb, bs, ws, ss = _case2d(1, 2, 8, 12, 5, 2, True, dtype=1, pdtype=1)

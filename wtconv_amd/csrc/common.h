@@ -416,6 +416,20 @@ __device__ __forceinline__ float wave_xor(float v, int lane4, int mask) {
 #endif
 }
 
+// Rows of 16 lanes change places: a lane of an odd row gives its `a` to the lane 16 below, whose `b` it takes for it
+// (v_permlane16_swap_b32).  Every lane of the wavefront takes part.
+__device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {
+#ifdef WT_EMULATE
+  const bool odd = (threadIdx.x & 16u) != 0;
+  const uint32_t got = __float_as_uint(__shfl_xor(__uint_as_float(odd ? a : b), 16, kWave));
+  (odd ? a : b) = got;
+#else
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+#endif
+}
+
 // Sum over the 64 lanes of a wavefront; every lane gets the total.  On the GPU: six DPP adds
 // (quad permutes, row mirrors, row broadcasts) and one v_readlane, no LDS traffic -- the
 // weight-gradient kernels reduce up to 76 running sums per workgroup this way.

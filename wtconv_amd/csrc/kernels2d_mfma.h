@@ -6,9 +6,18 @@
 // 8 x 8 patch of inputs (K <= 5), so for 16 blocks of one filter
 //     D[16 outputs of a block][16 blocks] = Wt[16 outputs][64 patch elements] * Patch[64][16 blocks]
 // is two MFMAs (patch rows 0-3 and 4-7).  Wt is the filter laid out as a Toeplitz matrix
-// (39 % non-zero); the fold kernel writes it in the compact form the lanes pick their
+// (39 % non-zero), kept in the compact form that the lanes pick their
 // fragment from.  Lane (n = lane % 16, q = lane / 16) supplies row q (+4) of block n's patch
-// -- 8 consecutive bf16 of an LDS row -- and receives outputs (row q, columns 0..3) of block n.
+// -- 8 consecutive bf16 of an LDS row -- and receives four outputs of block n: its row q at the coarse levels, a square or
+// a lattice of it in the pixels and at level 1 (see the kernel).
+//
+// What bounds it: vector code (commit with two levels of analysis, synthesis), LDS round trips and the two barriers of a
+// unit, at four waves a SIMD for want of registers; the matrix cores are busy an eighth of the time.  us per launch, before
+// level 1 and base convolution met in registers (with the base convolution through LDS as fp32, levels 3 and up behind a
+// barrier each and one table entry a lane in the fold) -> now: [128,96,56,56], three levels 61.3 -> 54.2; [256,96,56,56],
+// five 164 -> 145; [128,192,28,28] 36.3 -> 32.2; [256,384,14,14] 48.5 -> 40.0; [128,768,7,7] 21.3 -> 15.5; a single image
+// of 14 x 14 x 384 12.4 -> 10.7; 120 drawn shapes 0.86 at the geometric mean, from 0.37 to 1.2 (batches of [34,36], whose
+// fifteen block rows make eight tiles for four waves, 20.4 -> 23.5).
 //
 // Activations live in LDS as bf16 planes with a zero halo of 2.  bf16 tensors take one plane
 // per buffer (NS = 1).  fp32 tensors are split into NS = 3 bf16 planes (v = h0 + h1 + h2
@@ -25,6 +34,7 @@
 namespace wt {
 
 constexpr int kFragEntries = 21;     // 5 kernel rows x 4 column shifts, then one all-zero entry
+constexpr int kTapRow = 12;          // elements of a filter row with the zeros around it
 constexpr int kMfmaBlock = 256;
 constexpr int kDivShift = 20;        // magic reciprocals: exact for dividends < 4096, divisors <= 256
 
@@ -46,10 +56,13 @@ struct MPlan {
   int prows[kMaxLevels + 1];         // LDS rows from one stacked plane to the next: 4 nbr + 2
   int aoff[kMaxLevels + 1];          // byte offset of (slot 0, row -2, column -2) of sub-band 0, split 0
   int asub[kMaxLevels + 1];          // bytes from one plane stack to the next (sub-bands, then splits)
-  int zoff[kMaxLevels + 2], zpitch[kMaxLevels + 2], zpl[kMaxLevels + 2];   // fp32 Z_l, l = 1..L
+  int zoff[kMaxLevels + 2], zpitch[kMaxLevels + 2], zpl[kMaxLevels + 2];   // fp32 Z_l, l = 2..L
   int lloff[kMaxLevels + 1], llpl[kMaxLevels + 1];                         // fp32 raw LL of level l, 2 <= l < L
-  int toff;                          // byte offset of the fragment table of the current channel ...
-  int tfirst;                        // ... which starts at this filter (the filters before it live in registers)
+  int toff;                          // byte offset of the fragment table of the current channel: the base filter, then
+  int tskip;                         // the others but this many (those of level 1, where they live in registers)
+  int taps, tap_rows;                // byte offset of the folded filters as rows of taps; rows, the last one of zeros
+  int behind;                        // planes that hold what the last rows' loads take along: (4 nbr - H) W + 3 elements
+  int uq, ur;                        // units of a workgroup: uq, the first ur of them one more
   int lds_bytes;
 };
 
@@ -79,8 +92,8 @@ constexpr bool make_mplan_geometry(int H, int W, int L, int NS, int pb, MPlan* o
   for (int l = 1; l <= L; ++l) { pl.h[l] = (pl.h[l - 1] + 1) / 2; pl.w[l] = (pl.w[l - 1] + 1) / 2; }
   int off = 0;
   pl.toff = off;
-  pl.tfirst = NS == 1 ? 5 : 0;       // one split plane: base conv and level 1 stay in registers
-  off += NS * (pl.nfilt - pl.tfirst) * kFragEntries * 16;
+  pl.tskip = NS == 1 ? 4 : 0;        // one split plane: level 1 stays in registers
+  off += NS * (pl.nfilt - pl.tskip) * kFragEntries * 16;
   for (int l = 0; l <= L; ++l) {
     pl.nbr[l] = cdiv(pl.h[l], 4);
     pl.nbc[l] = cdiv(pl.w[l], 4);
@@ -107,14 +120,15 @@ constexpr bool make_mplan_geometry(int H, int W, int L, int NS, int pb, MPlan* o
     off += pl.asub[l] * NS * (l == 0 ? 1 : 4);
     if (off > (1 << 20)) return false;
   }
-  for (int l = 1; l <= L; ++l) {
+  pl.behind = cdiv((4 * pl.nbr[0] - H) * W + 3, H * W);
+  pl.tap_rows = NS * pl.nfilt * 5 + 1;
+  pl.taps = off;
+  off += rup(pl.tap_rows * kTapRow * 2 + 4, 16);
+  for (int l = 2; l <= L; ++l) {
     pl.zpitch[l] = 4 * pl.nbc[l - 1];
     pl.zpl[l] = 4 * pl.nbr[l - 1] * pl.zpitch[l];
     pl.zoff[l] = off;
-    int zbytes = pb * pl.zpl[l] * 4;
-    const int staging = NS * pl.tfirst * kFragEntries * 16;      // Z_1 doubles as staging area when a channel's parameters are folded
-    if (l == 1 && zbytes < staging) zbytes = staging;
-    off += zbytes;
+    off += pb * pl.zpl[l] * 4;
     if (off > (1 << 20)) return false;
   }
   for (int l = 2; l < L; ++l) {
@@ -254,79 +268,6 @@ __device__ __forceinline__ void split_pair(float lo, float hi, uint32_t (&w)[NS]
   }
 }
 
-// ------------------------------------------------------------------ fragment table (fold)
-// Entry e = 4 kh + cs of filter f of channel c: kernel row kh of the filter (embedded in 5 x 5,
-// scaled by gamma and 4^-level, rotated by 180 degrees when flip != 0) shifted right by cs in a
-// window of 8 -- the 8 bf16 a lane feeds the MFMA with -- as NS split words; entry 20 is zero.
-// Filter 0 is the base conv, filter 1 + 4 (l - 1) + s sub-band s of level l.
-template <int NS>
-__device__ __forceinline__ void fold_entry(const ParamTable& p, int pdtype, int K, int flip, int c, int f, int e,
-                                           uint4 (&out)[NS]) {
-  const int KK = K * K, o = 2 - K / 2;
-  float v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = 0.f;
-  if (e < 20) {
-    const int kh = e >> 2, cs = e & 3;
-    const int ih = kh - o;
-    float scale;
-    const void* wp;
-    int ch;
-    if (f == 0) {
-      wp = p.base_weight; ch = c;
-      scale = load_param(p.base_scale, pdtype, c);
-    } else {
-      const int l = (f - 1) >> 2, s = (f - 1) & 3;
-      wp = p.wt_weight[l]; ch = c * 4 + s;
-      scale = load_param(p.wt_scale[l], pdtype, ch);
-#pragma unroll 1
-      for (int i = 0; i <= l; ++i) scale *= 0.25f;
-    }
-    // the (up to five) taps of the entry's kernel row, fetched together whether or not the entry uses them: loads
-    // behind per-tap conditions would complete one after the other, and a channel switch waits for this fold
-    const bool row_ok = ih >= 0 && ih < K;
-    const int frow = row_ok ? (flip ? K - 1 - ih : ih) : 0;
-    const int rowi = ch * KK + frow * K;
-    float wr[5];
-    if (pdtype == WTCONV_F32) {
-      const float* w = static_cast<const float*>(wp) + rowi;
-#pragma unroll
-      for (int i = 0; i < 5; ++i) wr[i] = w[i < K ? i : K - 1];
-    } else {
-      const uint16_t* w = static_cast<const uint16_t*>(wp) + rowi;
-      uint16_t h[5];
-#pragma unroll
-      for (int i = 0; i < 5; ++i) h[i] = w[i < K ? i : K - 1];
-#pragma unroll
-      for (int i = 0; i < 5; ++i) wr[i] = pdtype == WTCONV_F16 ? f16_bits_to_f32(h[i]) : bf16_to_f32(h[i]);
-    }
-    if (row_ok) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int iw = j - cs - o;
-        if (iw >= 0 && iw < K && j - cs < 5 && j - cs >= 0) {
-          const int fi = flip ? K - 1 - iw : iw;
-          float t = wr[0];
-#pragma unroll
-          for (int i = 1; i < 5; ++i) t = fi == i ? wr[i] : t;
-          v[j] = t * scale;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int js = 0; js < NS; ++js) {
-    uint32_t w[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      w[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-      v[2 * i] -= __uint_as_float(w[i] << 16);
-      v[2 * i + 1] -= __uint_as_float(w[i] & 0xffff0000u);
-    }
-    out[js].x = w[0]; out[js].y = w[1]; out[js].z = w[2]; out[js].w = w[3];
-  }
-}
-
 // ------------------------------------------------------------------ pixel blocks in registers
 template <typename T> struct PixRow;
 template <> struct PixRow<float> { float4 v; };
@@ -439,8 +380,14 @@ __device__ __forceinline__ TileLane tile_lane(const char* lds, int T, int n, int
 // ------------------------------------------------------------------------------ the kernel
 // Grid: persistent workgroups, each takes a contiguous range of units (pb planes of one
 // channel).  NBL: 4x4 pixel blocks a thread loads per unit.  VEC: plane rows are whole,
-// aligned 4-element vectors.  RES: the Toeplitz fragments of the base conv and of level 1 stay
-// in registers while the channel does not change.
+// aligned 4-element vectors.  RES: the Toeplitz fragments of level 1 stay in registers while the channel does not change.
+//
+// A wave computes its 8 x 8 pixels of a level-1 block whole: the four sub-bands' convolutions of the 4 x 4 coefficients and
+// the base convolution of the four pixel blocks above them.  The output rows of the products are dealt so that a lane's
+// results of both meet: accumulator 4 q + v of a sub-band is coefficient (2 (v / 2) + q / 2, 2 (v % 2) + q % 2), and of the
+// base convolution of block v pixel (2 (q / 2) + i, 2 (q % 2) + j) of it -- the 2 x 2 pixels that the inverse Haar
+// transform makes of that coefficient.  The base convolution therefore never passes through LDS (as fp32 it took a third of
+// a 56 x 56 plane's LDS), and nothing but Z_2 has to be waited for between the convolutions and the stores.
 template <typename T, int NS, int NBL, bool VEC, bool RES, typename Geo>
 __global__ void __launch_bounds__(kMfmaBlock, NS == 1 ? 4 : 2)      // waves per SIMD the register budget must allow
 wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable prm, int pdtype, int K, int flip,
@@ -451,6 +398,7 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
       constexpr MPlan g = Geo::template plan<NS>();
       MPlan p = g;
       p.B = plarg.B; p.C = plarg.C; p.upc = plarg.upc; p.nunits = plarg.nunits; p.bq = plarg.bq; p.br = plarg.br;
+      p.uq = plarg.uq; p.ur = plarg.ur;
       return p;
     } else {
       return plarg;
@@ -462,28 +410,22 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
   const int n = lane & 15, q = lane >> 4;
   const int L = pl.L, H = pl.H, W = pl.W;
   const int HW = H * W;
+  // every 4x4 pixel block that exists is whole
+  const bool whole = Geo::kStatic && H % 4 == 0 && W % 4 == 0;
   // the channel tickets of a parameter-gradient pass that follows on the stream
   if (blockIdx.x == 0)
     for (int i = tid; i < nzero; i += kMfmaBlock) zero_words[i] = 0u;
 
-  // Toeplitz fragment entries of this lane: output (row ar, column ac) of a block, patch row q (+4)
-  const int ar = n >> 2, ac = n & 3;
-  const int ent_top = (q - ar >= 0) ? (q - ar) * 4 + ac : 20;
-  const int ent_bot = (q - ar <= 0) ? (4 + q - ar) * 4 + ac : 20;
-  const int tsplit = (pl.nfilt - pl.tfirst) * kFragEntries * 16;      // bytes between the split tables in LDS
-
-  for (int o = tid * 16; o < pl.lds_bytes; o += kMfmaBlock * 16) {
-    uint4 z; z.x = z.y = z.z = z.w = 0u;
-    lds_st<uint4>(lds, o, z);
-  }
-  WT_LDS_BARRIER();
-  levels_up<Geo, 0>(L, [&](auto lc) {
-    const int l = lc;
-    for (int R = tid; R < pl.nrow[l]; R += kMfmaBlock) {
-      const int p = R / pl.nbr[l], bi = R - p * pl.nbr[l];
-      lds_st<uint32_t>(lds, pl.rtoff[l] + 4 * R, rowtab_entry(p * pl.prows[l] + 4 * bi, p, bi));
-    }
-  });
+  // Toeplitz fragment entries of this lane for patch row q (+4) and output (row r, column c) of a block
+  auto entry_top = [&](int r, int c) { return q - r >= 0 ? (q - r) * 4 + c : 20; };
+  auto entry_bot = [&](int r, int c) { return q - r <= 0 ? (4 + q - r) * 4 + c : 20; };
+  // coarse levels: output n of a block in rows; level 1 and base conv as said above
+  const int ent_top = entry_top(n >> 2, n & 3), ent_bot = entry_bot(n >> 2, n & 3);
+  const int r1 = 2 * ((n >> 1) & 1) + (n >> 3), c1 = 2 * (n & 1) + ((n >> 2) & 1);
+  const int ent1_top = entry_top(r1, c1), ent1_bot = entry_bot(r1, c1);
+  const int r0 = 2 * (n >> 3) + ((n >> 1) & 1), c0 = 2 * ((n >> 2) & 1) + (n & 1);
+  const int ent0_top = entry_top(r0, c0), ent0_bot = entry_bot(r0, c0);
+  const int tsplit = (pl.nfilt - pl.tskip) * kFragEntries * 16;      // bytes between the split tables in LDS
 
   // ---- per-thread constants of the commit role: which 4x4 pixel blocks this thread owns
   int c_goff[NBL], c_x0[NBL], c_a1[NBL], c_a2[NBL], c_ll[NBL], c_p[NBL];
@@ -514,47 +456,147 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
   // plan fields of the two finest levels, used in every unit
   const int asub0 = pl.asub[0], asub1 = pl.asub[1], asub2 = pl.asub[2];
   const int pitchB0 = pl.pitch[0] * 2, pitchB1 = pl.pitch[1] * 2;
-  const int aoff0 = pl.aoff[0], aoff1 = pl.aoff[1];
-  const int tcs0 = pl.tcs[0], tcs1 = pl.tcs[1], nrow0 = pl.nrow[0], nrow1 = pl.nrow[1];
-  const int nbc0 = pl.nbc[0], nbc1 = pl.nbc[1], ntile0 = pl.ntile[0], ntile1 = pl.ntile[1];
-  const int rtoff0 = pl.rtoff[0], rtoff1 = pl.rtoff[1];
-  const int zoff1 = pl.zoff[1], zpitch1 = pl.zpitch[1], zpl1 = pl.zpl[1];
+  const int aoff0 = pl.aoff[0], aoff1 = pl.aoff[1], prows0 = pl.prows[0];
+  const int tcs1 = pl.tcs[1], nrow1 = pl.nrow[1], nbc1 = pl.nbc[1], ntile1 = pl.ntile[1], rtoff1 = pl.rtoff[1];
   const int zoff2 = pl.zoff[2], zpitch2 = pl.zpitch[2], zpl2 = pl.zpl[2];
   const int toff = pl.toff, upc = pl.upc, pb = pl.pb, C = pl.C, B = pl.B;
 
   const int G = gridDim.x;
   const int wg = xcd_contiguous(blockIdx.x, G);
-  const int u_begin = static_cast<int>(static_cast<long long>(wg) * pl.nunits / G);
-  const int u_end = static_cast<int>(static_cast<long long>(wg + 1) * pl.nunits / G);
+  const int u_begin = wg * pl.uq + (wg < pl.ur ? wg : pl.ur);
+  const int u_end = u_begin + pl.uq + (wg < pl.ur ? 1 : 0);
+
+  // A unit's channel, its number among the channel's units, and the batch items it takes: the batch is spread evenly over
+  // the units of a channel, at most pb items each, all units within one plane of each other (a short last unit would leave
+  // the workgroups that get it with less work than the rest).
+  struct Unit { int c, ub; };
+  auto first_item = [&](const Unit& u) { return u.ub * pl.bq + (u.ub < pl.br ? u.ub : pl.br); };
+  auto items = [&](const Unit& u) { return pl.bq + (u.ub < pl.br ? 1 : 0); };
+
+  // ---- a channel's filters, folded: gamma * w * 4^-level, rotated by 180 degrees when flip != 0, embedded in 5 x 5.  They
+  // come from memory one tap a lane, all of them in flight at once (one entry of the fragment table a lane, which wants up
+  // to five taps and a scale, took a single unit's workgroup 9000 of its 22 000 cycles), and go to LDS as rows of twelve
+  // bf16: three zeros, five taps, four zeros.  A fragment entry is eight neighbours of such a row.
+  // Two waves take a level (0: the base filter, and its bias), so that its tables are addressed through scalar registers.
+  constexpr int kTapItems = ((Geo::kStatic ? Geo::kL : kMaxLevels) + 2) / 2;
+  uint32_t tap_w[kTapItems], tap_s[kTapItems];
+  struct Tap { int s, row, col; };
+  auto tap_of = [&](int r) {
+    Tap t;
+    t.s = r / 25;
+    const int e = r - t.s * 25;
+    t.row = e / 5;
+    t.col = e - t.row * 5;
+    return t;
+  };
+  auto load_taps = [&](int c) {
+    int r = tid & 127;
+    WT_LAUNDER_LANE_INT(r);      // (nothing that follows from it is kept for the next channel)
+    const Tap t = tap_of(r);
+    const int o = 2 - K / 2, ih = t.row - o, iw = t.col - o, in = ih * K + iw;
+    const bool inside = ih >= 0 && ih < K && iw >= 0 && iw < K;
+    const int tap = flip ? K * K - 1 - in : in;
+#pragma unroll
+    for (int k = 0; k < kTapItems; ++k) {
+      const int l = (wave >> 1) + 2 * k;
+      tap_w[k] = tap_s[k] = 0u;
+      if (l > L) continue;
+      const void *w = l > 0 ? prm.wt_weight[l - 1] : prm.base_weight, *g = l > 0 ? prm.wt_scale[l - 1] : prm.base_scale;
+      const int ch = l > 0 ? 4 * c + t.s : c;
+      if (inside && t.s < (l > 0 ? 4 : 1)) {
+        if (pdtype == WTCONV_F32) {
+          tap_w[k] = static_cast<const uint32_t*>(w)[ch * K * K + tap];
+          tap_s[k] = static_cast<const uint32_t*>(g)[ch];
+        } else {
+          tap_w[k] = static_cast<const uint16_t*>(w)[ch * K * K + tap];
+          tap_s[k] = static_cast<const uint16_t*>(g)[ch];
+        }
+      } else if (l == 0 && r == 25 && use_bias && prm.base_bias != nullptr) {
+        if (pdtype == WTCONV_F32) {
+          tap_w[k] = static_cast<const uint32_t*>(prm.base_bias)[c];
+          tap_s[k] = static_cast<const uint32_t*>(g)[c];
+        } else {
+          tap_w[k] = static_cast<const uint16_t*>(prm.base_bias)[c];
+          tap_s[k] = static_cast<const uint16_t*>(g)[c];
+        }
+      }
+    }
+  };
+  auto store_taps = [&] {
+    int r = tid & 127;
+    WT_LAUNDER_LANE_INT(r);
+    const Tap t = tap_of(r);
+#pragma unroll
+    for (int k = 0; k < kTapItems; ++k) {
+      const int l = (wave >> 1) + 2 * k;
+      if (l > L) continue;
+      float v = __uint_as_float(tap_w[k]), scale = __uint_as_float(tap_s[k]);
+      if (pdtype == WTCONV_F16) {
+        v = f16_bits_to_f32(static_cast<uint16_t>(tap_w[k]));
+        scale = f16_bits_to_f32(static_cast<uint16_t>(tap_s[k]));
+      } else if (pdtype == WTCONV_BF16) {
+        v = bf16_to_f32(static_cast<bf16_t>(tap_w[k]));
+        scale = bf16_to_f32(static_cast<bf16_t>(tap_s[k]));
+      }
+      v *= ldexpf(scale, -2 * l);
+      if (t.s < (l > 0 ? 4 : 1)) {
+        const int f = l > 0 ? 4 * l - 3 + t.s : 0;
+#pragma unroll
+        for (int js = 0; js < NS; ++js) {
+          const bf16_t h = f32_to_bf16(v);
+          lds_st<bf16_t>(lds, pl.taps + (((js * pl.nfilt + f) * 5 + t.row) * kTapRow + 3 + t.col) * 2, h);
+          v -= bf16_to_f32(h);
+        }
+      } else if (l == 0 && r == 25) {
+        lds_st<float>(lds, pl.taps + pl.tap_rows * kTapRow * 2, v);
+      }
+    }
+  };
+  // entry e = 4 kh + cs of filter f: row kh, shifted right by cs in a window of eight; entry 20 is zero (a row of zeros)
+  auto entry_of = [&](int js, int f, int e) {
+    const int row = e < 20 ? (js * pl.nfilt + f) * 5 + (e >> 2) : pl.tap_rows - 1, at = 3 - (e & 3);
+    const int o = pl.taps + row * (kTapRow * 2) + (at & 2) * 2;
+    uint32_t d[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) d[j] = lds_ld<uint32_t>(lds, o + 4 * j);
+    Frag fr;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) fr.d[j] = at & 1 ? (d[j] >> 16 | d[j + 1] << 16) : d[j];
+    return fr;
+  };
 
   PixRow<T> pf[NBL][4];
-  const size_t total_elems = static_cast<size_t>(B) * C * HW;
-  auto fetch = [&](int u) {
-    const int c = u / upc;
-    const int ubf = u - c * upc;
-    const int b0 = ubf * pl.bq + (ubf < pl.br ? ubf : pl.br);      // the batch is spread evenly over the channel's units (see below)
-    const size_t base_off = (static_cast<size_t>(b0) * C + c) * HW;
-    const T* base = x + base_off;
+  // 16-bit planes whose rows are not whole vectors move as one unaligned 8-byte load a row, all four rows of a block: what
+  // comes along from past the row or the plane is cleared at the commit.  The planes at the tensor's end that do not have
+  // that much behind them (pl.behind) go element by element.
+  constexpr bool kOver = !VEC && sizeof(T) == 2;
+  auto fetch = [&](const Unit& u) {
+    const int b0 = first_item(u), np = items(u);
+    const T* base = x + (static_cast<size_t>(b0) * C + u.c) * HW;
+    const bool at_end = (B - b0 - np) * C + (C - 1 - u.c) < pl.behind;
 #pragma unroll
     for (int i = 0; i < NBL; ++i) {
-      const bool plane_ok = (c_mask[i] & 0x100u) && c_p[i] < pl.bq + (ubf < pl.br ? 1 : 0);
+      // (a plane that does not exist keeps what an earlier one left: its results are not stored)
+      if (!(c_mask[i] & 0x100u) || c_p[i] >= np) continue;
+      // (a uniform base and a 32-bit offset in bytes, which a 16-bit unit's elements fit, not added up ahead of the loop)
+      int goff = c_goff[i];
+      WT_LAUNDER_LANE_INT(goff);
+      const T* from = sizeof(T) == 2 ? reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + static_cast<size_t>(static_cast<uint32_t>(goff) * 2))
+                                     : base + goff;
+      if constexpr (kOver) {
+        if (!at_end) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pix_load4u(pf[i][r].v, from + r * W);
+          continue;
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pix_zero(pf[i][r]);
-        if (plane_ok && (c_mask[i] >> r & 1u)) {
-          const T* src = base + c_goff[i] + r * W;
+        if (!whole) pix_zero(pf[i][r]);
+        if (whole || (c_mask[i] >> r & 1u)) {
+          const T* src = from + r * W;
           if constexpr (VEC) {
-            if (c_mask[i] & 16u) pix_load4(pf[i][r], src);
-          } else if constexpr (sizeof(T) == 2) {
-            // one unaligned 8-byte load per row (columns past the row end are cleared at the commit); only a row
-            // whose four elements would reach past the end of the tensor goes element by element
-            if (base_off + c_goff[i] + r * W + 4 <= total_elems) {
-              pix_load4u(pf[i][r].v, src);
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (c_mask[i] >> (4 + e) & 1u) pix_set(pf[i][r], e, src[e]);
-            }
+            pix_load4(pf[i][r], src);      // (a block's first column exists, and with it the other three)
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -564,59 +606,240 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
       }
     }
   };
-  if (u_begin < u_end) fetch(u_begin);
+#pragma unroll
+  for (int i = 0; i < NBL; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pix_zero(pf[i][r]);
+  Unit nxt;
+  nxt.c = u_begin / upc;
+  nxt.ub = u_begin - nxt.c * upc;
+  if (u_begin < u_end) fetch(nxt);
+  load_taps(nxt.c);
+
+  // ---- while they are on their way: halos, and the block-row tables
+  for (int o = tid * 16; o < pl.lds_bytes; o += kMfmaBlock * 16) {
+    uint4 z; z.x = z.y = z.z = z.w = 0u;
+    lds_st<uint4>(lds, o, z);
+  }
+  WT_LDS_BARRIER();
+  levels_up<Geo, 1>(L, [&](auto lc) {
+    const int l = lc;
+    const float per_plane = 1.f / static_cast<float>(pl.nbr[l]);
+    for (int R = tid; R < pl.nrow[l]; R += kMfmaBlock) {
+      const int p = static_cast<int>((R + 0.5f) * per_plane), bi = R - p * pl.nbr[l];      // (whole below 500 block rows a plane)
+      lds_st<uint32_t>(lds, pl.rtoff[l] + 4 * R, rowtab_entry(p * pl.prows[l] + 4 * bi, p, bi));
+    }
+  });
+
+  // ---- level-1 tiles: where a lane finds its block's patches and Z_2, and where its results go
+  struct Tile {
+    int b1, b0, z2;      // LDS offsets: patch row q of the block's sub-band 0, of its pixels, Z_2 of its first coefficient
+    int p, to, y, x;     // plane slot; element offset of row y = 8 bi + q, column x = 8 tc in the unit's output
+    bool valid;
+  };
+  auto tile_of = [&](int t) {
+    Tile o;
+    int n = lane & 15, q = lane >> 4;
+    if constexpr (!Geo::kStatic) {
+      WT_LAUNDER_LANE_INT(n);
+      WT_LAUNDER_LANE_INT(q);
+    }
+    const int tc = n & ((1 << tcs1) - 1);
+    const int R = (t << (4 - tcs1)) + (n >> tcs1);
+    o.valid = R < nrow1 && tc < nbc1;
+    const unsigned e = lds_ld<uint32_t>(lds, rtoff1 + 4 * (R < nrow1 ? R : nrow1 - 1));
+    o.p = static_cast<int>((e >> 12) & 0xffu);
+    const int bi = static_cast<int>(e >> 20);
+    o.b1 = aoff1 + imul(static_cast<int>(e & 0xfffu) + q, pitchB1) + 8 * tc;
+    o.b0 = aoff0 + imul(imul(o.p, prows0) + 8 * bi + q, pitchB0) + 16 * tc;
+    o.z2 = zoff2 + (imul(o.p, zpl2) + imul(4 * bi + (q >> 1), zpitch2) + 4 * tc + (q & 1)) * 4;
+    o.y = 8 * bi + q;
+    o.x = 8 * tc;
+    o.to = o.p * C * HW + o.y * W + o.x;
+    return o;
+  };
 
   constexpr int NR = RES ? NS : 1;
-  Frag ra0t[NR], ra0b[NR], ra1t[4][NR], ra1b[4][NR];     // resident fragments (RES only)
-  int cur_c = -1;
+  Frag ra1t[4][NR], ra1b[4][NR];     // resident fragments (RES only)
   float bias = 0.f;
+  // the base convolution of the four pixel blocks and the sub-band convolutions of a tile
+  auto convolve = [&](const Tile& tl, Acc (&base)[4], Acc (&band)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      base[v].v[0] = base[v].v[1] = base[v].v[2] = base[v].v[3] = bias;
+      band[v].v[0] = band[v].v[1] = band[v].v[2] = band[v].v[3] = 0.f;
+    }
+    {
+      uint2 w[NS][3][3];      // patch rows q, q + 4, q + 8: twelve columns each
+#pragma unroll
+      for (int js = 0; js < NS; ++js)
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) w[js][r][k] = lds_ld<uint2>(lds, tl.b0 + js * asub0 + 4 * r * pitchB0 + 8 * k);
+      Frag at[NS], ab[NS];
+      load_a<NS>(lds, toff, tsplit, ent0_top, ent0_bot, at, ab);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        Frag bt[NS], bb[NS];
+#pragma unroll
+        for (int js = 0; js < NS; ++js) {
+          const uint2 a = w[js][v >> 1][v & 1], b = w[js][v >> 1][(v & 1) + 1];
+          const uint2 c = w[js][(v >> 1) + 1][v & 1], d = w[js][(v >> 1) + 1][(v & 1) + 1];
+          bt[js].d[0] = a.x; bt[js].d[1] = a.y; bt[js].d[2] = b.x; bt[js].d[3] = b.y;
+          bb[js].d[0] = c.x; bb[js].d[1] = c.y; bb[js].d[2] = d.x; bb[js].d[3] = d.y;
+        }
+        mma_tile<NS>(at, ab, bt, bb, base[v]);
+      }
+    }
+    WT_SCHED_FENCE();      // (all of a tile's reads at once would not fit the registers)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      Frag bt[NS], bb[NS];
+      load_b<NS>(lds, tl.b1 + s * asub1, 4 * asub1, 4 * pitchB1, bt, bb);
+      if constexpr (RES) {
+        mma_tile<NS>(ra1t[s], ra1b[s], bt, bb, band[s]);
+      } else {
+        Frag at[NS], ab[NS];
+        load_a<NS>(lds, toff + (1 + s - pl.tskip) * kFragEntries * 16, tsplit, ent1_top, ent1_bot, at, ab);
+        mma_tile<NS>(at, ab, bt, bb, band[s]);
+      }
+      if (s == 1) WT_SCHED_FENCE();
+    }
+  };
+  // Z_2, the inverse Haar transform, the sum with the base convolution, and the way to memory
+  auto finish = [&](const Tile& tl, Acc (&base)[4], Acc (&band)[4], T* obase, int np, bool wait) {
+    if (L >= 2) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) band[0].v[v] += lds_ld<float>(lds, tl.z2 + (2 * (v >> 1) * zpitch2 + 2 * (v & 1)) * 4);
+    }
+    float row[2][8];      // pixel rows y and y + 4, after the exchange
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float s1 = band[0].v[v] + band[1].v[v], d1 = band[0].v[v] - band[1].v[v];
+      const float s2 = band[2].v[v] + band[3].v[v], d2 = band[2].v[v] - band[3].v[v];
+      // a lane has 2 x 2 pixels of each block, the lane 16 further (or back) the ones beside them: after the exchange the
+      // first has the upper row of four, the second the lower one
+      if constexpr (sizeof(T) == 2) {
+        uint32_t up = pack_bf16x2(s1 + s2 + base[v].v[0], s1 - s2 + base[v].v[1]);
+        uint32_t lo = pack_bf16x2(d1 + d2 + base[v].v[2], d1 - d2 + base[v].v[3]);
+        swap_rows16(up, lo);
+        row[v >> 1][2 * (v & 1)] = __uint_as_float(up);
+        row[v >> 1][2 * (v & 1) + 1] = __uint_as_float(lo);
+      } else {
+        uint32_t up[2] = {__float_as_uint(s1 + s2 + base[v].v[0]), __float_as_uint(s1 - s2 + base[v].v[1])};
+        uint32_t lo[2] = {__float_as_uint(d1 + d2 + base[v].v[2]), __float_as_uint(d1 - d2 + base[v].v[3])};
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          swap_rows16(up[j], lo[j]);
+          row[v >> 1][4 * (v & 1) + j] = __uint_as_float(up[j]);
+          row[v >> 1][4 * (v & 1) + 2 + j] = __uint_as_float(lo[j]);
+        }
+      }
+    }
+    // the prefetch of the next unit has had this tile's convolutions to land; waiting for it here, ahead of
+    // the first store, lets the stores drain behind the next unit's work instead of being waited for at its commit
+    if (wait) WT_WAIT_VMEM();
+    if (!tl.valid || tl.p >= np) return;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (tl.y + 4 * half >= H) continue;
+      int to = tl.to;
+      WT_LAUNDER_LANE_INT(to);      // (not added to the tensor's address ahead of the loop)
+      T* dst = sizeof(T) == 2 ? reinterpret_cast<T*>(reinterpret_cast<char*>(obase) + static_cast<size_t>(static_cast<uint32_t>(to) * 2)) + 4 * half * W
+                              : obase + to + 4 * half * W;
+      const int left = W - tl.x;      // columns of the row from here on
+      if constexpr (sizeof(T) == 2) {
+        const uint32_t d[4] = {__float_as_uint(row[half][0]), __float_as_uint(row[half][1]),
+                               __float_as_uint(row[half][2]), __float_as_uint(row[half][3])};
+        if ((Geo::kStatic && W % 8 == 0) || left >= 8) {
+          __builtin_memcpy(dst, d, 16);
+        } else {
+          // 4, 2 and 1 of them
+          if (left & 4) __builtin_memcpy(dst, d, 8);
+          if constexpr (!VEC) {
+            const uint32_t two = left & 4 ? d[2] : d[0], one = left & 4 ? (left & 2 ? d[3] : d[2]) : (left & 2 ? d[1] : d[0]);
+            if (left & 2) __builtin_memcpy(dst + (left & 4), &two, 4);
+            if (left & 1) dst[left & 6] = static_cast<T>(one);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+          if (VEC) {
+            if (e < left) {
+              float4 o4; o4.x = row[half][e]; o4.y = row[half][e + 1]; o4.z = row[half][e + 2]; o4.w = row[half][e + 3];
+              *reinterpret_cast<float4*>(dst + e) = o4;
+            }
+          } else {
+#pragma unroll
+            for (int k = e; k < e + 4; ++k)
+              if (k < left) dst[k] = from_f32<T>(row[half][k]);
+          }
+        }
+      }
+    }
+  };
+  // the fragment table and the resident fragments from the loaded taps
+  auto take_channel = [&] {
+    store_taps();
+    WT_LDS_BARRIER();      // (in the first unit the block-row tables, too)
+    int first = tid;
+    WT_LAUNDER_LANE_INT(first);
+    for (int i = first; i < (pl.nfilt - pl.tskip) * kFragEntries; i += kMfmaBlock) {
+      const int slot = i / kFragEntries, e = i - slot * kFragEntries;
+#pragma unroll
+      for (int j = 0; j < NS; ++j) {
+        const Frag fr = entry_of(j, slot > 0 ? slot + pl.tskip : 0, e);
+        uint4 v; v.x = fr.d[0]; v.y = fr.d[1]; v.z = fr.d[2]; v.w = fr.d[3];
+        lds_st<uint4>(lds, toff + j * tsplit + i * 16, v);
+      }
+    }
+    if constexpr (RES) {
+      int top = ent1_top, bot = ent1_bot;
+      WT_LAUNDER_LANE_INT(top);
+      WT_LAUNDER_LANE_INT(bot);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        ra1t[s][0] = entry_of(0, 1 + s, top);
+        ra1b[s][0] = entry_of(0, 1 + s, bot);
+        WT_SCHED_FENCE();
+      }
+    }
+    bias = lds_ld<float>(lds, pl.taps + pl.tap_rows * kTapRow * 2);
+  };
+  take_channel();
+  Tile own = {};
+  if constexpr (Geo::kStatic) own = tile_of(wave < ntile1 ? wave : 0);      // a wave's first tile, the same in every unit
+  int cur_c = nxt.c;
 #pragma unroll 1
   for (int u = u_begin; u < u_end; ++u) {
-    const int c = u / upc;
-    // The batch is spread evenly over the units of a channel: at most pb items each, all units within one plane of
-    // each other (a short last unit would leave the workgroups that get it with less work than the rest).
-    const int ub = u - c * upc;
-    const int b0 = ub * pl.bq + (ub < pl.br ? ub : pl.br);
-    const int np = pl.bq + (ub < pl.br ? 1 : 0);   // planes of this unit that exist
-    if (c != cur_c) {     // (the previous unit ended with a barrier: nobody still reads the old table)
-      // fold this channel's parameters into the fragment table: filters from `tfirst` on into their
-      // LDS table, the ones before it (held in registers) through the idle Z_1 buffer
-      const int nent = pl.nfilt * kFragEntries;
-      const int nf_lds = (pl.nfilt - pl.tfirst) * kFragEntries;
-      for (int i = tid; i < nent; i += kMfmaBlock) {
-        const int f = i / kFragEntries, e = i - f * kFragEntries;
-        uint4 w[NS];
-        fold_entry<NS>(prm, pdtype, K, flip, c, f, e, w);
-#pragma unroll
-        for (int j = 0; j < NS; ++j) {
-          const int o = f >= pl.tfirst ? toff + (j * nf_lds + i - pl.tfirst * kFragEntries) * 16 : zoff1 + (j * pl.tfirst * kFragEntries + i) * 16;
-          lds_st<uint4>(lds, o, w[j]);
-        }
-      }
-      bias = (use_bias && prm.base_bias != nullptr)
-                 ? load_param(prm.base_bias, pdtype, c) * load_param(prm.base_scale, pdtype, c) : 0.f;
+    const Unit un = nxt;
+    const int c = un.c, b0 = first_item(un), np = items(un);
+    if (++nxt.ub == upc) { nxt.ub = 0; ++nxt.c; }
+    if (c != cur_c) {      // (every read of the old filters lies behind a barrier)
+      load_taps(c);
+      take_channel();
       cur_c = c;
-      if constexpr (RES) {
-        WT_LDS_BARRIER();
-        ra0t[0] = lds_frag16(lds, zoff1 + ent_top * 16);
-        ra0b[0] = lds_frag16(lds, zoff1 + ent_bot * 16);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          ra1t[s][0] = lds_frag16(lds, zoff1 + ((1 + s) * kFragEntries + ent_top) * 16);
-          ra1b[s][0] = lds_frag16(lds, zoff1 + ((1 + s) * kFragEntries + ent_bot) * 16);
-        }
-      }
     }
 
     // ---- commit: pixels -> level-0 planes; analysis levels 1 and 2 from registers
 #pragma unroll
     for (int i = 0; i < NBL; ++i) {
       if (!(c_mask[i] & 0x100u)) continue;
+      int x0 = c_x0[i], a1 = c_a1[i], a2 = c_a2[i];
+      WT_LAUNDER_LANE_INT(x0);      // (the sums with the plan's fields below are not kept from unit to unit)
+      WT_LAUNDER_LANE_INT(a1);
+      WT_LAUNDER_LANE_INT(a2);
       float v[4][4];
-      if constexpr (!VEC && sizeof(T) == 2) {      // clear the columns that came along from past the row end
+      if constexpr (kOver) {      // clear what came along from past the row and the plane
         const uint2 m = pix_col_mask(c_mask[i]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) { pf[i][r].v.x &= m.x; pf[i][r].v.y &= m.y; }
+        for (int r = 0; r < 4; ++r) {
+          const bool row = c_mask[i] >> r & 1u;
+          pf[i][r].v.x &= row ? m.x : 0u;
+          pf[i][r].v.y &= row ? m.y : 0u;
+        }
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) pix_get(pf[i][r], v[r]);
@@ -633,7 +856,7 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
         }
 #pragma unroll
         for (int j = 0; j < NS; ++j) {
-          const int o = c_x0[i] + j * asub0 + r * pitchB0;
+          const int o = x0 + j * asub0 + r * pitchB0;
           lds_st<uint32_t>(lds, o, w0[j]);
           lds_st<uint32_t>(lds, o + 4, w1[j]);
         }
@@ -656,7 +879,7 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
           split_pair<NS>(cf[s][0], cf[s][1], w);
 #pragma unroll
           for (int j = 0; j < NS; ++j)
-            lds_st<uint32_t>(lds, c_a1[i] + (j * 4 + s) * asub1 + i2 * pitchB1, w[j]);
+            lds_st<uint32_t>(lds, a1 + (j * 4 + s) * asub1 + i2 * pitchB1, w[j]);
         }
       }
       if (L >= 2) {
@@ -669,75 +892,61 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
           split_pair<NS>(cf[s], 0.f, w);
 #pragma unroll
           for (int j = 0; j < NS; ++j)
-            lds_st<uint16_t>(lds, c_a2[i] + (j * 4 + s) * asub2, static_cast<uint16_t>(w[j]));
+            lds_st<uint16_t>(lds, a2 + (j * 4 + s) * asub2, static_cast<uint16_t>(w[j]));
         }
         if (L >= 3) lds_st<float>(lds, c_ll[i], cf[0]);
       }
     }
-    if (u + 1 < u_end) fetch(u + 1);
+    if (u + 1 < u_end) fetch(nxt);
     WT_LDS_BARRIER();
 
-    // ---- analysis levels 3..L from the raw LL of the level above (fp32 in LDS)
-    levels_up<Geo, 3>(L, [&](auto lc) {
-      const int l = lc;
-      const int hl = pl.h[l], wl = pl.w[l], npos = pb * hl * wl;
-      for (int idx = tid; idx < npos; idx += kMfmaBlock) {
-        const int p = fast_div(idx, pl.mg_hw[l]);
-        const int rem = idx - imul(p, hl * wl);
-        const int i = fast_div(rem, pl.mg_w[l]);
-        const int j = rem - imul(i, wl);
-        const int hs = pl.h[l - 1], wsrc = pl.w[l - 1];
-        const int so = pl.lloff[l - 1] + (imul(p, pl.llpl[l - 1]) + imul(2 * i, wsrc) + 2 * j) * 4;
-        const bool r1 = 2 * i + 1 < hs, c1 = 2 * j + 1 < wsrc;
-        const float a = lds_ld<float>(lds, so);
-        const float b = c1 ? lds_ld<float>(lds, so + 4) : 0.f;
-        const float cc = r1 ? lds_ld<float>(lds, so + wsrc * 4) : 0.f;
-        const float d = (r1 && c1) ? lds_ld<float>(lds, so + wsrc * 4 + 4) : 0.f;
-        const float s1 = a + b, d1 = a - b, s2 = cc + d, d2 = cc - d;
-        const float cf[4] = {s1 + s2, s1 - s2, d1 + d2, d1 - d2};
-        const int ao = pl.aoff[l] + (imul(imul(p, pl.prows[l]) + i + 2, pl.pitch[l]) + j + 2) * 2;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          uint32_t w[NS];
-          split_pair<NS>(cf[s], 0.f, w);
-#pragma unroll
-          for (int js = 0; js < NS; ++js)
-            lds_st<uint16_t>(lds, ao + (js * 4 + s) * pl.asub[l], static_cast<uint16_t>(w[js]));
-        }
-        if (l < L) lds_st<float>(lds, pl.lloff[l] + (imul(p, pl.llpl[l]) + imul(i, wl) + j) * 4, cf[0]);
-      }
-      WT_LDS_BARRIER();
-    });
-
-    // ---- stage 1: the last wave runs levels L..2 (conv + inverse Haar -> Z_l), the others the base
-    // conv and, when every wave has at most one level-1 tile, the detail sub-bands of that tile
-    const int base_waves = L >= 2 ? 3 : 4;
-    // level-1 convolution of sub-band s of a tile into acc (resident or table fragments)
-    auto conv1 = [&](const TileLane& tl, int s, Acc& acc) {
-      Frag bt[NS], bb[NS];
-      load_b<NS>(lds, tl.boff + s * asub1, 4 * asub1, 4 * pitchB1, bt, bb);
-      if constexpr (RES) {
-        mma_tile<NS>(ra1t[s], ra1b[s], bt, bb, acc);
-      } else {
-        Frag at[NS], ab[NS];
-        load_a<NS>(lds, toff + (1 + s - pl.tfirst) * kFragEntries * 16, tsplit, ent_top, ent_bot, at, ab);
-        mma_tile<NS>(at, ab, bt, bb, acc);
-      }
-    };
-    const bool early = ntile1 <= 4 && L >= 2;   // every wave's single level-1 tile starts before the barrier
-    TileLane tl1 = {};
-    Acc acc1[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc1[s].v[0] = acc1[s].v[1] = acc1[s].v[2] = acc1[s].v[3] = 0.f;
+    // ---- the last wave: levels L..2 on its own (the others wait for this chain at the barrier)
     if (L >= 2 && wave == 3) {
-      WT_WAVE_PRIORITY(3);        // the other waves wait for this chain at the barrier
+      WT_WAVE_PRIORITY(3);
+      // (lane numbers that the compiler cannot see through: it would keep every address below in registers from unit to unit)
+      int n = lane & 15, q = lane >> 4, lane_ = lane;
+      WT_LAUNDER_LANE_INT(n);
+      WT_LAUNDER_LANE_INT(q);
+      WT_LAUNDER_LANE_INT(lane_);
+      // analysis levels 3..L from the raw LL of the level above (fp32 in LDS)
+      levels_up<Geo, 3>(L, [&](auto lc) {
+        const int l = lc;
+        const int hl = pl.h[l], wl = pl.w[l], npos = pb * hl * wl;
+        for (int idx = lane_; idx < npos; idx += 64) {
+          const int p = fast_div(idx, pl.mg_hw[l]);
+          const int rem = idx - imul(p, hl * wl);
+          const int i = fast_div(rem, pl.mg_w[l]);
+          const int j = rem - imul(i, wl);
+          const int hs = pl.h[l - 1], wsrc = pl.w[l - 1];
+          const int so = pl.lloff[l - 1] + (imul(p, pl.llpl[l - 1]) + imul(2 * i, wsrc) + 2 * j) * 4;
+          const bool r1 = 2 * i + 1 < hs, c1 = 2 * j + 1 < wsrc;
+          const float a = lds_ld<float>(lds, so);
+          const float b = c1 ? lds_ld<float>(lds, so + 4) : 0.f;
+          const float cc = r1 ? lds_ld<float>(lds, so + wsrc * 4) : 0.f;
+          const float d = (r1 && c1) ? lds_ld<float>(lds, so + wsrc * 4 + 4) : 0.f;
+          const float s1 = a + b, d1 = a - b, s2 = cc + d, d2 = cc - d;
+          const float cf[4] = {s1 + s2, s1 - s2, d1 + d2, d1 - d2};
+          const int ao = pl.aoff[l] + (imul(imul(p, pl.prows[l]) + i + 2, pl.pitch[l]) + j + 2) * 2;
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            uint32_t w[NS];
+            split_pair<NS>(cf[s], 0.f, w);
+#pragma unroll
+            for (int js = 0; js < NS; ++js)
+              lds_st<uint16_t>(lds, ao + (js * 4 + s) * pl.asub[l], static_cast<uint16_t>(w[js]));
+          }
+          if (l < L) lds_st<float>(lds, pl.lloff[l] + (imul(p, pl.llpl[l]) + imul(i, wl) + j) * 4, cf[0]);
+        }
+        WT_WAVE_SYNC_DIVERGENT();
+      });
+      // convolutions and inverse Haar transforms -> Z_l
       levels_down<Geo, 2>(L, [&](auto lc) {
         const int l = lc;
         const int ntile = pl.ntile[l];
         const int pitchB = pl.pitch[l] * 2, asub = pl.asub[l];
         const int zo_in = pl.zoff[l + 1], zp_in = pl.zpitch[l + 1], zpl_in = pl.zpl[l + 1];
         const int zo = pl.zoff[l], zp = pl.zpitch[l], zpl_o = pl.zpl[l], zrows = 4 * pl.nbr[l - 1];
-        const int tab = toff + (1 + 4 * (l - 1) - pl.tfirst) * kFragEntries * 16;
+        const int tab = toff + (1 + 4 * (l - 1) - pl.tskip) * kFragEntries * 16;
 #pragma unroll 1
         for (int t = 0; t < ntile; ++t) {
           const TileLane tl = tile_lane(lds, t, n, q, pl.tcs[l], pl.nrow[l], pl.nbc[l], pl.rtoff[l], pl.aoff[l], pitchB);
@@ -748,23 +957,17 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
             const float4 z = lds_ld<float4>(lds, zo_in + (imul(tl.p, zpl_in) + imul(4 * tl.bi + q, zp_in) + 4 * tl.tc) * 4);
             acc[0].v[0] = z.x; acc[0].v[1] = z.y; acc[0].v[2] = z.z; acc[0].v[3] = z.w;
           }
-          if constexpr (NS == 1) {       // every LDS read of the tile is issued before the first MFMA
-            Frag at[4][NS], ab[4][NS], bt[4][NS], bb[4][NS];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-              load_b<NS>(lds, tl.boff + s * asub, 4 * asub, 4 * pitchB, bt[s], bb[s]);
-              load_a<NS>(lds, tab + s * kFragEntries * 16, tsplit, ent_top, ent_bot, at[s], ab[s]);
+          for (int s2 = 0; s2 < 4; s2 += 2) {      // (the LDS reads of all four sub-bands at once would not fit the registers)
+            Frag at[2][NS], ab[2][NS], bt[2][NS], bb[2][NS];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              load_b<NS>(lds, tl.boff + (s2 + k) * asub, 4 * asub, 4 * pitchB, bt[k], bb[k]);
+              load_a<NS>(lds, tab + (s2 + k) * kFragEntries * 16, tsplit, ent_top, ent_bot, at[k], ab[k]);
             }
 #pragma unroll
-            for (int s = 0; s < 4; ++s) mma_tile<NS>(at[s], ab[s], bt[s], bb[s], acc[s]);
-          } else {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-              Frag at[NS], ab[NS], bt[NS], bb[NS];
-              load_b<NS>(lds, tl.boff + s * asub, 4 * asub, 4 * pitchB, bt, bb);
-              load_a<NS>(lds, tab + s * kFragEntries * 16, tsplit, ent_top, ent_bot, at, ab);
-              mma_tile<NS>(at, ab, bt, bb, acc[s]);
-            }
+            for (int k = 0; k < 2; ++k) mma_tile<NS>(at[k], ab[k], bt[k], bb[k], acc[s2 + k]);
+            WT_SCHED_FENCE();
           }
           float top[8], bot[8];
           synth_rows(acc, top, bot);
@@ -787,131 +990,26 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
       });
       WT_WAVE_PRIORITY(0);
     }
-    if (wave < base_waves) {
-      // contiguous tile range per wave; with one plane per unit and one block-row per tile the lower
-      // patch half of a tile is the upper half of the next one and is loaded once
-      const int t0 = wave * ntile0 / base_waves, t1 = (wave + 1) * ntile0 / base_waves;
-      const bool chain = pb == 1 && tcs0 == 4;
-      Frag at[NS], ab[NS], bt[NS], bb[NS];
-      if constexpr (!RES) load_a<NS>(lds, toff - pl.tfirst * kFragEntries * 16, tsplit, ent_top, ent_bot, at, ab);
-      bool have_top = false;
-#pragma unroll 1
-      for (int t = t0; t < t1; ++t) {
-        const TileLane tl = tile_lane(lds, t, n, q, tcs0, nrow0, nbc0, rtoff0, aoff0, pitchB0);
-        if (chain && have_top) {
-#pragma unroll
-          for (int j = 0; j < NS; ++j) {
-            bt[j] = bb[j];
-            bb[j] = lds_frag8(lds, tl.boff + j * asub0 + 4 * pitchB0);
-          }
-        } else {
-          load_b<NS>(lds, tl.boff, asub0, 4 * pitchB0, bt, bb);
-        }
-        have_top = true;
-        Acc acc;
-        acc.v[0] = acc.v[1] = acc.v[2] = acc.v[3] = bias;
-        if constexpr (RES) mma_tile<NS>(ra0t, ra0b, bt, bb, acc);
-        else mma_tile<NS>(at, ab, bt, bb, acc);
-        if (tl.valid) {
-          float4 a; a.x = acc.v[0]; a.y = acc.v[1]; a.z = acc.v[2]; a.w = acc.v[3];
-          lds_st<float4>(lds, zoff1 + (imul(tl.p, zpl1) + imul(4 * tl.bi + q, zpitch1) + 4 * tl.tc) * 4, a);
-        }
-      }
-    }
-    // the detail sub-bands of this wave's level-1 tile: they need nothing of this stage (the coarse-chain wave
-    // runs them after its chain, which is shorter than the base-conv share of the others)
-    if (early && wave < ntile1) {
-      tl1 = tile_lane(lds, wave, n, q, tcs1, nrow1, nbc1, rtoff1, aoff1, pitchB1);
-#pragma unroll
-      for (int s = 1; s < 4; ++s) conv1(tl1, s, acc1[s]);
+    // ---- level 1 and base conv: each wave's first tile up to the barrier, which Z_2 is waited for at
+    Acc base[4], band[4];
+    T* obase = out + (static_cast<size_t>(b0) * C + c) * HW;
+    if (wave < ntile1) {
+      if constexpr (!Geo::kStatic) own = tile_of(wave);      // (the run-time plan's fields leave no registers to keep it in)
+      convolve(own, base, band);
     }
     WT_LDS_BARRIER();
-
-    // ---- stage 2: level 1 (conv, inverse Haar), plus the base conv from Z_1, to HBM
-    {
-      T* obase = out + (static_cast<size_t>(b0) * C + c) * HW;
-      bool first_store = true;
+    if (wave < ntile1) finish(own, base, band, obase, np, true);
+    if (ntile1 > 4) {
 #pragma unroll 1
-      for (int t = wave; t < ntile1; t += 4) {
-        if (!early) {
-          tl1 = tile_lane(lds, t, n, q, tcs1, nrow1, nbc1, rtoff1, aoff1, pitchB1);
-#pragma unroll
-          for (int s = 0; s < 4; ++s) acc1[s].v[0] = acc1[s].v[1] = acc1[s].v[2] = acc1[s].v[3] = 0.f;
-        }
-        const int y = 2 * (4 * tl1.bi + q), xx = 8 * tl1.tc;
-        const bool store_ok = tl1.valid && tl1.p < np;
-        // the base-conv part of this lane's 2 x 8 pixels, read ahead of the convolutions
-        const int zbase = zoff1 + (imul(tl1.p, zpl1) + imul(y, zpitch1) + xx) * 4;
-        float4 z1[2][2];
-#pragma unroll
-        for (int rr = 0; rr < 2; ++rr)
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            z1[rr][half].x = z1[rr][half].y = z1[rr][half].z = z1[rr][half].w = 0.f;
-            if (store_ok && y + rr < H && xx + 4 * half < W)
-              z1[rr][half] = lds_ld<float4>(lds, zbase + (rr * zpitch1 + 4 * half) * 4);
-          }
-        if (L >= 2) {
-          const float4 z = lds_ld<float4>(lds, zoff2 + (imul(tl1.p, zpl2) + imul(4 * tl1.bi + q, zpitch2) + 4 * tl1.tc) * 4);
-          acc1[0].v[0] = z.x; acc1[0].v[1] = z.y; acc1[0].v[2] = z.z; acc1[0].v[3] = z.w;
-        }
-        conv1(tl1, 0, acc1[0]);
-        if (!early) {
-#pragma unroll
-          for (int s = 1; s < 4; ++s) conv1(tl1, s, acc1[s]);
-        }
-        float top[8], bot[8];
-        synth_rows(acc1, top, bot);
-        if (first_store) {
-          // the prefetch of the next unit has had this tile's convolutions to land; waiting for it here, ahead of
-          // the first store, lets the stores drain behind the next unit's work instead of being waited for at its commit
-          WT_WAIT_VMEM();
-          first_store = false;
-        }
-        if (store_ok) {
-          T* dbase = obase + static_cast<size_t>(tl1.p) * C * HW + imul(y, W) + xx;
-#pragma unroll
-          for (int rr = 0; rr < 2; ++rr) {
-            if (y + rr >= H) continue;
-            float* vals = rr ? bot : top;
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-              const int x0 = xx + 4 * half;
-              if (x0 >= W) continue;
-              const float4 z = z1[rr][half];
-              const float r0 = vals[4 * half] + z.x, r1 = vals[4 * half + 1] + z.y;
-              const float r2 = vals[4 * half + 2] + z.z, r3 = vals[4 * half + 3] + z.w;
-              T* dst = dbase + rr * W + 4 * half;
-              if constexpr (VEC) {
-                if constexpr (sizeof(T) == 4) {
-                  float4 o4; o4.x = r0; o4.y = r1; o4.z = r2; o4.w = r3;
-                  *reinterpret_cast<float4*>(dst) = o4;
-                } else {
-                  uint2 o2; o2.x = pack_bf16x2(r0, r1); o2.y = pack_bf16x2(r2, r3);
-                  *reinterpret_cast<uint2*>(dst) = o2;
-                }
-              } else if constexpr (sizeof(T) == 2) {
-                if (x0 + 3 < W) {      // four columns inside the row: one (unaligned) 8-byte store
-                  uint2 o2; o2.x = pack_bf16x2(r0, r1); o2.y = pack_bf16x2(r2, r3);
-                  pix_store4u(dst, o2);
-                } else {
-                  const float r[4] = {r0, r1, r2, r3};
-#pragma unroll
-                  for (int e = 0; e < 4; ++e)
-                    if (x0 + e < W) dst[e] = from_f32<T>(r[e]);
-                }
-              } else {
-                const float r[4] = {r0, r1, r2, r3};
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                  if (x0 + e < W) dst[e] = from_f32<T>(r[e]);
-              }
-            }
-          }
-        }
+      for (int t = wave + 4; t < ntile1; t += 4) {
+        const Tile tl = tile_of(t);
+        convolve(tl, base, band);
+        finish(tl, base, band, obase, np, false);
       }
+      WT_LDS_BARRIER();      // the next unit's commit overwrites what these tiles read
     }
-    WT_LDS_BARRIER();
+    // (With one tile a wave nothing but Z_2 is read behind the barrier above, and Z_2 is written next behind the barrier
+    // that follows the next commit.)
   }
 }
 

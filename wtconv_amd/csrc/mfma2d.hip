@@ -105,6 +105,15 @@ bool choose_mplan_uncached(int B, int C, int H, int W, int L, int NS, MPlan* out
       }
     }
   }
+  // a tile of level-1 blocks less, where it costs no more than a tenth of the planes (7 x 7: 32 of them instead of 33 fill two),
+  // and four tiles, one a wave, instead of more, where it costs no more than a quarter (12 x 12: 16 instead of 19)
+  for (int p2 = pb - 1; p2 * 4 >= pb * 3; --p2) {
+    MPlan alt;
+    if (make_mplan(B, C, H, W, L, NS, p2, &alt) && alt.ntile[1] < pl.ntile[1] && (alt.ntile[1] == 4 || p2 * 10 >= pb * 9)) {
+      pl = alt;
+      break;
+    }
+  }
   if (static_cast<size_t>(pl.lds_bytes) > lds_budget()) return false;
   const int per_thread = ceil_div(pl.nblk[0], kMfmaBlock);
   if (per_thread > 4) return false;
@@ -128,8 +137,11 @@ int launch_mfma(const void* x, void* out, const MfmaArgs& a, const MPlan& pl, hi
   if (int e = allow_lds(kern, lds)) return e;
   int nwg = compute_units() * resident_per_cu(kern, kMfmaBlock, lds);
   if (nwg > pl.nunits) nwg = pl.nunits;
+  MPlan arg = pl;
+  arg.uq = pl.nunits / nwg;
+  arg.ur = pl.nunits % nwg;
   WT_LAUNCH(kern, dim3(nwg), dim3(kMfmaBlock), lds, stream, static_cast<const T*>(x), static_cast<T*>(out), a.prm,
-            a.pdtype, a.K, a.flip, a.use_bias, pl, a.zero_words, a.nzero);
+            a.pdtype, a.K, a.flip, a.use_bias, arg, a.zero_words, a.nzero);
   return check_launch("wt2d_mfma_kernel");
 }
 
@@ -158,8 +170,8 @@ int launch_mfma_nbl(int nbl, bool vec, const void* x, void* out, const MfmaArgs&
 #define WT_TRY(H_, L_, PB_, VEC_) \
   if (try_static<T, NS, H_, L_, PB_, VEC_>(vec, x, out, a, pl, stream, &rc)) return rc;
   if constexpr (NS == 1) {
-    WT_TRY(56, 3, 1, true) WT_TRY(28, 3, 4, true) WT_TRY(14, 2, 11, false) WT_TRY(7, 2, 29, false)
-    WT_TRY(56, 5, 1, true) WT_TRY(28, 4, 4, true) WT_TRY(14, 3, 9, false)
+    WT_TRY(56, 3, 1, true) WT_TRY(28, 3, 4, true) WT_TRY(14, 2, 15, false) WT_TRY(7, 2, 32, false)
+    WT_TRY(56, 5, 1, true) WT_TRY(28, 4, 4, true) WT_TRY(14, 3, 12, false)
   } else {
     WT_TRY(56, 3, 1, true) WT_TRY(28, 3, 2, true) WT_TRY(14, 2, 9, false) WT_TRY(7, 2, 21, false)
   }
