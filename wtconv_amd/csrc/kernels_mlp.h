@@ -20,10 +20,16 @@
 //
 // LayerNorm needs all channels of a pixel and the wave has them: the statistics are two exact passes over its registers.
 //
-// What bounds it: with few channels the vector pipe (GELU, 28 cycles a value against 6 of matrix work at C = 96), with many
-// the LDS that feeds the matrix cores (one fragment read for NT products; at C = 384, NT = 1, both are busy all the time).
+// What bounds it: with few channels the vector pipe (busy 91 % of the time at C = 96, most of it GELU, which costs 59 us of
+// 226 there, 33 of 175 at C = 192, 24 of 175 at C = 384), with many nothing alone: at C = 384 the vector pipe is busy a third of
+// the time, LDS 29 % and the matrix cores 27 %; the pixels' way in and out with LayerNorm is 30 % of a tile's time, and 392 tiles
+// are 1.53 rounds of the compute units.  Two pixel tiles a wave and one wave a SIMD there (accumulators in accumulation
+// registers, half the LDS reads) took 205: a lone wave issues half as often.  Smaller tiles for the last round gave nothing
+// (a SIMD with two waves takes as long as all with two) and 192 channels 1 % less.
 // Measured at batch 256, us a block, the passes it replaces (norm, fc1, GELU, fc2, residual) -> this kernel: 56 x 56 x 96
-// 917 -> 243 (490 TFLOP/s), 28 x 28 x 192 455 -> 187, 14 x 14 x 384 295 -> 182 (650 TFLOP/s); 56 x 56 x 128 1059 -> 350, 28 x 28 x 256 609 -> 346.
+// 917 -> 222 (530 TFLOP/s), 28 x 28 x 192 455 -> 168, 14 x 14 x 384 295 -> 171 (690 TFLOP/s); 56 x 56 x 128 1059 -> 342,
+// 28 x 28 x 256 609 -> 338.  (228, 173, 179, 352 and 349 with a stage's loads in one piece, the first one's behind LayerNorm
+// and a clamp in GELU.)
 #pragma once
 
 #include "gelu.h"
@@ -62,11 +68,14 @@ struct MlpShape {
   static constexpr int kStageBytes = 2 * kSliceBytes;       // W1's slice i and W2's slice i - 1
   static_assert(C % 32 == 0 && kGranules % 64 == 0, "slices are loaded by whole waves");
   // The pixels of the workgroup pass through LDS on the way in and out, [channel][pixel] with a padding that puts the
-  // rows 8q apart on different banks.  (Before the first and after the last slice: the memory is the ring's.)
+  // rows 8q apart on different banks.  (The memory is the ring's.  On the way in they lie at its end, behind W1's first
+  // slice, which is on its way meanwhile; on the way out all slices are done with.)
   static constexpr int kPitch = PX + 4;
   static constexpr int kTileBytes = C * kPitch * 2;
   static_assert(RING == 3, "see the pipeline");
   static constexpr int kRegionBytes = RING * kStageBytes > kTileBytes ? RING * kStageBytes : kTileBytes;
+  static constexpr int kTileAt = kRegionBytes - kTileBytes / 16 * 16 - 16;
+  static_assert(kTileAt >= kSliceBytes, "W1's first slice lies before the pixels");
   static constexpr size_t lds_bytes(int hidden_here) { return kRegionBytes + 4 * static_cast<size_t>(hidden_here); }
 
   // Where granule g of row r sits within its row.  The LDS serves a 16-byte read in four goes of 16 lanes -- lanes 0-3,
@@ -113,26 +122,25 @@ block_mlp_kernel(MlpArgs a) {
   }
   const lds_addr lds0 = WT_LDS_ADDR(mlp_lds);
   auto holds = [&](int k) { return (k + 1) * S::kThreads <= S::kGranules || k * S::kThreads + wave * 64 < S::kGranules; };
-  // stage i of the ring: W1's slice i and W2's slice i - 1, as far as they exist (slices counted from s_begin)
-  auto load_stage = [&](int i, int at) {
+  // stage i of the ring: W1's slice i and W2's slice i - 1, as far as they exist (slices counted from s_begin); its loads
+  // k = 0 .. 2 kLoads
+  auto load_piece = [&](int i, int at, int k) {
     const lds_addr dst = WT_UNIFORM(lds0 + at * S::kStageBytes + wave * 1024);
-    if (i < nsl) {
-      const bf16_t* w1 = a.w1 + static_cast<size_t>(h0 + i * HC) * C;
-#pragma unroll
-      for (int k = 0; k < S::kLoads; ++k)
-        if (holds(k)) granules_to_lds(w1, src1[k], dst + k * (S::kThreads * 16));
+    if (k < S::kLoads) {
+      if (i < nsl && holds(k)) granules_to_lds(a.w1 + static_cast<size_t>(h0 + i * HC) * C, src1[k], dst + k * (S::kThreads * 16));
+    } else if (i > 0 && i <= nsl && holds(k - S::kLoads)) {
+      granules_to_lds(a.w2 + (h0 + (i - 1) * HC), src2[k - S::kLoads], dst + S::kSliceBytes + (k - S::kLoads) * (S::kThreads * 16));
     }
-    if (i > 0) {
-      const bf16_t* w2 = a.w2 + (h0 + (i - 1) * HC);
+  };
+  auto load_stage = [&](int i, int at) {
 #pragma unroll
-      for (int k = 0; k < S::kLoads; ++k)
-        if (holds(k)) granules_to_lds(w2, src2[k], dst + S::kSliceBytes + k * (S::kThreads * 16));
-    }
+    for (int k = 0; k < 2 * S::kLoads; ++k) load_piece(i, at, k);
   };
   for (int i = tid; i < nsl * HC; i += S::kThreads) bias_lds[i] = bf16_to_f32(a.b1[h0 + i]);
 
   // ---- the pixels, into LDS.  This thread's group of them, and the channels it moves: row, row + rows, ...
-  bf16_t* tile = reinterpret_cast<bf16_t*>(mlp_lds);
+  load_stage(0, 0);
+  bf16_t* tile = reinterpret_cast<bf16_t*>(mlp_lds + S::kTileAt);
   auto for_pixels = [&](auto vec, auto&& load, auto&& use) {      // load(offset in memory), use(value, channel, offset, offset in the tile)
     constexpr int V = decltype(vec)::value, groups = S::PX / V, rows = S::kThreads / groups, iters = C / rows;
     constexpr int U = iters % 12 == 0 ? 12 : (iters % 8 == 0 ? 8 : 6);      // in flight at once
@@ -249,10 +257,11 @@ block_mlp_kernel(MlpArgs a) {
       if (s % 2 == 1) WT_CHUNK_FENCE();
     }
   }
+  WT_WAIT_VMEM();       // (the first slice)
   __syncthreads();      // the tile has been read: the ring may be filled
 
-  load_stage(0, 0);
   load_stage(1, 1);
+  load_stage(2, 2);
   auto frag = [](const uint32_t (&v)[4]) { return frag_of(uint4{v[0], v[1], v[2], v[3]}); };
 
   mat_acc acc[MT][NT];
@@ -270,8 +279,6 @@ block_mlp_kernel(MlpArgs a) {
   for (int s = 0; s < KS; ++s) go1[s] = S::swz1(row1, 4 * s + q) * 16;
 #pragma unroll
   for (int g = 0; g < HC / 32; ++g) go2[g] = S::swz2(n, 4 * g + q) * 16;
-  WT_WAIT_VMEM();
-  __syncthreads();
 
   // ---- the slices, in a software pipeline: iteration i multiplies W1's slice i while the vector pipe is at the GELU of
   // slice i - 1, and then W2's slice i - 1.  The one barrier of an iteration is in its middle: behind it stage i + 1 has
@@ -304,13 +311,11 @@ block_mlp_kernel(MlpArgs a) {
     const int g = k / (NT * 4), t = k / 4 % NT, m = k / 2 % 2, r = k % 2 * 2;
     hf[g][t][2 * m + k % 2] = pack_bf16x2(gelu_erf(h[g][m][t][r]), gelu_erf(h[g][m][t][r + 1]));
   };
-  auto middle = [&](int i) {
+  auto middle = [&] {
     asm volatile("" ::: "memory");
     WT_WAIT_VMEM();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (i + 2 <= nsl) load_stage(i + 2, fill);
-    fill = fill == 2 ? 0 : fill + 1;
   };
   auto after = [&](const unsigned char* st) { return st == mlp_lds + 2 * S::kStageBytes ? mlp_lds : st + S::kStageBytes; };
   // A product step is one fragment read (kAhead steps before it is used) and its NT products; the GELU of a pair of values
@@ -333,7 +338,8 @@ block_mlp_kernel(MlpArgs a) {
       WT_SCHED_FENCE();
     }
   };
-  auto second_product = [&](const unsigned char* next, int ahead, auto then_first) {
+  // (`load`: the stage whose loads are issued on the way)
+  auto second_product = [&](const unsigned char* next, int ahead, int load, auto then_first) {
 #pragma unroll
     for (int j = 0; j < N2; ++j) {
 #pragma unroll
@@ -346,8 +352,14 @@ block_mlp_kernel(MlpArgs a) {
         if (j + kAhead == N2) start(next, ahead);
         w[j % kAhead] = fetch1(next, j + kAhead - N2);
       }
+      if (decltype(then_first)::value) {
+#pragma unroll
+        for (int k = 0; k < 2 * S::kLoads; ++k)
+          if (k * N2 / (2 * S::kLoads) == j) load_piece(load, fill, k);
+      }
       WT_SCHED_FENCE();
     }
+    fill = fill == 2 ? 0 : fill + 1;
   };
   auto keep = [&] {
 #pragma unroll
@@ -364,7 +376,8 @@ block_mlp_kernel(MlpArgs a) {
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) w[j] = fetch1(stage, j);
   first_product(false_type{}, false_type{});
-  middle(0);
+  middle();
+  fill = 0;
   stage = after(stage);
   keep();
   if (nsl > 1) {
@@ -377,10 +390,10 @@ block_mlp_kernel(MlpArgs a) {
     // that, the last one again (which costs 1 to 3 %: 384 channels 190 -> 192 us, 96 channels 222 -> 229)
     const int ahead = ROOM || i + 1 < nsl ? i + 1 : i;
     first_product(true_type{}, true_type{});
-    middle(i);
+    middle();
     keep();
     const unsigned char* next = after(stage);
-    second_product(next, ahead, true_type{});      // (behind the last slice the reads ahead are of a stage nobody fills: unused)
+    second_product(next, ahead, i + 2, true_type{});      // (behind the last slice the reads ahead are of a stage nobody fills: unused)
     stage = next;
   }
   // the last slice through W2
@@ -388,10 +401,11 @@ block_mlp_kernel(MlpArgs a) {
   for (int k = 0; k < PACKS; ++k) activate(k);
 #pragma unroll
   for (int j = 0; j < kAhead; ++j) w[j] = fetch2(stage, j);
-  second_product(stage, nsl, false_type{});
+  second_product(stage, nsl, 0, false_type{});
   __syncthreads();
 
   // ---- lane (n, q) holds channels 16 m + 4 q + 0..3 of its pixels
+  tile = reinterpret_cast<bf16_t*>(mlp_lds);
   if (a.splits > 1) {
     float* part = a.partial + static_cast<size_t>(blockIdx.y) * C * a.padded + blockIdx.x * S::PX + p_lane;
 #pragma unroll
