@@ -24,6 +24,9 @@ pytestmark = pytest.mark.gpu
     ((40, 9, 45, 50), 3, 2, torch.float32),       # K = 3: strips of two, odd rows a pass
     ((300, 1, 87, 66), 7, 1, torch.float32),      # 512 threads a plane, rows of 17 strips
     ((2, 130, 5, 77), 7, 2, torch.float32),       # three rows of 39 coefficients
+    ((3, 4, 13, 255), 5, 2, torch.float32),       # parameter gradients: one row of 64 strips a wave
+    ((4, 6, 30, 9), 3, 2, torch.float32),         # 21 rows of three strips
+    ((5, 4, 21, 82), 7, 1, torch.float16),        # three rows of 21, one lane without
 ])
 def test_layer_against_fp64(hip_device, shape, K, L, dtype):
     import wtconv

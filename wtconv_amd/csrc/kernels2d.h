@@ -33,6 +33,8 @@ __device__ __forceinline__ int row_of(const RowSplit& s, int t) {
 }
 
 // LDS layout of one plane, computed on the host (plan.h).
+constexpr int kStripMinWidth = 12;   // coarse levels of the weight-gradient kernel: strips from this width on
+
 struct Plan2D {
   int C, H, W, L;
   int P;                       // halo width of the pyramid buffers: max(K/2, 1)
@@ -63,7 +65,8 @@ struct Plan2D {
   int fw_skip;                 //   floats between where the level filters would follow the base filter and where they
                                //   are (a sub-layer's base filter is the LL filter of the level above it)
   RowSplit strips1;            // plane kernel: the strips of level 1 over the threads of a plane
-  RowSplit coefs[kMaxLevels + 1];      // and the single coefficients of level l >= 2 (analysis and synthesis)
+  RowSplit coefs[kMaxLevels + 1];      // and the single coefficients of level l >= 2 (synthesis)
+  RowSplit corr[kMaxLevels + 1];       // weight-gradient kernel: strips (or coefficients) of level l over the lanes of a wave
 };
 
 // ------------------------------------------------------------------ parameter folding
@@ -941,23 +944,20 @@ __device__ __forceinline__ void corr_strip2(const float* __restrict__ a, int ast
 // row under every stacked plane).
 template <int K, int TJ, int VW, bool PAIR>
 __device__ __forceinline__ void corr_level(const float* __restrict__ A, int astr, const float* __restrict__ G,
-                                           int gstr, int h, int w, int lane, int pass_row0, int pass_step,
+                                           int gstr, int h, const RowSplit split, int lane, int pass_row0, int pass_step,
                                            float (&acc)[K * K]) {
-  const int nstrip = (w + TJ - 1) / TJ;
-  const int gsh = group_shift(nstrip);
-  const int strip = lane & ((1 << gsh) - 1);
-  if (strip >= nstrip) return;
-  const int j0 = strip * TJ;
-  const int rpp = kWave >> gsh;          // row items per pass of one wave (>= 1: kMaxWgradWidth, plan.h)
+  const int row = row_of(split, lane), rpp = split.rows;      // row items per pass of one wave (>= 1: kMaxWgradWidth, plan.h)
+  if (row >= rpp) return;
+  const int j0 = (lane - imul(row, split.per_row)) * TJ;
   if constexpr (PAIR) {
     const int npair = (h + 1) >> 1;
-    for (int ip = pass_row0 * rpp + (lane >> gsh); ip < npair; ip += pass_step * rpp) {
+    for (int ip = pass_row0 * rpp + row; ip < npair; ip += pass_step * rpp) {
       const int i = 2 * ip;
       const float* gy = G + imul(i, gstr) + j0;
       corr_strip2<K, TJ, VW>(A + imul(i, astr) + j0, astr, gy, gy + gstr, acc);
     }
   } else {
-    for (int i = pass_row0 * rpp + (lane >> gsh); i < h; i += pass_step * rpp) {
+    for (int i = pass_row0 * rpp + row; i < h; i += pass_step * rpp) {
       const float* gy = G + imul(i, gstr) + j0;
       corr_strip<K, TJ, VW>(A + imul(i, astr) + j0, astr, gy, acc);   // A already points R rows/cols up-left
     }
@@ -965,7 +965,6 @@ __device__ __forceinline__ void corr_level(const float* __restrict__ A, int astr
 }
 
 constexpr int wgrad_sets(int L) { return L >= 4 ? 3 : (L >= 2 ? 2 : 1); }
-constexpr int kStripMinWidth = 12;   // coarse levels of the weight-gradient kernel: strips from this width on
 
 // Registers: with up to three sets of 49 sums K = 7 needs more than the 128 that two workgroups a CU leave each lane (it
 // spilled 300 to 640 bytes a lane): [16,64,56,56] fp32, three levels, training step 154 -> 128.5 us with 256.
@@ -1090,7 +1089,7 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
     {
       const int l = role_a ? 0 : 1;            // set 0, strips of TJ: base conv rows (A) / level 1 (B)
       corr_level<K, TJ, VW, true>(a_plane(l, role_a ? 0 : q), pl.astr[l], g_plane(l, role_a ? 0 : q), pl.gstr[l],
-                            rows(l), pl.w[l], lane, role_a ? q : 0, role_a ? 4 : 1, acc[0]);
+                            rows(l), pl.corr[l], lane, role_a ? q : 0, role_a ? 4 : 1, acc[0]);
     }
     if (wave == 0) {
       // bias gradient: the sum of grad_out is 2^L times the sum of its coarsest LL band (every
@@ -1106,17 +1105,17 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
         // first set (one pass of a wave instead of four at 14 x 14), a narrower one by single
         // coefficients (more lanes busy)
         if (pl.w[l] >= kStripMinWidth)
-          corr_level<K, TJ, VW, true>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.w[l], lane, 0,
+          corr_level<K, TJ, VW, true>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0,
                                       1, acc[1]);
         else
-          corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.w[l], lane, 0,
+          corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0,
                                      1, acc[1]);
       }
     }
     if constexpr (NSET >= 3) {                 // set 2: level 5 (A) / level 4 (B)
       const int l = role_a ? 5 : 4;
       if (l <= L) {
-        corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.w[l], lane, 0, 1,
+        corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0, 1,
                                    acc[2]);
       }
     }

@@ -17,6 +17,10 @@ constexpr int kTJC = 1;     // coarser levels of the plane kernel: single coeffi
                             // (measured against strips of 2: 28x28 planes 106 -> 100 us, 14x14 73 -> 71, 56x56 equal)
 constexpr int kTJW = 4;     // weight-gradient correlation strips
 
+constexpr RowSplit row_split(int per_row, int threads) {
+  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row};
+}
+
 constexpr int pow2_ceil(int v) { int p = 1; while (p < v) p *= 2; return p; }
 constexpr int log2_int(int v) { int s = 0; while ((1 << s) < v) ++s; return s; }
 
@@ -119,10 +123,6 @@ constexpr Plan2D make_plan2d_geometry(int B, int C, int H, int W, int K, int L, 
 
 inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_grad_pyramid, int nthreads, int pb = 1) {
   return make_plan2d_geometry(B, C, H, W, K, L, with_grad_pyramid, nthreads, pb);
-}
-
-constexpr RowSplit row_split(int per_row, int threads) {
-  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row};
 }
 
 // Completes a plan for the plane kernel: threads per plane, slots per workgroup, prefetch.
@@ -242,6 +242,11 @@ constexpr void finish_wgrad_plan(Plan2D* pl, int K) {
   // than the pyramids of a single tiny plane take
   const int red_floats = round_up(8 * (wgrad_sets(pl->L) * K * K + 1), 4);
   if (pl->lds_floats < red_floats) pl->lds_floats = red_floats;
+  // A wave's lanes take as many whole rows as they hold.  A power of two of lanes to each left out lanes wherever a row has not
+  // just as many strips: 78x66 planes (K = 5, L = 2, 17 strips of 32 lanes) 148.3 -> 127.3 us, 45x37 (K = 7, 10 of 16) 44.5 -> 39.6,
+  // 15x17 (K = 7) 93.6 -> 82.3, 40x34 229.7 -> 211.4, 70x75 (K = 3) 73.4 -> 67.9; 56x56 167.6 -> 167.7, 12x10 44.4 -> 45.3.
+  for (int l = 0; l <= pl->L; ++l)
+    pl->corr[l] = row_split(l < 2 || (l < 4 && pl->w[l] >= kStripMinWidth) ? (pl->w[l] + kTJW - 1) / kTJW : pl->w[l], kWave);
   const int slots = pow2_ceil(pl->pb);
   pl->slot_shift = log2_int(512 / slots);
   const int nps = 512 / slots;

@@ -32,8 +32,9 @@ static int run_plane2d_static(int K, int tj1, const void* x, void* out, const fl
   if (pl.H == H_ && pl.L == L_) {                                                                       \
     using G = PlaneGeoStatic<H_, H_, 5, L_>;                                                            \
     constexpr Plan2D g = G::plan();                                                                     \
-    if (tj1 == G::tj1() && same_plane_geometry(g, pl))                                                  \
-      return run_plane2d_mode<T, 5, G::tj1(), G::mode(), G>(x, out, fw, fb, pl, fold, stream);                \
+    constexpr int tj = G::tj1();                                                                        \
+    if (tj1 == tj && same_plane_geometry(g, pl))                                                        \
+      return run_plane2d_mode<T, 5, tj, G::mode(), G>(x, out, fw, fb, pl, fold, stream);                \
     return 1;                                                                                           \
   }
   WT_TRY(56, 3) WT_TRY(28, 3) WT_TRY(14, 2) WT_TRY(7, 2)
