@@ -59,6 +59,8 @@ def test_layer_against_fp64(hip_device, shape, K, L, dtype):
     ((9, 2, 64, 40), 5, 5),       # as wide and deep as the kernel takes, five tiles
     ((37, 9, 4, 4), 1, 1), ((70, 4, 7, 7), 5, 2), ((1, 1, 5, 6), 3, 2),      # many planes a unit; one plane, the tensor's last
     ((26, 4, 14, 14), 5, 3),      # a compile-time plan, the last unit not full
+    ((1, 5, 14, 14), 5, 3), ((5, 3, 14, 14), 5, 3), ((13, 4, 14, 14), 5, 2),      # and units of fewer planes than it has places for
+    ((1, 3, 28, 28), 5, 4), ((3, 4, 28, 28), 5, 3), ((1, 9, 7, 7), 5, 2), ((17, 5, 7, 7), 5, 2), ((33, 2, 7, 7), 5, 2),
 ])
 def test_matrix_core_layer_against_fp64(hip_device, shape, K, L):
     import wtconv

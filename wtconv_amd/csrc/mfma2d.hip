@@ -133,7 +133,11 @@ struct MfmaArgs {
 template <typename T, int NS, int NBL, bool VEC, typename Geo>
 int launch_mfma(const void* x, void* out, const MfmaArgs& a, const MPlan& pl, hipStream_t stream) {
   auto kern = wt2d_mfma_kernel<T, NS, NBL, VEC, NS == 1, Geo>;
-  const size_t lds = static_cast<size_t>(pl.lds_bytes);
+  size_t lds = static_cast<size_t>(pl.lds_bytes);
+  if constexpr (Geo::kStatic) {
+    constexpr MPlan g = Geo::template plan<NS>();
+    lds = g.lds_bytes;      // (the layout of as many planes as the kernel is for)
+  }
   if (int e = allow_lds(kern, lds)) return e;
   int nwg = compute_units() * resident_per_cu(kern, kMfmaBlock, lds);
   if (nwg > pl.nunits) nwg = pl.nunits;
@@ -157,7 +161,7 @@ int launch_mfma_vec(bool vec, const void* x, void* out, const MfmaArgs& a, const
 template <typename T, int NS, int H, int L, int PB, bool VEC>
 bool try_static(bool vec, const void* x, void* out, const MfmaArgs& a, const MPlan& pl,
                 hipStream_t stream, int* rc) {
-  if (pl.H != H || pl.W != H || pl.L != L || pl.pb != PB || vec != VEC) return false;
+  if (pl.H != H || pl.W != H || pl.L != L || pl.pb > PB || vec != VEC) return false;
   *rc = launch_mfma<T, NS, 1, VEC, GeoStatic<H, H, L, PB>>(x, out, a, pl, stream);
   return true;
 }
