@@ -184,3 +184,52 @@ def test_compiling_comes_before_the_binding(monkeypatch):
     assert block_ops.block_mlp(x, x, blk.norm, blk.mlp, blk.gamma) is None
     assert block_ops.patch_conv(x, model.stem, model.stem[0], model.stem[1], True) is None
     assert block_ops.mlp_fn(x, blk.mlp) is None
+
+
+@pytest.mark.parametrize("kind", ["plain", "pruned", "parametrized", "weight norm", "no bias", "no affine", "approximate", "subclass",
+                                  "no layer scale", "hook", "own forward"])
+def test_lookups_of_the_binding_find_what_python_finds(kind):
+    """The native look-ups of a block's modules against the Python ones, also where a name is no ordinary parameter."""
+    from torch.nn.utils import parametrize, prune, weight_norm
+    from wtconv_amd import _ext, block_ops, modules
+    from wtconvnext.wtconvnext import WTConvNeXtBlock
+    native = _ext.lookups()
+    if native is None:
+        pytest.skip("the binding is not built")
+    blk = WTConvNeXtBlock(8, wt_levels=3, ls_init_value=None if kind == "no layer scale" else 1.)
+    fc1, level = blk.mlp.fc1, blk.conv_dw.wavelet_convs[1]
+    if kind == "pruned":
+        for m in (fc1, level):
+            prune.random_unstructured(m, "weight", amount=0.5)
+    elif kind == "parametrized":
+        for m in (fc1, level):
+            parametrize.register_parametrization(m, "weight", torch.nn.Identity())
+    elif kind == "weight norm":
+        for m in (fc1, blk.conv_dw.base_conv):
+            weight_norm(m)
+    elif kind == "no bias":
+        fc1.bias = blk.conv_dw.base_conv.bias = None
+    elif kind == "no affine":
+        blk.norm = torch.nn.LayerNorm(8, elementwise_affine=False)
+    elif kind == "approximate":
+        blk.mlp.act = torch.nn.GELU(approximate="tanh")
+    elif kind == "subclass":
+        fc1.weight = torch.nn.Parameter(_Quantised(fc1.weight.detach()), requires_grad=False)
+    elif kind == "hook":
+        blk.norm.register_forward_pre_hook(lambda *a: None)
+    elif kind == "own forward":
+        blk.mlp.act.forward = lambda t: t
+    same = lambda a, b: a is b or (type(a) is type(b) and torch.equal(a, b))
+    x, y = torch.zeros(2), torch.ones(2)
+    got, want = (f(x, y, blk.norm, blk.mlp, blk.gamma) for f in (native.mlp_args, block_ops._mlp_args))
+    assert (got is None) == (want is None) == (kind not in ("plain", "no bias", "no layer scale"))
+    if got is not None:
+        assert len(got) == len(want) and got[4] == want[4] and all(same(a, b) for i, (a, b) in enumerate(zip(got, want)) if i != 4)
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(_ext, "lookups", lambda: None)
+        want = modules._layer_params(blk.conv_dw)
+    got = native.layer_params(blk.conv_dw)
+    assert all(same(a, b) for a, b in zip(got[:3], want[:3]))
+    assert all(len(g) == len(w) == 3 and all(same(a, b) for a, b in zip(g, w)) for g, w in zip(got[3:], want[3:]))
+    with pytest.raises(AttributeError):
+        native.mlp_args(x, y, blk.norm, torch.nn.Identity(), None)

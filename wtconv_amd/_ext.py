@@ -41,3 +41,6 @@ def get():
     mod.bind([ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _ENTRY_POINTS])
     _mod = mod
     return _mod
+
+
+lookups = get      # for the functions that look into modules: the binding's own also where something stands in for its kernels

@@ -54,6 +54,9 @@ def _watched(*modules):
     """Whether something expects to see these modules called, or the functions they call: hooks of the modules or of all
     modules, a `forward` put on a module itself, a dispatch or function mode (FLOP counters, tracers).  The function mode
     of a default device only looks at factory functions."""
+    native = _ext.lookups()
+    if native is not None:
+        return native.watched(*modules)
     if _nn._global_forward_hooks or _nn._global_forward_pre_hooks or torch._C._len_torch_dispatch_stack():
         return True
     for m in modules:
@@ -85,18 +88,22 @@ def block_mlp(x, shortcut, norm, mlp, gamma):
     ext = _ext.get()
     if ext is None:
         return None
+    native = _ext.lookups()
+    args = (_mlp_args if native is None else native.mlp_args)(x, shortcut, norm, mlp, gamma)
+    return None if args is None else ext.block_mlp(*args)
+
+
+def _mlp_args(x, shortcut, norm, mlp, gamma):
+    """What the binding's mlp_args() gives."""
     fc1, act, fc2 = mlp.fc1, mlp.act, mlp.fc2
     if (type(fc1) is not torch.nn.Linear or type(fc2) is not torch.nn.Linear or type(act) is not torch.nn.GELU
             or act.approximate != "none" or _watched(norm, mlp, fc1, act, fc2)):
         return None
-    nw, nb = _param(norm), _param(norm, "bias")
-    args = (nw, nb, norm.eps, _param(fc1), _param(fc1, "bias"), _param(fc2), _param(fc2, "bias"), gamma)
-    if nw is None or nb is None:
+    args = (x, shortcut, _param(norm), _param(norm, "bias"), norm.eps, _param(fc1), _param(fc1, "bias"), _param(fc2),
+            _param(fc2, "bias"), gamma)
+    if args[2] is None or args[3] is None or any(type(t) not in _PLAIN for t in args[:4] + args[5:]):
         return None
-    for t in (x, shortcut, nw, nb, *args[3:]):
-        if type(t) not in _PLAIN:
-            return None
-    return ext.block_mlp(x, shortcut, *args)
+    return args
 
 
 def patch_conv(x, seq, conv, norm, stem):

@@ -12,7 +12,9 @@
 // kernel dtypes.  layer() returns None for anything else and the caller takes the Python path, which converts.
 #include <torch/extension.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/function.h>
@@ -21,6 +23,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 
 #include <chrono>
 #include <mutex>
@@ -83,6 +86,12 @@ template <typename F>
 void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
 // Addresses in the order of the names in wtconv_amd/_ext.py.
+// What the look-ups below compare with, imported by bind(): an import within a call could let another thread in while a
+// static's initialisation is under way.
+struct Python {
+  PyObject *module, *device_context, *linear, *gelu;
+} python;
+
 void bind(const std::vector<uintptr_t>& a) {
   TORCH_CHECK(a.size() == 30, "bind: expected 30 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
@@ -93,6 +102,10 @@ void bind(const std::vector<uintptr_t>& a) {
   take(abi.patch_ok, a[18]); take(abi.patch_ws, a[19]); take(abi.patch, a[20]);
   take(abi.mlpt_ok, a[21]); take(abi.mlpt_fwd, a[22]); take(abi.mlpt_ws, a[23]); take(abi.mlpt_bwd, a[24]);
   take(abi.norm, a[25]); take(abi.residual, a[26]); take(abi.block_ws, a[27]); take(abi.norm_bwd, a[28]); take(abi.residual_bwd, a[29]);
+  const py::object nn = py::module_::import("torch.nn");
+  python = {py::module_::import("torch.nn.modules.module").release().ptr(),
+            py::module_::import("torch.utils._device").attr("DeviceContext").cast<py::object>().release().ptr(),
+            nn.attr("Linear").cast<py::object>().release().ptr(), nn.attr("GELU").cast<py::object>().release().ptr()};
   abi.bound = true;
 }
 
@@ -556,39 +569,214 @@ py::object haar(const Tensor& x, const std::optional<Tensor>& bank, int64_t dims
 
 // The block behind its WTConv layer in one kernel (inference): None if the kernel does not take these arguments or
 // autograd would record the call.
-py::object block_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm_w, const Tensor& norm_b, double eps,
-                     const Tensor& w1, const std::optional<Tensor>& b1, const Tensor& w2, const std::optional<Tensor>& b2,
-                     const std::optional<Tensor>& gamma) {
+// The result; undefined if the kernels do not take these tensors.  b1, b2 and gamma may be undefined.
+Tensor fused_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm_w, const Tensor& norm_b, double eps, const Tensor& w1,
+                 const Tensor& b1, const Tensor& w2, const Tensor& b2, const Tensor& gamma) {
   TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
-  if (x.dim() != 4 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous()) return py::none();
-  if (shortcut.sizes() != x.sizes() || !b1.has_value() || !b2.has_value()) return py::none();
+  if (x.dim() != 4 || !x.is_cuda() || x.scalar_type() != at::kBFloat16 || !x.is_contiguous()) return Tensor();
+  if (shortcut.sizes() != x.sizes() || !b1.defined() || !b2.defined()) return Tensor();
   const int64_t B = x.size(0), C = x.size(1), HW = x.size(2) * x.size(3);
-  if (w1.dim() != 2 || w2.dim() != 2 || w1.size(1) != C || w2.size(0) != C || w1.size(0) != w2.size(1)) return py::none();
+  if (w1.dim() != 2 || w2.dim() != 2 || w1.size(1) != C || w2.size(0) != C || w1.size(0) != w2.size(1)) return Tensor();
   const int64_t hidden = w1.size(0);
-  if (norm_w.numel() != C || norm_b.numel() != C || b1->numel() != hidden || b2->numel() != C) return py::none();
-  if (gamma.has_value() && gamma->numel() != C) return py::none();
+  if (norm_w.numel() != C || norm_b.numel() != C || b1.numel() != hidden || b2.numel() != C) return Tensor();
+  if (gamma.defined() && gamma.numel() != C) return Tensor();
   const bool grad = at::GradMode::is_enabled();
-  if (grad && x.requires_grad()) return py::none();
-  const Tensor* all[] = {&shortcut, &norm_w, &norm_b, &w1, &*b1, &w2, &*b2, gamma.has_value() ? &*gamma : nullptr};
+  if (grad && x.requires_grad()) return Tensor();
+  if (x._fw_grad(0).defined()) return Tensor();
   uintptr_t bits = 0;
-  for (const Tensor* t : all) {
-    if (t == nullptr) continue;
-    if (!canonical(*t, x.device(), at::kBFloat16) || (grad && t->requires_grad())) return py::none();
-    if (t != &shortcut) bits |= reinterpret_cast<uintptr_t>(t->data_ptr());
+  for (const Tensor* t : {&shortcut, &norm_w, &norm_b, &w1, &b1, &w2, &b2, &gamma}) {
+    if (!t->defined()) continue;
+    if (!canonical(*t, x.device(), at::kBFloat16) || (grad && t->requires_grad()) || t->_fw_grad(0).defined()) return Tensor();
+    if (t != &shortcut) bits |= reinterpret_cast<uintptr_t>(t->const_data_ptr());
   }
-  if (bits % 16 || x.numel() == 0 || B * HW > (1LL << 30) || !abi.mlp_ok(B, C, HW, hidden)) return py::none();
+  if (bits % 16 || x.numel() == 0 || B * HW > (1LL << 30) || !abi.mlp_ok(B, C, HW, hidden)) return Tensor();
   const c10::DeviceGuard guard(x.device());
-  Tensor out = at::empty_like(x, at::MemoryFormat::Contiguous);
+  Tensor out = at::empty(x.sizes(), x.options());
   const size_t wsz = abi.mlp_ws(B, C, HW, hidden);
-  Tensor ws;
-  if (wsz) ws = at::empty({static_cast<int64_t>(wsz)}, x.options().dtype(at::kByte));
-  const wtconv_mlp_params p = {norm_w.data_ptr(), norm_b.data_ptr(), w1.data_ptr(), b1->data_ptr(), w2.data_ptr(),
-                               b2->data_ptr(), gamma.has_value() ? gamma->data_ptr() : nullptr};
-  const int rc = abi.mlp(x.data_ptr(), shortcut.data_ptr(), out.data_ptr(), &p, B, C, HW, hidden, static_cast<float>(eps),
-                         WTCONV_BF16, WTCONV_BF16, wsz ? ws.data_ptr() : nullptr, wsz,
+  c10::DataPtr ws;
+  if (wsz) ws = scratch(x, wsz);
+  const wtconv_mlp_params p = {norm_w.const_data_ptr(), norm_b.const_data_ptr(), w1.const_data_ptr(), b1.const_data_ptr(),
+                               w2.const_data_ptr(), b2.const_data_ptr(), gamma.defined() ? gamma.const_data_ptr() : nullptr};
+  const int rc = abi.mlp(x.const_data_ptr(), shortcut.const_data_ptr(), out.mutable_data_ptr(), &p, B, C, HW, hidden,
+                         static_cast<float>(eps), WTCONV_BF16, WTCONV_BF16, ws.get(), wsz,
                          c10::hip::getCurrentHIPStream(x.device().index()).stream());
   if (rc) fail(rc, "wtconv block mlp");
-  return py::cast(out);
+  return out;
+}
+
+// (x, shortcut, norm weight, norm bias, eps, fc1 weight, fc1 bias, fc2 weight, fc2 bias, gamma)
+PyObject* block_mlp(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 10, "block_mlp: expected 10 arguments, got ", nargs);
+  Tensor t[10];
+  for (int i = 0; i < 10; ++i) {
+    if (i == 4 || (args[i] == Py_None && (i == 6 || i == 8 || i == 9))) continue;
+    TORCH_CHECK_TYPE(THPVariable_Check(args[i]), "block_mlp: argument ", i, " is no tensor");
+    t[i] = THPVariable_Unpack(args[i]);
+  }
+  const double eps = PyFloat_AsDouble(args[4]);
+  if (eps == -1. && PyErr_Occurred()) return nullptr;
+  const Tensor out = fused_mlp(t[0], t[1], t[2], t[3], eps, t[5], t[6], t[7], t[8], t[9]);
+  if (!out.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- modules, looked into without the interpreter: a block at inference asks for some forty attributes, which cost as much
+// host time as two launches (one image, 14 x 14 x 384: a block 20.9 -> 16.3 us of host time, of these the MLP 11.9 -> 8.1;
+// WTConvNeXt-T on one image, which the host bounds, 500 -> 442 us).
+
+// A name that lives as long as the process.
+PyObject* name_of(const char* s) { return PyUnicode_InternFromString(s); }
+
+// A module's own attributes (borrowed); nullptr if it has none.
+PyObject* own_dict(PyObject* module) {
+  PyObject** at = _PyObject_GetDictPtr(module);
+  return at != nullptr && *at != nullptr && PyDict_Check(*at) ? *at : nullptr;
+}
+
+// module.<name>, an ordinary parameter or sub-module (of the dict `kind`) first, else as Python looks it up; throws.
+py::object member(PyObject* module, PyObject* kind, PyObject* name) {
+  if (PyObject* own = own_dict(module))
+    if (PyObject* of = PyDict_GetItemWithError(own, kind))
+      if (PyDict_Check(of))
+        if (PyObject* v = PyDict_GetItemWithError(of, name))
+          if (v != Py_None) return py::reinterpret_borrow<py::object>(v);
+  if (PyErr_Occurred()) throw py::error_already_set();
+  PyObject* v = PyObject_GetAttr(module, name);
+  if (v == nullptr) throw py::error_already_set();
+  return py::reinterpret_steal<py::object>(v);
+}
+py::object parameter(PyObject* module, PyObject* name) {
+  static PyObject* const kind = name_of("_parameters");
+  return member(module, kind, name);
+}
+py::object submodule(PyObject* module, PyObject* name) {
+  static PyObject* const kind = name_of("_modules");
+  return member(module, kind, name);
+}
+
+// An attribute that the module itself holds, or as Python looks it up; throws.
+py::object attribute(PyObject* module, PyObject* name) {
+  if (PyObject* own = own_dict(module))
+    if (PyObject* v = PyDict_GetItemWithError(own, name)) return py::reinterpret_borrow<py::object>(v);
+  if (PyErr_Occurred()) throw py::error_already_set();
+  PyObject* v = PyObject_GetAttr(module, name);
+  if (v == nullptr) throw py::error_already_set();
+  return py::reinterpret_steal<py::object>(v);
+}
+
+bool truth(PyObject* o) {
+  const int t = PyObject_IsTrue(o);
+  if (t < 0) throw py::error_already_set();
+  return t != 0;
+}
+
+// Whether something expects to see these modules called, or the functions they call: hooks of the modules or of all
+// modules, a `forward` put on a module itself, a dispatch or function mode (FLOP counters, tracers).  The function mode
+// of a default device only looks at factory functions.
+bool watched_modules(PyObject* const* modules, Py_ssize_t n) {
+  static PyObject* const all[] = {name_of("_global_forward_hooks"), name_of("_global_forward_pre_hooks")};
+  static PyObject* const one[] = {name_of("_forward_hooks"), name_of("_forward_pre_hooks")};
+  static PyObject* const forward = name_of("forward");
+  for (PyObject* name : all) {
+    const py::object hooks = py::reinterpret_steal<py::object>(PyObject_GetAttr(python.module, name));
+    if (!hooks) throw py::error_already_set();
+    if (truth(hooks.ptr())) return true;
+  }
+  if (c10::impl::TorchDispatchModeTLS::stack_len()) return true;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    for (PyObject* name : one)
+      if (truth(attribute(modules[i], name).ptr())) return true;
+    PyObject* own = own_dict(modules[i]);
+    if (own == nullptr) return true;
+    const int has = PyDict_Contains(own, forward);
+    if (has < 0) throw py::error_already_set();
+    if (has) return true;
+  }
+  for (int64_t i = 0, m = at::impl::PythonTorchFunctionTLS::stack_len(); i < m; ++i) {
+    PyObject* mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+    if (reinterpret_cast<PyObject*>(Py_TYPE(mode)) != python.device_context) return true;
+  }
+  return false;
+}
+
+PyObject* watched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  return PyBool_FromLong(watched_modules(args, nargs));
+  END_HANDLE_TH_ERRORS
+}
+
+// Base weight, bias and scale, level weights and level scales of a WTConv2d / WTConv1d, as layer() takes them; None if the
+// module is built another way (lists of modules that are no plain dicts).
+PyObject* layer_params(PyObject*, PyObject* module) {
+  HANDLE_TH_ERRORS
+  static PyObject* const modules = name_of("_modules");
+  static PyObject* const weight = name_of("weight");
+  static PyObject* const bias = name_of("bias");
+  static PyObject* const parts[] = {name_of("base_conv"), name_of("base_scale"), name_of("wavelet_convs"), name_of("wavelet_scale")};
+  auto dict_of = [&](PyObject* m) -> PyObject* {
+    PyObject* own = own_dict(m);
+    PyObject* of = own != nullptr ? PyDict_GetItemWithError(own, modules) : nullptr;
+    return of != nullptr && PyDict_CheckExact(of) ? of : nullptr;
+  };
+  PyObject* sub = dict_of(module);
+  PyObject* part[4] = {};
+  for (int i = 0; i < 4 && sub != nullptr; ++i)
+    if ((part[i] = PyDict_GetItemWithError(sub, parts[i])) == nullptr) sub = nullptr;
+  PyObject* lists[2] = {sub != nullptr ? dict_of(part[2]) : nullptr, sub != nullptr ? dict_of(part[3]) : nullptr};
+  if (PyErr_Occurred()) throw py::error_already_set();
+  if (lists[0] == nullptr || lists[1] == nullptr) Py_RETURN_NONE;
+  py::object levels[2];
+  for (int k = 0; k < 2; ++k) {
+    const py::object of = py::reinterpret_steal<py::object>(PyDict_Values(lists[k]));      // (a look-up may run Python code)
+    if (!of) throw py::error_already_set();
+    const Py_ssize_t n = PyList_GET_SIZE(of.ptr());
+    levels[k] = py::reinterpret_steal<py::object>(PyList_New(n));
+    if (!levels[k]) throw py::error_already_set();
+    for (Py_ssize_t i = 0; i < n; ++i)
+      PyList_SET_ITEM(levels[k].ptr(), i, parameter(PyList_GET_ITEM(of.ptr(), i), weight).release().ptr());
+  }
+  const py::object base = py::reinterpret_borrow<py::object>(part[0]), scale = py::reinterpret_borrow<py::object>(part[1]);
+  const py::object found[] = {parameter(base.ptr(), weight), parameter(base.ptr(), bias), parameter(scale.ptr(), weight)};
+  return PyTuple_Pack(5, found[0].ptr(), found[1].ptr(), found[2].ptr(), levels[0].ptr(), levels[1].ptr());
+  END_HANDLE_TH_ERRORS
+}
+
+// What block_mlp() is called with, from (x, shortcut, norm, mlp, gamma); None where the block's passes have to be the modules'
+// own: another activation than the exact GELU, observers, a tensor of a subclass, a LayerNorm without parameters.
+PyObject* mlp_args(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 5, "mlp_args: expected 5 arguments, got ", nargs);
+  static PyObject* const weight = name_of("weight");
+  static PyObject* const bias = name_of("bias");
+  static PyObject* const parts[] = {name_of("fc1"), name_of("act"), name_of("fc2")};
+  static PyObject* const approximate = name_of("approximate");
+  static PyObject* const eps_name = name_of("eps");
+  PyObject *norm = args[2], *mlp = args[3];
+  const py::object fc1 = submodule(mlp, parts[0]), act = submodule(mlp, parts[1]), fc2 = submodule(mlp, parts[2]);
+  auto is = [](const py::object& o, PyObject* type) { return reinterpret_cast<PyObject*>(Py_TYPE(o.ptr())) == type; };
+  if (!is(fc1, python.linear) || !is(fc2, python.linear) || !is(act, python.gelu)) Py_RETURN_NONE;
+  const py::object kind = attribute(act.ptr(), approximate);
+  if (!PyUnicode_Check(kind.ptr()) || PyUnicode_CompareWithASCIIString(kind.ptr(), "none") != 0) Py_RETURN_NONE;
+  PyObject* modules[] = {norm, mlp, fc1.ptr(), act.ptr(), fc2.ptr()};
+  if (watched_modules(modules, 5)) Py_RETURN_NONE;
+  const py::object found[] = {parameter(norm, weight),      parameter(norm, bias),      attribute(norm, eps_name),
+                              parameter(fc1.ptr(), weight), parameter(fc1.ptr(), bias), parameter(fc2.ptr(), weight),
+                              parameter(fc2.ptr(), bias)};
+  PyObject* given[] = {args[0], args[1], found[0].ptr(), found[1].ptr(), found[2].ptr(), found[3].ptr(), found[4].ptr(), found[5].ptr(),
+                       found[6].ptr(), args[4]};
+  if (given[2] == Py_None || given[3] == Py_None) Py_RETURN_NONE;
+  for (int i = 0; i < 10; ++i)
+    if (i != 4 && given[i] != Py_None && !THPVariable_CheckExact(given[i])) Py_RETURN_NONE;
+  PyObject* out = PyTuple_New(10);
+  if (out == nullptr) throw py::error_already_set();
+  for (int i = 0; i < 10; ++i) {
+    Py_INCREF(given[i]);
+    PyTuple_SET_ITEM(out, i, given[i]);
+  }
+  return out;
+  END_HANDLE_TH_ERRORS
 }
 
 // ---- a block's MLP in training: fc2(gelu(fc1(x))) over the last extent of x.
@@ -954,9 +1142,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   static PyMethodDef functions[] = {
       {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&layer)), METH_FASTCALL,
        "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical"},
+      {"watched", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&watched)), METH_FASTCALL,
+       "whether something expects to see these modules called"},
+      {"layer_params", &layer_params, METH_O, "the parameters of a WTConv module as layer() takes them; None if it is built otherwise"},
+      {"mlp_args", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&mlp_args)), METH_FASTCALL,
+       "the arguments of block_mlp from x, shortcut, the modules norm and mlp, and gamma; None where the modules are to be called"},
+      {"block_mlp", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&block_mlp)), METH_FASTCALL,
+       "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken"},
       {nullptr, nullptr, 0, nullptr}};
   if (PyModule_AddFunctions(m.ptr(), functions) != 0) throw py::error_already_set();
-  m.def("block_mlp", &block_mlp, "LayerNorm, MLP, layer scale and shortcut of a WTConvNeXt block; None if not taken");
   m.def("mlp", &mlp, "a block's MLP with a C++ autograd node; None if not taken", py::arg("x"), py::arg("fc1_weight"), py::arg("fc1_bias"),
         py::arg("fc2_weight"), py::arg("fc2_bias"), py::arg("twice") = false);
   m.def("channel_norm", &channel_norm, "LayerNorm over the channels with a C++ autograd node; None if not taken");

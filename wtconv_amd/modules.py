@@ -15,6 +15,7 @@ import math
 import torch
 import torch.nn as nn
 
+from . import _ext
 from . import functional as Fn
 
 _R = 0.7071067811865476
@@ -68,6 +69,11 @@ def _param(module, name="weight"):
 def _layer_params(module):
     """base weight, bias, scale, level weights, level scales of a WTConv2d / WTConv1d (a call reads 3 + 2 L of them, and
     through `module.base_conv.weight` and the like that alone takes 4 us)."""
+    native = None if torch.compiler.is_compiling() else _ext.lookups()
+    if native is not None:
+        found = native.layer_params(module)
+        if found is not None:
+            return found
     sub = module._modules
     base = sub["base_conv"]
     return (_param(base), _param(base, "bias"), _param(sub["base_scale"]),
