@@ -12,7 +12,7 @@
 extern "C" {
 #endif
 
-#define WTCONV_OPS_VERSION 1
+#define WTCONV_OPS_VERSION 2
 
 /* Version of this part in the loaded library (== WTCONV_OPS_VERSION). */
 int wtconv_ops_version(void);
@@ -90,6 +90,14 @@ size_t wtconv_mlp_backward_workspace_bytes(long long pixels, int C, int hidden, 
 int wtconv_mlp_backward(const void* x, const void* h, const void* act, const void* dy, const wtconv_mlp_params* params,
                         void* dx, const wtconv_mlp_grads* grads, long long pixels, int C, int hidden, int dtype,
                         int param_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/* ---- what precedes the classifier (the head at wtconvnext/wtconvnext.py:358-369 of the reference): out (B, C) =
+ * LayerNorm over the channels of the means over the pixels of x (B, C, HW), the means rounded to `dtype` as between two
+ * operators.  Float or bfloat16 with parameters of either, C even and at most 2048, x aligned to four bytes.
+ * wtconv_pool_norm_supported says whether one workgroup an image is the faster way. */
+int wtconv_pool_norm_supported(int B, int C, int HW);
+int wtconv_pool_norm(const void* x, void* out, const void* weight, const void* bias, int B, int C, int HW, float eps, int dtype,
+                     int param_dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -407,3 +407,47 @@ def test_fused_block_is_left_alone_where_modules_are_watched(hip_device):
     assert seen and (fused.float() - apart.float()).norm() < 1e-2 * apart.float().norm()
     blk(x).float().sum().backward()
     assert blk.mlp.fc1.weight.grad is not None
+
+
+@pytest.mark.parametrize("B,C,H,W,dtype,pdtype", [
+    (1, 768, 7, 7, torch.bfloat16, torch.bfloat16), (300, 768, 7, 7, torch.bfloat16, torch.float32),      # odd rows: pairs share a word
+    (3, 2, 1, 1, torch.bfloat16, torch.bfloat16), (2, 6, 1, 3, torch.float32, torch.bfloat16), (5, 10, 8, 8, torch.bfloat16, torch.bfloat16),
+    (2, 766, 5, 13, torch.float32, torch.float32), (2, 2048, 8, 8, torch.bfloat16, torch.bfloat16),       # a pass of pairs not full; as many as it takes
+    (4, 770, 12, 14, torch.bfloat16, torch.bfloat16), (2, 130, 14, 14, torch.float32, torch.float32),     # several trips a channel
+])
+def test_pool_norm_matches_the_two_operators(hip_device, B, C, H, W, dtype, pdtype):
+    from wtconv_amd import _ext
+    torch.manual_seed(C + H)
+    x = (torch.randn(B, C, H, W, device=hip_device) + 3.).to(dtype)
+    w, b = torch.randn(C, device=hip_device).to(pdtype), torch.randn(C, device=hip_device).to(pdtype)
+    with torch.no_grad():
+        got = _ext.get().pool_norm(x, w, b, 1e-6)
+        mean = x.double().mean(dim=(2, 3))
+        rounded = mean.to(dtype).double()
+        want = torch.nn.functional.layer_norm(rounded, (C,), w.double(), b.double(), 1e-6)
+    assert got.shape == (B, C) and got.dtype == dtype
+    # Float sums of H W values: the mean is off by up to H W 2^-24 of itself.  Where that moves a mean across a rounding
+    # boundary of bfloat16, it is off by a unit, 2^-8 of its 3 + eps; divided by the deviation over the channels, that enters
+    # one value and, through the statistics, all of an image a little.
+    std = rounded.std(dim=1, unbiased=False, keepdim=True) + 1e-3
+    unit = (2. ** -7 if dtype == torch.bfloat16 else H * W * 2. ** -24) * rounded.abs() / std * (w.double().abs() + 1e-3)
+    err = (got.double() - want).abs()
+    assert (err <= 2 * unit + (2. ** -8 if dtype == torch.bfloat16 else 1e-5) * (want.abs() + 1)).all()
+    # nearly all means round alike
+    assert (err <= (2. ** -8 if dtype == torch.bfloat16 else 1e-4) * (want.abs() + 1)).double().mean() > 0.97
+
+
+def test_pool_norm_hands_on_what_is_not_finite_and_leaves_the_rest(hip_device):
+    from wtconv_amd import _ext
+    fn = _ext.get().pool_norm
+    x, w, b = torch.randn(3, 20, 7, 7, device=hip_device), torch.ones(20, device=hip_device), torch.zeros(20, device=hip_device)
+    x[1, 4, 6, 6] = float("inf")
+    with torch.no_grad():
+        got = fn(x, w, b, 1e-6)
+        clean = fn(x[::2].contiguous(), w, b, 1e-6)
+        assert torch.equal(got[::2], clean) and not got[1].isfinite().any()
+        assert fn(x[:, :19].contiguous(), w[:19], b[:19], 1e-6) is None and fn(x.half(), w, b, 1e-6) is None
+        assert fn(x.transpose(2, 3)[:, :, :5], w, b, 1e-6) is None and fn(x[:0], w, b, 1e-6) is None
+        assert fn(x, w.double(), b, 1e-6) is None and fn(x, w, None, 1e-6) is None
+        assert fn(torch.zeros(1, 2, 300, 300, device=hip_device), w[:2], b[:2], 1e-6) is None
+    assert fn(x.requires_grad_(), w, b, 1e-6) is None

@@ -19,7 +19,8 @@ _ENTRY_POINTS = ("wtconv2d_forward", "wtconv2d_backward_typed", "wtconv2d_backwa
                  "wtconv_patch_conv_supported", "wtconv_patch_conv_workspace_bytes", "wtconv_patch_conv",
                  "wtconv_mlp_supported", "wtconv_mlp_forward", "wtconv_mlp_backward_workspace_bytes", "wtconv_mlp_backward",
                  "wtconv_channel_norm", "wtconv_block_residual", "wtconv_block_workspace_bytes",
-                 "wtconv_channel_norm_backward_typed", "wtconv_block_residual_backward_typed")
+                 "wtconv_channel_norm_backward_typed", "wtconv_block_residual_backward_typed",
+                 "wtconv_pool_norm_supported", "wtconv_pool_norm")
 
 _mod = None
 _tried = False

@@ -9,7 +9,7 @@ MAX_LEVELS = 5
 F32, BF16, F16 = 0, 1, 2
 PASS_FORWARD, PASS_BACKWARD_INPUT, PASS_BACKWARD_PARAMS, PASS_BACKWARD = 0, 1, 2, 3
 ABI_VERSION = 6      # of wtconv_hip.h
-OPS_VERSION = 1      # of wtconv_ops.h
+OPS_VERSION = 2      # of wtconv_ops.h
 
 
 class Params(ctypes.Structure):
@@ -91,6 +91,8 @@ OPS_EXPORTS = {
     "wtconv_mlp_forward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _ll] + [_i] * 4 + [_p]),
     "wtconv_mlp_backward_workspace_bytes": (_z, [_ll, _i, _i, _i]),
     "wtconv_mlp_backward": (_i, [_p] * 4 + [ctypes.POINTER(MlpParams), _p, ctypes.POINTER(MlpGrads), _ll] + [_i] * 4 + [_p, _z, _p]),
+    "wtconv_pool_norm_supported": (_i, [_i] * 3),
+    "wtconv_pool_norm": (_i, [_p] * 4 + [_i] * 3 + [_f, _i, _i, _p]),
     "wtconv_patch_conv": (_i, [_i, _p, _p, ctypes.POINTER(PatchParams)] + [_i] * 5 + [_f, _i, _i, _p, _z, _p]),
 }
 

@@ -127,6 +127,21 @@ def patch_conv(x, seq, conv, norm, stem):
     return ext.patch_conv(x, *args, norm.eps, stem)
 
 
+def pool_norm(x, norm):
+    """`norm` (a LayerNorm over the channels) of the mean of x (B, C, H, W) over its pixels, (B, C), as one kernel; None where
+    it does not apply: autograd records, other dtypes than float32 and bfloat16, observers that expect to see the module
+    called, or tensors of a subclass."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled():      # (first: loading the binding is not traceable)
+        return None
+    ext = _ext.get()
+    if ext is None or _watched(norm):
+        return None
+    weight, bias = _param(norm), _param(norm, "bias")
+    if weight is None or bias is None or not usable(x, weight, bias) or any(type(t) not in _PLAIN for t in (x, weight, bias)):
+        return None
+    return channel_norm(x, weight, bias, norm.eps, nhwc=False, pool=True).flatten(1)
+
+
 def mlp_fn(x, mlp, twice=True):
     """A block's `mlp` (fc1, exact GELU, fc2) on x (B, H, W, C) where autograd records it, products, GELU and bias sums as
     kernels of this library; None where that does not apply (see block_mlp).  Second derivatives are PyTorch's; with
@@ -163,8 +178,14 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-def channel_norm(x, weight, bias, eps, nhwc):
-    """LayerNorm over the channels of x (B, C, H, W); returns (B, H, W, C) if `nhwc` else (B, C, H, W).  Not recorded."""
+def channel_norm(x, weight, bias, eps, nhwc, pool=False):
+    """LayerNorm over the channels of x (B, C, H, W); returns (B, H, W, C) if `nhwc` else (B, C, H, W).  Not recorded.
+    With `pool`, of its mean over the pixels."""
+    if pool:
+        out = _native("pool_norm", x, weight, bias, eps)
+        if out is not None:
+            return out[:, None, None] if nhwc else out[:, :, None, None]
+        x = x.mean(dim=(2, 3), keepdim=True)
     out = _native("channel_norm", x, weight, bias, eps, nhwc) if not records(x, weight, bias) else None
     if out is not None:
         return out

@@ -211,6 +211,37 @@ extern "C" int wtconv_channel_norm(const void* x, void* out, const void* weight,
              : launch(channel_norm_kernel<bf16_t, bf16_t, false>, static_cast<bf16_t*>(nullptr));
 }
 
+// One workgroup an image: a few trips of its loads.  Longer rows are serial (128 channels of 32 x 32: 28.9 us, the two passes
+// 7.6; 512 of 16 x 16 in float 11.0 and 10.6); at the limits one image of 640 channels of 14 x 14 takes 10.2 us (12.0), of 768
+// of 12 x 12 9.0 (12.4).
+extern "C" int wtconv_pool_norm_supported(int B, int C, int HW) {
+  return B > 0 && C > 0 && HW > 0 && C % 2 == 0 && C <= kPoolChannels && HW <= 200 && C * HW <= 1 << 17;
+}
+
+extern "C" int wtconv_pool_norm(const void* x, void* out, const void* weight, const void* bias, int B, int C, int HW, float eps,
+                                int dtype, int param_dtype, void* stream_) {
+  const char* fn = "wtconv_pool_norm";
+  if (B <= 0 || C <= 0 || HW <= 0) return fail(WTCONV_E_ARG, "%s: sizes must be positive (got B=%d C=%d HW=%d)", fn, B, C, HW);
+  if (C % 2 || C > kPoolChannels || static_cast<long long>(C) * HW > 0x3fffffffLL)
+    return fail(WTCONV_E_UNSUPPORTED, "%s: an even number of at most %d channels (got %d)", fn, kPoolChannels, C);
+  if ((dtype != WTCONV_F32 && dtype != WTCONV_BF16) || (param_dtype != WTCONV_F32 && param_dtype != WTCONV_BF16))
+    return fail(WTCONV_E_ARG, "%s: unknown dtype code", fn);
+  if (x == nullptr || out == nullptr || weight == nullptr || bias == nullptr) return fail(WTCONV_E_ARG, "%s: null pointer", fn);
+  if (reinterpret_cast<uintptr_t>(x) % 4 || reinterpret_cast<uintptr_t>(out) % (dtype == WTCONV_F32 ? 4 : 2))
+    return fail(WTCONV_E_ARG, "%s: tensor pointer not aligned (input to four bytes, output to an element)", fn);
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const size_t lds = sizeof(float) * (C + kPoolThreads / kWave);
+  auto launch = [&](auto kern, auto* tag) {
+    using T = std::remove_pointer_t<decltype(tag)>;
+    if (int e = allow_lds(kern, lds)) return e;
+    WT_LAUNCH(kern, dim3(B), dim3(kPoolThreads), lds, stream, static_cast<const T*>(x), static_cast<T*>(out), weight, bias,
+              param_dtype, eps, C, HW);
+    return check_launch("pool_norm_kernel");
+  };
+  return dtype == WTCONV_F32 ? launch(pool_norm_kernel<float>, static_cast<float*>(nullptr))
+                             : launch(pool_norm_kernel<bf16_t>, static_cast<bf16_t*>(nullptr));
+}
+
 extern "C" int wtconv_block_residual(const void* y, const void* shortcut, const void* gamma, void* out, int B, int C,
                                      int HW, int dtype, int param_dtype, void* stream_) {
   const char* fn = "wtconv_block_residual";

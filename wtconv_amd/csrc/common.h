@@ -430,6 +430,24 @@ __device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {
 #endif
 }
 
+// Sum over the 16 lanes of a row; every lane has it.
+__device__ __forceinline__ float row_sum(float v) {
+#ifdef WT_EMULATE
+#pragma unroll
+  for (int m = 8; m >= 1; m >>= 1) v += __shfl_xor(v, m, kWave);
+#else
+  using std::integral_constant;
+  auto dpp = [](float x, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v += dpp(v, integral_constant<int, 0xB1>{});     // quad_perm [1,0,3,2]
+  v += dpp(v, integral_constant<int, 0x4E>{});     // quad_perm [2,3,0,1]
+  v += dpp(v, integral_constant<int, 0x141>{});    // row_half_mirror
+  v += dpp(v, integral_constant<int, 0x140>{});    // row_mirror
+#endif
+  return v;
+}
+
 // Sum over the 64 lanes of a wavefront; every lane gets the total.  On the GPU: six DPP adds
 // (quad permutes, row mirrors, row broadcasts) and one v_readlane, no LDS traffic -- the
 // weight-gradient kernels reduce up to 76 running sums per workgroup this way.

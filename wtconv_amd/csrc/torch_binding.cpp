@@ -79,6 +79,8 @@ struct Abi {
   int (*norm_bwd)(const void*, const void*, const void*, void*, void*, void*, int, int, int, int, float, int, int, int, void*,
                   size_t, void*);
   int (*residual_bwd)(const void*, const void*, const void*, void*, void*, int, int, int, int, int, int, void*, size_t, void*);
+  int (*pool_ok)(int, int, int);
+  int (*pool)(const void*, void*, const void*, const void*, int, int, int, float, int, int, void*);
   bool bound = false;
 } abi;
 
@@ -93,7 +95,7 @@ struct Python {
 } python;
 
 void bind(const std::vector<uintptr_t>& a) {
-  TORCH_CHECK(a.size() == 30, "bind: expected 30 addresses, got ", a.size());
+  TORCH_CHECK(a.size() == 32, "bind: expected 32 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
   take(abi.fwd1, a[5]); take(abi.bwd1, a[6]); take(abi.bwdin1, a[7]); take(abi.bwdpar1, a[8]); take(abi.ws1, a[9]);
   take(abi.last_error, a[10]);
@@ -102,6 +104,7 @@ void bind(const std::vector<uintptr_t>& a) {
   take(abi.patch_ok, a[18]); take(abi.patch_ws, a[19]); take(abi.patch, a[20]);
   take(abi.mlpt_ok, a[21]); take(abi.mlpt_fwd, a[22]); take(abi.mlpt_ws, a[23]); take(abi.mlpt_bwd, a[24]);
   take(abi.norm, a[25]); take(abi.residual, a[26]); take(abi.block_ws, a[27]); take(abi.norm_bwd, a[28]); take(abi.residual_bwd, a[29]);
+  take(abi.pool_ok, a[30]); take(abi.pool, a[31]);
   const py::object nn = py::module_::import("torch.nn");
   python = {py::module_::import("torch.nn.modules.module").release().ptr(),
             py::module_::import("torch.utils._device").attr("DeviceContext").cast<py::object>().release().ptr(),
@@ -1135,6 +1138,38 @@ py::object patch_conv(const Tensor& x, const Tensor& conv_w, const Tensor& conv_
   return py::cast(out);
 }
 
+// ---- the head: mean over the pixels, LayerNorm over the channels; (B, C), or None if the kernel does not take these arguments.
+// (x, weight, bias, eps)
+PyObject* pool_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(nargs == 4, "pool_norm: expected 4 arguments, got ", nargs);
+  TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
+  for (int i = 0; i < 3; ++i)
+    if (!THPVariable_CheckExact(args[i])) Py_RETURN_NONE;
+  const Tensor &x = THPVariable_Unpack(args[0]), &weight = THPVariable_Unpack(args[1]), &bias = THPVariable_Unpack(args[2]);
+  const double eps = PyFloat_AsDouble(args[3]);
+  if (eps == -1. && PyErr_Occurred()) return nullptr;
+  if (!x.is_cuda() || !x.has_storage() || x.dim() != 4 || !block_dtype(x.scalar_type()) || !x.is_contiguous() || x.numel() == 0)
+    Py_RETURN_NONE;
+  const int64_t B = x.size(0), C = x.size(1), HW = x.size(2) * x.size(3);
+  const bool grad = at::GradMode::is_enabled();
+  if ((grad && x.requires_grad()) || x._fw_grad(0).defined()) Py_RETURN_NONE;
+  for (const Tensor* t : {&weight, &bias})
+    if (!canonical(*t, x.device(), weight.scalar_type()) || !block_dtype(t->scalar_type()) || t->numel() != C || t->dim() != 1 ||
+        (grad && t->requires_grad()) || t->_fw_grad(0).defined())
+      Py_RETURN_NONE;
+  if (reinterpret_cast<uintptr_t>(x.const_data_ptr()) % 4 || x.numel() > (1LL << 40) || B > (1LL << 30) || C > (1LL << 20) ||
+      HW > (1LL << 20) || !abi.pool_ok(B, C, HW))
+    Py_RETURN_NONE;
+  const c10::DeviceGuard guard(x.device());
+  Tensor out = at::empty({B, C}, x.options().requires_grad(false));
+  const int rc = abi.pool(x.const_data_ptr(), out.mutable_data_ptr(), weight.const_data_ptr(), bias.const_data_ptr(), B, C, HW,
+                          static_cast<float>(eps), dtype_code(x.scalar_type()), dtype_code(weight.scalar_type()), stream_of(x));
+  if (rc) fail(rc, "wtconv pool norm");
+  return THPVariable_Wrap(out);
+  END_HANDLE_TH_ERRORS
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -1142,6 +1177,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   static PyMethodDef functions[] = {
       {"layer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&layer)), METH_FASTCALL,
        "WTConv layer (2-D or 1-D) with a C++ autograd node; None if the arguments are not canonical"},
+      {"pool_norm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&pool_norm)), METH_FASTCALL,
+       "mean over the pixels and LayerNorm over the channels; None if not taken"},
       {"watched", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&watched)), METH_FASTCALL,
        "whether something expects to see these modules called"},
       {"layer_params", &layer_params, METH_O, "the parameters of a WTConv module as layer() takes them; None if it is built otherwise"},

@@ -180,8 +180,9 @@ class _Head(nn.Module):
         self.fc = nn.Linear(self.norm.normalized_shape[0], num_classes) if num_classes > 0 else nn.Identity()
 
     def forward(self, x, pre_logits: bool = False):
-        x = x.mean(dim=(2, 3), keepdim=True)
-        x = self.norm(x).flatten(1)
+        ops = _block_ops()
+        y = ops.pool_norm(x, self.norm) if ops is not None and type(self.norm) is LayerNorm2d else None
+        x = self.norm(x.mean(dim=(2, 3), keepdim=True)).flatten(1) if y is None else y
         return x if pre_logits else self.fc(x)
 
 
