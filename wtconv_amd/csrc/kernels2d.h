@@ -25,8 +25,9 @@ constexpr int kFetchPasses = 2;  // 2x4 pieces of the next plane a thread may ho
 // How a plane's threads walk a level: thread t takes item t % per_row of rows t / per_row, + rows, ...  The quotient comes
 // from a reciprocal (exact below 1024 threads and 512 items: the error of v * magic is under v * per_row < 2^20).
 struct RowSplit {
-  int per_row, rows;           // work items of a row; rows that the threads take at once
+  int per_row, rows;           // threads of a row; rows that the threads take at once
   unsigned magic;              // ceil(2^20 / per_row)
+  int used;                    // work items of a row: per_row, or fewer where a power of two takes as many passes
 };
 __device__ __forceinline__ int row_of(const RowSplit& s, int t) {
   return static_cast<int>((static_cast<unsigned>(t) * s.magic) >> 20);
@@ -552,8 +553,9 @@ __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2
   const int hl = pl.h[l];
   const RowSplit split = pl.coefs[l];
   const int row = row_of(split, ltid);
-  if (row >= split.rows) return;
-  const int j0 = (ltid - imul(row, split.per_row)) * TJ;
+  const int strip = ltid - imul(row, split.per_row);
+  if (row >= split.rows || strip >= split.used) return;
+  const int j0 = strip * TJ;
   const int astr = pl.astr[l], apl = pl.apl[l], P = pl.P;
   const float* A = lds + pl.aoff[l];
   const bool has_carry = l < pl.L;
@@ -618,8 +620,9 @@ __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2
   const int hl = pl.h[1];
   const RowSplit split = pl.strips1;
   const int row = row_of(split, ltid);
-  if (row >= split.rows) return;
-  const int j0 = (ltid - imul(row, split.per_row)) * TJ;
+  const int strip = ltid - imul(row, split.per_row);
+  if (row >= split.rows || strip >= split.used) return;
+  const int j0 = strip * TJ;
   const int astr = pl.astr[1], apl = pl.apl[1], P = pl.P;
   const float* A = lds + pl.aoff[1];
   const float* X = lds + pl.aoff[0];
@@ -947,8 +950,9 @@ __device__ __forceinline__ void corr_level(const float* __restrict__ A, int astr
                                            int gstr, int h, const RowSplit split, int lane, int pass_row0, int pass_step,
                                            float (&acc)[K * K]) {
   const int row = row_of(split, lane), rpp = split.rows;      // row items per pass of one wave (>= 1: kMaxWgradWidth, plan.h)
-  if (row >= rpp) return;
-  const int j0 = (lane - imul(row, split.per_row)) * TJ;
+  const int strip = lane - imul(row, split.per_row);
+  if (row >= rpp || strip >= split.used) return;
+  const int j0 = strip * TJ;
   if constexpr (PAIR) {
     const int npair = (h + 1) >> 1;
     for (int ip = pass_row0 * rpp + row; ip < npair; ip += pass_step * rpp) {

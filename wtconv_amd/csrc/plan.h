@@ -17,11 +17,18 @@ constexpr int kTJC = 1;     // coarser levels of the plane kernel: single coeffi
                             // (measured against strips of 2: 28x28 planes 106 -> 100 us, 14x14 73 -> 71, 56x56 equal)
 constexpr int kTJW = 4;     // weight-gradient correlation strips
 
-constexpr RowSplit row_split(int per_row, int threads) {
-  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row};
-}
-
 constexpr int pow2_ceil(int v) { int p = 1; while (p < v) p *= 2; return p; }
+
+// Rows of `used` items over the threads: dense, or a power of two of threads each where that takes `height` rows, and half as
+// many, in as many passes (shifts instead of products where the plan is a constant: 56x56 step 421.9 -> 420.6 us, gradients of
+// 28x28 planes 111.0 -> 107.6).
+constexpr RowSplit row_split(int used, int threads, int height) {
+  const int p = pow2_ceil(used);
+  auto passes = [&](int n, int per_row) { const int rows = threads / per_row; return rows > 0 ? (n + rows - 1) / rows : n + 1; };
+  const bool even = passes(height, p) == passes(height, used) && passes((height + 1) / 2, p) == passes((height + 1) / 2, used);
+  const int per_row = even && p <= threads ? p : used;
+  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row, used};
+}
 constexpr int log2_int(int v) { int s = 0; while ((1 << s) < v) ++s; return s; }
 
 // Lanes that a row of a plane takes: one for each piece of four pixels it is loaded in, which is also one for each
@@ -129,8 +136,8 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
 constexpr void finish_plane_plan(Plan2D* pl, int tj1, int sg_shift) {
   pl->sg_shift = sg_shift;
   const int sg = 1 << pl->sg_shift;
-  pl->strips1 = row_split((pl->w[1] + tj1 - 1) / tj1, sg);
-  for (int l = 2; l <= pl->L; ++l) pl->coefs[l] = row_split(pl->w[l], sg);
+  pl->strips1 = row_split((pl->w[1] + tj1 - 1) / tj1, sg, pl->h[1]);
+  for (int l = 2; l <= pl->L; ++l) pl->coefs[l] = row_split(pl->w[l], sg, pl->h[l]);
   pl->block = sg > 256 ? sg : 256;   // (two whole planes per 512-thread workgroup measured slower: lockstep phases)
   const int slots = pl->block / sg;
   pl->lds_floats = pl->plane_lds_floats * slots;
@@ -246,7 +253,8 @@ constexpr void finish_wgrad_plan(Plan2D* pl, int K) {
   // just as many strips: 78x66 planes (K = 5, L = 2, 17 strips of 32 lanes) 148.3 -> 127.3 us, 45x37 (K = 7, 10 of 16) 44.5 -> 39.6,
   // 15x17 (K = 7) 93.6 -> 82.3, 40x34 229.7 -> 211.4, 70x75 (K = 3) 73.4 -> 67.9; 56x56 167.6 -> 167.7, 12x10 44.4 -> 45.3.
   for (int l = 0; l <= pl->L; ++l)
-    pl->corr[l] = row_split(l < 2 || (l < 4 && pl->w[l] >= kStripMinWidth) ? (pl->w[l] + kTJW - 1) / kTJW : pl->w[l], kWave);
+    pl->corr[l] = row_split(l < 2 || (l < 4 && pl->w[l] >= kStripMinWidth) ? (pl->w[l] + kTJW - 1) / kTJW : pl->w[l], kWave,
+                            pl->pb == 1 ? pl->h[l] : 512);      // (stacked planes: dense)
   const int slots = pow2_ceil(pl->pb);
   pl->slot_shift = log2_int(512 / slots);
   const int nps = 512 / slots;
