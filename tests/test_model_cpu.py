@@ -233,3 +233,47 @@ def test_lookups_of_the_binding_find_what_python_finds(kind):
     assert all(len(g) == len(w) == 3 and all(same(a, b) for a, b in zip(g, w)) for g, w in zip(got[3:], want[3:]))
     with pytest.raises(AttributeError):
         native.mlp_args(x, y, blk.norm, torch.nn.Identity(), None)
+
+
+@pytest.mark.parametrize("where", ["base_conv", "base_scale", "wavelet_convs", "wavelet_scale"])
+@pytest.mark.parametrize("replaced", ["base_conv", "base_scale", "wavelet_convs", "wavelet_scale"])
+def test_lookups_of_the_binding_outlive_what_a_parametrization_replaces(where, replaced):
+    """A parametrized weight runs Python code while a layer's parameters are looked up, and that code may put another module
+    in the place of one that the look-up began with: the old one goes, and the answer is the one of Python's own look-up."""
+    from torch.nn.utils import parametrize
+    import wtconv
+    from wtconv_amd import _ext, modules
+    if _ext.lookups() is None:
+        pytest.skip("the binding is not built")
+
+    class Replaces(torch.nn.Module):
+        def __init__(self, layer):
+            super().__init__()
+            self.layer, self.made = [layer], 0
+
+        def forward(self, w):
+            self.made += 1
+            fresh = getattr(wtconv.WTConv2d(2, 2, kernel_size=3, wt_levels=2), replaced)
+            for p in fresh.parameters():
+                p.data.fill_(self.made)
+            setattr(self.layer[0], replaced, fresh)
+            return w + self.made
+
+    def look_up():
+        torch.manual_seed(0)
+        layer = wtconv.WTConv2d(2, 2, kernel_size=3, wt_levels=2)
+        part = getattr(layer, where)
+        replaces = Replaces(layer)
+        parametrize.register_parametrization(part if where.startswith("base") else part[0], "weight", replaces, unsafe=True)
+        setattr(layer, where, part)      # (registering evaluates the parametrization)
+        found = modules._layer_params(layer)
+        for _ in range(50):      # (freed memory is not put to another use at once)
+            modules._layer_params(layer)
+        return [t for p in found for t in (p if isinstance(p, (list, tuple)) else [p])], replaces.made
+
+    got, made = look_up()
+    with pytest.MonkeyPatch.context() as patch:
+        patch.setattr(_ext, "lookups", lambda: None)
+        want, made_in_python = look_up()
+    assert made == made_in_python and len(got) == len(want) == 7
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -711,28 +711,40 @@ PyObject* watched(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // Base weight, bias and scale, level weights and level scales of a WTConv2d / WTConv1d, as layer() takes them; None if the
-// module is built another way (lists of modules that are no plain dicts).
+// module is built another way (lists of modules that are no plain dicts).  A look-up of a parameter may run Python code
+// (parametrizations), and that may replace any sub-module, or let another thread do so: a part is looked up in its turn, in
+// the order in which Python reads them, and held while it is read.
 PyObject* layer_params(PyObject*, PyObject* module) {
   HANDLE_TH_ERRORS
   static PyObject* const modules = name_of("_modules");
   static PyObject* const weight = name_of("weight");
   static PyObject* const bias = name_of("bias");
   static PyObject* const parts[] = {name_of("base_conv"), name_of("base_scale"), name_of("wavelet_convs"), name_of("wavelet_scale")};
-  auto dict_of = [&](PyObject* m) -> PyObject* {
-    PyObject* own = own_dict(m);
-    PyObject* of = own != nullptr ? PyDict_GetItemWithError(own, modules) : nullptr;
-    return of != nullptr && PyDict_CheckExact(of) ? of : nullptr;
+  auto held = [](PyObject* borrowed) {
+    if (borrowed == nullptr && PyErr_Occurred()) throw py::error_already_set();
+    return py::reinterpret_borrow<py::object>(borrowed);
   };
-  PyObject* sub = dict_of(module);
-  PyObject* part[4] = {};
-  for (int i = 0; i < 4 && sub != nullptr; ++i)
-    if ((part[i] = PyDict_GetItemWithError(sub, parts[i])) == nullptr) sub = nullptr;
-  PyObject* lists[2] = {sub != nullptr ? dict_of(part[2]) : nullptr, sub != nullptr ? dict_of(part[3]) : nullptr};
-  if (PyErr_Occurred()) throw py::error_already_set();
-  if (lists[0] == nullptr || lists[1] == nullptr) Py_RETURN_NONE;
+  auto dict_of = [&](PyObject* m) -> py::object {
+    PyObject* own = own_dict(m);
+    const py::object of = own != nullptr ? held(PyDict_GetItemWithError(own, modules)) : py::object();
+    return of && PyDict_CheckExact(of.ptr()) ? of : py::object();
+  };
+  const py::object sub = dict_of(module);
+  auto part = [&](int i) { return held(PyDict_GetItemWithError(sub.ptr(), parts[i])); };
+  auto list = [&](int i) {
+    const py::object p = part(i);
+    return p ? dict_of(p.ptr()) : py::object();
+  };
+  if (!sub || !part(0) || !part(1) || !list(2) || !list(3)) Py_RETURN_NONE;
+  const py::object base = part(0), base_w = parameter(base.ptr(), weight), base_b = parameter(base.ptr(), bias);
+  const py::object scale = part(1);
+  if (!scale) Py_RETURN_NONE;
+  const py::object base_s = parameter(scale.ptr(), weight);
   py::object levels[2];
   for (int k = 0; k < 2; ++k) {
-    const py::object of = py::reinterpret_steal<py::object>(PyDict_Values(lists[k]));      // (a look-up may run Python code)
+    const py::object dict = list(2 + k);
+    if (!dict) Py_RETURN_NONE;
+    const py::object of = py::reinterpret_steal<py::object>(PyDict_Values(dict.ptr()));
     if (!of) throw py::error_already_set();
     const Py_ssize_t n = PyList_GET_SIZE(of.ptr());
     levels[k] = py::reinterpret_steal<py::object>(PyList_New(n));
@@ -740,9 +752,7 @@ PyObject* layer_params(PyObject*, PyObject* module) {
     for (Py_ssize_t i = 0; i < n; ++i)
       PyList_SET_ITEM(levels[k].ptr(), i, parameter(PyList_GET_ITEM(of.ptr(), i), weight).release().ptr());
   }
-  const py::object base = py::reinterpret_borrow<py::object>(part[0]), scale = py::reinterpret_borrow<py::object>(part[1]);
-  const py::object found[] = {parameter(base.ptr(), weight), parameter(base.ptr(), bias), parameter(scale.ptr(), weight)};
-  return PyTuple_Pack(5, found[0].ptr(), found[1].ptr(), found[2].ptr(), levels[0].ptr(), levels[1].ptr());
+  return PyTuple_Pack(5, base_w.ptr(), base_b.ptr(), base_s.ptr(), levels[0].ptr(), levels[1].ptr());
   END_HANDLE_TH_ERRORS
 }
 
