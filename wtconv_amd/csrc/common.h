@@ -416,6 +416,15 @@ __device__ __forceinline__ float wave_xor(float v, int lane4, int mask) {
 #endif
 }
 
+// This lane's number in its wavefront.  `zero`: 0, laundered where the number is not to be kept.
+__device__ __forceinline__ int lane_number(int zero) {
+#ifdef WT_EMULATE
+  return static_cast<int>(threadIdx.x & (kWave - 1)) + zero;
+#else
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+#endif
+}
+
 // Rows of 16 lanes change places: a lane of an odd row gives its `a` to the lane 16 below, whose `b` it takes for it
 // (v_permlane16_swap_b32).  Every lane of the wavefront takes part.
 __device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {

@@ -22,25 +22,28 @@ namespace wt {
 
 constexpr int kFetchPasses = 2;  // 2x4 pieces of the next plane a thread may hold in registers
 
-// How a plane's threads walk a level: thread t takes item t % per_row of rows t / per_row, + rows, ...  The quotient comes
-// from a reciprocal (exact below 1024 threads and 512 items: the error of v * magic is under v * per_row < 2^20).
-struct RowSplit {
-  int per_row, rows;           // threads of a row; rows that the threads take at once
-  unsigned magic;              // ceil(2^20 / per_row)
-  int used;                    // work items of a row: per_row, or fewer where a power of two takes as many passes
-};
-__device__ __forceinline__ int row_of(const RowSplit& s, int t) {
-  return static_cast<int>((static_cast<unsigned>(t) * s.magic) >> 20);
+// How threads walk the rows of a level: thread t takes item t % per_row of rows t / per_row, + rows, ...  A plan has it in one
+// word a level, next to the level's extents: per_row above a reciprocal, ceil(2^20 / per_row), whose quotients are exact below
+// 1024 threads and 512 items (the error of v * magic is under v * per_row < 2^20).  (Four words a level at the plan's end, the
+// quotients among them, were arguments that a launch fetched late and one after the other: 0.1 us for one level, 0.4 for five, up
+// to 0.9 with K = 7, of 8 to 30.)
+struct RowWalk { int row, strip, rows; };      // this thread's first row and item; rows that the threads take at once
+__device__ __forceinline__ RowWalk walk_rows(unsigned split, int t, int threads) {
+  const unsigned magic = split & 0x1fffffu, from = static_cast<unsigned>(t) & 0x3ffu;      // (factors of 24 bits to the compiler)
+  const unsigned row = from * magic >> 20;
+  return {static_cast<int>(row), static_cast<int>(from - row * (split >> 21)), static_cast<int>(static_cast<unsigned>(threads) * magic >> 20)};
 }
 
-// LDS layout of one plane, computed on the host (plan.h).
 constexpr int kStripMinWidth = 12;   // coarse levels of the weight-gradient kernel: strips from this width on
 
+// LDS layout of one plane, computed on the host (plan.h).
 struct Plan2D {
   int C, H, W, L;
   int P;                       // halo width of the pyramid buffers: max(K/2, 1)
   int h[kMaxLevels + 1];       // grid of level l (l = 0 is the input plane)
   int w[kMaxLevels + 1];
+  unsigned split[kMaxLevels + 1];      // rows over threads (walk_rows): plane kernel, the strips of level 1 and the coefficients of
+                               //   the levels above it over a plane's; weight-gradient kernel, strips or coefficients over a wave's
   int aoff[kMaxLevels + 1];    // float offset of level l (level 0: 1 plane; l >= 1: 4 planes)
   int astr[kMaxLevels + 1];    // row stride
   int apl[kMaxLevels + 1];     // size of one sub-band plane
@@ -65,9 +68,6 @@ struct Plan2D {
   int fw_stride;               // plane kernel: folded filters of a channel to the next channel's (floats)
   int fw_skip;                 //   floats between where the level filters would follow the base filter and where they
                                //   are (a sub-layer's base filter is the LL filter of the level above it)
-  RowSplit strips1;            // plane kernel: the strips of level 1 over the threads of a plane
-  RowSplit coefs[kMaxLevels + 1];      // and the single coefficients of level l >= 2 (synthesis)
-  RowSplit corr[kMaxLevels + 1];       // weight-gradient kernel: strips (or coefficients) of level l over the lanes of a wave
 };
 
 // ------------------------------------------------------------------ parameter folding
@@ -547,15 +547,13 @@ __device__ __forceinline__ void ihaar4(float ll, float lh, float hl, float hh,
 // inverse Haar, cropped store into Z_l.
 template <int K, int TJ>
 __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2D& pl, int l,
-                                            wt_uniform_ptr wl_f, int ltid) {
+                                            wt_uniform_ptr wl_f, int ltid, int nth) {
   constexpr int R = K / 2;
   constexpr int VW = (R >= 1) ? TJ : 1;   // window starts at column j0 when the halo equals R
-  const int hl = pl.h[l];
-  const RowSplit split = pl.coefs[l];
-  const int row = row_of(split, ltid);
-  const int strip = ltid - imul(row, split.per_row);
-  if (row >= split.rows || strip >= split.used) return;
-  const int j0 = strip * TJ;
+  const int hl = pl.h[l], wl = pl.w[l];
+  const RowWalk at = walk_rows(pl.split[l], ltid, nth);
+  if (at.row >= at.rows || at.strip >= (wl + TJ - 1) / TJ) return;
+  const int j0 = at.strip * TJ;
   const int astr = pl.astr[l], apl = pl.apl[l], P = pl.P;
   const float* A = lds + pl.aoff[l];
   const bool has_carry = l < pl.L;
@@ -564,7 +562,7 @@ __device__ __forceinline__ void synth_inner(float* __restrict__ lds, const Plan2
   float* Zout = lds + pl.zoff[l];
   const int zout_str = pl.zstr[l];
   const int ho = pl.h[l - 1], wo = pl.w[l - 1];
-  for (int i = row; i < hl; i += split.rows) {
+  for (int i = at.row; i < hl; i += at.rows) {
     float o0[2 * TJ], o1[2 * TJ];
     subband_chunks<K, TJ, VW>(A + imul(i - R + P, astr) + (j0 - R + P), astr, apl, wl_f,
                                  has_carry ? Zin + imul(i, zin_str) + j0 : nullptr, o0, o1);
@@ -612,17 +610,15 @@ __device__ __forceinline__ void store_row(T* __restrict__ dst, const float (&v)[
 template <typename T, int K, int TJ>
 __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2D& pl,
                                             wt_uniform_ptr wb_f, wt_uniform_ptr w1_f, float bias,
-                                            T* __restrict__ out_plane, int ltid) {
+                                            T* __restrict__ out_plane, int ltid, int nth) {
   constexpr int R = K / 2;
   constexpr int NO = 2 * TJ;
   constexpr int VW = (R >= 1) ? TJ : 1;
   constexpr int VWX = (R >= 1) ? (NO >= 4 ? 4 : NO) : 1;
-  const int hl = pl.h[1];
-  const RowSplit split = pl.strips1;
-  const int row = row_of(split, ltid);
-  const int strip = ltid - imul(row, split.per_row);
-  if (row >= split.rows || strip >= split.used) return;
-  const int j0 = strip * TJ;
+  const int hl = pl.h[1], wl = pl.w[1];
+  const RowWalk at = walk_rows(pl.split[1], ltid, nth);
+  if (at.row >= at.rows || at.strip >= (wl + TJ - 1) / TJ) return;
+  const int j0 = at.strip * TJ;
   const int astr = pl.astr[1], apl = pl.apl[1], P = pl.P;
   const float* A = lds + pl.aoff[1];
   const float* X = lds + pl.aoff[0];
@@ -631,7 +627,7 @@ __device__ __forceinline__ void synth_final(float* __restrict__ lds, const Plan2
   const float* Zin = lds + pl.zoff[2];
   const int zin_str = pl.zstr[2];
   const int H = pl.H, W = pl.W;
-  for (int i = row; i < hl; i += split.rows) {
+  for (int i = at.row; i < hl; i += at.rows) {
     float o0[NO], o1[NO];
     subband_chunks<K, TJ, VW>(A + imul(i - R + P, astr) + (j0 - R + P), astr, apl, w1_f,
                                  has_carry ? Zin + imul(i, zin_str) + j0 : nullptr, o0, o1);
@@ -855,12 +851,12 @@ __global__ __launch_bounds__(1024, 4) void wt2d_plane_kernel(const T* __restrict
     }
     for (int lv = pl.L; lv >= 2; --lv) {
       const int l = WT_UNIFORM(lv);
-      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + fw_skip + (1 + 4 * (l - 1)) * KK, ltid);
+      if (live) synth_inner<K, TJC>(lds, pl, l, fwc + fw_skip + (1 + 4 * (l - 1)) * KK, ltid, sg);
       plane_sync(wave_local);
     }
     WT_WAIT_VMEM();     // next plane's loads have landed; the stores below are not waited for
     WT_WAVE_PRIORITY(0);
-    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, bias_of(c), out + plane_off, ltid);
+    if (live) synth_final<T, K, TJ1>(lds, pl, fwc, fwc + fw_skip + KK, bias_of(c), out + plane_off, ltid, sg);
     plane_sync(wave_local);   // the next plane overwrites the buffers read above
   }
 }
@@ -947,12 +943,11 @@ __device__ __forceinline__ void corr_strip2(const float* __restrict__ a, int ast
 // row under every stacked plane).
 template <int K, int TJ, int VW, bool PAIR>
 __device__ __forceinline__ void corr_level(const float* __restrict__ A, int astr, const float* __restrict__ G,
-                                           int gstr, int h, const RowSplit split, int lane, int pass_row0, int pass_step,
+                                           int gstr, int h, const RowWalk at, int pass_row0, int pass_step,
                                            float (&acc)[K * K]) {
-  const int row = row_of(split, lane), rpp = split.rows;      // row items per pass of one wave (>= 1: kMaxWgradWidth, plan.h)
-  const int strip = lane - imul(row, split.per_row);
-  if (row >= rpp || strip >= split.used) return;
-  const int j0 = strip * TJ;
+  const int row = at.row, rpp = at.rows;      // row items per pass of one wave (>= 1: kMaxWgradWidth, plan.h)
+  if (row >= rpp) return;
+  const int j0 = at.strip * TJ;
   if constexpr (PAIR) {
     const int npair = (h + 1) >> 1;
     for (int ip = pass_row0 * rpp + row; ip < npair; ip += pass_step * rpp) {
@@ -989,7 +984,7 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
   const int chunk = blockIdx.y;
   const int tid = threadIdx.x;
   const int wave = WT_UNIFORM(tid >> 6);
-  int lane = tid & (kWave - 1);
+  const int first_lane = tid & (kWave - 1);
   const int q = wave & 3;
   const bool role_a = wave < 4;
   const int P = pl.P;
@@ -1019,6 +1014,29 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
   auto a_plane = [&](int l, int s) { return lds + pl.aoff[l] + s * pl.apl[l] + (P - R) * pl.astr[l] + (P - R); };
   auto g_plane = [&](int l, int s) { return lds + pl.goff[l] + s * pl.gpl[l]; };
   auto rows = [&](int l) { return pb * (pl.h[l] + P) - P; };
+  // strips that a row of level l is walked in, or single coefficients (see below)
+  auto in_strips = [&](int l) { return l < 2 || pl.w[l] >= kStripMinWidth; };
+  // Where this lane is in the rows of the two finest sets, level 0 (A) / 1 (B) and 3 (A) / 2 (B): row below strip in 16 bits each,
+  // 0xff for a lane without one.  Found once where a register is left to hold it, 56x56 planes 162.7 -> 157.6 us; with K = 5 the
+  // run-time plan's kernel has none (sums spilled for it: 45x42 planes, four levels 57.6 -> 63.9 us).
+  constexpr bool kHeld = Geo::kStatic || NSET == 1 || K <= 3 || (K == 7 && NSET == 2);
+  auto pack = [&](int l) {
+    const RowWalk at = walk_rows(pl.split[l], first_lane, kWave);
+    return at.row < at.rows ? static_cast<unsigned>(at.row | at.strip << 8) : 0xffu;
+  };
+  unsigned held = 0u;
+  int rows0 = 0, rows1 = 0;
+  if constexpr (kHeld) {
+    auto wave_rows = [&](int l) { return walk_rows(pl.split[l], 0, kWave).rows; };
+    held = role_a ? pack(0) : pack(1);
+    rows0 = role_a ? wave_rows(0) : wave_rows(1);
+    if constexpr (NSET >= 2) {
+      held |= (role_a ? pack(3) : pack(2)) << 16;
+      rows1 = role_a ? wave_rows(3) : wave_rows(2);
+    }
+  }
+  auto walk0 = [&](int l, int lane) { return kHeld ? RowWalk{static_cast<int>(held & 0xffu), static_cast<int>(held >> 8 & 0xffu), rows0} : walk_rows(pl.split[l], lane, kWave); };
+  auto walk1 = [&](int l, int lane) { return kHeld ? RowWalk{static_cast<int>(held >> 16 & 0xffu), static_cast<int>(held >> 24), rows1} : walk_rows(pl.split[l], lane, kWave); };
 
   const int b_begin = chunk * bchunk;
   const int b_end = b_begin + bchunk < B ? b_begin + bchunk : B;
@@ -1036,7 +1054,10 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
     const int b0 = WT_UNIFORM(bv);
     WT_LAUNDER_LANE_INT(slot);
     WT_LAUNDER_LANE_INT(ltid);
+    // (the lane's number once more instead of a register through the loop)
+    int lane = 0;
     WT_LAUNDER_LANE_INT(lane);
+    lane = lane_number(lane);
     const bool valid = has_slot && b0 + slot < b_end;
     const size_t plane_off = (static_cast<size_t>(valid ? b0 + slot : b0) * nC + c) * plane_elems;
     int l0 = 2;
@@ -1093,7 +1114,7 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
     {
       const int l = role_a ? 0 : 1;            // set 0, strips of TJ: base conv rows (A) / level 1 (B)
       corr_level<K, TJ, VW, true>(a_plane(l, role_a ? 0 : q), pl.astr[l], g_plane(l, role_a ? 0 : q), pl.gstr[l],
-                            rows(l), pl.corr[l], lane, role_a ? q : 0, role_a ? 4 : 1, acc[0]);
+                            rows(l), walk0(l, lane), role_a ? q : 0, role_a ? 4 : 1, acc[0]);
     }
     if (wave == 0) {
       // bias gradient: the sum of grad_out is 2^L times the sum of its coarsest LL band (every
@@ -1108,19 +1129,16 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
         // a level at least kStripMinWidth wide is walked in row pairs of TJ-wide strips like the
         // first set (one pass of a wave instead of four at 14 x 14), a narrower one by single
         // coefficients (more lanes busy)
-        if (pl.w[l] >= kStripMinWidth)
-          corr_level<K, TJ, VW, true>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0,
-                                      1, acc[1]);
+        if (in_strips(l))
+          corr_level<K, TJ, VW, true>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), walk1(l, lane), 0, 1, acc[1]);
         else
-          corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0,
-                                     1, acc[1]);
+          corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), walk1(l, lane), 0, 1, acc[1]);
       }
     }
     if constexpr (NSET >= 3) {                 // set 2: level 5 (A) / level 4 (B)
       const int l = role_a ? 5 : 4;
       if (l <= L) {
-        corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), pl.corr[l], lane, 0, 1,
-                                   acc[2]);
+        corr_level<K, 1, 1, false>(a_plane(l, q), pl.astr[l], g_plane(l, q), pl.gstr[l], rows(l), walk_rows(pl.split[l], lane, kWave), 0, 1, acc[2]);
       }
     }
     WT_LDS_BARRIER();
@@ -1134,11 +1152,11 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
 #pragma unroll
     for (int t = 0; t < KK; ++t) {
       const float v = wave_sum(acc[s][t]);
-      if (lane == 0) red[wave * NRED + s * KK + t] = v;
+      if (first_lane == 0) red[wave * NRED + s * KK + t] = v;
     }
   {
     const float v = wave_sum(gsum) * static_cast<float>(1 << L);
-    if (lane == 0) red[wave * NRED + NRED - 1] = v;
+    if (first_lane == 0) red[wave * NRED + NRED - 1] = v;
   }
   WT_LDS_BARRIER();
   float* dst = partial + (static_cast<size_t>(chunk) * nC + c) * (NF * KK + 1);

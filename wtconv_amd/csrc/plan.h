@@ -19,15 +19,16 @@ constexpr int kTJW = 4;     // weight-gradient correlation strips
 
 constexpr int pow2_ceil(int v) { int p = 1; while (p < v) p *= 2; return p; }
 
+// A row of per_row threads as walk_rows takes it.
+constexpr unsigned dense_rows(int per_row) { return static_cast<unsigned>(per_row) << 21 | ((1u << 20) + per_row - 1) / per_row; }
+
 // Rows of `used` items over the threads: dense, or a power of two of threads each where that takes `height` rows, and half as
-// many, in as many passes (shifts instead of products where the plan is a constant: 56x56 step 421.9 -> 420.6 us, gradients of
-// 28x28 planes 111.0 -> 107.6).
-constexpr RowSplit row_split(int used, int threads, int height) {
+// many, in as many passes (which is 0.2 % faster at the geometric mean, now and then a tenth or more either way: banks).
+constexpr unsigned row_split(int used, int threads, int height) {
   const int p = pow2_ceil(used);
   auto passes = [&](int n, int per_row) { const int rows = threads / per_row; return rows > 0 ? (n + rows - 1) / rows : n + 1; };
   const bool even = passes(height, p) == passes(height, used) && passes((height + 1) / 2, p) == passes((height + 1) / 2, used);
-  const int per_row = even && p <= threads ? p : used;
-  return {per_row, threads / per_row, ((1u << 20) + per_row - 1) / per_row, used};
+  return dense_rows(even && p <= threads ? p : used);
 }
 constexpr int log2_int(int v) { int s = 0; while ((1 << s) < v) ++s; return s; }
 
@@ -136,8 +137,8 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
 constexpr void finish_plane_plan(Plan2D* pl, int tj1, int sg_shift) {
   pl->sg_shift = sg_shift;
   const int sg = 1 << pl->sg_shift;
-  pl->strips1 = row_split((pl->w[1] + tj1 - 1) / tj1, sg, pl->h[1]);
-  for (int l = 2; l <= pl->L; ++l) pl->coefs[l] = row_split(pl->w[l], sg, pl->h[l]);
+  pl->split[1] = row_split((pl->w[1] + tj1 - 1) / tj1, sg, pl->h[1]);
+  for (int l = 2; l <= pl->L; ++l) pl->split[l] = row_split(pl->w[l], sg, pl->h[l]);
   pl->block = sg > 256 ? sg : 256;   // (two whole planes per 512-thread workgroup measured slower: lockstep phases)
   const int slots = pl->block / sg;
   pl->lds_floats = pl->plane_lds_floats * slots;
@@ -216,7 +217,7 @@ inline bool same_plane_geometry(const Plan2D& a, const Plan2D& b) {
       a.fuse != b.fuse || a.block != b.block || a.fw_stride != b.fw_stride || a.fw_skip != b.fw_skip)
     return false;
   for (int l = 0; l <= a.L; ++l)
-    if (a.h[l] != b.h[l] || a.w[l] != b.w[l] || a.aoff[l] != b.aoff[l] || a.astr[l] != b.astr[l] ||
+    if (a.h[l] != b.h[l] || a.w[l] != b.w[l] || a.split[l] != b.split[l] || a.aoff[l] != b.aoff[l] || a.astr[l] != b.astr[l] ||
         a.apl[l] != b.apl[l] || a.zoff[l] != b.zoff[l] || a.zstr[l] != b.zstr[l])
       return false;
   return true;
@@ -253,8 +254,7 @@ constexpr void finish_wgrad_plan(Plan2D* pl, int K) {
   // just as many strips: 78x66 planes (K = 5, L = 2, 17 strips of 32 lanes) 148.3 -> 127.3 us, 45x37 (K = 7, 10 of 16) 44.5 -> 39.6,
   // 15x17 (K = 7) 93.6 -> 82.3, 40x34 229.7 -> 211.4, 70x75 (K = 3) 73.4 -> 67.9; 56x56 167.6 -> 167.7, 12x10 44.4 -> 45.3.
   for (int l = 0; l <= pl->L; ++l)
-    pl->corr[l] = row_split(l < 2 || (l < 4 && pl->w[l] >= kStripMinWidth) ? (pl->w[l] + kTJW - 1) / kTJW : pl->w[l], kWave,
-                            pl->pb == 1 ? pl->h[l] : 512);      // (stacked planes: dense)
+    pl->split[l] = dense_rows(l < 2 || (l < 4 && pl->w[l] >= kStripMinWidth) ? (pl->w[l] + kTJW - 1) / kTJW : pl->w[l]);
   const int slots = pow2_ceil(pl->pb);
   pl->slot_shift = log2_int(512 / slots);
   const int nps = 512 / slots;
@@ -283,7 +283,7 @@ inline bool same_wgrad_geometry(const Plan2D& a, const Plan2D& b) {
       a.plane_lds_floats != b.plane_lds_floats)
     return false;
   for (int l = 0; l <= a.L; ++l)
-    if (a.h[l] != b.h[l] || a.w[l] != b.w[l] || a.aoff[l] != b.aoff[l] || a.astr[l] != b.astr[l] ||
+    if (a.h[l] != b.h[l] || a.w[l] != b.w[l] || a.split[l] != b.split[l] || a.aoff[l] != b.aoff[l] || a.astr[l] != b.astr[l] ||
         a.apl[l] != b.apl[l] || a.goff[l] != b.goff[l] || a.gstr[l] != b.gstr[l] || a.gpl[l] != b.gpl[l])
       return false;
   return true;
