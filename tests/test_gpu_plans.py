@@ -24,6 +24,12 @@ pytestmark = pytest.mark.gpu
     ((40, 9, 45, 50), 3, 2, torch.float32),       # K = 3: strips of two, odd rows a pass
     ((300, 1, 87, 66), 7, 1, torch.float32),      # 512 threads a plane, rows of 17 strips
     ((2, 130, 5, 77), 7, 2, torch.float32),       # three rows of 39 coefficients
+    ((1, 7, 33, 36), 7, 1, torch.float32),        # few planes: 512 threads each, strips of one
+    ((1, 5, 66, 58), 5, 3, torch.float16),        # and 1024
+    ((4, 3, 99, 79), 3, 2, torch.float32),        # 512 threads, strips of two
+    ((300, 5, 6, 5), 7, 1, torch.float32),        # four planes a wave, strips of one
+    ((209, 4, 13, 16), 7, 3, torch.float32),      # a wave a plane
+    ((1, 2, 3, 130), 5, 1, torch.float32),        # two rows of 65 coefficients
     ((3, 4, 13, 255), 5, 2, torch.float32),       # parameter gradients: one row of 64 strips a wave
     ((4, 6, 30, 9), 3, 2, torch.float32),         # 21 rows of three strips
     ((5, 4, 21, 82), 7, 1, torch.float16),        # three rows of 21, one lane without

@@ -189,6 +189,21 @@ static size_t stream_sub_records(const Stream2D& s, int B, int C, int K, int L) 
   return round_up64(static_cast<size_t>(wgrad_split(B, C, s.h[d], s.w[d], K, L - d).nchunk) * C * ((1 + 4 * (L - d)) * K * K + 1));
 }
 
+// choose_plane_shape's answer, kept for the sizes asked for last: it weighs up to twenty pairs, two microseconds of host time that
+// a small call would show.
+static void plane_shape(const Plan2D& pl, int K, int* tj1, int* sg_shift) {
+  struct Known { int B, C, H, W, K, L, tj1, sg_shift; };
+  static thread_local Known known[64] = {};
+  const unsigned at = (pl.B * 31u + pl.C) * 31u + pl.H * 97u + pl.W * 7u + K * 5u + pl.L;
+  Known& k = known[(at ^ at >> 6) % 64];
+  if (k.B != pl.B || k.C != pl.C || k.H != pl.H || k.W != pl.W || k.K != K || k.L != pl.L) {
+    k = {pl.B, pl.C, pl.H, pl.W, K, pl.L, 4, 8};
+    choose_plane_shape(pl, K, &k.tj1, &k.sg_shift);
+  }
+  *tj1 = k.tj1;
+  *sg_shift = k.sg_shift;
+}
+
 // One launch of the plane-resident kernels on planes that fit LDS; `fw` / `fb` folded parameters, those of a channel
 // `fw_stride` floats from the next one's, the level filters `fw_skip` floats behind their usual place.
 static int resident2d(const char* fn, const void* x, void* out, const float* fw, const float* fb, int B, int C, int H,
@@ -196,11 +211,8 @@ static int resident2d(const char* fn, const void* x, void* out, const float* fw,
                       const PlaneFold& fold = PlaneFold{}) {
   Plan2D pl = make_plan2d(B, C, H, W, K, L, false, 256);
   int tj1 = 4, sg_shift = 8;
-  choose_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
-  // keep the slots of a workgroup within LDS: fewer, larger plane groups if needed
-  while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
-  if (!plane_shape_is_static(K, H, W, L))
-    widen_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, pl.nplanes, &tj1, &sg_shift);
+  if (plane_shape_is_static(K, H, W, L)) static_plane_shape(H, &tj1, &sg_shift);
+  else plane_shape(pl, K, &tj1, &sg_shift);
   finish_plane_plan(&pl, tj1, sg_shift);
   pl.fw_stride = fw_stride;
   pl.fw_skip = fw_skip;

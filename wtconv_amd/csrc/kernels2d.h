@@ -687,7 +687,7 @@ __device__ __forceinline__ void zero_lds(float* lds, int nfloats) {
 
 // Forward (and, with flipped folded weights and zero fb, input-gradient) kernel.
 // Persistent: grid.x = min(work units, resident workgroups), block = 256 threads, or 512 or 1024 that share one plane
-// where few planes run on a CU at once (widen_plane_shape).
+// where few planes run on a CU at once (choose_plane_shape).
 // 2^sg_shift threads share a plane, so a workgroup holds blockDim >> sg_shift planes, each in
 // its own LDS slot (small planes: up to 16 per workgroup).  When a plane takes less than a wave,
 // the planes of one wave are the same channel of consecutive batch items, so the folded

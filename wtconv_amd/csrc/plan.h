@@ -42,44 +42,6 @@ static_assert(kTJC == 1, "row_lanes counts single coefficients of level 2");
 // Widest plane of the weight-gradient kernel: a wave sums strips of kTJW pixels of whole rows.
 constexpr int kMaxWgradWidth = kWave * kTJW;
 
-// What level 1 costs in strips of `tj` over `threads` threads, in lane-instructions: the lanes that are taken up -- half of
-// it counted by the waves that have any strip, half by whole passes (an idle wave costs no issue slots, but its workgroup
-// waits) -- times a strip's 8 K^2 tj multiply-adds, divided by what its LDS reads leave of them (a 5 x 5 window does 1.7, 0.9
-// or 0.6 multiply-adds for a float it reads), and 100 instructions a thread in the plane's other phases.
-// Fitted to every width and thread count on 308 shapes (fp32, 6 to 110 pixels, K = 3 to 7): the pick is 2 % slower than the
-// best pair at the geometric mean, picks by busy lanes alone 5 %, up to half slower.  Those took (forward, us)
-// [16,72,45,37], K = 7, two levels 33.9, now 27.5; [17,140,87,66], K = 7, one level 129 -> 90; [148,168,19,17], K = 5, one
-// level 64 -> 46; [20,252,44,43], K = 7, two levels 100 -> 77.
-constexpr double strip_cost(int K, int h1, int w1, int tj, int threads) {
-  const int per_row = (w1 + tj - 1) / tj, rows = threads / per_row, full = h1 / rows, rest = h1 - full * rows;
-  auto waves_of = [](int lanes) { return (lanes + kWave - 1) / kWave * kWave; };
-  const double passes = static_cast<double>(threads) * (full + (rest > 0 ? 1 : 0));
-  const double busy = threads >= kWave ? static_cast<double>(full) * waves_of(rows * per_row) + waves_of(rest * per_row) : passes;
-  return 0.5 * (passes + busy) * 8 * K * K * tj / (tj == 1 ? (K > 5 ? 0.4 : 0.65) : tj == 2 && K > 3 ? 0.9 : 1.0) + 100.0 * threads;
-}
-
-// Level-1 strip width and threads per plane of the plane kernel: the cheaper pair (ties: the
-// wider strip), which counts for more when the slots of a workgroup (256 / threads-per-plane planes of
-// `plane_lds_bytes` each) leave room for fewer than three workgroups per CU: with two, the
-// phases of a plane are latency bound (measured on 14x14 planes: 88 -> 76 us with 32 instead
-// of 16 threads per plane, i.e. half the slots).
-constexpr void choose_plane_shape(int K, int h1, int w1, size_t plane_lds_bytes, int* tj1, int* sg_shift) {
-  double best = 0.0;
-  const int lanes = row_lanes(2 * w1), most = lanes > 256 ? lanes : 256;
-  for (int tj = 4; tj >= 1; tj /= 2) {
-    const int per_row = (w1 + tj - 1) / tj;
-    if (per_row > most) continue;
-    int sg = per_row * h1 < most ? pow2_ceil(per_row * h1) : most;
-    if (sg < 16) sg = 16;
-    if (sg < lanes) sg = lanes;
-    double cost = strip_cost(K, h1, w1, tj, sg);
-    const size_t wg_lds = plane_lds_bytes * (256 / sg);
-    const int resident = wg_lds ? static_cast<int>(kLdsLimitBytes / wg_lds) : 3;
-    if (resident < 3) cost *= 3.0 / (resident > 0 ? resident : 0.5);
-    if (best == 0.0 || cost < best - 1e-9) { best = cost; *tj1 = tj; *sg_shift = log2_int(sg); }
-  }
-}
-
 // Fills the LDS layout of one plane.  Planes are stacked in one column: x, then the four
 // sub-band planes of level 1, level 2, ...; consecutive planes are separated by one gap of
 // P zero rows that serves as bottom halo of the upper and top halo of the lower plane.
@@ -133,6 +95,55 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
   return make_plan2d_geometry(B, C, H, W, K, L, with_grad_pyramid, nthreads, pb);
 }
 
+// Time of the plane kernel on a plan's planes (pl.B of them for each of pl.C channels), up to a factor and a constant, with
+// level-1 strips of `tj` and 2^sg_shift threads a plane.  A unit is what takes up whole waves: a plane, or the planes of one
+// channel that a wave holds.  Each of 256 compute units has `units` of them, n at a time, and takes
+//   rounds * latency of one + units * issue slots of one
+// where the last round counts half.  A level-1 strip is w = 8 K^2 tj multiply-adds, for narrow strips times what their LDS reads
+// add (a 5 x 5 window does 1.7, 0.9 or 0.6 multiply-adds for a float it reads); a wave by itself takes seven cycles for one, four
+// SIMDs together issue one a cycle.  Levels from 2 on are single coefficients, one after the other; a pass of 2 x 4 pieces is
+// 160 slots, and 600 cycles a level go to barriers and latencies.  Registers leave room for 1280 threads.
+// Fitted for the pick alone to every pair on 1803 shapes (fp32, 5 to 110 pixels, K = 3 to 7, 1 to 256 images, 16 to 512 channels):
+// 1 % slower than the best pair at the geometric mean.  Two simpler rules, most busy lanes (A) and fewest slots (B), both with
+// up to 256 threads and more only where few planes leave that many, were 7 % and 4 % slower than the best.  On 409 shapes that the
+// fit has not seen it takes 0.95 of A's time and 0.96 of B's; with K = 7 it is over a tenth slower than the faster of them on one
+// shape in forty.  Forward us, A / B / now: [64,64,33,21], K = 3, two levels 21.0 / 21.5 / 18.5; [8,32,64,64], K = 5, three levels
+// 14.5 / 14.6 / 13.4; [16,72,45,37], K = 7, two levels 32.8 / 26.4 / 26.6; [209,22,13,16], K = 7, three levels 27.5 / 40.2 / 27.6;
+// [1,83,33,36], K = 7, one level 10.3 / 13.3 / 9.1; and the worst, [134,433,9,10], K = 7, two levels 131 / 107 / 136.
+constexpr double plane_cost(const Plan2D& pl, int K, int tj, int sg_shift) {
+  const int threads = 1 << sg_shift, h1 = pl.h[1], per_row = (pl.w[1] + tj - 1) / tj, rows = threads / per_row;
+  const int full = h1 / rows, rest = h1 - full * rows, waves = threads > kWave ? threads / kWave : 1;
+  auto waves_of = [&](int lanes) { return threads > kWave ? (lanes + kWave - 1) / kWave : lanes > 0 ? 1 : 0; };
+  auto passes = [](int n, int at_once) { return (n + at_once - 1) / at_once; };
+  int coarse = 0;
+  for (int l = 2; l <= pl.L; ++l) coarse += passes(pl.h[l], threads / pl.w[l]);
+  const int pieces = passes(h1, threads / row_lanes(pl.W));
+  const double wide = 8.0 * K * K, w = wide * tj * (tj == 4 ? 1.0 : tj == 2 ? (K <= 3 ? 1.0 : K <= 5 ? 1.25 : 1.6) : K <= 3 ? 1.6 : K <= 5 ? 2.1 : 3.0);
+  const double latency = 7.0 * w * passes(h1, rows) + 3.0 * wide * coarse + 600.0 * (1 + pl.L) + 160.0 * pieces;
+  const double issue = w * (static_cast<double>(full) * waves_of(rows * per_row) + waves_of(rest * per_row)) + 160.0 * pieces * waves;
+  const int planes = threads < kWave ? kWave / threads : 1, block = threads > 256 ? threads : 256;
+  const double units = static_cast<double>(pl.C) * passes(pl.B, planes) / 256.0;
+  const int by_lds = kLdsLimitBytes / (pl.plane_lds_floats * 4 * (block / threads)), by_threads = block < 1280 ? 1280 / block : 1;
+  const double n = static_cast<double>(by_lds < by_threads ? by_lds : by_threads) * (block / (waves * kWave));
+  return (units <= n ? 1.0 : units / n + 0.5) * latency + (units < 1.0 ? 1.0 : units) * issue / 4;
+}
+
+// Level-1 strip width and threads per plane of the plane kernel: the cheapest pair (ties: the wider strip, the fewer threads)
+// of those whose rows fit the threads and whose planes, of a workgroup of 256, fit half of LDS.
+constexpr void choose_plane_shape(const Plan2D& pl, int K, int* tj1, int* sg_shift) {
+  double best = 0.0;
+  const size_t lds = static_cast<size_t>(pl.plane_lds_floats) * 4;
+  for (int tj = 4; tj >= 1; tj /= 2) {
+    const int per_row = (pl.w[1] + tj - 1) / tj;
+    for (int s = 4; s <= 10; ++s) {
+      if ((1 << s) < row_lanes(pl.W) || (1 << s) < per_row || ((1 << s) > 16 && (1 << s) > 4 * pow2_ceil(per_row * pl.h[1]))) continue;
+      if (s < 8 ? lds * (256 >> s) > kLdsLimitBytes / 2 : lds > kLdsLimitBytes) continue;
+      const double cost = plane_cost(pl, K, tj, s);
+      if (best == 0.0 || cost < best) { best = cost; *tj1 = tj; *sg_shift = s; }
+    }
+  }
+}
+
 // Completes a plan for the plane kernel: threads per plane, slots per workgroup, prefetch.
 constexpr void finish_plane_plan(Plan2D* pl, int tj1, int sg_shift) {
   pl->sg_shift = sg_shift;
@@ -165,38 +176,22 @@ struct PlaneGeoFold : PlaneGeoRuntime {
   static constexpr bool kFold = true;
   using Fold = PlaneFold;
 };
-constexpr Plan2D static_plane_plan(int H, int W, int K, int L, int* tj1_out) {
-  Plan2D pl = make_plan2d_geometry(1, 1, H, W, K, L, false, 256, 1);
-  int tj1 = 4, sg_shift = 8;
-  choose_plane_shape(K, pl.h[1], pl.w[1], static_cast<size_t>(pl.plane_lds_floats) * 4, &tj1, &sg_shift);
-  while (sg_shift < 8 && static_cast<size_t>(pl.plane_lds_floats) * 4 * (256 >> sg_shift) > kLdsLimitBytes / 2) ++sg_shift;
-  finish_plane_plan(&pl, tj1, sg_shift);
-  if (tj1_out != nullptr) *tj1_out = tj1;
-  return pl;
-}
-// Shapes with a compile-time plan of the plane kernel (plane2d.hip): the WTConvNeXt stages.
+// Shapes with a compile-time plan of the plane kernel (plane2d.hip): the WTConvNeXt stages, with the pairs that are fastest
+// there for many planes (few take them, too: [2,96,56,56] fp32 15.2 us, with more threads 18.4).
 constexpr bool plane_shape_is_static(int K, int H, int W, int L) {
   return K == 5 && H == W && ((H == 56 && L == 3) || (H == 28 && L == 3) || (H == 14 && L == 2) || (H == 7 && L == 2));
 }
-
-// More threads for a plane, when the workgroups a CU can hold at once -- by LDS, or for want of planes -- leave it with
-// fewer than twelve waves: the phases of a plane are bound by the latency of LDS then, and halving what a thread does
-// shortens them.  The level-1 strip is the cheapest one.
-// Forward us, fp32, K = 5, three levels, 256 threads -> widened: [16,64,80,80] (two by LDS) 53.6 -> 43.6, [16,64,72,72]
-// (K = 3, two levels) 35.7 -> 26.4, [16,64,68,68] (five levels) 67.2 -> 49.6; [1,64,40,40] (64 planes) 19.2 -> 17.7,
-// [8,32,64,64] 19.2 -> 18.6.  Planes with a compile-time plan stay with it: [2,96,56,56] 15.2, widened 18.4.
-inline void widen_plane_shape(int K, int h1, int w1, size_t plane_lds_bytes, int nplanes, int* tj1, int* sg_shift) {
-  if (*sg_shift != 8) return;
-  int wgs = plane_lds_bytes ? static_cast<int>(kLdsLimitBytes / plane_lds_bytes) : 1;
-  if (wgs > (nplanes + 255) / 256) wgs = (nplanes + 255) / 256;
-  while (*sg_shift < 10 && (wgs << *sg_shift) < 768) ++*sg_shift;
-  if (*sg_shift == 8) return;
-  double best = 0.0;
-  for (int tj = 4; tj >= 1; tj /= 2) {
-    if ((w1 + tj - 1) / tj > 1 << *sg_shift) continue;
-    const double cost = strip_cost(K, h1, w1, tj, 1 << *sg_shift);
-    if (best == 0.0 || cost < best - 1e-9) { best = cost; *tj1 = tj; }
-  }
+constexpr void static_plane_shape(int H, int* tj1, int* sg_shift) {
+  *tj1 = H >= 28 ? 4 : H == 14 ? 2 : 1;
+  *sg_shift = H == 56 ? 8 : H == 28 ? 6 : H == 14 ? 5 : 4;
+}
+constexpr Plan2D static_plane_plan(int H, int W, int K, int L, int* tj1_out) {
+  Plan2D pl = make_plan2d_geometry(1, 1, H, W, K, L, false, 256, 1);
+  int tj1 = 4, sg_shift = 8;
+  static_plane_shape(H, &tj1, &sg_shift);
+  finish_plane_plan(&pl, tj1, sg_shift);
+  if (tj1_out != nullptr) *tj1_out = tj1;
+  return pl;
 }
 
 template <int H, int W, int K, int L>
