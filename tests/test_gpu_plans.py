@@ -26,7 +26,7 @@ pytestmark = pytest.mark.gpu
     ((2, 130, 5, 77), 7, 2, torch.float32),       # three rows of 39 coefficients
     ((1, 7, 33, 36), 7, 1, torch.float32),        # few planes: 512 threads each, strips of one
     ((1, 5, 66, 58), 5, 3, torch.float16),        # and 1024
-    ((4, 3, 99, 79), 3, 2, torch.float32),        # 512 threads, strips of two
+    ((4, 3, 99, 79), 3, 2, torch.float32),        # the same, K = 3
     ((300, 5, 6, 5), 7, 1, torch.float32),        # four planes a wave, strips of one
     ((209, 4, 13, 16), 7, 3, torch.float32),      # a wave a plane
     ((1, 2, 3, 130), 5, 1, torch.float32),        # two rows of 65 coefficients

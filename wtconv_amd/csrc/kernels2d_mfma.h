@@ -62,7 +62,7 @@ struct MPlan {
   int tskip;                         // the others but this many (those of level 1, where they live in registers)
   int taps, tap_rows;                // byte offset of the folded filters as rows of taps; rows, the last one of zeros
   int behind;                        // planes that hold what the last rows' loads take along: (4 nbr - H) W + 3 elements
-  int uq, ur;                        // units of a workgroup: uq, the first ur of them one more
+  int uq, ur;                        // units of a workgroup: uq, ur of them one more
   int lds_bytes;
 };
 
@@ -463,8 +463,15 @@ wt2d_mfma_kernel(const T* __restrict__ x, T* __restrict__ out, const ParamTable 
 
   const int G = gridDim.x;
   const int wg = xcd_contiguous(blockIdx.x, G);
-  const int u_begin = wg * pl.uq + (wg < pl.ur ? wg : pl.ur);
-  const int u_end = u_begin + pl.uq + (wg < pl.ur ? 1 : 0);
+  // The workgroups with a unit more are the first to be dispatched, and so the first few of each XCD's and on different CUs.  With
+  // the first ranges longer instead, the first XCDs had twice the work of the last: us [30,48,57,64], two levels 18.4 -> 15.8,
+  // [256,264,8,6], one level 18.9 -> 15.6, [256,384,14,14], three levels 38.9 -> 36.3; 614 drawn shapes 0.99, one in eight over 5 %
+  // faster, two over 5 % slower, at most 9 %.  (Spread evenly over the ranges they meet on one CU: [256,33,16,18] 16.3 -> 20.6.)
+  const int xcds = (G & 7) == 0 ? 3 : 0, xcd = blockIdx.x & ((1 << xcds) - 1), nth = blockIdx.x >> xcds;
+  const int longer = (pl.ur + (1 << xcds) - 1 - xcd) >> xcds;                              // of this XCD, and of those before it
+  const int before = xcd * (pl.ur >> xcds) + min(xcd, pl.ur & ((1 << xcds) - 1));
+  const int u_begin = wg * pl.uq + before + min(nth, longer);
+  const int u_end = u_begin + pl.uq + (nth < longer ? 1 : 0);
 
   // A unit's channel, its number among the channel's units, and the batch items it takes: the batch is spread evenly over
   // the units of a channel, at most pb items each, all units within one plane of each other (a short last unit would leave
