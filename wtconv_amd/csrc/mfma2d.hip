@@ -46,6 +46,28 @@ size_t lds_budget() {
   return kLdsLimitBytes;
 }
 
+// Planes a unit of the kernels with a constant plan (the WTConvNeXt stage shapes: 56/28/14/7 squares; 3/3/2/2 levels as single
+// layers, 5/4/3/2 in the model); 0 for other shapes.
+constexpr int static_planes(int NS, int H, int W, int L) {
+  if (H != W) return 0;
+  if (NS != 1) return L == 3 ? (H == 56 ? 1 : H == 28 ? 2 : 0) : L == 2 ? (H == 14 ? 9 : H == 7 ? 21 : 0) : 0;
+  return H == 56 ? (L == 3 || L == 5 ? 1 : 0) : H == 28 ? (L == 3 || L == 4 ? 4 : 0) : H == 14 ? (L == 2 ? 15 : L == 3 ? 12 : 0) : H == 7 && L == 2 ? 32 : 0;
+}
+
+// Time of a launch with this plan, up to a factor.  Workgroups are persistent, and the one with most units is waited for: its
+// `rounds` units, each with a latency and with what the n workgroups of a CU take turns at -- to four fifths as if all had as many,
+// to one fifth by the units there are.  Fitted to all plans on 1141 shapes (bf16, up to 64 pixels), for the pick alone: 1.2 % slower
+// than the best of them at the geometric mean.
+double unit_cost(const MPlan& pl) {
+  const int by_lds = kLdsLimitBytes / pl.lds_bytes, per_cu = ceil_div(pl.nunits, 256);
+  int n = by_lds < 4 ? by_lds : 4;
+  if (n > per_cu) n = per_cu;
+  const int planes = pl.bq + (pl.br > 0 ? 1 : 0), rounds = ceil_div(pl.nunits, 256 * n);
+  double share = 6.0 + 4.0 / 4096 * planes * pl.H * pl.W;
+  for (int l = 1; l <= pl.L; ++l) share += 3.0 * ceil_div(planes * pl.nbr[l], 16 >> pl.tcs[l]);
+  return rounds * (20.0 + 0.8 * n * share) + 0.2 * (pl.nunits > 256 ? pl.nunits / 256.0 : 1.0) * share;
+}
+
 // Planes per unit: as many as keep every thread's share at one 4x4 block, shrunk until a
 // workgroup's LDS leaves room for several workgroups per CU.
 bool choose_mplan_uncached(int B, int C, int H, int W, int L, int NS, MPlan* out, int* nbl);
@@ -84,6 +106,7 @@ bool choose_mplan_uncached(int B, int C, int H, int W, int L, int NS, MPlan* out
   int pb = kMfmaBlock / bpp0;
   if (pb < 1) pb = 1;
   if (pb > B) pb = B;
+  const int fixed = NS == 1 ? static_planes(NS, H, W, L) : 0;
   // Four workgroups per CU (40 KB each) where the planes allow it; three (53 KB) if that puts
   // clearly more threads to work in the load phase of planes of 14 x 14 and larger (measured, bf16,
   // stage shapes: 28 x 28 planes 48 -> 44 us with 4 instead of 3 planes; 7 x 7 planes are faster
@@ -91,27 +114,38 @@ bool choose_mplan_uncached(int B, int C, int H, int W, int L, int NS, MPlan* out
   const size_t want = NS == 1 ? 40 * 1024 : 80 * 1024, relaxed = NS == 1 ? 53 * 1024 : 80 * 1024;
   const int pb_max = pb;
   MPlan pl;
-  for (;; --pb) {
-    if (!make_mplan(B, C, H, W, L, NS, pb, &pl)) return false;
-    if (static_cast<size_t>(pl.lds_bytes) <= want || pb == 1) break;
-  }
-  if (bpp0 >= 16 && pl.nblk[0] * 10 < kMfmaBlock * 6) {
-    for (int p2 = pb_max; p2 > pb; --p2) {
-      MPlan alt;
-      if (B % p2 == 0 && make_mplan(B, C, H, W, L, NS, p2, &alt) && static_cast<size_t>(alt.lds_bytes) <= relaxed) {
-        pl = alt;
-        pb = p2;
-        break;
+  if (fixed > 0) {
+    if (!make_mplan(B, C, H, W, L, NS, fixed < B ? fixed : B, &pl)) return false;
+  } else {
+    for (;; --pb) {
+      if (!make_mplan(B, C, H, W, L, NS, pb, &pl)) return false;
+      if (static_cast<size_t>(pl.lds_bytes) <= want || pb == 1) break;
+    }
+    if (bpp0 >= 16 && pl.nblk[0] * 10 < kMfmaBlock * 6) {
+      for (int p2 = pb_max; p2 > pb; --p2) {
+        MPlan alt;
+        if (B % p2 == 0 && make_mplan(B, C, H, W, L, NS, p2, &alt) && static_cast<size_t>(alt.lds_bytes) <= relaxed) {
+          pl = alt;
+          pb = p2;
+          break;
+        }
       }
     }
-  }
-  // a tile of level-1 blocks less, where it costs no more than a tenth of the planes (7 x 7: 32 of them instead of 33 fill two),
-  // and four tiles, one a wave, instead of more, where it costs no more than a quarter (12 x 12: 16 instead of 19)
-  for (int p2 = pb - 1; p2 * 4 >= pb * 3; --p2) {
-    MPlan alt;
-    if (make_mplan(B, C, H, W, L, NS, p2, &alt) && alt.ntile[1] < pl.ntile[1] && (alt.ntile[1] == 4 || p2 * 10 >= pb * 9)) {
-      pl = alt;
-      break;
+    // And of these planes or fewer, down to a third, what costs least.  us forward, bf16, with the most planes / what this picks:
+    // [101,102,17,13], two levels 15.7 / 15.7 of 11, 17.4 with the 10 that fill four tiles; [11,385,24,22], K = 3 17.3 / 16.1;
+    // [53,41,19,24], K = 3 11.2 / 10.3; [256,296,6,5], one level 15.4 / 14.8.  1141 shapes 0.98 of the time with a few planes less
+    // where that saves a tile or leaves four, one a wave (at most 13 % slower, 28 of them over 3 %).
+    if (NS == 1) {
+      double least = unit_cost(pl);
+      for (int p2 = pb - 1; p2 > 0 && p2 * 3 >= pb; --p2) {
+        MPlan alt;
+        if (!make_mplan(B, C, H, W, L, NS, p2, &alt)) continue;
+        const double cost = unit_cost(alt);
+        if (cost < least) {
+          least = cost;
+          pl = alt;
+        }
+      }
     }
   }
   if (static_cast<size_t>(pl.lds_bytes) > lds_budget()) return false;
@@ -156,11 +190,11 @@ int launch_mfma_vec(bool vec, const void* x, void* out, const MfmaArgs& a, const
              : launch_mfma<T, NS, NBL, false, GeoRuntime>(x, out, a, pl, stream);
 }
 
-// The WTConvNeXt stage shapes (56/28/14/7 squares; 3/3/2/2 levels as single layers, 5/4/3/2 in the
-// model) have kernels whose whole LDS layout is a compile-time constant.
-template <typename T, int NS, int H, int L, int PB, bool VEC>
+// A shape with a kernel whose whole LDS layout is a compile-time constant; fewer planes than it has places for run on it, too.
+template <typename T, int NS, int H, int L, bool VEC>
 bool try_static(bool vec, const void* x, void* out, const MfmaArgs& a, const MPlan& pl,
                 hipStream_t stream, int* rc) {
+  constexpr int PB = static_planes(NS, H, H, L);
   if (pl.H != H || pl.W != H || pl.L != L || pl.pb > PB || vec != VEC) return false;
   *rc = launch_mfma<T, NS, 1, VEC, GeoStatic<H, H, L, PB>>(x, out, a, pl, stream);
   return true;
@@ -171,14 +205,10 @@ int launch_mfma_nbl(int nbl, bool vec, const void* x, void* out, const MfmaArgs&
                     hipStream_t stream) {
 #ifndef WT_EMULATE
   int rc = 0;
-#define WT_TRY(H_, L_, PB_, VEC_) \
-  if (try_static<T, NS, H_, L_, PB_, VEC_>(vec, x, out, a, pl, stream, &rc)) return rc;
-  if constexpr (NS == 1) {
-    WT_TRY(56, 3, 1, true) WT_TRY(28, 3, 4, true) WT_TRY(14, 2, 15, false) WT_TRY(7, 2, 32, false)
-    WT_TRY(56, 5, 1, true) WT_TRY(28, 4, 4, true) WT_TRY(14, 3, 12, false)
-  } else {
-    WT_TRY(56, 3, 1, true) WT_TRY(28, 3, 2, true) WT_TRY(14, 2, 9, false) WT_TRY(7, 2, 21, false)
-  }
+#define WT_TRY(H_, L_, VEC_) \
+  if (try_static<T, NS, H_, L_, VEC_>(vec, x, out, a, pl, stream, &rc)) return rc;
+  WT_TRY(56, 3, true) WT_TRY(28, 3, true) WT_TRY(14, 2, false) WT_TRY(7, 2, false)
+  if constexpr (NS == 1) { WT_TRY(56, 5, true) WT_TRY(28, 4, true) WT_TRY(14, 3, false) }
 #undef WT_TRY
 #endif
   switch (nbl) {
