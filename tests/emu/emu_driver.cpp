@@ -187,6 +187,20 @@ int main(int argc, char** argv) {
     fclose(fo);
     return 0;
   }
+  if (dims == 8) {
+    // the head: header {8, B, C, H, W, 0, 0, dtype, pdtype, unused}; in x, weight, bias -> out (B, C)
+    Buf bx = read_buf(fp, static_cast<size_t>(B) * C * H * W, dtype), w = read_buf(fp, C, pdtype), b = read_buf(fp, C, pdtype);
+    fclose(fp);
+    Buf o = out_buf(static_cast<size_t>(B) * C, dtype);
+    const int rc = wtconv_pool_norm(bx.ptr(), o.ptr(), w.ptr(), b.ptr(), B, C, H * W, 1e-6f, dtype, pdtype, nullptr);
+    if (rc) { fprintf(stderr, "pool_norm: %s\n", wtconv_last_error()); return 3; }
+    o.unpack();
+    FILE* fo = fopen(argv[2], "wb");
+    if (!fo) { perror("open out"); return 2; }
+    fwrite(o.f.data(), 4, o.f.size(), fo);
+    fclose(fo);
+    return 0;
+  }
   const int S = dims == 2 ? 4 : 2;
   const size_t KK = dims == 2 ? static_cast<size_t>(K) * K : K;
   const size_t P = static_cast<size_t>(B) * C * H * W;   // 1-D: H == 1, W == N

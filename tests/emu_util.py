@@ -193,6 +193,24 @@ def run_patch_conv(stem, x, cw, cb, nw, nb, eps=1e-6, timeout=600):
         return np.fromfile(fout, dtype=np.float32).reshape(B, cw.shape[0], H // P, W // P)
 
 
+def run_pool_norm(x, weight, bias, dtype=0, pdtype=0, timeout=600):
+    """wtconv_pool_norm on the host; x (B,C,H,W), float32 arrays.  Returns (B,C)."""
+    exe = build()
+    B, C, H, W = x.shape
+    hdr = np.array([8, B, C, H, W, 0, 0, dtype, pdtype, 0], dtype=np.int32)
+    parts = [hdr.tobytes()] + [np.ascontiguousarray(a, dtype=np.float32).tobytes() for a in (x, weight, bias)]
+    with tempfile.TemporaryDirectory() as td:
+        fin, fout = os.path.join(td, "in.bin"), os.path.join(td, "out.bin")
+        with open(fin, "wb") as f:
+            f.write(b"".join(parts))
+        env = dict(os.environ)
+        env["ASAN_OPTIONS"] = "detect_leaks=0"
+        r = subprocess.run([exe, fin, fout], capture_output=True, text=True, timeout=timeout, env=env)
+        if r.returncode != 0:
+            raise RuntimeError(f"emu_driver failed ({r.returncode}):\n{r.stderr[-4000:]}")
+        return np.fromfile(fout, dtype=np.float32).reshape(B, C)
+
+
 def run_mlp(x, dy, w1, b1, w2, b2, timeout=600):
     """wtconv_mlp_forward and wtconv_mlp_backward on the host; x, dy (pixels, C), bf16 values in float32 arrays.  Returns
     y, dx and the gradients of the parameters in the order of the arguments."""

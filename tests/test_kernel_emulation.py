@@ -237,6 +237,14 @@ def test_emulated_2d_mfma_loads_stay_inside_the_tensor(B, C, H, W, K, L):
     _compare(got, _oracle(2, x, g, bw, bb, bs, ws, ss), rtol=2e-2, atol_scale=2e-2)
 
 
+@pytest.mark.parametrize("B,C,H,L", [(1, 2, 14, 3), (5, 1, 14, 3), (13, 1, 14, 3), (3, 2, 7, 2), (33, 1, 7, 2)])
+def test_emulated_2d_mfma_constant_plans(B, C, H, L):
+    """Compile-time plans: units of fewer planes than they have places for, and a unit more than one."""
+    x, g, bw, bb, bs, ws, ss = _case2d(B, C, H, H, 5, L, True, dtype=1, pdtype=1)
+    got = emu_util.run(2, x, g, bw, bb, bs, ws, ss, 5, dtype=1, pdtype=1, mfma=1)
+    _compare(got, _oracle(2, x, g, bw, bb, bs, ws, ss), rtol=2e-2, atol_scale=2e-2)
+
+
 def test_emulated_2d_bf16_vector_alu_kernels():
     """bf16 tensors on the vector-ALU kernels (what K = 7 or planes wider than 64 take)."""
     x, g, bw, bb, bs, ws, ss = _case2d(1, 2, 8, 12, 5, 2, True, dtype=1, pdtype=1)
@@ -525,3 +533,23 @@ def test_emulated_mlp_training(M, C, hidden):
 def test_emulated_block_mlp_few_pixels(B, C, H, W, hidden, layer_scale):
     """The two-kernel form of wtconv_block_mlp on the host under the sanitizers."""
     test_emulated_block_mlp(B, C, H, W, hidden, layer_scale)
+
+
+@pytest.mark.parametrize("B,C,H,W,dtype,pdtype", [
+    (1, 2, 1, 1, 1, 1), (2, 2, 3, 5, 1, 0), (1, 130, 7, 7, 1, 1), (2, 770, 3, 3, 0, 0), (1, 6, 9, 15, 0, 1),
+])
+def test_emulated_pool_norm(B, C, H, W, dtype, pdtype):
+    """wtconv_pool_norm on the host under the sanitizers: odd rows, channels that fill no pass, several trips a channel."""
+    rng = np.random.default_rng(C + H)
+    rd = lambda a, t: _bf16_round(a) if t else a
+    x = rd(rng.standard_normal((B, C, H, W)).astype(np.float32) + 3, dtype)
+    w, b = (rd(rng.standard_normal(C).astype(np.float32), pdtype) for _ in range(2))
+    got = emu_util.run_pool_norm(x, w, b, dtype, pdtype)
+    mean = rd(x.astype(np.float64).mean(axis=(2, 3)).astype(np.float32), dtype).astype(np.float64)
+    d = mean - mean.mean(axis=1, keepdims=True)
+    want = d / np.sqrt((d * d).mean(axis=1, keepdims=True) + 1e-6) * w + b
+    # a mean that falls on the other side of a boundary of bfloat16 is off by a unit, 2^-7 of its 3 or so, over a deviation of 1 / sqrt(H W);
+    # the result is rounded once
+    tol = 2. ** -7 * 4 * np.sqrt(H * W) + 2. ** -8 * np.abs(want) if dtype else 2e-5 * np.sqrt(H * W) * (1 + np.abs(want))
+    assert (np.abs(got - want) <= tol * (1 + np.abs(w))).all()
+    assert np.median(np.abs(got - want)) <= (2. ** -8 if dtype else 1e-5) * np.median(np.abs(want) + 1e-3)

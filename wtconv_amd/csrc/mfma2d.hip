@@ -203,14 +203,16 @@ bool try_static(bool vec, const void* x, void* out, const MfmaArgs& a, const MPl
 template <typename T, int NS>
 int launch_mfma_nbl(int nbl, bool vec, const void* x, void* out, const MfmaArgs& a, const MPlan& pl,
                     hipStream_t stream) {
-#ifndef WT_EMULATE
   int rc = 0;
 #define WT_TRY(H_, L_, VEC_) \
   if (try_static<T, NS, H_, L_, VEC_>(vec, x, out, a, pl, stream, &rc)) return rc;
-  WT_TRY(56, 3, true) WT_TRY(28, 3, true) WT_TRY(14, 2, false) WT_TRY(7, 2, false)
-  if constexpr (NS == 1) { WT_TRY(56, 5, true) WT_TRY(28, 4, true) WT_TRY(14, 3, false) }
-#undef WT_TRY
+  if constexpr (NS == 1) { WT_TRY(7, 2, false) WT_TRY(14, 3, false) }      // (the two that the host emulation runs, too)
+#ifndef WT_EMULATE
+  WT_TRY(56, 3, true) WT_TRY(28, 3, true) WT_TRY(14, 2, false)
+  if constexpr (NS == 1) { WT_TRY(56, 5, true) WT_TRY(28, 4, true) }
+  else { WT_TRY(7, 2, false) }
 #endif
+#undef WT_TRY
   switch (nbl) {
     case 1: return launch_mfma_vec<T, NS, 1>(vec, x, out, a, pl, stream);
     case 2: return launch_mfma_vec<T, NS, 2>(vec, x, out, a, pl, stream);
