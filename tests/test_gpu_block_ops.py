@@ -451,3 +451,36 @@ def test_pool_norm_hands_on_what_is_not_finite_and_leaves_the_rest(hip_device):
         assert fn(x, w.double(), b, 1e-6) is None and fn(x, w, None, 1e-6) is None
         assert fn(torch.zeros(1, 2, 300, 300, device=hip_device), w[:2], b[:2], 1e-6) is None
     assert fn(x.requires_grad_(), w, b, 1e-6) is None
+
+
+@pytest.mark.parametrize("kind,part", [("block", "input"), ("block", "norm.weight"), ("block", "mlp.fc1.weight"), ("block", "gamma"),
+                                       ("head", "input"), ("head", "norm.bias")])
+def test_tangents_take_pytorchs_own_passes(hip_device, kind, part):
+    """Forward-mode differentiation at inference: no kernel here has tangents, and none may lose them.  On the CPU, where no
+    kernel runs, the same module in double gives the tangent that is wanted."""
+    import copy
+    import torch.autograd.forward_ad as fwd
+    from wtconvnext import wtconvnext as N
+    torch.manual_seed(7)
+    module = N.WTConvNeXtBlock(96, wt_levels=1, ls_init_value=0.5) if kind == "block" else N._Head(96, 10)
+    if kind == "block":
+        module.conv_dw = torch.nn.Identity()      # (the layer itself refuses tangents)
+    x, step = torch.randn(2, 96, 8, 8), torch.randn(2, 96, 8, 8)
+
+    def tangent(device, dtype):
+        m = copy.deepcopy(module).to(device, dtype).requires_grad_(False)
+        xin = x.to(device, dtype)
+        with fwd.dual_level():
+            if part == "input":
+                xin = fwd.make_dual(xin, step.to(xin))
+            else:
+                owner, _, name = part.rpartition(".")
+                owner = m.get_submodule(owner)
+                p = getattr(owner, name).detach()
+                delattr(owner, name)
+                setattr(owner, name, fwd.make_dual(p, torch.linspace(-1, 2, p.numel()).square().view(p.shape).to(p)))
+            return fwd.unpack_dual(m(xin)).tangent
+
+    got, want = tangent(hip_device, torch.float32), tangent("cpu", torch.float64)
+    assert got is not None, "the tangent was lost"
+    torch.testing.assert_close(got.cpu().double(), want, rtol=1e-4, atol=1e-4 * want.abs().max().item())

@@ -8,6 +8,7 @@ Reference semantics: `x.permute(0, 2, 3, 1)` + `nn.LayerNorm` after `conv_dw`
 import ctypes
 
 import torch
+from torch.autograd import forward_ad as _forward_ad
 from torch.nn.modules import module as _nn
 from torch.utils._device import DeviceContext
 
@@ -22,9 +23,15 @@ def records(x, *params):
     return torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
 
 
+def _tangents(*tensors):
+    """Whether forward-mode differentiation follows any of these tensors."""
+    return _forward_ad._current_level >= 0 and any(t is not None and _forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def usable(x, *params, training=False):
     """Whether the kernels take this call: a contiguous fp32 / bf16 GPU tensor with an even channel count, parameters
-    of one fp32 / bf16 dtype on the same device, no autocast, not under torch.compile.  With training=False also:
+    of one fp32 / bf16 dtype on the same device, no autocast, no forward-mode differentiation (the kernels have no tangents
+    and raw pointers would lose them without a word), not under torch.compile.  With training=False also:
     nothing recorded for autograd (the plain functions below take raw pointers; the *_fn variants are the ones that
     autograd can differentiate)."""
     if not training and records(x, *params):
@@ -34,6 +41,8 @@ def usable(x, *params, training=False):
     if torch.is_autocast_enabled():      # autocast keeps LayerNorm outputs and the residual stream in fp32; the kernels return x.dtype
         return False
     if not x.is_cuda or x.dtype not in _DT or x.dim() != 4 or x.shape[1] % 2 or not x.is_contiguous():
+        return False
+    if _tangents(x, *params):
         return False
     pd = None
     for p in params:
@@ -47,7 +56,7 @@ def usable(x, *params, training=False):
 
 def usable_nhwc(y, shortcut):
     """Whether the residual kernels take the MLP output `y` (B, H, W, C) for this shortcut: same dtype and device."""
-    return y.dtype == shortcut.dtype and y.device == shortcut.device and y.dim() == 4
+    return y.dtype == shortcut.dtype and y.device == shortcut.device and y.dim() == 4 and not _tangents(y, shortcut)
 
 
 def _watched(*modules):
