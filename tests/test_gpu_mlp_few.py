@@ -10,6 +10,7 @@ pytestmark = pytest.mark.gpu
     ((1, 96, 4, 8), 384), ((1, 96, 3, 11), 64), ((3, 96, 29, 38), 384),      # a tile; a tile and one; nearly the last number taken
     ((1, 128, 7, 7), 512), ((2, 192, 28, 28), 768), ((1, 256, 31, 40), 1024),
     ((1, 384, 14, 14), 1536), ((17, 384, 7, 7), 192), ((1, 384, 8, 8), 4096),
+    ((1, 384, 17, 49), 2496), ((4, 192, 8, 16), 4096), ((2, 256, 23, 25), 1792),      # up to the most pixels times hidden units
     ((1, 512, 14, 14), 2048), ((1, 768, 7, 7), 3072), ((8, 768, 4, 13), 64), ((1, 1024, 7, 7), 4096), ((6, 1024, 4, 13), 1024),
 ])
 @pytest.mark.parametrize("layer_scale", [True, False])

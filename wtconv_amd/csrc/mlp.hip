@@ -83,8 +83,8 @@ int launch(MlpArgs a, size_t workspace_bytes, hipStream_t stream) {
 
 // ---- few pixels: two kernels (kernels_mlp_few.h), for these channel counts.  (Behind the shape: few_pays's limits, the hidden
 // units up to which the pixels do not matter, and the most pixels times hidden units.)
-#define WT_FEW_SHAPES(X) X(96, 2, 1, 768, 1280000) X(128, 2, 1, 256, 1280000) X(192, 2, 2, kMaxHidden, 1280000)         \
-                         X(256, 2, 2, kMaxHidden, 1280000) X(384, 4, 2, kMaxHidden, 1280000) X(512, 4, 2, kMaxHidden, 1280000) \
+#define WT_FEW_SHAPES(X) X(96, 2, 1, 768, 2 << 20) X(128, 2, 1, 256, 1280000) X(192, 2, 2, kMaxHidden, 2 << 20)       \
+                         X(256, 2, 2, kMaxHidden, 2 << 20) X(384, 4, 2, kMaxHidden, 2 << 20) X(512, 4, 2, kMaxHidden, 1280000) \
                          X(768, 4, 2, kMaxHidden, 1280000) X(1024, 4, 2, kMaxHidden, 1 << 20)
 constexpr long long kFewPixelChannels = 320000;
 constexpr int kFewTiles = 2;
@@ -105,19 +105,22 @@ bool has_few(int B, int C, int HW, int hidden) {
 
 // Whether the two kernels are the faster way.  Each tile of 32 pixels goes through all weights on its own, 2 C times the hidden
 // units, while the one kernel's time hardly depends on the pixels before its workgroups fill the chip: the lines of equal time
-// lie near a constant number of pixels * hidden units.  Where the one kernel needs no second launch (few channels), a second
-// launch pays from some hundred pixels on.  Measured (graph replay), us, two kernels / one kernel with its combination, from
-// 512 channels the separate passes, pixels by hidden units:
-//    96   32 x 64 5.9/7.9    3332 x 384 13.0/13.8   1664 x 768 10.1/15.2  | 96 x 2048 10.7/10.1  488 x 2048 10.6/15.4  1666 x 4096 39.9/21.3
-//   128   32 x 64 8.3/8.7    2340 x 256 13.1/15.2   | 64 x 512 9.5/9.0   256 x 512 9.1/9.9   1952 x 512 13.8/19.9   2500 x 512 17.4/16.2   1120 x 1024 16.5/14.6
-//   192   196 x 768 8.0/14.7   1664 x 768 13.3/21.5   312 x 4096 19.4/20.5   833 x 4096 38.4/24.8
-//   256   196 x 1024 11.6/15.7   976 x 1024 18.2/27.6   312 x 4096 23.2/23.1   625 x 4096 38.9/28.7
-//   384   196 x 1536 11.6/22.7   832 x 1536 22.0/28.3   312 x 4096 23.1/28.6   833 x 4096 54.1/36.3
-//   512   196 x 2048 16.9/29.7   624 x 2048 29.6/37.3   768   49 x 3072 15.6/40.7   416 x 3072 36.2/44.2   416 x 4096 47.8/44.2
-//  1024   49 x 4096 20.4/55.8   256 x 4096 36.9/39.8   312 x 4096 49.9/44.6
+// lie near a constant number of pixels * hidden units.  Measured (graph replay), us, two kernels / one kernel with its combination,
+// from 512 channels the separate passes, pixels by hidden units:
+//    96   196 x 384 7.7/12.1   3136 x 384 12.8/14.3   196 x 768 7.7/11.9   2500 x 768 15.5/17.8   3136 x 768 17.0/16.3
+//   128   196 x 512 8.0/10.8   2500 x 512 15.4/16.9   224 x 4096 16.4/18.4   312 x 4096 17.1/16.2
+//   192   196 x 768 8.5/15.5   1280 x 1024 14.5/20.6   512 x 4096 18.9/24.3   1280 x 2048 22.3/24.7   784 x 4096 33.9/21.8
+//   256   196 x 1024 10.2/16.2   1024 x 2048 22.4/26.0   512 x 4096 21.0/25.3   640 x 4096 30.1/26.0
+//   384   196 x 1536 11.9/23.2   784 x 1536 23.7/28.0   512 x 4096 29.7/32.2   784 x 2048 32.0/30.2   784 x 4096 47.9/33.1
+//   512   196 x 2048 16.1/30.6   256 x 4096 23.9/34.3   312 x 4096 35.1/38.0   392 x 4096 40.8/37.5
+//   768   49 x 3072 16.4/41.8   312 x 3072 28.1/38.0   312 x 4096 36.4/41.3   392 x 4096 47.2/43.9
+//  1024   49 x 4096 20.6/55.7   256 x 4096 37.6/39.9   312 x 4096 50.5/43.4
+// Of 208 other sizes of 192 to 384 channels five are over 5 % slower than the faster way, at most 10 %.  With 96 and 128 channels and
+// more hidden units than the first limit the line dates from a slower pair of kernels and lies too low: there 65 of 154 sizes
+// would be 5 to 48 % faster as two kernels (128, 196 x 768 8.1/13.2; 96, 1024 x 2048 12.8/17.1), up to about the 2 M of the others.
 bool few_pays(int pixels, int C, int hidden) {
   const long long work = static_cast<long long>(pixels) * hidden;
-#define WT_CASE(c, ng, kg, any, most) if (C == c) return hidden <= any ? work <= most : pixels >= 224 && work <= (1 << 20);
+#define WT_CASE(c, ng, kg, any, most) if (C == c) return hidden <= any ? work <= (most) : pixels >= 224 && work <= (1 << 20);
   WT_FEW_SHAPES(WT_CASE)
 #undef WT_CASE
   return false;
