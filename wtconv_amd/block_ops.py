@@ -189,11 +189,11 @@ def _stream():
 
 def channel_norm(x, weight, bias, eps, nhwc, pool=False):
     """LayerNorm over the channels of x (B, C, H, W); returns (B, H, W, C) if `nhwc` else (B, C, H, W).  Not recorded.
-    With `pool`, of its mean over the pixels."""
+    With `pool` (and without `nhwc`), of its mean over the pixels, (B, C, 1, 1)."""
     if pool:
         out = _native("pool_norm", x, weight, bias, eps)
         if out is not None:
-            return out[:, None, None] if nhwc else out[:, :, None, None]
+            return out[:, :, None, None]
         x = x.mean(dim=(2, 3), keepdim=True)
     out = _native("channel_norm", x, weight, bias, eps, nhwc) if not records(x, weight, bias) else None
     if out is not None:

@@ -11,13 +11,14 @@
 // -- 8 consecutive bf16 of an LDS row -- and receives four outputs of block n: its row q at the coarse levels, a square or
 // a lattice of it in the pixels and at level 1 (see the kernel).
 //
-// What bounds it: vector code (commit with two levels of analysis, synthesis), LDS round trips and the two barriers of a
-// unit, at four waves a SIMD for want of registers; the matrix cores are busy an eighth of the time.  us per launch, before
-// level 1 and base convolution met in registers (with the base convolution through LDS as fp32, levels 3 and up behind a
-// barrier each and one table entry a lane in the fold) -> now: [128,96,56,56], three levels 61.3 -> 54.2; [256,96,56,56],
-// five 164 -> 145; [128,192,28,28] 36.3 -> 32.2; [256,384,14,14] 48.5 -> 40.0; [128,768,7,7] 21.3 -> 15.5; a single image
-// of 14 x 14 x 384 12.4 -> 10.7; 120 drawn shapes 0.86 at the geometric mean, from 0.37 to 1.2 (batches of [34,36], whose
-// fifteen block rows make eight tiles for four waves, 20.4 -> 23.5).
+// What bounds it: LDS (busy 63 % of a 56 x 56 launch, 24 % on bank conflicts), vector code (44 %: commit with two levels of
+// analysis, synthesis) and the two barriers of a unit, at four waves a SIMD for want of registers (the constant plans spill one to
+// four of 128, the run-time plan more); the matrix cores are busy an eighth of the time.  us per launch, before level 1 and base
+// convolution met in registers (with the base convolution through LDS as fp32, levels 3 and up behind a barrier each and one table
+// entry a lane in the fold) -> now: [128,96,56,56], three levels 56.5 -> 49.6; [256,96,56,56], five 161 -> 141; [128,192,28,28]
+// 36.1 -> 31.7; [256,384,14,14] 47.3 -> 36.6; [128,768,7,7] 21.3 -> 15.5; a single image of 14 x 14 x 384 12.0 -> 7.2;
+// 250 drawn shapes 0.87 at the geometric mean, from 0.64 to 1.06 (two over 1.05: single images of few channels and two levels,
+// 8.5 -> 9.0; [34,36], whose fifteen block rows make eight tiles for four waves, 20.9 -> 21.2).
 //
 // Activations live in LDS as bf16 planes with a zero halo of 2.  bf16 tensors take one plane
 // per buffer (NS = 1).  fp32 tensors are split into NS = 3 bf16 planes (v = h0 + h1 + h2
@@ -51,7 +52,7 @@ struct MPlan {
   // MFMA tiles: 16 blocks = TR block-rows x TC block-columns, TC = 2^tcs >= nbc; the block-rows of
   // the stacked planes of a unit are numbered R = p * nbr + bi
   int tcs[kMaxLevels + 1], nrow[kMaxLevels + 1], ntile[kMaxLevels + 1];
-  int rtoff[kMaxLevels + 1];         // byte offset of the block-row table of level l
+  int rtoff[kMaxLevels + 1];         // byte offset of the block-row table of level l >= 1
   int pitch[kMaxLevels + 1];         // LDS row pitch of a level-l plane in bf16 elements (multiple of 4)
   int prows[kMaxLevels + 1];         // LDS rows from one stacked plane to the next: 4 nbr + 2
   int aoff[kMaxLevels + 1];          // byte offset of (slot 0, row -2, column -2) of sub-band 0, split 0
@@ -136,7 +137,7 @@ constexpr bool make_mplan_geometry(int H, int W, int L, int NS, int pb, MPlan* o
     pl.lloff[l] = off;
     off += rup(pb * pl.llpl[l] * 4, 16);
   }
-  for (int l = 0; l <= L; ++l) {
+  for (int l = 1; l <= L; ++l) {
     pl.rtoff[l] = off;
     off += rup(pl.nrow[l] * 4, 16);
   }
@@ -277,7 +278,6 @@ template <> struct PixRow<bf16_t> { uint2 v; };
 // address).  Columns past the row end come along and are cleared before use; nothing is computed on the loaded
 // words before the commit, so all the loads of a block stay in flight.
 __device__ __forceinline__ void pix_load4u(uint2& v, const bf16_t* p) { __builtin_memcpy(&v, p, 8); }
-__device__ __forceinline__ void pix_store4u(bf16_t* p, const uint2& v) { __builtin_memcpy(p, &v, 8); }
 // words that keep the valid columns of a block row: bits 4..7 of `cmask` say which of its four columns exist
 __device__ __forceinline__ uint2 pix_col_mask(unsigned cmask) {
   uint2 m;

@@ -87,13 +87,13 @@ struct Abi {
 template <typename F>
 void take(F& slot, uintptr_t addr) { slot = reinterpret_cast<F>(addr); }
 
-// Addresses in the order of the names in wtconv_amd/_ext.py.
 // What the look-ups below compare with, imported by bind(): an import within a call could let another thread in while a
 // static's initialisation is under way.
 struct Python {
   PyObject *module, *device_context, *linear, *gelu;
 } python;
 
+// Addresses in the order of the names in wtconv_amd/_ext.py.
 void bind(const std::vector<uintptr_t>& a) {
   TORCH_CHECK(a.size() == 32, "bind: expected 32 addresses, got ", a.size());
   take(abi.fwd2, a[0]); take(abi.bwd2, a[1]); take(abi.bwdin2, a[2]); take(abi.bwdpar2, a[3]); take(abi.ws2, a[4]);
@@ -570,9 +570,8 @@ py::object haar(const Tensor& x, const std::optional<Tensor>& bank, int64_t dims
   return py::cast(out);
 }
 
-// The block behind its WTConv layer in one kernel (inference): None if the kernel does not take these arguments or
-// autograd would record the call.
-// The result; undefined if the kernels do not take these tensors.  b1, b2 and gamma may be undefined.
+// The block behind its WTConv layer in one kernel (inference): undefined if the kernels do not take these tensors, or autograd
+// would record the call.  b1, b2 and gamma may be undefined.
 Tensor fused_mlp(const Tensor& x, const Tensor& shortcut, const Tensor& norm_w, const Tensor& norm_b, double eps, const Tensor& w1,
                  const Tensor& b1, const Tensor& w2, const Tensor& b2, const Tensor& gamma) {
   TORCH_CHECK(abi.bound, "wtconv binding used before bind()");
