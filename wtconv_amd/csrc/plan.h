@@ -110,6 +110,10 @@ inline Plan2D make_plan2d(int B, int C, int H, int W, int K, int L, bool with_gr
 // shape in forty.  Forward us, A / B / now: [64,64,33,21], K = 3, two levels 21.0 / 21.5 / 18.5; [8,32,64,64], K = 5, three levels
 // 14.5 / 14.6 / 13.4; [16,72,45,37], K = 7, two levels 32.8 / 26.4 / 26.6; [209,22,13,16], K = 7, three levels 27.5 / 40.2 / 27.6;
 // [1,83,33,36], K = 7, one level 10.3 / 13.3 / 9.1; and the worst, [134,433,9,10], K = 7, two levels 131 / 107 / 136.
+// 1500 more shapes that the fit has not seen, 449 of them fp16: 2 % slower than the best pair in both types, 0.90 of the time of the kernels
+// that went with A; 40 are over 3 % slower than those, 15 over a tenth (tall or wide planes of which LDS holds two or three, rows that
+// fall on the same banks), at most [113,17,43,98], K = 7, one level, 57.5 -> 70.4.  A new fit to half of them gained 0.3 % there
+// and 0.15 % on the other half.
 constexpr double plane_cost(const Plan2D& pl, int K, int tj, int sg_shift) {
   const int threads = 1 << sg_shift, h1 = pl.h[1], per_row = (pl.w[1] + tj - 1) / tj, rows = threads / per_row;
   const int full = h1 / rows, rest = h1 - full * rows, waves = threads > kWave ? threads / kWave : 1;
