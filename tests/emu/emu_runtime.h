@@ -74,6 +74,17 @@ inline float __shfl_xor(float v, int mask, int /*width*/) {
 
 namespace emu {
 
+// Value of the lane `d` (-1, 1) further in the wavefront, 0 from beyond it.  Every lane must call it.
+inline float lane_next_to(float v, int d) {
+  BlockState* b = tls_block;
+  b->xchg[threadIdx.x] = v;
+  wave_barrier();
+  const int l = static_cast<int>(threadIdx.x % 64) + d;
+  const float r = l < 0 || l > 63 ? 0.f : b->xchg[threadIdx.x + d];
+  wave_barrier();
+  return r;
+}
+
 // D = A (16x32) * B (32x16) + C on bfloat16 operands with float accumulation, operands and
 // result distributed over the 64 lanes of a wavefront as v_mfma_f32_16x16x32_bf16 holds them:
 // lane l carries A[l % 16][8 * (l / 16) + j], B[8 * (l / 16) + j][l % 16] (j = 0..7) and

@@ -27,8 +27,10 @@
 #define WT_CHUNK_FENCE() do {} while (0)
 #define WT_COMPILER_FENCE() asm volatile("" ::: "memory")
 #define WT_LAUNDER_UNIFORM_PTR(p) do {} while (0)
+#define WT_LAUNDER_UNIFORM(v) do {} while (0)
 #define WT_LAUNDER_LANE_INT(v) do {} while (0)
 #define WT_WAVE_PRIORITY(n) do {} while (0)
+#define WT_ANY_LANE(p) (p)
 typedef const float* wt_uniform_ptr;
 #else
 // Folded weights are read-only for the whole launch and indexed uniformly: the constant
@@ -73,6 +75,8 @@ typedef const float __attribute__((address_space(4)))* wt_uniform_ptr;
 // are issued here (25 SGPRs live) instead of being hoisted out of the row loop all at once
 // (hundreds of SGPRs, spilled to VGPR lanes).
 #define WT_LAUNDER_UNIFORM_PTR(p) asm volatile("" : "+s"(p))
+// The same for any wave-uniform value.
+#define WT_LAUNDER_UNIFORM(v) asm volatile("" : "+s"(v))
 // Makes a per-lane index opaque inside a loop body, so that the addresses derived from it
 // are recomputed per iteration (a few integer ops) instead of being hoisted out of the loop
 // into long-lived registers that end up spilled.
@@ -82,6 +86,8 @@ typedef const float __attribute__((address_space(4)))* wt_uniform_ptr;
 // priority so that they are not slowed down to a quarter of their speed by the arithmetic-heavy
 // phases of the other workgroups on the same SIMD, which fill whatever issue slots are left.
 #define WT_WAVE_PRIORITY(n) __builtin_amdgcn_s_setprio(n)
+// Whether a predicate holds in any lane of the wave, as a wave-uniform condition (the host emulation: this lane's own).
+#define WT_ANY_LANE(p) __any(p)
 #endif
 
 namespace wt {
@@ -436,6 +442,35 @@ __device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {
   const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
   a = r[0];
   b = r[1];
+#endif
+}
+
+// Value of the lane before / behind this one in its wavefront, 0 from beyond it.  Every lane takes part.  (DPP wave_shr:1,
+// wave_shl:1: a vector instruction.)
+__device__ __forceinline__ float wave_before(float v) {
+#ifdef WT_EMULATE
+  return ::emu::lane_next_to(v, -1);
+#else
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, true));
+#endif
+}
+__device__ __forceinline__ float wave_behind(float v) {
+#ifdef WT_EMULATE
+  return ::emu::lane_next_to(v, 1);
+#else
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, true));
+#endif
+}
+
+// w * x + c to a register of its own: sums that move from one name to the next as a loop goes on (a row of results up by
+// one) take no copies then, which they do where the compiler adds in place.  w is wave-uniform.
+__device__ __forceinline__ float fma_apart(float w, float x, float c) {
+#ifdef WT_EMULATE
+  return fmaf(w, x, c);
+#else
+  float d;
+  asm("v_fma_f32 %0, %1, %2, %3" : "=v"(d) : "s"(w), "v"(x), "v"(c));
+  return d;
 #endif
 }
 

@@ -29,20 +29,18 @@ namespace wt {
 constexpr int kStreamPad = 4;       // column halo of the LDS tiles in coefficients (>= K/2, keeps rows 16-byte aligned)
 constexpr int kStreamThreads = 256;
 
-// Eight elements to any element address.
+// Four elements, or the `n` < 4 that exist, to any element address.
 template <typename T>
-__device__ __forceinline__ void store8_any(T* __restrict__ p, const float (&v)[8]) {
-  uint4 q;
-  if constexpr (sizeof(T) == 4) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      q.x = __float_as_uint(v[4 * k]); q.y = __float_as_uint(v[4 * k + 1]);
-      q.z = __float_as_uint(v[4 * k + 2]); q.w = __float_as_uint(v[4 * k + 3]);
-      store_u4<4>(p + 4 * k, q);
-    }
+__device__ __forceinline__ void store4_any(T* __restrict__ p, int n, const float (&v)[4]) {
+  if (n >= 4) {
+    if constexpr (sizeof(T) == 4)
+      store_u4<4>(p, uint4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])});
+    else
+      store_u2<2>(p, uint2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])});
   } else {
-    q.x = pack2<T>(v[0], v[1]); q.y = pack2<T>(v[2], v[3]); q.z = pack2<T>(v[4], v[5]); q.w = pack2<T>(v[6], v[7]);
-    store_u4<2>(p, q);
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < n) p[e] = from_f32<T>(v[e]);
   }
 }
 
@@ -193,115 +191,328 @@ __device__ __forceinline__ void haar_tile(const float* __restrict__ Xt, float* _
   }
 }
 
-// One step of the layer on tiles of TW x TH level-1 coefficients (2 TW x 2 TH pixels).  `sub` (CARRY) = the sub-layer's
-// result on the LL band, (planes, hl, wl); without it the LL band is convolved here (the last level).  A thread owns four
-// adjacent coefficients of a row (2 x 8 output pixels): every LDS row it reads as 16-byte vectors feeds 4K (sub-bands)
-// or 8K (base conv) products.  fw[c * fstride]: the channel's folded filters; `fbase` / `fband` = offsets of the base
-// filter and of the four sub-band filters.  fb == nullptr: no bias.
-// Bound by vector issue and LDS reads in turn.  [8,96,160,160] fp32, K = 5, three levels: 99 us with 64-column tiles and
-// all four bands convolved here, 69.5 us now (2.3 TB/s).
-// grid = (tiles_x * tiles_y, gy, gz) with gy * gz >= planes, block = 256.
-template <typename T, int K, typename Shape, bool CARRY>
-__global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_kernel(const T* __restrict__ x, T* __restrict__ out,
-                                                                         const float* __restrict__ sub, int H, int W,
-                                                                         int hl, int wl, const float* __restrict__ fw,
-                                                                         const float* __restrict__ fb, int C,
-                                                                         int fstride, int fbase, int fband,
-                                                                         int nplanes) {
-  constexpr int R = K / 2, KK = K * K;
-  constexpr int TH = Shape::TH, TW = Shape::TW, HP = kStreamPad, TJ = 4, NT = TW / TJ;
-  constexpr int AH = TH + 2 * R, AWD = TW + 2 * HP, S0 = CARRY ? 1 : 0;
-  constexpr int XH = 2 * AH, XWD = 2 * AWD;
-  __shared__ alignas(16) float At[(4 - S0) * AH * AWD];
-  __shared__ alignas(16) float Xt[XH * XWD];
-  const int plane = WT_UNIFORM(static_cast<int>(blockIdx.z * gridDim.y + blockIdx.y));
-  if (plane >= nplanes) return;
-  const int tiles_x = (wl + TW - 1) / TW;
-  const int ty = blockIdx.x / tiles_x, tx = blockIdx.x - ty * tiles_x;
-  const int i0 = ty * TH, j0 = tx * TW;
-  const int tid = threadIdx.x;
-  const int r = tid / NT, c0 = (tid - r * NT) * TJ;
-  const int ch = plane % C;
-  const size_t psz = static_cast<size_t>(H) * W;
-  stage_window<T, XH, XWD>(x + plane * psz, H, W, 2 * (i0 - R), 2 * (j0 - HP), Xt, tid);
-  __syncthreads();
-  haar_tile<AH, AWD, S0>(Xt, At, tid);
-  __syncthreads();
-  const int i = i0 + r, j = j0 + c0;
-  if (r >= TH || i >= hl || j >= wl) return;
-  wt_uniform_ptr fwc = (wt_uniform_ptr)(fw + static_cast<size_t>(ch) * fstride);
-  float y[4][TJ];
+// ---- rows over the lanes of a wave ------------------------------------------------------------------------------------
+// A lane owns four pixels of a row (two coefficients) and walks down the plane; what it needs of its neighbours' rows comes
+// from their registers (wave_before, wave_behind), so there is no LDS, no barrier, and a wave only ever waits for its loads.
+// A unit is a stretch of rows of one tile (a column of lanes) of a plane; a wave takes `per` units of one channel side by
+// side.  Lanes whose pixels lie outside the plane hold zeros, which are the zero padding of the convolutions and of odd
+// extents; where two units that end at the plane's edge meet, lanes between them hold zeros as well.
+struct LaneSplit {
+  int tiles, own;          // tiles of a plane, lanes that each owns
+  int pitch, gap;          // lanes from unit to unit; more lanes behind each second one (two tiles a plane)
+  int per;                 // units of a wave
+  int segs, rows;          // stretches of a tile and their rows of coefficients
+  int units, blocks;       // of a channel
+};
+
+// Lanes that a lane's K x K windows reach to either side: the coefficients' reach further than the pixels'.
+constexpr int lane_halo(int K) { return (K / 2 + 1) / 2; }
+
+// v and its neighbours' values, R to either side.
+template <int N, int R>
+__device__ __forceinline__ void widen(const float (&v)[N], float (&w)[N + 2 * R]) {
 #pragma unroll
-  for (int s = S0; s < 4; ++s) {
-    wt_uniform_ptr w = fwc + fband + s * KK;
+  for (int e = 0; e < N; ++e) w[R + e] = v[e];
 #pragma unroll
-    for (int t = 0; t < TJ; ++t) y[s][t] = 0.f;
-#pragma unroll
-    for (int kh = 0; kh < K; ++kh) {
-      float v[12];
-      lds_read<12>(At + ((s - S0) * AH + r + kh) * AWD + c0, v);
-#pragma unroll
-      for (int kw = 0; kw < K; ++kw)
-#pragma unroll
-        for (int t = 0; t < TJ; ++t) y[s][t] = fmaf(w[kh * K + kw], v[t + kw - R + HP], y[s][t]);
-      if (K > 5 && kh == R) {            // (seven rows and 49 weights are more than the registers hold)
-        pin_values(y[s]);
-        WT_CHUNK_FENCE();
-      }
+  for (int d = 1; d <= R; ++d) {
+    float l = wave_before(v[(4 * N - d) % N]), r = wave_behind(v[(d - 1) % N]);
+    if (d > N) {
+      l = wave_before(l);
+      r = wave_behind(r);
     }
-    WT_CHUNK_FENCE();                    // one sub-band's LDS rows in registers at a time
+    w[R - d] = l;
+    w[R + N - 1 + d] = r;
   }
-  if constexpr (CARRY) {
-    const float* zp = sub + static_cast<size_t>(plane) * hl * wl + static_cast<size_t>(i) * wl + j;
-    if (j + TJ <= wl) {
-      load4_any<float>(zp, y[0]);
+}
+
+// Two rows of four pixels as they come from memory.
+template <typename T>
+struct RowPair {
+  static constexpr int N = sizeof(T) == 4 ? 4 : 2;      // words of a row
+  uint32_t w[2][N];
+
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int k = 0; k < N; ++k) w[0][k] = w[1][k] = 0u;
+  }
+  __device__ __forceinline__ void load(int row, const T* __restrict__ p) {
+    if constexpr (N == 4) {
+      const uint4 q = load_u4<4>(p);
+      w[row][0] = q.x; w[row][1] = q.y; w[row][2] = q.z; w[row][3] = q.w;
     } else {
-#pragma unroll
-      for (int t = 0; t < TJ; ++t) y[0][t] = j + t < wl ? zp[t] : 0.f;
+      const uint2 q = load_u2<2>(p);
+      w[row][0] = q.x; w[row][1] = q.y;
     }
   }
+  // (planes less than four pixels wide)
+  __device__ __forceinline__ void load_few(int row, const T* __restrict__ p, int n) {
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+      if (e < n) v[e] = to_f32<T>(p[e]);
+    if constexpr (N == 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[row][e] = __float_as_uint(v[e]);
+    } else {
+      w[row][0] = pack2<T>(v[0], v[1]);
+      w[row][1] = pack2<T>(v[2], v[3]);
+    }
+  }
+  __device__ __forceinline__ void get(int row, float (&v)[4]) const {
+    if constexpr (N == 4) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(w[row][e]);
+    } else {
+      unpack2<T>(w[row][0], v[0], v[1]);
+      unpack2<T>(w[row][1], v[2], v[3]);
+    }
+  }
+};
+
+// This lane's unit and place in it.
+struct LaneUnit {
+  int b, tile, seg;
+  int j;             // its first coefficient's column
+  bool have, owns;   // within the plane; owned by the unit
+};
+template <int HL>
+__device__ __forceinline__ LaneUnit lane_unit(const LaneSplit& sp, int u0, int lane, int wl) {
+  LaneUnit r;
+  // with two tiles a plane the gap follows each right one
+  const int first = sp.gap > 0 ? u0 & 1 : 0, pair = 2 * sp.pitch + sp.gap, l = lane + first * sp.pitch;
+  int slot, q;
+  if (sp.gap > 0) {
+    const int p = l / pair, in = l - p * pair;
+    slot = 2 * p + (in >= sp.pitch ? 1 : 0);
+    q = in - (in >= sp.pitch ? sp.pitch : 0);
+    slot -= first;
+  } else {
+    slot = lane / sp.pitch;
+    q = lane - slot * sp.pitch;
+  }
+  const int u = u0 + slot, bs = u / sp.tiles;
+  r.tile = u - bs * sp.tiles;
+  r.b = bs / sp.segs;
+  r.seg = bs - r.b * sp.segs;
+  if (r.tile > 0 || sp.tiles > 2) q -= HL;
+  r.j = 2 * (r.tile * sp.own + q);
+  r.have = slot < sp.per && u < sp.units && q < sp.own + HL && r.j >= 0 && r.j < wl;
+  r.owns = r.have && q >= 0 && q < sp.own;
+  return r;
+}
+
+// One step of the layer.  `sub` (CARRY) = the sub-layer's result on the LL band, (planes, hl, wl); without it the LL band is
+// convolved here (the last level).  A lane takes its rows of coefficients one after the other: each adds to the K rows of
+// band results around it and to as many rows of pixels, which move up by one (two) as the row ends; the first K - 1 rows and
+// the last, which reach beyond the stretch, skip what they would add outside it.  Coefficients are sums and differences
+// without their factor 1/2 (a power of two, made up for at the inverse).
+// fw[c * fstride]: the channel's folded filters; `fbase` / `fband` = offsets of the base filter and of the four sub-band
+// filters, in SGPRs a filter at a time.  fb == nullptr: no bias.
+// A row of coefficients at K = 5 is 350 multiply-adds of about 450 vector instructions, and [8,96,160,160] fp32 52 us (47 from
+// the caches), where the memory that it moves takes 35; tiles in LDS with a thread for four coefficients took 68.
+// grid = 1-D, a multiple of eight, at least C * sp.blocks; block = 256 (waves on their own).
+template <typename T, int K, bool CARRY>
+__global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_kernel(
+    const T* __restrict__ x, T* __restrict__ out, const float* __restrict__ sub, int H, int W, int hl, int wl,
+    const float* __restrict__ fw, const float* __restrict__ fb, int C, int fstride, int fbase, int fband, LaneSplit sp) {
+  constexpr int R = K / 2, KK = K * K, S0 = CARRY ? 1 : 0, NP = 3 * R + 2;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int at = xcd_contiguous(blockIdx.x, gridDim.x);      // (an XCD's workgroups share rows)
+  const int ch = WT_UNIFORM(at / sp.blocks);
+  const int u0 = WT_UNIFORM(((at - ch * sp.blocks) * (kStreamThreads / kWave) + (tid >> 6)) * sp.per);
+  if (ch >= C || u0 >= sp.units) return;
+  const LaneUnit un = lane_unit<lane_halo(K)>(sp, u0, lane, wl);
+  const bool have = un.have;
+  const int i0 = un.seg * sp.rows, i1 = un.owns ? min(i0 + sp.rows, hl) : i0, c0 = 2 * un.j;
+  const int steps = sp.rows + 2 * R;
+  const long long row0 = (static_cast<long long>(un.b) * C + ch) * H + 2 * i0;
+  const T* px = x + (row0 - 2 * R) * W + (W >= 4 ? piece_start(c0, W) : c0);
+  T* po = out + row0 * W + c0;
+  const float* pz = CARRY ? sub + ((static_cast<long long>(un.b) * C + ch) * hl + i0) * wl + un.j : nullptr;
+  wt_uniform_ptr fwc = (wt_uniform_ptr)(fw + static_cast<size_t>(ch) * fstride);
   const float bias = fb != nullptr ? fb[ch] : 0.f;
-  float o[2][2 * TJ];
+  // rows of pixels 2 (i - R) ..., and of band results i - R ..., around the row i of the step
+  float P[NP][4], Y[4][K][2];
 #pragma unroll
-  for (int t = 0; t < TJ; ++t) {
-    const float p = y[0][t] + y[1][t], m = y[0][t] - y[1][t], q = y[2][t] + y[3][t], d = y[2][t] - y[3][t];
-    o[0][2 * t] = fmaf(0.5f, p + q, bias);
-    o[0][2 * t + 1] = fmaf(0.5f, p - q, bias);
-    o[1][2 * t] = fmaf(0.5f, m + d, bias);
-    o[1][2 * t + 1] = fmaf(0.5f, m - d, bias);
-  }
-  wt_uniform_ptr wb = fwc + fbase;
+  for (int k = 0; k < NP; ++k)
 #pragma unroll
-  for (int xr = 0; xr < K + 1; ++xr) {
-    float v[16];
-    lds_read<16>(Xt + (2 * r + xr + R) * XWD + 2 * c0 + HP, v);
+    for (int e = 0; e < 4; ++e) P[k][e] = bias;
 #pragma unroll
-    for (int dr = 0; dr < 2; ++dr) {
-      const int kh = xr - dr;
-      if (kh < 0 || kh >= K) continue;
+  for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int kw = 0; kw < K; ++kw)
-#pragma unroll
-        for (int u = 0; u < 2 * TJ; ++u) o[dr][u] = fmaf(wb[kh * K + kw], v[u + kw - R + HP], o[dr][u]);
+    for (int k = 0; k < K; ++k) Y[s][k][0] = Y[s][k][1] = 0.f;
+
+  // (lanes without pixels keep the zeros that they start with)
+  auto fetch = [&](int t, int width, RowPair<T>& r) __attribute__((always_inline)) {
+    const int i = i0 - R + t;
+    const bool top = have && i >= 0 && 2 * i < H, bottom = have && i >= 0 && 2 * i + 1 < H;
+    if (WT_ANY_LANE(have && !bottom)) r.clear();
+    if (width >= 4) {
+      if (top) r.load(0, px);
+      if (bottom) r.load(1, px + width);
+    } else {
+      if (top) r.load_few(0, px, width - c0);
+      if (bottom) r.load_few(1, px + width, width - c0);
     }
-    if (xr & 1) WT_CHUNK_FENCE();      // two input rows in registers at a time
-  }
-  const int oj = 2 * j;
-  const int nvalid = W - oj;
+    px += 2 * width;
+  };
+  // Row t of the stretch: it adds to rows KLO .. KHI - 1 of the K around it.
+  auto step = [&](auto klo, auto khi, auto ends, int t, const RowPair<T>& now, RowPair<T>& next) __attribute__((always_inline)) {
+    constexpr int KLO = decltype(klo)::value, KHI = decltype(khi)::value;
+    constexpr bool ENDS = decltype(ends)::value;      // (and a row of results ends with it)
+    const int o = i0 + t - 2 * R;
+    // (what follows from these is not kept over the loop: the SGPRs are for the weights)
+    int at_c = c0, width = W;
+    WT_LAUNDER_LANE_INT(at_c);
+    WT_LAUNDER_UNIFORM(width);
+    float a[4], c[4], z[2] = {0.f, 0.f};
+    now.get(0, a);
+    now.get(1, c);
+    if (width >= 4) {
+      piece_shift(a, at_c, width);
+      piece_shift(c, at_c, width);
+    }
+    if (t + 1 < steps) fetch(t + 1, width, next);
+    if constexpr (ENDS && CARRY) {
+      if (o < i1) {
+        if (at_c + 2 < width) {
+          const uint2 v = load_u2<2>(pz);
+          z[0] = __uint_as_float(v.x);
+          z[1] = __uint_as_float(v.y);
+        } else {
+          z[0] = *pz;
+        }
+      }
+      pz += wl;
+    }
+    {
+      float ar[4 + 2 * R], cr[4 + 2 * R];
+      widen<4, R>(a, ar);
+      widen<4, R>(c, cr);
+      wt_uniform_ptr w = fwc + fbase;
+      WT_LAUNDER_UNIFORM(w);
 #pragma unroll
-  for (int dr = 0; dr < 2; ++dr) {
-    const int oi = 2 * i + dr;
-    if (oi < H) {
-      T* dst = out + plane * psz + static_cast<size_t>(oi) * W + oj;
-      if (nvalid >= 2 * TJ) {
-        store8_any<T>(dst, o[dr]);
-      } else {
+      for (int k = 0; k < NP; ++k) {
+        if (K > 3 && k > R && (k - R) % 2 == 0) {      // (three rows of a filter at a time)
+          pin_values(P[k - 1]);
+          pin_values(P[k - 2]);
+          WT_SCHED_FENCE();
+          WT_LAUNDER_UNIFORM(w);
+        }
+        const int up = 3 * R - k, low = up + 1;      // rows of the filter that the two rows of pixels meet
+        const bool adds = k >= R && k / 2 >= KLO && k / 2 < KHI;
 #pragma unroll
-        for (int e = 0; e < 2 * TJ; ++e)
-          if (e < nvalid) dst[e] = from_f32<T>(o[dr][e]);
+        for (int e = 0; e < 4; ++e) {
+          float v = k + 2 < NP ? P[k + 2][e] : bias;
+          if (adds && up >= 0) {
+#pragma unroll
+            for (int kw = 0; kw < K; ++kw) v = kw == 0 ? fma_apart(w[up * K], ar[e], v) : fmaf(w[up * K + kw], ar[e + kw], v);
+          }
+          if (adds && low < K) {
+#pragma unroll
+            for (int kw = 0; kw < K; ++kw)
+              v = kw == 0 && up < 0 ? fma_apart(w[low * K], cr[e], v) : fmaf(w[low * K + kw], cr[e + kw], v);
+          }
+          P[k][e] = v;
+        }
       }
     }
+    WT_SCHED_FENCE();
+#pragma unroll
+    for (int s = S0; s < 4; ++s) {
+      float v[2], vr[2 + 2 * R];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float sac = a[2 * e] + c[2 * e], sbd = a[2 * e + 1] + c[2 * e + 1];
+        const float dac = a[2 * e] - c[2 * e], dbd = a[2 * e + 1] - c[2 * e + 1];
+        v[e] = s == 0 ? sac + sbd : s == 1 ? dac + dbd : s == 2 ? sac - sbd : dac - dbd;
+      }
+      widen<2, R>(v, vr);
+      wt_uniform_ptr w = fwc + fband + s * KK;
+      WT_LAUNDER_UNIFORM(w);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        if (K > 3 && k == (K + 1) / 2) {
+#pragma unroll
+          for (int d = 0; d < (K + 1) / 2; ++d) pin_values(Y[s][d]);
+          WT_SCHED_FENCE();
+          WT_LAUNDER_UNIFORM(w);
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          float y = k + 1 < K ? Y[s][k + 1][e] : 0.f;
+          if (k >= KLO && k < KHI) {
+#pragma unroll
+            for (int kw = 0; kw < K; ++kw)
+              y = kw == 0 ? fma_apart(w[(2 * R - k) * K], vr[e], y) : fmaf(w[(2 * R - k) * K + kw], vr[e + kw], y);
+          }
+          Y[s][k][e] = y;
+        }
+      }
+      WT_SCHED_FENCE();      // (a filter at a time in SGPRs)
+    }
+    if constexpr (ENDS) {
+      if (o < i1) {
+        float r[2][4];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float y1 = Y[1][0][e];
+          const float p = CARRY ? fmaf(2.f, z[e], y1) : Y[0][0][e] + y1, m = CARRY ? fmaf(2.f, z[e], -y1) : Y[0][0][e] - y1;
+          const float q = Y[2][0][e] + Y[3][0][e], d = Y[2][0][e] - Y[3][0][e];
+          r[0][2 * e] = fmaf(0.25f, p + q, P[0][2 * e]);
+          r[0][2 * e + 1] = fmaf(0.25f, p - q, P[0][2 * e + 1]);
+          r[1][2 * e] = fmaf(0.25f, m + d, P[1][2 * e]);
+          r[1][2 * e + 1] = fmaf(0.25f, m - d, P[1][2 * e + 1]);
+        }
+        store4_any<T>(po, width - at_c, r[0]);
+        if (2 * o + 1 < H) store4_any<T>(po + width, width - at_c, r[1]);
+      }
+      po += 2 * width;
+    }
+  };
+  // (both ways round, so that no row moves from register to register)
+  using std::false_type;
+  using std::true_type;
+#define WT_ROWS(n) std::integral_constant<int, (n)>{}
+  RowPair<T> ra, rb;
+  ra.clear();
+  rb.clear();
+  fetch(0, W, ra);
+  if constexpr (R >= 1) {
+    step(WT_ROWS(2 * R), WT_ROWS(K), false_type{}, 0, ra, rb);
+    step(WT_ROWS(2 * R - 1), WT_ROWS(K), false_type{}, 1, rb, ra);
   }
+  if constexpr (R >= 2) {
+    step(WT_ROWS(2 * R - 2), WT_ROWS(K), false_type{}, 2, ra, rb);
+    step(WT_ROWS(2 * R - 3), WT_ROWS(K), false_type{}, 3, rb, ra);
+  }
+  if constexpr (R >= 3) {
+    step(WT_ROWS(2 * R - 4), WT_ROWS(K), false_type{}, 4, ra, rb);
+    step(WT_ROWS(2 * R - 5), WT_ROWS(K), false_type{}, 5, rb, ra);
+  }
+  int t = 2 * R;
+  for (; t + 1 < sp.rows; t += 2) {
+    step(WT_ROWS(0), WT_ROWS(K), true_type{}, t, ra, rb);
+    step(WT_ROWS(0), WT_ROWS(K), true_type{}, t + 1, rb, ra);
+  }
+  if (t < sp.rows) {
+    step(WT_ROWS(0), WT_ROWS(K), true_type{}, t, ra, rb);
+    ++t;
+    ra = rb;
+  }
+  if constexpr (R >= 1) {
+    step(WT_ROWS(0), WT_ROWS(2 * R), true_type{}, t, ra, rb);
+    step(WT_ROWS(0), WT_ROWS(2 * R - 1), true_type{}, t + 1, rb, ra);
+  }
+  if constexpr (R >= 2) {
+    step(WT_ROWS(0), WT_ROWS(2 * R - 2), true_type{}, t + 2, ra, rb);
+    step(WT_ROWS(0), WT_ROWS(2 * R - 3), true_type{}, t + 3, rb, ra);
+  }
+  if constexpr (R >= 3) {
+    step(WT_ROWS(0), WT_ROWS(2 * R - 4), true_type{}, t + 4, ra, rb);
+    step(WT_ROWS(0), WT_ROWS(2 * R - 5), true_type{}, t + 5, rb, ra);
+  }
+#undef WT_ROWS
 }
 
 // Where the sums of stream_corr_kernel go: partial[(chunk * C + c) * rec + f * K*K + t].
