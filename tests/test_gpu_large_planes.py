@@ -80,3 +80,18 @@ def test_infinities_stay_within_their_windows(hip_device):
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     fin = torch.isfinite(want)
     assert_fp32(got[fin], want[fin], "finite outputs")
+
+
+@pytest.mark.parametrize("row,col", [(70, 79), (70, 80), (70, 0), (139, 159), (0, 3)])
+def test_infinities_stay_within_their_sums(hip_device, row, col):
+    """An infinity of x makes those sums of the base filter's gradient infinite whose windows hold it, and no other: a lane
+    beside its unit's own ones, or below the plane, adds nothing (an infinity times no gradient is not a number)."""
+    H, W, K = 140, 160, 5
+    ref, x, g = seeded_case("2d", 2, K, 1, (1, 2, H, W))
+    x[0, 0, row, col] = float("inf")
+    got = hip_run(copy_to_hip_module(ref, _modules(), "2d", K, 1), x, g, hip_device)[2]["base_conv.weight"].reshape(2, K, K)
+    r = K // 2
+    want = torch.tensor([[0 <= row - kh + r < H and 0 <= col - kw + r < W for kw in range(K)] for kh in range(K)])
+    assert torch.equal(torch.isinf(got[0]).cpu(), want)
+    assert torch.equal(torch.isfinite(got[0]).cpu(), ~want)
+    assert torch.isfinite(got[1]).all()

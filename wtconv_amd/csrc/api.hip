@@ -133,9 +133,9 @@ static bool wgrad_fits_lds(int B, int C, int H, int W, int K, int L) {
 
 constexpr long long kMaxPlaneElems = 1LL << 28;
 
-// Workgroups of stream_corr_kernel that run at once (three per CU on 256 CUs; a constant, as workspace sizes must not
-// depend on the device queried): one round of them, at most one per batch item and 16 x 64 tile.
-constexpr int kStreamResident = 768;
+// Workgroups of stream_corr_kernel that run at once (two per CU on 256 CUs; a constant, as workspace sizes must not depend on
+// the device queried): one round of them, at most one per batch item and 16 x 64 coefficients.
+constexpr int kStreamResident = 512;
 static int stream_chunks(int B, int C, int H, int W) {
   const long long units = static_cast<long long>(B) * ((H + 31) / 32) * ((W + 127) / 128);
   long long want = kStreamResident / C;

@@ -8,15 +8,13 @@
 // sixteenth, ... of the pixels:
 //   stream_ll_kernel       X_1 of x, a quarter of the pixels, fp32
 //   (the sub-layer, by the same rule: plane-resident or another step)
-//   stream_final_kernel    tiles: detail bands of level 1 from the pixels in LDS, their convs, the sub-layer's result,
-//                          inverse Haar, base conv
+//   stream_final_kernel    detail bands of level 1, their convs, the sub-layer's result, inverse Haar, base conv
 // Parameter gradients follow the same recursion: stream_corr_kernel sums the base conv's and the detail bands' filters
 // from the pixels of x and grad_out, and the sub-layer's filters are its parameter gradients on X_1 and G_1.
 // Nothing of a level but its LL band goes through memory.
 //
-// Measured, us a training step (forward): [8,96,160,160] fp32 523 -> 380 (167 -> 118) against one launch per level and
-// pass with every band in memory; [8,64,141,155] fp16, K = 7 1018 -> 556 (350 -> 156); [4,64,199,230] fp32, five levels
-// 443 -> 325 (138 -> 109).
+// Measured, us a training step: [8,96,160,160] fp32 523 with a launch per level and pass and every band in memory, 366 with
+// tiles of a step in LDS, 310 with rows over the lanes of a wave.
 //
 // Rows start at any element's address and may have any length (16-byte accesses need no more than that).
 #pragma once
@@ -26,7 +24,6 @@
 
 namespace wt {
 
-constexpr int kStreamPad = 4;       // column halo of the LDS tiles in coefficients (>= K/2, keeps rows 16-byte aligned)
 constexpr int kStreamThreads = 256;
 
 // Four elements, or the `n` < 4 that exist, to any element address.
@@ -96,101 +93,6 @@ __global__ void stream_ll_kernel(const T* __restrict__ src, int hs, int ws, floa
   }
 }
 
-// Window of a plane -> LDS: dst[r * WD + c] = plane[gi0 + r][gj0 + c], zero outside the plane; gj0 a multiple of 4.
-// Four elements at a time; the position of a thread's next piece advances without divisions.  All loads of a thread
-// are issued before the first LDS write.
-template <typename T, int ROWS, int WD>
-__device__ __forceinline__ void stage_window(const T* __restrict__ src, int h, int w, int gi0, int gj0,
-                                             float* __restrict__ dst, int tid) {
-  constexpr int W4 = WD / 4;
-  constexpr int N = ROWS * W4;
-  constexpr int IT = (N + kStreamThreads - 1) / kStreamThreads;
-  constexpr int DR = kStreamThreads / W4, DC = kStreamThreads % W4;
-  static_assert(WD % 4 == 0, "whole vectors");
-  float v[IT][4];
-  {
-    int row = tid / W4, col = tid - row * W4;
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-      const int gi = gi0 + row, gj = gj0 + col * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[it][e] = 0.f;
-      if (row < ROWS && gi >= 0 && gi < h && gj >= 0 && gj < w) {
-        const T* q = src + (static_cast<size_t>(gi) * w + gj);
-        if (gj + 4 <= w) {
-          load4_any<T>(q, v[it]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 3; ++e)
-            if (gj + e < w) v[it][e] = to_f32<T>(q[e]);
-        }
-      }
-      col += DC;
-      row += DR;
-      if (col >= W4) { col -= W4; ++row; }
-    }
-  }
-#pragma unroll
-  for (int it = 0; it < IT; ++it) {
-    const int p = it * kStreamThreads + tid;
-    if (p < N) {
-      float4 t4;
-      t4.x = v[it][0]; t4.y = v[it][1]; t4.z = v[it][2]; t4.w = v[it][3];
-      reinterpret_cast<float4*>(dst)[p] = t4;
-    }
-  }
-}
-
-// Twelve / sixteen floats of an LDS row from a 16-byte aligned address.
-template <int N>
-__device__ __forceinline__ void lds_read(const float* __restrict__ p, float (&v)[N]) {
-#pragma unroll
-  for (int q = 0; q < N / 4; ++q) {
-    const float4 t4 = reinterpret_cast<const float4*>(p)[q];
-    v[4 * q] = t4.x; v[4 * q + 1] = t4.y; v[4 * q + 2] = t4.z; v[4 * q + 3] = t4.w;
-  }
-}
-
-// Tile shapes: TW x TH coefficients, four adjacent ones of a row a thread.  Tiles of 64 columns left a third of the
-// threads of an 80-column level (160-pixel planes) without work; the launch takes the shape that covers the level with
-// the fewest tiles.
-template <int TW_, int TH_>
-struct StreamShape {
-  static constexpr int TW = TW_, TH = TH_;
-  static_assert(TW / 4 * TH <= kStreamThreads, "one thread per four coefficients");
-};
-
-// Level-1 Haar bands S0..3 of a pixel tile in LDS: coefficient (rr, cc) of the AH x AWD tile comes from pixels
-// (2rr .. 2rr+1, 2cc .. 2cc+1) of the 2AH x 2AWD pixel tile.  Pixels outside the plane were staged as zeros, which is
-// both the zero padding of odd sizes and the zero halo of the sub-band convs (a coefficient outside the level has all
-// four pixels outside the plane).
-template <int AH, int AWD, int S0>
-__device__ __forceinline__ void haar_tile(const float* __restrict__ Xt, float* __restrict__ At, int tid) {
-  constexpr int XWD = 2 * AWD;
-  constexpr int PAIRS = AWD / 2;             // two coefficients (four pixels of each row) per step
-  for (int e = tid; e < AH * PAIRS; e += kStreamThreads) {
-    const int rr = e / PAIRS, cp = e - rr * PAIRS;
-    const float4 top = *reinterpret_cast<const float4*>(Xt + (2 * rr) * XWD + 4 * cp);
-    const float4 bot = *reinterpret_cast<const float4*>(Xt + (2 * rr + 1) * XWD + 4 * cp);
-    const float a[2] = {top.x, top.z}, b[2] = {top.y, top.w}, c[2] = {bot.x, bot.z}, d[2] = {bot.y, bot.w};
-    float o[4][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const float sac = a[t] + c[t], sbd = b[t] + d[t], dac = a[t] - c[t], dbd = b[t] - d[t];
-      o[0][t] = 0.5f * (sac + sbd);
-      o[1][t] = 0.5f * (dac + dbd);
-      o[2][t] = 0.5f * (sac - sbd);
-      o[3][t] = 0.5f * (dac - dbd);
-    }
-#pragma unroll
-    for (int s = S0; s < 4; ++s) {
-      float2 t2;
-      t2.x = o[s][0]; t2.y = o[s][1];
-      *reinterpret_cast<float2*>(At + ((s - S0) * AH + rr) * AWD + 2 * cp) = t2;
-    }
-  }
-}
-
 // ---- rows over the lanes of a wave ------------------------------------------------------------------------------------
 // A lane owns four pixels of a row (two coefficients) and walks down the plane; what it needs of its neighbours' rows comes
 // from their registers (wave_before, wave_behind), so there is no LDS, no barrier, and a wave only ever waits for its loads.
@@ -244,20 +146,6 @@ struct RowPair {
       w[row][0] = q.x; w[row][1] = q.y;
     }
   }
-  // (planes less than four pixels wide)
-  __device__ __forceinline__ void load_few(int row, const T* __restrict__ p, int n) {
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int e = 0; e < 3; ++e)
-      if (e < n) v[e] = to_f32<T>(p[e]);
-    if constexpr (N == 4) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) w[row][e] = __float_as_uint(v[e]);
-    } else {
-      w[row][0] = pack2<T>(v[0], v[1]);
-      w[row][1] = pack2<T>(v[2], v[3]);
-    }
-  }
   __device__ __forceinline__ void get(int row, float (&v)[4]) const {
     if constexpr (N == 4) {
 #pragma unroll
@@ -268,6 +156,60 @@ struct RowPair {
     }
   }
 };
+
+// A lane's rows 2 i and 2 i + 1 of a plane of H rows, from p on (`lanes`: whether it has any there).  The loads are the last
+// thing that happens to r until take_rows, whatever the width: a value that one of several paths may have written is moved
+// where they meet, and waited for there.  (A path of its own for narrow planes cost both kernels below each load's latency: 50
+// and 72 us, 44 and 63 without, at [8,96,160,160] fp32, K = 5.)
+// Rows of less than four pixels are read on into the next ones, the tensor's last up to three pixels early: `left` = rows from
+// the first one to the tensor's end.
+__device__ __forceinline__ int narrow_back(long long left, int width) {
+  return left * width < 4 ? 4 - static_cast<int>(left) * width : 0;
+}
+template <typename T>
+__device__ __forceinline__ void fetch_rows(bool lanes, int i, int H, const T* __restrict__ p, int width, long long left,
+                                           RowPair<T>& r) {
+  const bool in = lanes && i >= 0;
+  int b0 = 0, b1 = 0;
+  if (width < 4) {
+    b0 = narrow_back(left, width);
+    b1 = narrow_back(left - 1, width);
+  }
+  if (in && 2 * i < H) r.load(0, p - b0);
+  if (in && 2 * i + 1 < H) r.load(1, p + (width - b1));
+}
+// The values, zero outside the plane; lanes that never load hold the zeros that they start with.
+template <typename T>
+__device__ __forceinline__ void take_rows(const RowPair<T>& r, bool lanes, int i, int H, int c0, int width, long long left,
+                                          float (&a)[4], float (&c)[4]) {
+  r.get(0, a);
+  r.get(1, c);
+  if (width >= 4) {
+    piece_shift(a, c0, width);
+    piece_shift(c, c0, width);
+  } else {
+    const int b0 = narrow_back(left, width), b1 = narrow_back(left - 1, width);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float va = 0.f, vc = 0.f;
+#pragma unroll
+      for (int d = 0; e + d < 4; ++d) {
+        if (d == b0) va = a[e + d];
+        if (d == b1) vc = c[e + d];
+      }
+      a[e] = e < width ? va : 0.f;
+      c[e] = e < width ? vc : 0.f;
+    }
+  }
+  const bool top = i >= 0 && 2 * i < H, bottom = i >= 0 && 2 * i + 1 < H;
+  if (WT_ANY_LANE(lanes && !bottom)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a[e] = top ? a[e] : 0.f;
+      c[e] = bottom ? c[e] : 0.f;
+    }
+  }
+}
 
 // This lane's unit and place in it.
 struct LaneUnit {
@@ -308,8 +250,8 @@ __device__ __forceinline__ LaneUnit lane_unit(const LaneSplit& sp, int u0, int l
 // without their factor 1/2 (a power of two, made up for at the inverse).
 // fw[c * fstride]: the channel's folded filters; `fbase` / `fband` = offsets of the base filter and of the four sub-band
 // filters, in SGPRs a filter at a time.  fb == nullptr: no bias.
-// A row of coefficients at K = 5 is 350 multiply-adds of about 450 vector instructions, and [8,96,160,160] fp32 52 us (47 from
-// the caches), where the memory that it moves takes 35; tiles in LDS with a thread for four coefficients took 68.
+// A row of coefficients at K = 5 is 350 multiply-adds of about 450 vector instructions, and [8,96,160,160] fp32 44 us, where
+// the memory that it moves takes 35; tiles in LDS with a thread for four coefficients took 68.
 // grid = 1-D, a multiple of eight, at least C * sp.blocks; block = 256 (waves on their own).
 template <typename T, int K, bool CARRY>
 __global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_kernel(
@@ -342,18 +284,9 @@ __global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_k
 #pragma unroll
     for (int k = 0; k < K; ++k) Y[s][k][0] = Y[s][k][1] = 0.f;
 
-  // (lanes without pixels keep the zeros that they start with)
+  const long long rows_end = W < 4 ? static_cast<long long>(sp.units / (sp.tiles * sp.segs)) * C * H : 0;
   auto fetch = [&](int t, int width, RowPair<T>& r) __attribute__((always_inline)) {
-    const int i = i0 - R + t;
-    const bool top = have && i >= 0 && 2 * i < H, bottom = have && i >= 0 && 2 * i + 1 < H;
-    if (WT_ANY_LANE(have && !bottom)) r.clear();
-    if (width >= 4) {
-      if (top) r.load(0, px);
-      if (bottom) r.load(1, px + width);
-    } else {
-      if (top) r.load_few(0, px, width - c0);
-      if (bottom) r.load_few(1, px + width, width - c0);
-    }
+    fetch_rows<T>(have, i0 - R + t, H, px, width, rows_end - row0 + 2 * (R - t), r);
     px += 2 * width;
   };
   // Row t of the stretch: it adds to rows KLO .. KHI - 1 of the K around it.
@@ -366,12 +299,7 @@ __global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_k
     WT_LAUNDER_LANE_INT(at_c);
     WT_LAUNDER_UNIFORM(width);
     float a[4], c[4], z[2] = {0.f, 0.f};
-    now.get(0, a);
-    now.get(1, c);
-    if (width >= 4) {
-      piece_shift(a, at_c, width);
-      piece_shift(c, at_c, width);
-    }
+    take_rows<T>(now, have, i0 - R + t, H, at_c, width, rows_end - row0 + 2 * (R - t), a, c);
     if (t + 1 < steps) fetch(t + 1, width, next);
     if constexpr (ENDS && CARRY) {
       if (o < i1) {
@@ -526,81 +454,128 @@ struct StreamCorrOut {
 
 // One step of the parameter gradients: correlation sums of x with grad_out (BASE) and of their level-1 detail bands
 // (BANDS), dWt[kh][kw] = sum_{b,i,j} G[i][j] * X[i+kh-R][j+kw-R], and the LL bands of both for the sub-layer (where
-// xll / gll are given; BASE only).  A workgroup takes a contiguous range of the (batch item, tile) units of a channel;
-// a thread owns four coefficients (2 x 8 pixels of grad_out, in registers) and keeps the sums of all four filters, so
-// that x and grad_out are read once.  K = 7 has too many sums for that (196): two launches.
-// [8,96,160,160] fp32, K = 5: 82 us; a workgroup per filter over bands from memory took 43 + 65 for the same filters,
-// after 26 us for writing the bands.
-// grid = (C, nchunk), block = 256.
-template <typename T, int K, typename Shape, bool BASE, bool BANDS>
-__global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_corr_kernel(const T* __restrict__ x,
-                                                                        const T* __restrict__ g,
-                                                                        float* __restrict__ xll,
-                                                                        float* __restrict__ gll, int H, int W, int hl,
-                                                                        int wl, int B, int C, StreamCorrOut outp) {
-  constexpr int R = K / 2, KK = K * K;
-  constexpr int TH = Shape::TH, TW = Shape::TW, HP = kStreamPad, TJ = 4, NT = TW / TJ;
-  constexpr int AH = TH + 2 * R, AWD = TW + 2 * HP;
-  constexpr int XH = 2 * AH, XWD = 2 * AWD;
-  constexpr int NS = (BASE ? 1 : 0) + (BANDS ? 3 : 0);
-  __shared__ alignas(16) float At[BANDS ? 3 * AH * AWD : 4];
-  __shared__ alignas(16) float Xt[XH * XWD];
-  __shared__ float red[4][NS * KK + 1];
-  const int cc = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
-  const int r = tid / NT, c0 = (tid - r * NT) * TJ;
-  const int tiles_x = (wl + TW - 1) / TW, tiles = tiles_x * ((hl + TH - 1) / TH);
-  const int units = B * tiles;
-  const int per = (units + static_cast<int>(gridDim.y) - 1) / static_cast<int>(gridDim.y);
-  const int u_begin = chunk * per;
-  const int u_end = u_begin + per < units ? u_begin + per : units;
-  const size_t psz = static_cast<size_t>(H) * W, lsz = static_cast<size_t>(hl) * wl;
-  float acc[NS][KK];
-  float gsum = 0.f;
+// xll / gll are given; BASE only).  Rows over the lanes of a wave, as above: a lane walks down its rows of grad_out, keeps the
+// rows of x and of its bands around them in registers (a ring, whose place follows from the row: the loop is unrolled over a
+// round of it) and the sums of all four filters, so that x and grad_out are read once and every multiply-add is one of the
+// sums'.  K = 7 has too many sums for that (196): two launches.
+// A wave takes every `waves`-th group of `per` units of its channel, an even number apart: a lane beside its unit's own ones
+// is beside them in all its groups, and its sums (an infinity of x times the zero of no grad_out) are left out at the end.
+// Coefficients are sums and differences without their factor 1/2, products take the 1/4 at the end.
+// A row at K = 5 is 350 multiply-adds, 84 moves from the neighbours and some 90 others, and two waves fit a SIMD (229
+// registers).  [8,96,160,160] fp32: 63 us, of which the issue of its instructions is 43; tiles in LDS with a thread for four
+// coefficients took 81, two thirds of it LDS reads and their bank conflicts.
+// grid = (C, nchunk), block = 256 (waves on their own until their sums meet).
+template <typename T, int K, bool BASE, bool BANDS>
+__global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T* __restrict__ x, const T* __restrict__ g,
+                                                                        float* __restrict__ xll, float* __restrict__ gll,
+                                                                        int H, int W, int hl, int wl, int C,
+                                                                        StreamCorrOut outp, LaneSplit sp) {
+  constexpr int R = K / 2, KK = K * K, HP = (R + 1) / 2;
+  constexpr int LEAD = BANDS ? R : HP, P = 2 * LEAD + 1;      // rows of x ahead of grad_out's; rows of the ring
+  constexpr int NS = (BASE ? 1 : 0) + (BANDS ? 3 : 0), A0 = BASE ? 1 : 0;
+  constexpr int NR = (NS * KK + 4) / 4 * 4;                    // the sums and grad_out's own, in fours
+  __shared__ float red[kStreamThreads / kWave][NR];
+  const int ch = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = WT_UNIFORM(tid >> 6), waves = static_cast<int>(gridDim.y) * (kStreamThreads / kWave);
+  float acc[NS][KK], gsum = 0.f;
+  const long long rows_end = W < 4 ? static_cast<long long>(sp.units / (sp.tiles * sp.segs)) * C * H : 0;
+  bool keep = false;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
     for (int t = 0; t < KK; ++t) acc[s][t] = 0.f;
-  int b = u_begin / tiles, tile = u_begin - b * tiles;
-  for (int u = u_begin; u < u_end; ++u) {
-    const size_t plane = static_cast<size_t>(b) * C + cc;
-    const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
-    if (++tile == tiles) { tile = 0; ++b; }
-    const int i0 = ty * TH, j0 = tx * TW;
-    const int i = i0 + r, j = j0 + c0;
-    const bool own = r < TH && i < hl && j < wl;
-    float gv[2][2 * TJ];
+
+  for (int u0 = (chunk * (kStreamThreads / kWave) + wave) * sp.per; u0 < sp.units; u0 += waves * sp.per) {
+    const LaneUnit un = lane_unit<lane_halo(K)>(sp, u0, lane, wl);
+    const bool have = un.have, owns = un.owns;
+    keep = keep || owns;
+    const int i0 = un.seg * sp.rows, i1 = owns ? min(i0 + sp.rows, hl) : i0, c0 = 2 * un.j;
+    const long long plane = static_cast<long long>(un.b) * C + ch;
+    const int cl = W >= 4 ? piece_start(c0, W) : c0;
+    const T* px = x + (plane * H + 2 * (i0 - LEAD)) * W + cl;
+    const T* pg = g + (plane * H + 2 * i0) * W + cl;
+    long long pl = (plane * hl + i0) * wl + un.j;
+    float X[BASE ? P : 1][2][4], Z[BANDS ? P : 1][3][2];
+    RowPair<T> rx, rg;
+    rx.clear();
+    rg.clear();
+    // (row i of the coefficients')
+    auto left = [&](int i) __attribute__((always_inline)) { return rows_end - (plane * H + 2 * i); };
+    auto detail = [](const float (&a)[4], const float (&c)[4], float (&z)[3][2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int dr = 0; dr < 2; ++dr)
-      load8_row<T>(g + plane * psz + static_cast<size_t>(2 * i + dr) * W + 2 * j,
-                   own && 2 * i + dr < H ? W - 2 * j : 0, gv[dr]);
-    stage_window<T, XH, XWD>(x + plane * psz, H, W, 2 * (i0 - R), 2 * (j0 - HP), Xt, tid);
-    __syncthreads();
-    if constexpr (BANDS) {
-      haar_tile<AH, AWD, 1>(Xt, At, tid);
-      __syncthreads();
-    }
-    if (own) {
+      for (int e = 0; e < 2; ++e) {
+        const float sac = a[2 * e] + c[2 * e], sbd = a[2 * e + 1] + c[2 * e + 1];
+        const float dac = a[2 * e] - c[2 * e], dbd = a[2 * e + 1] - c[2 * e + 1];
+        z[0][e] = dac + dbd;
+        z[1][e] = sac - sbd;
+        z[2][e] = dac - dbd;
+      }
+    };
+    auto put = [&](auto slot, int i, int width, const RowPair<T>& r) __attribute__((always_inline)) {      // row i of x, which has come
+      constexpr int S = decltype(slot)::value;
+      float a[4], c[4];
+      take_rows<T>(r, have, i, H, c0, width, left(i), a, c);
       if constexpr (BASE) {
 #pragma unroll
-        for (int e = 0; e < 2 * TJ; ++e) gsum += gv[0][e] + gv[1][e];
-        if (gll != nullptr) {
-          float ll[TJ];
-#pragma unroll
-          for (int t = 0; t < TJ; ++t) ll[t] = 0.5f * ((gv[0][2 * t] + gv[1][2 * t]) + (gv[0][2 * t + 1] + gv[1][2 * t + 1]));
-          store4_row(gll + plane * lsz + static_cast<size_t>(i) * wl + j, wl - j, ll);
+        for (int e = 0; e < 4; ++e) {
+          X[S][0][e] = a[e];
+          X[S][1][e] = c[e];
         }
-        if (xll != nullptr) {
-          float a[8], c[8], ll[TJ];
-          lds_read<8>(Xt + (2 * (r + R)) * XWD + 2 * (c0 + HP), a);
-          lds_read<8>(Xt + (2 * (r + R) + 1) * XWD + 2 * (c0 + HP), c);
+      }
+      if constexpr (BANDS) detail(a, c, Z[S]);
+    };
+    // Row t of the stretch, t % P == PH: rows t .. t + P - 1 of x from the stretch's first one are in places PH, PH + 1, ...
+    auto step = [&](auto phase, int t) __attribute__((always_inline)) {
+      constexpr int PH = decltype(phase)::value;
+      const int o = i0 + t;
+      int width = W;
+      WT_LAUNDER_UNIFORM(width);
+      put(std::integral_constant<int, (PH + P - 1) % P>{}, o + LEAD, width, rx);
+      float gv[2][4];
+      take_rows<T>(rg, owns, o < i1 ? o : hl, H, c0, width, left(o), gv[0], gv[1]);
+      px += 2 * width;
+      pg += 2 * width;
+      if (t + 1 < sp.rows) {
+        fetch_rows<T>(have, o + LEAD + 1, H, px, width, left(o + LEAD + 1), rx);
+        fetch_rows<T>(owns && o + 1 < i1, o + 1, H, pg, width, left(o + 1), rg);
+      }
+      if (WT_ANY_LANE(have && o >= hl)) {      // (no row of grad_out meets the rows of x that are left)
+        const bool past = o >= hl;
 #pragma unroll
-          for (int t = 0; t < TJ; ++t) ll[t] = 0.5f * ((a[2 * t] + c[2 * t]) + (a[2 * t + 1] + c[2 * t + 1]));
-          store4_row(xll + plane * lsz + static_cast<size_t>(i) * wl + j, wl - j, ll);
+        for (int k = 0; k < P; ++k) {
+          if constexpr (BASE) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              X[k][0][e] = past ? 0.f : X[k][0][e];
+              X[k][1][e] = past ? 0.f : X[k][1][e];
+            }
+          }
+          if constexpr (BANDS) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+              Z[k][s][0] = past ? 0.f : Z[k][s][0];
+              Z[k][s][1] = past ? 0.f : Z[k][s][1];
+            }
+          }
         }
+      }
+      if constexpr (BASE) {
 #pragma unroll
-        for (int xr = 0; xr < K + 1; ++xr) {
-          float v[16];
-          lds_read<16>(Xt + (2 * r + xr + R) * XWD + 2 * c0 + HP, v);
+        for (int e = 0; e < 4; ++e) gsum += gv[0][e] + gv[1][e];
+        auto ll = [&](float* __restrict__ dst, const float (&a)[4], const float (&c)[4]) __attribute__((always_inline)) {
+          const float v0 = 0.5f * ((a[0] + c[0]) + (a[1] + c[1])), v1 = 0.5f * ((a[2] + c[2]) + (a[3] + c[3]));
+          if (un.j + 1 < wl) store_u2<2>(dst + pl, uint2{__float_as_uint(v0), __float_as_uint(v1)});
+          else dst[pl] = v0;
+        };
+        if (xll != nullptr && o < i1) ll(xll, X[(PH + LEAD) % P][0], X[(PH + LEAD) % P][1]);
+        if (gll != nullptr && o < i1) ll(gll, gv[0], gv[1]);
+        pl += wl;
+        WT_SCHED_FENCE();
+#pragma unroll
+        for (int xr = 0; xr < K + 1; ++xr) {      // row 2 o + xr - R of pixels
+          const int q = xr - R + 2 * HP;          // (from the first of the ring's middle 2 HP + 1 pairs)
+          float v[4 + 2 * R];
+          widen<4, R>(X[(PH + LEAD - HP + q / 2) % P][q & 1], v);
 #pragma unroll
           for (int dr = 0; dr < 2; ++dr) {
             const int kh = xr - dr;
@@ -608,65 +583,79 @@ __global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_corr_ke
 #pragma unroll
             for (int kw = 0; kw < K; ++kw)
 #pragma unroll
-              for (int e = 0; e < 2 * TJ; ++e)
-                acc[0][kh * K + kw] = fmaf(gv[dr][e], v[e + kw - R + HP], acc[0][kh * K + kw]);
+              for (int e = 0; e < 4; ++e) acc[0][kh * K + kw] = fmaf(v[e + kw], gv[dr][e], acc[0][kh * K + kw]);
           }
           if (xr & 1) {
             pin_values(acc[0]);
-            WT_CHUNK_FENCE();
+            WT_SCHED_FENCE();
           }
         }
       }
       if constexpr (BANDS) {
+        float gz[3][2];
+        detail(gv[0], gv[1], gz);
 #pragma unroll
-        for (int s = 1; s < 4; ++s) {
-          constexpr int A0 = BASE ? 0 : -1;
-          float gb[TJ];
-#pragma unroll
-          for (int t = 0; t < TJ; ++t) {
-            const float sac = gv[0][2 * t] + gv[1][2 * t], sbd = gv[0][2 * t + 1] + gv[1][2 * t + 1];
-            const float dac = gv[0][2 * t] - gv[1][2 * t], dbd = gv[0][2 * t + 1] - gv[1][2 * t + 1];
-            gb[t] = 0.5f * (s == 1 ? dac + dbd : s == 2 ? sac - sbd : dac - dbd);
-          }
+        for (int s = 0; s < 3; ++s) {
 #pragma unroll
           for (int kh = 0; kh < K; ++kh) {
-            float v[12];
-            lds_read<12>(At + ((s - 1) * AH + r + kh) * AWD + c0, v);
+            float v[2 + 2 * R];
+            widen<2, R>(Z[(PH + kh) % P][s], v);
 #pragma unroll
             for (int kw = 0; kw < K; ++kw)
 #pragma unroll
-              for (int t = 0; t < TJ; ++t)
-                acc[A0 + s][kh * K + kw] = fmaf(gb[t], v[t + kw - R + HP], acc[A0 + s][kh * K + kw]);
+              for (int e = 0; e < 2; ++e) acc[A0 + s][kh * K + kw] = fmaf(v[e + kw], gz[s][e], acc[A0 + s][kh * K + kw]);
           }
           pin_values(acc[A0 + s]);
-          WT_CHUNK_FENCE();
+          WT_SCHED_FENCE();
         }
       }
+    };
+    // (all the rows before the first one at once)
+    auto fill = [&](auto... q) __attribute__((always_inline)) {
+      RowPair<T> r[sizeof...(q)];
+      (r[decltype(q)::value].clear(), ...);
+      (fetch_rows<T>(have, i0 - LEAD + decltype(q)::value, H, px + 2LL * decltype(q)::value * W, W,
+                     left(i0 - LEAD + decltype(q)::value), r[decltype(q)::value]), ...);
+      px += 2LL * LEAD * 2 * W;
+      fetch_rows<T>(have, i0 + LEAD, H, px, W, left(i0 + LEAD), rx);
+      fetch_rows<T>(owns, i0, H, pg, W, left(i0), rg);
+      (put(q, i0 - LEAD + decltype(q)::value, W, r[decltype(q)::value]), ...);
+    };
+    auto round = [&](int t, auto... ph) __attribute__((always_inline)) {
+      (void)(... && (t + decltype(ph)::value < sp.rows ? (step(ph, t + decltype(ph)::value), true) : false));
+    };
+#define WT_PH(n) std::integral_constant<int, (n)>{}
+    if constexpr (LEAD == 1) fill(WT_PH(0), WT_PH(1));
+    if constexpr (LEAD == 2) fill(WT_PH(0), WT_PH(1), WT_PH(2), WT_PH(3));
+    if constexpr (LEAD == 3) fill(WT_PH(0), WT_PH(1), WT_PH(2), WT_PH(3), WT_PH(4), WT_PH(5));
+    if constexpr (LEAD == 0) {
+      fetch_rows<T>(have, i0, H, px, W, left(i0), rx);
+      fetch_rows<T>(owns, i0, H, pg, W, left(i0), rg);
     }
-    __syncthreads();
+    for (int t = 0; t < sp.rows; t += P) {
+      if constexpr (P == 1) round(t, WT_PH(0));
+      if constexpr (P == 3) round(t, WT_PH(0), WT_PH(1), WT_PH(2));
+      if constexpr (P == 5) round(t, WT_PH(0), WT_PH(1), WT_PH(2), WT_PH(3), WT_PH(4));
+      if constexpr (P == 7) round(t, WT_PH(0), WT_PH(1), WT_PH(2), WT_PH(3), WT_PH(4), WT_PH(5), WT_PH(6));
+    }
+#undef WT_PH
   }
-  const int wave = tid >> 6, lane = tid & (kWave - 1);
-#pragma unroll
-  for (int s = 0; s < NS; ++s)
-#pragma unroll
-    for (int t = 0; t < KK; ++t) {
-      const float v = wave_sum(acc[s][t]);
-      if (lane == 0) red[wave][s * KK + t] = v;
-    }
   {
-    const float v = wave_sum(gsum);
-    if (lane == 0) red[wave][NS * KK] = v;
+    float sums[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) sums[i] = !keep ? 0.f : i < NS * KK ? acc[i < NS * KK ? i / KK : 0][i % KK] : i == NS * KK ? gsum : 0.f;
+    wave_sums<NR>(sums, lane, red[wave]);
   }
   __syncthreads();
-  float* dst = outp.partial + (static_cast<size_t>(chunk) * C + cc) * outp.rec;
+  float* dst = outp.partial + (static_cast<size_t>(chunk) * C + ch) * outp.rec;
   for (int o = tid; o <= NS * KK; o += kStreamThreads) {
     const float v = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
     const int s = o / KK, t = o - s * KK;
     if (s == NS) {
       if (BASE && outp.with_gsum) dst[outp.rec - 1] = v;
     } else {
-      const int f = BASE && s == 0 ? outp.fbase : outp.fband + s - (BASE ? 1 : 0);
-      dst[f * KK + t] = v;
+      const int f = s < A0 ? outp.fbase : outp.fband + s - A0;
+      dst[f * KK + t] = s < A0 ? v : 0.25f * v;
     }
   }
 }

@@ -5,25 +5,9 @@
 
 namespace wt {
 
-// The tile shape that covers a level of hl x wl coefficients with the fewest tiles (a tile costs about the same time
-// whatever its shape, most of its threads being at work).
-template <typename F>
-static int by_stream_shape(int hl, int wl, F&& launch) {
-  auto tiles = [&](int tw, int th) {
-    return static_cast<long long>((wl + tw - 1) / tw) * ((hl + th - 1) / th);
-  };
-  const long long n64 = tiles(64, 16), n80 = tiles(80, 12), n48 = tiles(48, 20);
-  if (n64 <= n80 && n64 <= n48) return launch(StreamShape<64, 16>{}, n64);
-  return n80 <= n48 ? launch(StreamShape<80, 12>{}, n80) : launch(StreamShape<48, 20>{}, n48);
-}
-
-// How a level of hl x wl coefficients goes over the lanes: the tiles that take the fewest waves, and the stretches of rows of
-// least time, in rows of a wave: 2 R more rows count for half of them, 1.2 go to the start; a SIMD takes up to three waves side
-// by side (fewer than 1.6 leave it waiting), and where they make more than a round the last one is a third empty.
-// [8,96,160,160] fp32, K = 5, us by rows of a stretch: 20 59, 16 51, 14 47, 12 53, 10 53, 9 50, 8 52, 7 49, 5 51.
-static LaneSplit lane_split(int B, int C, int hl, int wl, int K) {
-  constexpr int kSimds = 1024;      // 256 compute units
-  const int R = K / 2, HL = lane_halo(K), lanes = (wl + 1) / 2, least = HL > 0 ? 2 * HL : 1;
+// How a level of hl x wl coefficients goes over the lanes: the tiles that take the fewest waves.
+static LaneSplit lane_tiles(int wl, int K) {
+  const int HL = lane_halo(K), lanes = (wl + 1) / 2, least = HL > 0 ? 2 * HL : 1;
   LaneSplit best = {};
   double waves = 0.;
   for (int n = (lanes + kWave - 1) / kWave; n <= (lanes + 7) / 8 || best.per == 0; ++n) {
@@ -40,6 +24,17 @@ static LaneSplit lane_split(int B, int C, int hl, int wl, int K) {
     const double w = static_cast<double>(s.tiles) / s.per;
     if (best.per == 0 || w < waves) { best = s; waves = w; }
   }
+  return best;
+}
+
+// The layer's step: stretches of rows of least time, in rows of a wave: 2 R more rows count for half of them, 1.2 go to the
+// start; a SIMD takes up to three waves side by side (fewer than 1.6 leave it waiting), and where they make more than a round
+// the last one is a third empty.
+// [8,96,160,160] fp32, K = 5, us by rows of a stretch: 20 59, 16 51, 14 47, 12 53, 10 53, 9 50, 8 52, 7 49, 5 51.
+static LaneSplit lane_split(int B, int C, int hl, int wl, int K) {
+  constexpr int kSimds = 1024;      // 256 compute units
+  const int R = K / 2;
+  LaneSplit best = lane_tiles(wl, K);
   double least_time = 0.;
   for (int n = 1; n <= hl; ++n) {
     const int rows = (hl + n - 1) / n < 2 * R ? 2 * R : (hl + n - 1) / n;
@@ -60,6 +55,27 @@ static LaneSplit lane_split(int B, int C, int hl, int wl, int K) {
   }
   constexpr int kWavesPerBlock = kStreamThreads / kWave;
   best.blocks = (best.units + kWavesPerBlock * best.per - 1) / (kWavesPerBlock * best.per);
+  return best;
+}
+
+// The correlations' step, whose nchunk workgroups a channel run side by side: the stretches whose shares of the waves are
+// shortest, in rows; the 2 R rows of x before a stretch's first are loaded and transformed only and count for two.
+static LaneSplit corr_split(int B, int hl, int wl, int K, int nchunk) {
+  LaneSplit best = lane_tiles(wl, K);
+  const long long waves = static_cast<long long>(nchunk) * (kStreamThreads / kWave);
+  long long least = 0;
+  for (int n = 1; n <= hl; ++n) {
+    const int rows = (hl + n - 1) / n, segs = (hl + rows - 1) / rows;
+    const long long units = static_cast<long long>(B) * best.tiles * segs;
+    const long long groups = (units + best.per - 1) / best.per, time = (groups + waves - 1) / waves * (rows + 2);
+    if (n == 1 || time < least) {
+      least = time;
+      best.segs = segs;
+      best.rows = rows;
+      best.units = static_cast<int>(units);
+    }
+    if (rows <= 4) break;
+  }
   return best;
 }
 
@@ -96,28 +112,26 @@ static int run_stream_corr(const StreamStep& st, const void* x_, const void* g_,
   const T* x = static_cast<const T*>(x_);
   const T* g = static_cast<const T*>(g_);
   const int hl = (st.H + 1) / 2, wl = (st.W + 1) / 2;
-  return by_stream_shape(hl, wl, [&](auto shape, long long) {
-    using Sh = decltype(shape);
-    const dim3 grid(st.C, nchunk);
-    if constexpr (K <= 5) {
-      if (bands) {
-        WT_LAUNCH((stream_corr_kernel<T, K, Sh, true, true>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H,
-                  st.W, hl, wl, st.B, st.C, outp);
-        return check_launch("stream_corr_kernel");
-      }
+  const dim3 grid(st.C, nchunk);
+  const LaneSplit sp = corr_split(st.B, hl, wl, K, nchunk);
+  if constexpr (K <= 5) {
+    if (bands) {
+      WT_LAUNCH((stream_corr_kernel<T, K, true, true>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H, st.W, hl,
+                wl, st.C, outp, sp);
+      return check_launch("stream_corr_kernel");
     }
-    WT_LAUNCH((stream_corr_kernel<T, K, Sh, true, false>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H,
-              st.W, hl, wl, st.B, st.C, outp);
-    if (int e = check_launch("stream_corr_kernel")) return e;
-    if constexpr (K > 5) {
-      if (bands) {
-        WT_LAUNCH((stream_corr_kernel<T, K, Sh, false, true>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H,
-                  st.W, hl, wl, st.B, st.C, outp);
-        return check_launch("stream_corr_kernel");
-      }
+  }
+  WT_LAUNCH((stream_corr_kernel<T, K, true, false>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H, st.W, hl, wl,
+            st.C, outp, sp);
+  if (int e = check_launch("stream_corr_kernel")) return e;
+  if constexpr (K > 5) {
+    if (bands) {
+      WT_LAUNCH((stream_corr_kernel<T, K, false, true>), grid, dim3(kStreamThreads), 0, stream, x, g, xll, gll, st.H, st.W, hl,
+                wl, st.C, outp, sp);
+      return check_launch("stream_corr_kernel");
     }
-    return 0;
-  });
+  }
+  return 0;
 }
 
 #define WT_BY_K(K, CALL)                                                              \
