@@ -493,8 +493,7 @@ __device__ __forceinline__ float row_sum(float v) {
 }
 
 // Sum over the 64 lanes of a wavefront; every lane gets the total.  On the GPU: six DPP adds
-// (quad permutes, row mirrors, row broadcasts) and one v_readlane, no LDS traffic -- the
-// weight-gradient kernels reduce up to 76 running sums per workgroup this way.
+// (quad permutes, row mirrors, row broadcasts) and one v_readlane, no LDS traffic.
 __device__ __forceinline__ float wave_sum(float v) {
 #ifdef WT_EMULATE
 #pragma unroll
@@ -516,14 +515,17 @@ __device__ __forceinline__ float wave_sum(float v) {
 #endif
 }
 
-// dst[i] = the sum of v[i] over the wavefront, from one lane of each 16 (v is used up; dst: LDS).  Halves, then quarters of
+// dst[i] = the sum of v[i] over the wavefront, i < M, from one lane of each 16 (v is used up; dst: LDS).  Halves, then quarters of
 // the wave swap values so that one add serves two of them, and a quarter's sums end in its own lanes: 3 instructions a value
 // that wait for nothing, against 18 with wave_sum, most of them waits of its six dependent adds.
-template <int N>
+// The gradient kernels' 50 to 101 sums a wave, us a launch with wave_sum and with this: 2-D [128,96,56,56] fp32 170 and 158,
+// [8,96,80,80] fp32 48.7 and 43.8, [16,72,45,37] fp16 K = 7 40.3 and 34.5; 1-D [64,64,4096] fp32 54.0 and 50.8 (the whole
+// backward pass), [8,48,20011] bf16 K = 7 28.0 and 23.9.
+template <int N, int M = N>
 __device__ __forceinline__ void wave_sums(float (&v)[N], int lane, float* __restrict__ dst) {
-  static_assert(N % 4 == 0, "four values at a time");
+  static_assert(N % 4 == 0 && M <= N, "four values at a time");
 #ifdef WT_EMULATE
-  for (int i = 0; i < N; ++i) {
+  for (int i = 0; i < M; ++i) {
     const float t = wave_sum(v[i]);
     if (lane == 0) dst[i] = t;
   }
@@ -545,7 +547,8 @@ __device__ __forceinline__ void wave_sums(float (&v)[N], int lane, float* __rest
   for (int i = 0; i < N; i += 4) v[i] = row_sum(v[i]);
   if ((lane & 15) == 0) {
 #pragma unroll
-    for (int i = 0; i < N; i += 4) dst[i + of_row] = v[i];
+    for (int i = 0; i < N; i += 4)
+      if (i + 4 <= M || i + of_row < M) dst[i + of_row] = v[i];
   }
 #endif
 }

@@ -539,18 +539,15 @@ __device__ __forceinline__ void row1d_store_partial(const float (&acc)[NF][K], f
                                                     float* __restrict__ red, float* __restrict__ dst, int tid, int nth) {
   constexpr int NRED = NF * K + 1;
   const int wave = tid >> 6, lane = tid & (kWave - 1);
+  float sums[(NRED + 3) / 4 * 4] = {};
 #pragma unroll
   for (int f = 0; f < NF; ++f)
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
+    for (int k = 0; k < K; ++k)
       // the sums of level l were formed from coefficients 2^(l/2) times the orthonormal ones on either side
-      const float v = wave_sum(own ? acc[f][k] : 0.f) * (f == 0 ? 1.f : 1.f / static_cast<float>(2 << ((f - 1) / 2)));
-      if (lane == 0) red[wave * NRED + f * K + k] = v;
-    }
-  {
-    const float v = wave_sum(own ? gsum : 0.f);
-    if (lane == 0) red[wave * NRED + NRED - 1] = v;
-  }
+      sums[f * K + k] = (own ? acc[f][k] : 0.f) * (f == 0 ? 1.f : 1.f / static_cast<float>(2 << ((f - 1) / 2)));
+  sums[NRED - 1] = own ? gsum : 0.f;
+  wave_sums<(NRED + 3) / 4 * 4, NRED>(sums, lane, red + wave * NRED);
   WT_LDS_BARRIER();
   const int nwaves = nth >> 6;
   for (int o = tid; o < NRED; o += nth) {

@@ -1147,16 +1147,14 @@ __global__ __launch_bounds__(512, K <= 5 ? 4 : 2) void wt2d_wgrad_kernel(const T
   // cross-lane reduction, then cross-wave through LDS (pyramid buffers are dead now)
   constexpr int NRED = NSET * KK + 1;
   float* red = lds;   // [8 waves][NRED]
-#pragma unroll
-  for (int s = 0; s < NSET; ++s)
-#pragma unroll
-    for (int t = 0; t < KK; ++t) {
-      const float v = wave_sum(acc[s][t]);
-      if (first_lane == 0) red[wave * NRED + s * KK + t] = v;
-    }
   {
-    const float v = wave_sum(gsum) * static_cast<float>(1 << L);
-    if (first_lane == 0) red[wave * NRED + NRED - 1] = v;
+    float sums[(NRED + 3) / 4 * 4] = {};
+#pragma unroll
+    for (int s = 0; s < NSET; ++s)
+#pragma unroll
+      for (int t = 0; t < KK; ++t) sums[s * KK + t] = acc[s][t];
+    sums[NRED - 1] = gsum * static_cast<float>(1 << L);
+    wave_sums<(NRED + 3) / 4 * 4, NRED>(sums, first_lane, red + wave * NRED);
   }
   WT_LDS_BARRIER();
   float* dst = partial + (static_cast<size_t>(chunk) * nC + c) * (NF * KK + 1);

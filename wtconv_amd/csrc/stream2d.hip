@@ -30,7 +30,8 @@ static LaneSplit lane_tiles(int wl, int K) {
 // The layer's step: stretches of rows of least time, in rows of a wave: 2 R more rows count for half of them, 1.2 go to the
 // start; a SIMD takes up to three waves side by side (fewer than 1.6 leave it waiting), and where they make more than a round
 // the last one is a third empty.
-// [8,96,160,160] fp32, K = 5, us by rows of a stretch: 20 59, 16 51, 14 47, 12 53, 10 53, 9 50, 8 52, 7 49, 5 51.
+// [8,96,160,160] fp32, K = 5, us by rows of a stretch: 20 59, 16 51, 14 47, 12 53, 10 53, 9 50, 8 52, 7 49, 5 51 (while each
+// row's loads were still waited for at once; 14, which it takes, is 44 since).
 static LaneSplit lane_split(int B, int C, int hl, int wl, int K) {
   constexpr int kSimds = 1024;      // 256 compute units
   const int R = K / 2;
