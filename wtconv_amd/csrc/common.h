@@ -31,6 +31,7 @@
 #define WT_LAUNDER_LANE_INT(v) do {} while (0)
 #define WT_WAVE_PRIORITY(n) do {} while (0)
 #define WT_ANY_LANE(p) (p)
+#define WT_INLINE_LAMBDA
 typedef const float* wt_uniform_ptr;
 #else
 // Folded weights are read-only for the whole launch and indexed uniformly: the constant
@@ -88,6 +89,8 @@ typedef const float __attribute__((address_space(4)))* wt_uniform_ptr;
 #define WT_WAVE_PRIORITY(n) __builtin_amdgcn_s_setprio(n)
 // Whether a predicate holds in any lane of the wave, as a wave-uniform condition (the host emulation: this lane's own).
 #define WT_ANY_LANE(p) __any(p)
+// A lambda that keeps its captures in registers.
+#define WT_INLINE_LAMBDA __attribute__((always_inline))
 #endif
 
 namespace wt {

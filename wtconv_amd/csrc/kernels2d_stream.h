@@ -285,12 +285,12 @@ __global__ __launch_bounds__(kStreamThreads, K <= 5 ? 3 : 2) void stream_final_k
     for (int k = 0; k < K; ++k) Y[s][k][0] = Y[s][k][1] = 0.f;
 
   const long long rows_end = W < 4 ? static_cast<long long>(sp.units / (sp.tiles * sp.segs)) * C * H : 0;
-  auto fetch = [&](int t, int width, RowPair<T>& r) __attribute__((always_inline)) {
+  auto fetch = [&](int t, int width, RowPair<T>& r) WT_INLINE_LAMBDA {
     fetch_rows<T>(have, i0 - R + t, H, px, width, rows_end - row0 + 2 * (R - t), r);
     px += 2 * width;
   };
   // Row t of the stretch: it adds to rows KLO .. KHI - 1 of the K around it.
-  auto step = [&](auto klo, auto khi, auto ends, int t, const RowPair<T>& now, RowPair<T>& next) __attribute__((always_inline)) {
+  auto step = [&](auto klo, auto khi, auto ends, int t, const RowPair<T>& now, RowPair<T>& next) WT_INLINE_LAMBDA {
     constexpr int KLO = decltype(klo)::value, KHI = decltype(khi)::value;
     constexpr bool ENDS = decltype(ends)::value;      // (and a row of results ends with it)
     const int o = i0 + t - 2 * R;
@@ -500,8 +500,8 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
     rx.clear();
     rg.clear();
     // (row i of the coefficients')
-    auto left = [&](int i) __attribute__((always_inline)) { return rows_end - (plane * H + 2 * i); };
-    auto detail = [](const float (&a)[4], const float (&c)[4], float (&z)[3][2]) __attribute__((always_inline)) {
+    auto left = [&](int i) WT_INLINE_LAMBDA { return rows_end - (plane * H + 2 * i); };
+    auto detail = [](const float (&a)[4], const float (&c)[4], float (&z)[3][2]) WT_INLINE_LAMBDA {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const float sac = a[2 * e] + c[2 * e], sbd = a[2 * e + 1] + c[2 * e + 1];
@@ -511,7 +511,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
         z[2][e] = dac - dbd;
       }
     };
-    auto put = [&](auto slot, int i, int width, const RowPair<T>& r) __attribute__((always_inline)) {      // row i of x, which has come
+    auto put = [&](auto slot, int i, int width, const RowPair<T>& r) WT_INLINE_LAMBDA {      // row i of x, which has come
       constexpr int S = decltype(slot)::value;
       float a[4], c[4];
       take_rows<T>(r, have, i, H, c0, width, left(i), a, c);
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
       if constexpr (BANDS) detail(a, c, Z[S]);
     };
     // Row t of the stretch, t % P == PH: rows t .. t + P - 1 of x from the stretch's first one are in places PH, PH + 1, ...
-    auto step = [&](auto phase, int t) __attribute__((always_inline)) {
+    auto step = [&](auto phase, int t) WT_INLINE_LAMBDA {
       constexpr int PH = decltype(phase)::value;
       const int o = i0 + t;
       int width = W;
@@ -562,7 +562,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
       if constexpr (BASE) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) gsum += gv[0][e] + gv[1][e];
-        auto ll = [&](float* __restrict__ dst, const float (&a)[4], const float (&c)[4]) __attribute__((always_inline)) {
+        auto ll = [&](float* __restrict__ dst, const float (&a)[4], const float (&c)[4]) WT_INLINE_LAMBDA {
           const float v0 = 0.5f * ((a[0] + c[0]) + (a[1] + c[1])), v1 = 0.5f * ((a[2] + c[2]) + (a[3] + c[3]));
           if (un.j + 1 < wl) store_u2<2>(dst + pl, uint2{__float_as_uint(v0), __float_as_uint(v1)});
           else dst[pl] = v0;
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
       }
     };
     // (all the rows before the first one at once)
-    auto fill = [&](auto... q) __attribute__((always_inline)) {
+    auto fill = [&](auto... q) WT_INLINE_LAMBDA {
       RowPair<T> r[sizeof...(q)];
       (r[decltype(q)::value].clear(), ...);
       (fetch_rows<T>(have, i0 - LEAD + decltype(q)::value, H, px + 2LL * decltype(q)::value * W, W,
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void stream_corr_kernel(const T*
       fetch_rows<T>(owns, i0, H, pg, W, left(i0), rg);
       (put(q, i0 - LEAD + decltype(q)::value, W, r[decltype(q)::value]), ...);
     };
-    auto round = [&](int t, auto... ph) __attribute__((always_inline)) {
+    auto round = [&](int t, auto... ph) WT_INLINE_LAMBDA {
       (void)(... && (t + decltype(ph)::value < sp.rows ? (step(ph, t + decltype(ph)::value), true) : false));
     };
 #define WT_PH(n) std::integral_constant<int, (n)>{}
